@@ -34,7 +34,7 @@
 // lplb_plan_sync_timeouts has reported the failures and cleared the block.
 #include "map_kernel.h"
 #include "plan_sync.h"
-#include "solve_kernel.h"
+#include "solve_spread.h"
 #include <atomic>
 #include <mutex>
 #include <stdio.h>
@@ -47,9 +47,9 @@ namespace lplb {
 constexpr int kPreferredSlices = 250;
 constexpr int kPlanLdsLimit = 160 * 1024 - 8 * 1024;   // dynamic LDS; the kernel has static LDS besides
 // An LP workgroup's dynamic LDS starts with the areas its (up to four) LP waves work in, then
-// come the staged counts: per wave the pivot rows (2 * kWave doubles) and the assembly tile.
-constexpr size_t plan_lp_area_bytes(int gm) {
-  return 2 * kWave * sizeof(double) + (size_t)assembly_tile_floats_of(gm) * sizeof(float);
+// come the staged counts: per wave the pivot rows and the assembly tile.
+template <int GM, int DM> constexpr size_t plan_lp_area_bytes() {
+  return lp_pivot_doubles<GM, DM>() * sizeof(double) + lp_tile_floats<GM, DM>() * sizeof(float);
 }
 constexpr int kDefaultMaxPolls = 1 << 22;   // a few seconds of polling before a wait gives up
 // LPs per LP workgroup: waves 0..3 of a workgroup sit on the CU's four SIMDs, and an LP
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(WAVES *kWave, (GM * DM <= 16 && GM <= 8) ? 4 : 2) v
     // slices, fetches the totals the slices have added up in memory and hands them over.
     __shared__ int counts_ready;
     // dynamic LDS of an LP workgroup: [LP wave][pivot rows | assembly tile], then the counts
-    constexpr size_t kLpArea = plan_lp_area_bytes(GM);
+    constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
     static_assert(kLpArea % 16 == 0, "the LP waves' areas keep 16-byte alignment");
     unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
     float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
@@ -267,9 +267,9 @@ __global__ __launch_bounds__(WAVES *kWave, (GM * DM <= 16 && GM <= 8) ? 4 : 2) v
     if (wave_s < n_lps) {
       // (own-histogram mode: every LP of the batch reads the one staged copy)
       float *mine = a.local_counts ? staged : staged + (size_t)wave_s * sa.staged_stride;
-      const int n_ok = solve_lp<GM, DM, EXACT, 1>(sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave,
-                                                  reinterpret_cast<double *>(my_area),
-                                                  reinterpret_cast<float *>(my_area + 2 * kWave * sizeof(double)));
+      const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
+          sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave, reinterpret_cast<double *>(my_area),
+          reinterpret_cast<float *>(my_area + lp_pivot_doubles<GM, DM>() * sizeof(double)));
       if (n_ok < 0) {
         // no counts, no solution: tell the slices not to wait for this LP's shares.  (If it was this wave's
         // own wait that ran out and not the poller's, nobody has counted the failure yet.)
@@ -878,7 +878,7 @@ static int launch_plan_shape(PlanArgs &a, hipStream_t s, bool *done) {
   const size_t lds_slices = plan_lds_bytes(a.sh.n_logical, a.n_rep, W, k);
   // LP workgroups: their waves' working areas, then the counts (one copy per LP if they fit,
   // else none and the LPs read global memory; own-histogram mode needs one copy in any case)
-  const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes(GM);
+  const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
   const size_t one_copy = (size_t)a.solve.n_experts * sizeof(float);
   const size_t all_copies = (size_t)min(a.solve.n_units, kLpsPerWorkgroup) * one_copy;
   size_t lds = max(lds_slices, lp_areas + (a.local_counts ? one_copy : 0));

@@ -1,6 +1,6 @@
 // LP solver entry points: batches of LPs, one per wave or four per wave.
-// The device code and the description of the method are in solve_kernel.h.
-#include "solve_kernel.h"
+// The device code and the description of the method are in solve_kernel.h and solve_spread.h.
+#include "solve_spread.h"
 
 namespace lplb {
 
@@ -15,12 +15,12 @@ template <int GM, int DM, bool EXACT, int ROWS, int EPL>
 __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
   extern __shared__ float staged_all[];   // a.staged_stride floats per LP of this wave
   __shared__ int rep_of_edge[EPL * kWave];
-  __shared__ __attribute__((aligned(16))) double pivot_rows[2 * kWave];
-  __shared__ __attribute__((aligned(16))) float tile[assembly_tile_floats<GM, EPL>()];
+  __shared__ __attribute__((aligned(16))) double pivot_rows[lp_pivot_doubles<GM, DM, ROWS, EPL>()];
+  __shared__ __attribute__((aligned(16))) float tile[lp_tile_floats<GM, DM, ROWS, EPL>()];
   if (blockIdx.x == 0 && threadIdx.x == 0)
     atomicAdd(a.avail, a.n_units);
   const int first_unit = blockIdx.x * ROWS;
-  const int n_ok = solve_lp<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_all, rep_of_edge, pivot_rows, tile);
+  const int n_ok = solve_lps<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_all, rep_of_edge, pivot_rows, tile);
   const int n_mine = min(max(a.n_units - first_unit, 0), ROWS);
   if (threadIdx.x == 0 && n_ok < n_mine)
     atomicAdd(a.avail, n_ok - n_mine);
