@@ -366,6 +366,34 @@ int lplb_plan_noalloc(const int64_t *idx, int64_t n_elements,
                       lplb_stream_t stream);
 
 /*
+ * Expert placement, on the host (all pointers are host pointers; nothing is enqueued).
+ * lplb_balanced_packing, lplb_replicate_experts and lplb_rebalance_experts are the
+ * reference's embedded EPLB (lplb/eplb.py:6-46, 49-77, 80-148), one row of weights per
+ * layer; lplb_build_mapping is what Planner.update_redundancy_mapping makes of it
+ * (lplb/planner.py:115-182).
+ *
+ *   weight, history  the load per logical expert as fp32 (for the packing) and as fp64
+ *                    (for the order inside a rank), or both NULL: index order
+ *   r2o              int32 [group_size, dup_per_rank]
+ *   phy2log          int32 [n_physical], out (see lplb_solve)
+ *   log2phy          int32 [n_logical, 2], out: the original's and the replica's slot, -1: none
+ *   logcnt           int32 [n_logical], out: copies of each expert
+ *
+ * LPLB_EINVAL for sizes that do not divide and unless some expert has two copies and none more.
+ */
+int lplb_balanced_packing(const float *weight, int n_layers, int n_items, int n_packs,
+                          int64_t *pack_index, int64_t *rank_in_pack);
+int lplb_replicate_experts(const float *weight, int n_rows, int n_logical, int n_physical,
+                           int64_t *phy2log, int64_t *rank, int64_t *logcnt);
+int lplb_rebalance_experts(const float *weight, int n_layers, int n_logical, int n_physical,
+                           int n_groups, int n_nodes, int n_gpus, int64_t *phy2log,
+                           int64_t *phyrank, int64_t *logcnt);
+int lplb_build_mapping(const float *weight, const double *history, const int32_t *r2o,
+                       int group_size, int dup_per_rank, int ep_size, int n_logical,
+                       int n_physical, int n_nodes, int32_t *phy2log, int32_t *log2phy,
+                       int32_t *logcnt);
+
+/*
  * No counterpart in the reference.  enabled = 0 makes lplb_plan always run the
  * chain of kernels (for callers that replay captured plans concurrently on
  * several streams, that let four or more plans execute at once, or that keep the

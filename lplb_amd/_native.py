@@ -57,6 +57,10 @@ _SIGNATURES = {
     "lplb_plan_one_launch_count": (_i, [_vp]),
     "lplb_plan_inject_fault": (_i, [_i, _i]),
     "lplb_plan": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
+    "lplb_balanced_packing": (_i, [_vp, _i, _i, _i, _vp, _vp]),
+    "lplb_replicate_experts": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp]),
+    "lplb_rebalance_experts": (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
+    "lplb_build_mapping": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "lplb_plan_noalloc": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
 }
 
@@ -136,6 +140,12 @@ def _check(rc: int) -> None:
     if rc != 0:
         kind = UnsupportedShape if rc == 2 else RuntimeError
         raise kind(f"lplb_hip error {rc}: {load().lplb_last_error().decode()}")
+
+
+def check_host(rc: int) -> None:
+    """Result of the host-side placement functions, whose argument checks are assertions like the reference's."""
+    if rc != 0:
+        raise AssertionError(load().lplb_last_error().decode())
 
 
 def _require(cond: bool, what: str) -> None:

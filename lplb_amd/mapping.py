@@ -1,4 +1,4 @@
-"""Physical <-> logical expert layout of the planner (host side, numpy).
+"""Physical <-> logical expert layout of the planner (host side; the work is done by csrc/mapping.hip).
 
 Per EP rank the physical slots are laid out as
 
@@ -12,56 +12,35 @@ from __future__ import annotations
 
 import numpy as np
 
-from .eplb import rebalance_experts
+from . import _native
 
 
 def build_redundancy_mapping(r2o: np.ndarray, ep_size: int, n_logical: int, n_physical: int,
-                             workload: np.ndarray | None = None, n_nodes: int = 1):
+                             workload: np.ndarray | None = None, n_nodes: int = 1, out: np.ndarray | None = None):
     """Returns (phy2log int32 [n_physical], log2phy int32 [n_logical, 2], logcnt int32 [n_logical]).
 
     workload: optional per-logical-expert history.  When given, experts are first
     spread over ranks with EPLB (reorder only, no replication) and each rank's
     experts are sorted heaviest first, so the heaviest C*D of every rank get the
     replicas (lplb/planner.py:127-147).  Equal histories keep index order.
+    out: optional int32 [n_physical + 3 * n_logical] buffer, contiguous, that the three arrays become parts of.
     Raises AssertionError unless every logical expert ends up with at most one
     replica and at least one expert has one (lplb/planner.py:173).
     """
-    r2o = np.asarray(r2o, dtype=np.int64)
+    r2o = np.ascontiguousarray(r2o, dtype=np.int32)
     G, D = r2o.shape
-    n_group = ep_size // G
-    L = n_logical // ep_size
-    P = n_physical // ep_size
-    C = (P - L) // D
-
-    if workload is None:
-        nored = np.arange(n_logical, dtype=np.int64)
-    else:
+    weight = history = None
+    if workload is not None:
         workload = np.asarray(workload).reshape(-1)
         assert workload.size == n_logical
-        nored = rebalance_experts(workload[None].astype(np.float32), n_logical, n_group,
-                                  n_nodes, ep_size)[0][0]
-    nored = nored.reshape(n_group, G, L)
-    if workload is not None:
-        order = np.argsort(-workload[nored].astype(np.float64), axis=-1, kind="stable")
-        nored = np.take_along_axis(nored, order, axis=-1)
-
-    tored = nored[:, :, :C * D].reshape(n_group, G, C, D)
-    # replica (c, d) on rank i <- original (c, d) of rank r2o[i, d]
-    dup = tored[:, r2o, :, np.arange(D)[None, :]]          # [G, D, n_group, C]
-    dup = dup.transpose(2, 0, 3, 1)                        # [n_group, G, C, D]
-    phy2log = np.concatenate([nored, dup.reshape(n_group, G, C * D)], axis=-1).reshape(-1)
-    assert phy2log.shape[0] == n_physical, (phy2log.shape, n_physical)
-
-    # log2phy lists originals before replicas: walk physical ids by (local slot, rank).
-    by_slot = np.arange(n_physical).reshape(ep_size, P).T.reshape(-1)
-    logs = phy2log[by_slot]
-    order = np.argsort(logs, kind="stable")
-    logcnt = np.bincount(logs, minlength=n_logical)
-    max_cnt = int(logcnt.max())
-    assert max_cnt == 2, f"every logical expert may have at most one replica (got {max_cnt} copies)"
-    starts = np.cumsum(logcnt) - logcnt
-    sorted_logs = logs[order]
-    pos = np.arange(order.size) - starts[sorted_logs]
-    log2phy = np.full((n_logical, max_cnt), -1, dtype=np.int32)
-    log2phy[sorted_logs, pos] = by_slot[order]
-    return phy2log.astype(np.int32), log2phy, logcnt.astype(np.int32)
+        weight = np.ascontiguousarray(workload, dtype=np.float32)
+        history = np.ascontiguousarray(workload, dtype=np.float64)
+    if out is None:
+        out = np.empty(n_physical + 3 * n_logical, dtype=np.int32)
+    assert out.shape == (n_physical + 3 * n_logical,)
+    at = out.ctypes.data
+    _native.check_host(_native.load().lplb_build_mapping(
+        None if weight is None else weight.ctypes.data, None if history is None else history.ctypes.data, r2o.ctypes.data,
+        G, D, ep_size, n_logical, n_physical, n_nodes, at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical)))
+    return (out[:n_physical], out[n_physical:n_physical + 2 * n_logical].reshape(n_logical, 2),
+            out[n_physical + 2 * n_logical:])

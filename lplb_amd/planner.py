@@ -10,7 +10,6 @@ from __future__ import annotations
 import functools
 import warnings
 
-import numpy as np
 import torch
 
 from . import _native
@@ -117,12 +116,14 @@ class Planner:
         :return: ``(phy2log [n_routed], log2phy [n_logical, 2], logcnt [n_logical])``, int32.
         """
         host = None if workload is None else workload.detach().cpu().numpy()
-        phy2log, log2phy, logcnt = build_redundancy_mapping(
-            self._r2o_host, self.ep_size, self.n_logical_routed_experts, self.n_routed_experts,
-            host, n_nodes=max(1, self.ep_size // self.gpus_per_node))
-        to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(self.device)  # noqa: E731
-        self.phy2log = to_dev(phy2log)
-        return self.phy2log, to_dev(log2phy), to_dev(logcnt)
+        # the three arrays are parts of one buffer, which goes to the GPU in one copy
+        n_phy, n_log = self.n_routed_experts, self.n_logical_routed_experts
+        staged = torch.empty(n_phy + 3 * n_log, dtype=torch.int32, pin_memory=self.device.type == "cuda")
+        build_redundancy_mapping(self._r2o_host, self.ep_size, n_log, n_phy, host,
+                                 n_nodes=max(1, self.ep_size // self.gpus_per_node), out=staged.numpy())
+        table = staged.to(self.device)
+        self.phy2log = table[:n_phy]
+        return self.phy2log, table[n_phy:n_phy + 2 * n_log].view(n_log, 2), table[n_phy + 2 * n_log:]
 
     def count_workload(self, idx: torch.Tensor, n_sms: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Histogram of ``idx`` (values in [-1, n_logical), -1 ignored) over ``n_sms`` slices.

@@ -63,6 +63,25 @@ def test_balanced_packing_properties():
     assert np.array_equal(pack1, np.broadcast_to(np.arange(6), (3, 6))) and not rank1.any()
 
 
+@pytest.mark.parametrize("n_log,n_phy,groups,nodes,gpus", [
+    (1, 1, 1, 1, 1), (7, 8, 1, 1, 8), (24, 24, 8, 8, 8), (63, 64, 3, 1, 4), (256, 256, 4, 2, 32), (258, 264, 2, 2, 8),
+    (1290, 1296, 10, 2, 16)])                               # groups of 1, 3, 8, 21, 64, 129 experts: every way of adding them up
+@pytest.mark.parametrize("weights", ["distinct", "ties", "spread", "nan"])
+def test_native_placement_equals_the_numpy_restatement(n_log, n_phy, groups, nodes, gpus, weights):
+    from oracle import eplb_numpy
+    rng = np.random.default_rng(n_log)
+    w = {"distinct": rng.random((2, n_log)) * 1e6, "ties": rng.integers(0, 4, (2, n_log)),
+         "spread": rng.lognormal(0, 3, (2, n_log)), "nan": np.where(rng.random((2, n_log)) < 0.1, np.nan, 1.0)}[weights]
+    for got, want in zip(eplb.rebalance_experts(w, n_phy, groups, nodes, gpus),
+                         eplb_numpy.rebalance_experts(w, n_phy, groups, nodes, gpus)):
+        np.testing.assert_array_equal(got, want)
+    if n_log % 8 == 0 and n_log >= 16:
+        args = (topology.CUBE_8P2E, 8, n_log, n_log + 16, w[0], nodes)
+        for got, want in zip(build_redundancy_mapping(*args), eplb_numpy.build_redundancy_mapping(*args)):
+            np.testing.assert_array_equal(got, want)
+            assert got.dtype == want.dtype and got.shape == want.shape
+
+
 # ------------------------------------------------------ redundancy mapping
 @pytest.mark.parametrize("case", REFERENCE_SOLVE_CASES, ids=[c[0] for c in REFERENCE_SOLVE_CASES])
 @pytest.mark.parametrize("with_history", [False, True])
