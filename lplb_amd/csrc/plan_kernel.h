@@ -1,0 +1,870 @@
+// The whole plan of a batch as one kernel launch: device code and the launch of one variant.
+// plan.hip holds the entry points, the admission of launches and the chain of kernels that serves
+// everything else; plan_8.hip, plan_16.hip and plan_32.hip instantiate this file by group size.
+//
+// Every kernel boundary of the chain (histogram, scan, LP, redirect) costs 3-5 us on this GPU although the
+// kernels have 1-8 us of work.  Here the LP workgroups (one per four LPs, first in the grid) and one
+// workgroup per slice of the indices run side by side in a single grid:
+//   slice workgroup: load the indices once (they stay in registers as 16-bit expert ids) -> histogram of the
+//     slice in LDS, bitmaps of the replicated sets -> publish both -> collect the other slices' counts of the
+//     replicated sets -> ordinals and hashes -> wait for the LP's shares -> choose original or replica, store;
+//   LP workgroup: (own-histogram mode: collect the slices' histograms ->) solve -> publish the shares.
+// A batch of up to 4096 indices that feeds the LP itself is one workgroup that does both (plan_in_one_workgroup):
+// nothing is exchanged and nothing has to be resident beside it.
+//
+// What crosses workgroups are 8-byte words that say themselves whether they are complete, so that there is no
+// counter of arrivals between a slice's counts and their readers and no acknowledgement to wait for:
+// every word carries the launch's tag in its high half, and a launch overwrites the words of the launch before it
+// (which has ended; so nothing has to be cleared either).
+//   * A slice publishes its counts, two of 16 bits per word: those of the replicated sets for every other slice, the
+//     whole histogram for the slices that add up the batch's totals.
+//   * The totals are added up by up to 64 of the slices, each for eight words of every slice's histogram, and
+//     published once more; the LP workgroups and the first slice collect those.  (One CU reads such words past the
+//     caches at 25 bytes per ns: collecting 64 whole rows takes an LP workgroup 2.8 us, 256 rows 8 us.  As atomic
+//     adds to shared totals they run into the rate of the atomic units, about 5 per ns over the whole GPU: 1.6 us
+//     for 64 slices, 6.6 us for 256.)
+// Measured per call, own histogram, against rows read once a counter of arrivals said that everybody's were there:
+// [8192 x 8] 12.0 -> 11.6 us, [16384 x 8] at 32 ranks 25.3 -> 24.1, [262144 x 8] 22.8 -> 19.6.  What bounds it at
+// [8192 x 8]: 3.7 us until the last slice's counts are out (1.0 of them until the last workgroup has started), 2.6 us
+// until the LP has the totals, 4.6 us of LP, 0.9 us until the last index is stored.
+// Words are written and read with agent-scope atomics (plan_sync.h).
+// The workgroups wait for each other, so the whole grid has to be resident: its size is bounded by what fits
+// the GPU, and the host admits a launch only while the plans still executing leave room for it.
+// Every wait is bounded all the same.  A wait that runs out is counted, the workgroup sends every token of its
+// slice to the expert's original slot (which needs nothing from other workgroups), physical_counts is filled
+// with -1 by the workgroup that writes them if it is among those, and the block of words is marked as unusable:
+// plans that use it later send every token to the original slot and count one more failure each, until
+// lplb_plan_sync_timeouts has reported the failures and cleared the block.
+#pragma once
+#include "map_kernel.h"
+#include "plan_sync.h"
+#include "solve_spread.h"
+
+namespace lplb {
+
+constexpr int kPlanWaves = 8, kPlanThreads = kPlanWaves * kWave;
+constexpr int kPlanLdsLimit = 160 * 1024 - 8 * 1024;   // dynamic LDS; the kernels have static LDS besides
+constexpr int kDefaultMaxPolls = 1 << 22;   // a few seconds of polling before a wait gives up
+// LPs per LP workgroup: waves 0..3 of a workgroup sit on the CU's four SIMDs, and an LP
+// wave is bound by instruction issue, so a fifth LP on the same CU would slow two of them
+// down (8 LPs in one workgroup: 17.0 us per plan against 13.5 us).  Batches with more
+// groups get more LP workgroups.
+constexpr int kLpsPerWorkgroup = 4, kMaxLpWorkgroups = 8;
+// Ahead of its use, an LP workgroup's dynamic LDS holds per LP wave the pivot rows and the assembly tile, then
+// the counts.
+template <int GM, int DM> constexpr size_t plan_lp_area_bytes() {
+  return lp_pivot_doubles<GM, DM>() * sizeof(double) + lp_tile_floats<GM, DM>() * sizeof(float);
+}
+
+// One block of these per stream that plans (kSyncSlots of them per device), offsets in ints:
+//   [kGenAt] launches that have used the block; (value + 1) tags what a launch publishes;
+//   [kPoisonAt] non-zero: a wait ran out in this block (see above); [kTimeoutsAt] waits that
+//   ran out since the library was loaded (never cleared);
+//   [kAvailAt + 2 p] (8 bytes) who has touched the caller's counter of feasible LPs in the launch with tag
+//   parity p: bit k = LP k was feasible and has been (or is being) added, bit 32 = a wait ran out, so the
+//   batch is not balanced as a whole and whoever set the bit took the LPs added so far back out; an LP
+//   that finds bit 32 set does not add itself.  The reference's callers read "counter == number of
+//   groups" as "this batch was balanced" (tests/test_solve.py:58, scripts/run_ep16_cube8p2e.py:61).
+//   every launch clears the word of the other parity;
+//   from kSharesAt: the LP's shares as words (tag << 32) | float bits with tag = (launch tag << 2) | 1 (valid)
+//   or 2 (there will be none); up to kShareCopies copies, kMaxShares words apart: polls of one line queue up in
+//   memory, so slice s polls copy s % copies;
+//   from kSetRowsAt: per slice set_words words with its tokens of the replicated sets, two sets per word;
+//   from kHistRowsAt: per slice hist_words words with its histogram, two experts per word;
+//   from kTotalsAt: one word per expert with the batch's tokens.
+constexpr int kGenAt = 0, kPoisonAt = 1, kTimeoutsAt = 4, kAvailAt = 10;
+constexpr unsigned long long kGaveUp = 1ull << 32;
+constexpr int kMaxSlices = 256, kMaxPlanExperts = 1024, kMaxShares = 1024, kShareCopies = 8;
+constexpr int kSharesAt = 16, kMaxSetWords = kMaxPlanExperts / 2, kMaxHistWords = kMaxPlanExperts / 2;
+constexpr int kSetRowsAt = kSharesAt + 2 * kMaxShares * kShareCopies;
+constexpr int kHistRowsAt = kSetRowsAt + 2 * kMaxSlices * kMaxSetWords;
+constexpr int kTotalsAt = kHistRowsAt + 2 * kMaxSlices * kMaxHistWords;
+constexpr int kSlotInts = kTotalsAt + 2 * kMaxPlanExperts, kSyncSlots = 8;
+static_assert(kSetRowsAt % 16 == 0 && kHistRowsAt % 16 == 0 && kTotalsAt % 16 == 0 && kSlotInts % 16 == 0, "rows start on 64-byte lines");
+
+struct PlanArgs {
+  const int64_t *idx;
+  int64_t n, per;
+  int n_slices, n_lp_workgroups;
+  int n_share_copies;    // copies of the LP's shares: a power of two, at most kShareCopies
+  int set_words;         // words per slice for its counts of the replicated sets: a power of two >= 8
+  int hist_words;        // ... for its histogram: a multiple of 8 that holds n_logical counts
+  int adders, adder_words;     // slices that add up the totals, for adder_words words (a power of two >= 8) of every histogram each
+  int expected_slices;   // = n_slices unless a fault is injected
+  int max_polls;
+  const int32_t *o2r, *phy2log;
+  int32_t *totals;   // [n_logical] this GPU's tokens per expert, out
+  int64_t *out;
+  int32_t *physical_counts;   // [n_ranks * P] tokens per physical expert, or null
+  int32_t *avail;
+  RedirectShape sh;
+  int n_rep;
+  uint32_t magic_L, magic_cd, magic_D, magic_G;   // fast_div_magic of L, C * D, D, G
+  SolveArgs solve;   // result = the shares (o_weight); workload is replaced by the batch's own counts if local_counts
+  int local_counts;
+  int *sync;
+  int *arrived_word;   // pinned host memory, or null: receives arrived_seq once every workgroup of the launch has arrived
+  int arrived_seq;
+};
+
+// plan.hip: admission and launch of one kernel (see there).  lds: dynamic LDS of the launch.
+struct KernelFootprint {   // one per kernel variant
+  std::atomic<int> regs{-1}, static_lds{0};
+  std::atomic<uint64_t> much_lds_allowed{0};   // bit per device: the kernel may use more than 64 KiB of dynamic LDS
+};
+typedef void (*PlanKernel)(PlanArgs);
+int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_others, PlanArgs &a, size_t lds, hipStream_t s,
+                bool *done);
+// plan_8.hip, plan_16.hip, plan_32.hip: the variants for group sizes up to 8, 16, 32.
+int launch_plan_up_to_8(PlanArgs &a, hipStream_t s, bool *done);
+int launch_plan_up_to_16(PlanArgs &a, hipStream_t s, bool *done);
+int launch_plan_up_to_32(PlanArgs &a, hipStream_t s, bool *done);
+
+// A wait ran out: count it, switch the block of words off, and make sure the caller's counter of
+// feasible LPs does not vouch for this batch (the first to give up takes back what the LPs have added).
+__device__ inline void give_up(const PlanArgs &a, unsigned long long *avail_state) {
+  agent_add(a.sync + kTimeoutsAt, 1);
+  agent_store(a.sync + kPoisonAt, 1);
+  const unsigned long long before = __hip_atomic_fetch_or(avail_state, kGaveUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int added = __popcll(before & 0xffffffffull);
+  if (!(before & kGaveUp) && added > 0)
+    atomicAdd(a.avail, -added);
+}
+
+// Debug builds: stamps of the first and the last slice workgroup and of the first LP workgroup.
+#define LPLB_PLAN_STAMP(k)                                                                     \
+  LPLB_STAMP_AT(a.solve.clocks == nullptr ? nullptr                                            \
+                : blockIdx.x == a.n_lp_workgroups ? a.solve.clocks + 64                        \
+                : blockIdx.x == gridDim.x - 1 ? a.solve.clocks + 80                            \
+                : blockIdx.x == 0 ? a.solve.clocks + 96 : nullptr, k)
+
+// Debug builds: stamps of every slice workgroup (the buffer must hold 128 + 8 * slices).
+#ifdef LPLB_PHASE_CLOCKS
+#define LPLB_SLICE_STAMP(k)                                                                    \
+  do {                                                                                         \
+    if (a.solve.clocks && threadIdx.x == 0)                                                    \
+      a.solve.clocks[128 + 8 * (blockIdx.x - a.n_lp_workgroups) + (k)] = wall_clock64();       \
+  } while (0)
+#else
+#define LPLB_SLICE_STAMP(k) do { } while (0)
+#endif
+
+// ---- a slice's tables in LDS ----
+// One ranking slot per (wave, replicated set, chunk of 64 indices), K chunks per wave.
+constexpr int64_t kLongestSlice = 16 * kPlanThreads;   // 16 chunks per wave
+template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
+  return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * rank_record_bytes_single(K) +
+         (size_t)(n_logical + 1) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
+         (size_t)(3 + kPlanWaves) * (n_rep + 1) * sizeof(int32_t) + 32;
+}
+struct SliceTables {
+  RepEntry *reps;           // [R + 1]
+  unsigned char *records;   // [waves][R + 1][record bytes]
+  Route *route;             // [n_logical + 1]
+  int32_t *set_expert;      // [R] the set's expert, -1: none
+  int32_t *before, *total;  // [R] tokens of the set before this slice, in the whole batch
+  int32_t *wave_total;      // [waves][R] ... in the chunks of the waves before each wave (one pass)
+  int32_t *hist;            // [n_logical up to a multiple of 16, + 1] the slice's histogram; once that is published, what it adds up of the
+                            // batch's; in the first slice at last the whole of the batch's
+};
+template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, int nl, int R) {
+  SliceTables t;
+  t.reps = reinterpret_cast<RepEntry *>(lds);
+  t.records = lds + (size_t)(R + 1) * sizeof(RepEntry);
+  t.route = reinterpret_cast<Route *>(t.records + (size_t)kPlanWaves * (R + 1) * rank_record_bytes_single(K));
+  t.set_expert = reinterpret_cast<int32_t *>(t.route + nl + 1);
+  t.before = t.set_expert + R;
+  t.total = t.before + R;
+  t.wave_total = t.total + R;
+  t.hist = t.wave_total + kPlanWaves * R;
+  return t;
+}
+
+// What the table build reads of global memory, as unconditional loads from clamped addresses ahead of the index
+// loads; and where a set belongs.
+struct SetOfPlan {
+  int ep_rank, place, d, group_rank;
+};
+__device__ inline SetOfPlan set_of_plan(const PlanArgs &a, int i) {
+  const int cd = a.sh.C * a.sh.D;
+  SetOfPlan s;
+  s.ep_rank = (int)fast_div((uint32_t)i, a.magic_cd);
+  s.place = i - s.ep_rank * cd;
+  s.d = s.place - (int)fast_div((uint32_t)s.place, a.magic_D) * a.sh.D;
+  s.group_rank = s.ep_rank - (int)fast_div((uint32_t)s.ep_rank, a.magic_G) * a.sh.G;
+  return s;
+}
+__device__ inline int slot_of_plan(const PlanArgs &a, int e) {
+  return e + (int)fast_div((uint32_t)e, a.magic_L) * (a.sh.P - a.sh.L);
+}
+struct PlanTableLoads {
+  int slot0, le0, rle0, host0;
+  int physical_le0;   // phy2log of physical slot tid
+  bool set0;
+  SetOfPlan s0;
+};
+__device__ inline PlanTableLoads issue_plan_table_loads(const PlanArgs &a, int tid) {
+  PlanTableLoads t;
+  t.slot0 = slot_of_plan(a, min(tid, a.sh.n_logical - 1));
+  t.le0 = a.phy2log[t.slot0];
+  t.set0 = tid < a.n_rep;
+  t.s0 = set_of_plan(a, t.set0 ? tid : 0);
+  t.rle0 = a.phy2log[t.s0.ep_rank * a.sh.P + t.s0.place];
+  t.host0 = a.o2r[t.s0.group_rank * a.sh.D + t.s0.d];
+  t.physical_le0 = a.phy2log[min(tid, a.sh.n_ranks * a.sh.P - 1)];
+  return t;
+}
+// Where an expert's tokens go when nothing is redirected and which replicated set (if any) it belongs to
+// (minilp.cu:466-496); everything else empty.  Ends with a workgroup barrier.
+template <int K>
+__device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t, const PlanTableLoads &l, int tid) {
+  constexpr int nt = kPlanThreads;
+  const int nl = a.sh.n_logical, R = a.n_rep, cd = a.sh.C * a.sh.D;
+  for (int e = tid; e <= nl; e += nt)
+    t.route[e] = Route{-1, R};
+  for (int e = tid; e <= nl; e += nt)
+    t.hist[e] = 0;
+  {
+    const i32x4 zero{0, 0, 0, 0};
+    i32x4 *z = reinterpret_cast<i32x4 *>(t.records);
+    for (int i = tid; i < kPlanWaves * (R + 1) * rank_record_bytes_single(K) / 16; i += nt)
+      z[i] = zero;
+  }
+  for (int q = tid; q < R; q += nt) {
+    t.before[q] = 0;
+    t.total[q] = 0;
+  }
+  if (tid == 0)
+    t.reps[R] = RepEntry{1, 0xffffffffu, INT32_MAX, -1};   // "no replica": every token stays
+  __syncthreads();
+  if (tid < nl && l.le0 >= 0 && l.le0 < nl)
+    t.route[l.le0].original = l.slot0;
+  for (int e = tid + nt; e < nl; e += nt) {
+    const int s = slot_of_plan(a, e), le = a.phy2log[s];
+    if (le >= 0 && le < nl)
+      t.route[le].original = s;
+  }
+  // A set's key is R - 1 - i, so that of two sets that name the same expert the later one
+  // wins (as a sequential pass over the sets would have it) with an atomic min.
+  auto enter_set = [&](int i, const SetOfPlan &s, int le, int host) {
+    const bool ok = le >= 0 && le < nl;
+    if (ok)
+      atomicMin(&t.route[le].rep, R - 1 - i);
+    t.reps[R - 1 - i] = RepEntry{0, 0u, 0, ((s.ep_rank - s.group_rank) + host + 1) * a.sh.P - cd + s.place};
+    t.set_expert[R - 1 - i] = ok ? le : -1;
+  };
+  if (l.set0)
+    enter_set(tid, l.s0, l.rle0, l.host0);
+  for (int i = tid + nt; i < R; i += nt) {
+    const SetOfPlan s = set_of_plan(a, i);
+    enter_set(i, s, a.phy2log[s.ep_rank * a.sh.P + s.place], a.o2r[s.group_rank * a.sh.D + s.d]);
+  }
+  __syncthreads();
+}
+
+// K chunks of 64 indices from w0 on (uniform), those before `end`.
+template <int K> __device__ inline void load_chunks(int64_t (&raw)[K], const int64_t *idx, int64_t w0, int64_t end, int lane) {
+  const int64_t *src = idx + w0 + lane;
+  if (w0 + K * kWave <= end) {
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      raw[c] = __builtin_nontemporal_load(src + c * kWave);
+  } else {
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      raw[c] = w0 + c * kWave + lane < end ? __builtin_nontemporal_load(src + c * kWave) : -1;
+  }
+}
+template <int K> __device__ inline void store_chunks(const int32_t (&o)[K], int64_t *out, int64_t w0, int64_t end, int lane) {
+  int64_t *dst = out + w0 + lane;
+  if (w0 + K * kWave <= end) {
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      __builtin_nontemporal_store((int64_t)o[c], dst + c * kWave);
+  } else {
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      if (w0 + c * kWave + lane < end)
+        __builtin_nontemporal_store((int64_t)o[c], dst + c * kWave);
+  }
+}
+// Between the phases a token is kept as its expert id only, two ids per register (the route is looked up
+// again where it is needed): the waits are long and registers bound how many workgroups are resident.
+template <int N> __device__ inline int packed_expert(const uint32_t (&packed)[N], int c) {
+  return (int)((packed[c / 2] >> (16 * (c % 2))) & 0xffffu);
+}
+template <int N> __device__ inline void pack_expert(uint32_t (&packed)[N], int c, int e) {
+  packed[c / 2] = (c % 2) ? packed[c / 2] | ((uint32_t)e << 16) : (uint32_t)e;
+}
+
+// ---- a slice's tokens: bitmaps and histogram, the tokens of the earlier chunks and waves ----
+template <int K> struct SliceTokens {
+  static constexpr int kRec = rank_record_bytes_single(K);
+  __device__ static ChunkSlot *slot(unsigned char *my_records, int set, int c) {
+    return reinterpret_cast<ChunkSlot *>(my_records + __umul24((uint32_t)set, (uint32_t)kRec)) + c;
+  }
+  // Enters the wave's tokens; afterwards t.hist is the slice's histogram, a slot's start the tokens of its set
+  // in the wave's earlier chunks, t.wave_total those in the earlier waves.  Ends with a workgroup barrier.
+  __device__ static void count(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, const int64_t (&raw)[K],
+                               uint32_t (&packed)[(K + 1) / 2], int tid, int lane, int wave_s) {
+    const int nl = a.sh.n_logical, R = a.n_rep;
+    const unsigned long long my_bit = 1ull << lane;
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const bool valid = (uint64_t)raw[c] < (uint64_t)nl;   // -1, other negatives and too large ids fail
+      const int e = valid ? (int)raw[c] : nl;
+      pack_expert(packed, c, e);
+      const int set = t.route[e].rep;
+      // a token of a replicated set is counted through the set's bitmaps (the sets hold the hot
+      // experts, whose tokens would queue up at one histogram counter), any other one here
+      if (set < R)
+        atomicOr(reinterpret_cast<unsigned long long *>(slot(my_records, set, c)), my_bit);
+      else if (valid)
+        atomicAdd(&t.hist[e], 1);
+    }
+    __syncthreads();
+    LPLB_PLAN_STAMP(8);
+    LPLB_SLICE_STAMP(1);
+    // inside the wave: lane = (set, chunk), chunk fastest
+    const int c = lane % K;
+    for (int p0 = 0; p0 < R * K; p0 += kWave) {
+      const bool live = p0 + lane < R * K;
+      const int q = live ? (p0 + lane) / K : R;   // lanes past the end read the stand-in record (zeros)
+      ChunkSlot *mine = slot(my_records, q, c);
+      const int own = __popcll(*reinterpret_cast<const unsigned long long *>(mine));
+      const int in_my_wave = group_sum<K>(own);
+      const int in_earlier_chunks = group_exclusive_scan<K>(own, c);
+      if (live) {
+        mine->start = in_earlier_chunks;
+        if (c == 0)
+          t.wave_total[wave_s * R + q] = in_my_wave;
+      }
+    }
+    __syncthreads();
+    for (int q = tid; q < R; q += kPlanThreads) {   // the sets' tokens in this slice, into the histogram
+      int32_t n = 0, of_wave[kPlanWaves];
+#pragma unroll
+      for (int w = 0; w < kPlanWaves; ++w)
+        of_wave[w] = t.wave_total[w * R + q];
+#pragma unroll
+      for (int w = 0; w < kPlanWaves; ++w) {   // (each wave's count becomes the count of the waves before it)
+        t.wave_total[w * R + q] = n;
+        n += of_wave[w];
+      }
+      const int le = t.set_expert[q];
+      if (le >= 0 && t.route[le].rep == q)   // (of two sets that name the same expert only one has the tokens)
+        t.hist[le] = n;
+    }
+    __syncthreads();
+  }
+  // Ordinal of the first token of every chunk: what is there already plus the tokens before this slice and in
+  // the waves before this one.  The wave's own slots only: no barrier.
+  __device__ static void add_starts(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, int lane, int wave_s) {
+    const int R = a.n_rep, c = lane % K;
+    for (int p0 = 0; p0 < R * K; p0 += kWave) {
+      const bool live = p0 + lane < R * K;
+      const int q = live ? (p0 + lane) / K : 0;
+      const int32_t base = t.before[q] + t.wave_total[wave_s * R + q];
+      if (live)
+        atomicAdd(&slot(my_records, q, c)->start, base);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  __device__ static int32_t hash(const SliceTables &t, unsigned char *my_records, int e, int c) {
+    const int set = t.route[e].rep;
+    const i32x4 s = *reinterpret_cast<const i32x4 *>(slot(my_records, set, c));   // bits_lo, bits_hi, start
+    const i32x4 x = *reinterpret_cast<const i32x4 *>(&t.reps[set]);               // total, magic, -, -
+    const int32_t k =
+        __builtin_amdgcn_mbcnt_hi((uint32_t)s.y, __builtin_amdgcn_mbcnt_lo((uint32_t)s.x, (uint32_t)s.z));
+    return ordinal_hash<false>(k, x.x, (uint32_t)x.y);
+  }
+};
+
+// Tokens per physical expert (= bincount of the output) from a slice's tables; hist: of the batch.
+// le0: phy2log of slot tid (or of any slot if there is none), read ahead of time.
+__device__ inline void plan_physical_counts(const PlanArgs &a, const SliceTables &t, int le0, bool ok, int tid) {
+  const int nl = a.sh.n_logical, R = a.n_rep;
+  for (int i = tid; i < a.sh.n_ranks * a.sh.P; i += kPlanThreads) {
+    const int le = !ok ? -1 : i == tid ? le0 : a.phy2log[i];
+    int32_t v = ok ? 0 : -1;
+    if (le >= 0 && le < nl) {
+      const Route rt = t.route[le];
+      if (rt.rep >= R) {
+        v = rt.original == i ? t.hist[le] : 0;
+      } else {
+        const RepEntry x = t.reps[rt.rep];
+        const int32_t kept = kept_on_original(x.total, x.expected);
+        v = rt.original == i ? kept : (x.replica == i ? x.total - kept : 0);
+      }
+    }
+    a.physical_counts[i] = v;
+  }
+}
+__device__ inline void set_total(RepEntry &x, int32_t total) {
+  x.total = total;
+  x.magic = total >= 1 ? 0xffffffffu / (uint32_t)total : 0u;
+}
+
+// ---- collecting words ----
+__device__ inline unsigned long long tagged_word(uint32_t tag, uint32_t v) { return ((unsigned long long)tag << 32) | v; }
+// Up to N words per lane (its first `mine`), all with the launch's tag: polls until they are or max_polls polls have
+// passed; words past `mine` are 0.  Whole waves; false: the wait ran out.
+template <int N, typename Address>
+__device__ inline bool collect_words(uint32_t (&words)[N], uint32_t tag, int mine, int max_polls, Address address) {
+  for (int polls = 0; polls < max_polls; ++polls) {
+    unsigned long long v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      v[k] = k < mine ? agent_load(address(k)) : (unsigned long long)tag << 32;
+    bool all_in = true;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      all_in = all_in && (uint32_t)(v[k] >> 32) == tag;
+      words[k] = (uint32_t)v[k];
+    }
+    if (__all(all_in))
+      return true;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return false;
+}
+// Adds up `words` words (two counts each) of every slice's row over the slices, into total[] and, over the slices
+// before this one, into before[] (LDS, zeroed; before may be null).  row_words: a power of two >= words; stride:
+// words from row to row.  By the whole workgroup: a thread takes one word of every (threads / row_words)-th slice,
+// IN_FLIGHT of them at a time.  Returns whether this wave's words all came.
+template <int IN_FLIGHT>
+__device__ inline bool add_up_rows_n(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int row_words,
+                                     uint32_t tag, int slice, int32_t *total, int32_t *before, int tid, int lane) {
+  const bool can_come = a.expected_slices == a.n_slices;   // (an injected fault: one slice never comes)
+  const int max_polls = can_come ? a.max_polls : 1;
+  const int q_lanes = min(row_words, kPlanThreads), p_lanes = kPlanThreads / q_lanes;   // powers of two
+  const int p_first = tid / q_lanes;
+  bool came = can_come;
+  for (int q0 = 0; q0 < words; q0 += q_lanes) {
+    const int q = q0 + tid % q_lanes;
+    const bool in_row = q < words;
+    int32_t sum[2] = {0, 0}, earlier[2] = {0, 0};
+    for (int p0 = 0; p0 < a.n_slices; p0 += IN_FLIGHT * p_lanes) {
+      const unsigned long long *at = rows + (int64_t)(p0 + p_first) * stride + q;
+      const int left = in_row ? (a.n_slices - p0 - p_first + p_lanes - 1) / p_lanes : 0;   // words of this thread, at most IN_FLIGHT now
+      uint32_t counts[IN_FLIGHT];
+      came = collect_words<IN_FLIGHT>(counts, tag, left, max_polls, [&](int k) { return at + (int64_t)k * p_lanes * stride; }) && came;
+#pragma unroll
+      for (int k = 0; k < IN_FLIGHT; ++k) {
+        const bool is_before = p0 + k * p_lanes + p_first < slice;
+        const int32_t lo = (int32_t)(counts[k] & 0xffffu), hi = (int32_t)(counts[k] >> 16);
+        sum[0] += lo;
+        sum[1] += hi;
+        earlier[0] += is_before ? lo : 0;
+        earlier[1] += is_before ? hi : 0;
+      }
+    }
+    // lanes of a wave that hold the same word add up first (updates of one LDS word queue up)
+    for (int m = q_lanes; m < kWave; m <<= 1)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        sum[h] += __shfl_xor(sum[h], m);
+        earlier[h] += before ? __shfl_xor(earlier[h], m) : 0;
+      }
+    if (in_row && lane < q_lanes)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        atomicAdd(&total[2 * q + h], sum[h]);
+        if (before)
+          atomicAdd(&before[2 * q + h], earlier[h]);
+      }
+  }
+  return came;
+}
+__device__ inline bool add_up_rows(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int row_words,
+                                   uint32_t tag, int slice, int32_t *total, int32_t *before, int tid, int lane) {
+  return a.n_slices * min(row_words, kPlanThreads) <= kPlanThreads
+             ? add_up_rows_n<1>(a, rows, stride, words, row_words, tag, slice, total, before, tid, lane)
+             : add_up_rows_n<4>(a, rows, stride, words, row_words, tag, slice, total, before, tid, lane);
+}
+// The batch's totals into `counts` (LDS, floats or ints; below 2^24 a count is exact as a float), by every wave of
+// the workgroup.  Returns whether this wave's have come.
+template <typename T>
+__device__ inline bool collect_totals(const PlanArgs &a, T *counts, uint32_t tag, int tid, int wave_s) {
+  const unsigned long long *totals = reinterpret_cast<const unsigned long long *>(a.sync + kTotalsAt);
+  const int nl = a.sh.n_logical;
+  if (a.expected_slices != a.n_slices)   // (an injected fault: one slice never comes)
+    return false;
+  for (int e0 = wave_s * kWave; e0 < nl; e0 += kPlanThreads) {
+    const int e = e0 + tid % kWave;
+    uint32_t count[1];
+    if (!collect_words<1>(count, tag, e < nl, a.max_polls, [&](int) { return totals + e; }))
+      return false;
+    if (e < nl)
+      counts[e] = (T)count[0];
+  }
+  return true;
+}
+
+// K: 64-index chunks per wave.
+// Registers: up to 16 ranks the kernel as a whole is held to 128 VGPRs (two workgroups per CU), which is what
+// lets 256 slices and the LPs be resident together; the LP of 32 ranks takes more.
+constexpr int plan_workgroups_per_cu(int group_size) { return group_size <= 16 ? 2 : 1; }
+template <int GM, int DM, bool EXACT, int K>
+__global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void plan_in_one_launch(PlanArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
+  __shared__ int missing[2];   // LP workgroup: [0] some counts did not come; slice: [0] the same, [1] some share will not come
+  const int nl = a.sh.n_logical, R = a.n_rep;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
+  const int pid = blockIdx.x;
+  // Which launch of this block of words this is (the same value in every workgroup: it is advanced only once
+  // all of them have read it), and whether the block is switched off.
+  const int gen = agent_load(a.sync + kGenAt);
+  const bool poisoned = agent_load(a.sync + kPoisonAt) != 0;
+  const uint32_t tag = (uint32_t)gen + 1u;
+  const uint32_t tag_valid = (tag << 2) | 1u, tag_none = tag_valid + 1u;
+  unsigned long long *shares = reinterpret_cast<unsigned long long *>(a.sync + kSharesAt);
+  unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen & 1);
+
+  if (pid < a.n_lp_workgroups) {
+    // ------------------------------------------------------------ the LPs
+    SolveArgs sa = a.solve;
+    const int first_lp = pid * kLpsPerWorkgroup;          // of this workgroup
+    const int n_lps = min(kLpsPerWorkgroup, sa.n_units - first_lp);
+    LPLB_PLAN_STAMP(0);
+    // dynamic LDS of an LP workgroup: [LP wave][pivot rows | assembly tile], then the counts
+    constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
+    static_assert(kLpArea % 16 == 0, "the LP waves' areas keep 16-byte alignment");
+    unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
+    float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
+    sa.tag_valid = tag_valid;
+    // Own-histogram mode: the LP waves' table loads are on their way when they and the other waves turn to the
+    // batch's histogram.  (Switched off: no slice will publish.)
+    auto counts_have_come = [&]() -> bool {
+      const bool mine = !poisoned && collect_totals(a, staged, tag, tid, wave_s);
+      if (!mine && lane == 0)
+        missing[0] = 1;
+      __syncthreads();
+      return missing[0] == 0;
+    };
+    if (a.local_counts) {
+      if (tid == 0)
+        missing[0] = 0;
+      __syncthreads();
+    }
+    LPLB_PLAN_STAMP(1);
+    if (wave_s < n_lps) {
+      // (own-histogram mode: every LP of the batch reads the one staged copy)
+      float *mine = a.local_counts ? staged : staged + (size_t)wave_s * sa.staged_stride;
+      const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
+          sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave, reinterpret_cast<double *>(my_area),
+          reinterpret_cast<float *>(my_area + lp_pivot_doubles<GM, DM>() * sizeof(double)), counts_have_come);
+      if (n_ok < 0) {
+        // no counts, no solution: tell the slices not to wait for this LP's shares
+        if (wave_s == 0 && lane == 0 && !poisoned)
+          give_up(a, avail_state);
+        const int n_edges = sa.G * sa.D;
+        for (int j = lane; j < n_edges; j += kWave)
+          for (int k = 0; k < a.n_share_copies; ++k)
+            agent_store(shares + (int64_t)k * kMaxShares + (int64_t)(first_lp + wave_s) * n_edges + j,
+                        (unsigned long long)tag_none << 32);
+      } else if (lane == 0 && n_ok > 0 && !poisoned) {
+        // feasible: count it for the caller unless some workgroup has already given up on this batch
+        const unsigned long long before = __hip_atomic_fetch_or(avail_state, 1ull << (first_lp + wave_s), __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT);
+        if (!(before & kGaveUp))
+          atomicAdd(a.avail, n_ok);
+      }
+    } else if (a.local_counts) {
+      counts_have_come();
+    }
+    LPLB_PLAN_STAMP(2);
+    return;
+  }
+
+  // --------------------------------------------------------------- a slice
+  const int slice = pid - a.n_lp_workgroups;
+  const SliceTables t = carve_tables<K>(smem_raw, nl, R);
+  unsigned char *my_records = t.records + (size_t)wave_s * ((R + 1) * rank_record_bytes_single(K));
+  const int64_t begin = slice_begin(a.n, a.per, slice);
+  const int64_t end = slice_begin(a.n, a.per, slice + 1);
+  LPLB_PLAN_STAMP(0);
+  LPLB_SLICE_STAMP(0);
+  // Where a slice shares a CU with an LP workgroup (grids with more workgroups than CUs), its
+  // waves go first: the LP wave issues an instruction nearly every cycle it may, and a slice
+  // wave on the same SIMD would be starved for as long as the LP runs, with every other slice
+  // waiting for it.  The slices spend most of their time asleep, so the LP loses little.
+  __builtin_amdgcn_s_setprio(2);
+
+  // ---- small table reads, the index loads right behind them, the tables while they are on their way ----
+  const PlanTableLoads tl = issue_plan_table_loads(a, tid);
+  const int64_t w0 = begin + (int64_t)wave_s * (K * kWave);   // first index of this wave's chunks (uniform)
+  int64_t raw[K];
+  load_chunks<K>(raw, a.idx, w0, end, lane);
+  if (tid == 0) {
+    missing[0] = 0;
+    missing[1] = 0;
+  }
+  build_plan_tables<K>(a, t, tl, tid);
+  LPLB_PLAN_STAMP(10);
+
+  // ---- the tokens ----
+  uint32_t packed[(K + 1) / 2];
+  SliceTokens<K>::count(a, t, my_records, raw, packed, tid, lane, wave_s);
+  LPLB_PLAN_STAMP(9);
+  // ---- this slice's counts, for every workgroup ----
+  unsigned long long *set_rows = reinterpret_cast<unsigned long long *>(a.sync + kSetRowsAt);
+  unsigned long long *hist_rows = reinterpret_cast<unsigned long long *>(a.sync + kHistRowsAt);
+  const int real_set_words = (R + 1) / 2;
+  if (!poisoned) {
+    auto count_of_set = [&](int q) {
+      const int le = q < R ? t.set_expert[q] : -1;
+      return le >= 0 && t.route[le].rep == q ? (uint32_t)t.hist[le] : 0u;
+    };
+    auto count_of = [&](int e) { return e < nl ? (uint32_t)t.hist[e] : 0u; };
+    for (int e2 = tid; e2 < a.hist_words; e2 += kPlanThreads)
+      agent_store(hist_rows + (int64_t)slice * a.hist_words + e2, tagged_word(tag, count_of(2 * e2) | count_of(2 * e2 + 1) << 16));
+    for (int q2 = tid; q2 < real_set_words; q2 += kPlanThreads)
+      agent_store(set_rows + (int64_t)slice * a.set_words + q2, tagged_word(tag, count_of_set(2 * q2) | count_of_set(2 * q2 + 1) << 16));
+  } else if (slice == 0 && tid == 0) {
+    agent_add(a.sync + kTimeoutsAt, 1);   // one more plan that this block of words could not serve
+  }
+  LPLB_PLAN_STAMP(1);
+  LPLB_SLICE_STAMP(2);
+  // ---- the batch's totals of eight words' experts (more if there are fewer slices than that takes), if this slice
+  //      is one that adds them up ----
+  bool mine_came = !poisoned;
+  if (!poisoned && slice < a.adders) {
+    const int first_word = slice * a.adder_words, words = min(a.adder_words, a.hist_words - first_word);
+    __syncthreads();   // (the histogram has been read)
+    for (int i = tid; i < 2 * words; i += kPlanThreads)
+      t.hist[i] = 0;
+    __syncthreads();
+    mine_came = add_up_rows(a, hist_rows + first_word, a.hist_words, words, a.adder_words, tag, slice, t.hist, nullptr, tid, lane);
+    __syncthreads();
+    unsigned long long *totals = reinterpret_cast<unsigned long long *>(a.sync + kTotalsAt);
+    if (mine_came)   // (a wave whose words did not come gives the batch up below)
+      for (int i = tid; i < 2 * words; i += kPlanThreads)
+        if (2 * first_word + i < nl)
+          agent_store(totals + 2 * first_word + i, tagged_word(tag, (uint32_t)t.hist[i]));
+  }
+  LPLB_PLAN_STAMP(11);
+  // ---- tokens of each replicated set before this slice and in the whole batch ----
+  if (!poisoned)
+    mine_came = add_up_rows(a, set_rows, a.set_words, real_set_words, a.set_words, tag, slice, t.total, t.before, tid, lane) && mine_came;
+  if (!mine_came)
+    missing[0] = 1;
+  __syncthreads();
+  LPLB_PLAN_STAMP(2);
+  LPLB_SLICE_STAMP(4);
+  bool ok = missing[0] == 0;   // (the same in every thread)
+  if (!ok && !poisoned && tid == 0)
+    give_up(a, avail_state);
+  int32_t h[K];   // hashes of this thread's tokens: worked out while the LP is still running
+  if (ok) {
+    for (int q = tid; q < R; q += kPlanThreads)
+      set_total(t.reps[q], t.total[q]);
+    SliceTokens<K>::add_starts(a, t, my_records, lane, wave_s);
+    if (slice == 0 && !collect_totals(a, t.hist, tag, tid, wave_s)) {   // for the caller (and for the counts below)
+      if (lane == 0)
+        give_up(a, avail_state);
+      missing[1] = 1;
+    }
+    __syncthreads();
+    LPLB_PLAN_STAMP(3);
+    if (slice == 0)
+      for (int e = tid; e < nl; e += kPlanThreads)
+        a.totals[e] = t.hist[e];
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      h[c] = SliceTokens<K>::hash(t, my_records, packed_expert(packed, c), c);
+      if (K > 8 && c % 8 == 7)
+        __builtin_amdgcn_sched_barrier(0);   // (the table reads of all 16 at once would not fit the registers)
+    }
+    LPLB_PLAN_STAMP(4);
+    // ---- the LP's shares: every set's thread polls its own; value and tag arrive in the same word ----
+    for (int i = tid; i < R; i += kPlanThreads) {
+      const SetOfPlan s = set_of_plan(a, i);
+      const unsigned long long *word_at = shares + (slice & (a.n_share_copies - 1)) * kMaxShares + s.ep_rank * a.sh.D + s.d;
+      unsigned long long word = 0;
+      int polls = 0;
+      uint32_t got = 0;
+      while ((got = (uint32_t)((word = agent_load(word_at)) >> 32)) != tag_valid && got != tag_none && ++polls < a.max_polls)
+        __builtin_amdgcn_s_sleep(1);
+      if (got == tag_valid) {
+        t.reps[R - 1 - i].expected = expected_on_original(__builtin_bit_cast(float, (uint32_t)word), t.total[R - 1 - i]);
+      } else {
+        if (got != tag_none)
+          give_up(a, avail_state);
+        missing[1] = 1;
+      }
+    }
+    __syncthreads();
+    LPLB_PLAN_STAMP(5);
+    ok = missing[1] == 0;
+    if (slice == 0 && tid == 0) {
+      // Every slice's counts and every LP's shares carry this launch's tag, so every workgroup has read it: the
+      // next launch takes the next one.  From here on no workgroup waits for one that is not resident yet: tell
+      // the host, which then stops counting this launch against what the GPU can hold at once (a posted write
+      // to host memory).
+      agent_store(a.sync + kGenAt, (gen + 1) & 0x3fffffff);
+      agent_store(reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (1 - (gen & 1)), 0ull);
+      if (a.arrived_word)
+        __hip_atomic_store(a.arrived_word, a.arrived_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  LPLB_PLAN_STAMP(6);
+  // ---- choose and store; if a wait ran out, every token goes to its original slot ----
+  int32_t o[K];
+#pragma unroll
+  for (int c = 0; c < K; ++c) {
+    const int e = packed_expert(packed, c);
+    const Route rt = t.route[e];
+    o[c] = rt.original;
+    if (ok) {
+      const RepEntry x = t.reps[rt.rep];
+      o[c] = h[c] >= x.expected ? x.replica : rt.original;
+    }
+    if (K > 8 && c % 8 == 7)
+      __builtin_amdgcn_sched_barrier(0);
+  }
+  if (slice == 0 && a.physical_counts)
+    plan_physical_counts(a, t, tl.physical_le0, ok, tid);
+  store_chunks<K>(o, a.out, w0, end, lane);
+  LPLB_PLAN_STAMP(7);
+  LPLB_SLICE_STAMP(3);
+}
+
+// A short batch that feeds the LP itself, as one workgroup: the LPs are solved by its first waves between the
+// histogram and the choice.  Bound by the chain table loads -> indices -> histogram -> LP (4 us of 7.7) -> choice,
+// of which the slices' form above adds two round trips through memory between slices and LP: [7 x 8] indices 11.3 ->
+// 9.0 us per call, [128 x 8] 11.6 -> 9.5 us, where the calling thread needs 8 us for a call.  Up to
+// kSingleMaxIndices, eight per lane: past that a wave's chunks take longer than the exchange.  The LP waves come last
+// in the order of the indices, so that they have none unless the batch fills all eight waves.
+constexpr int kSingleMaxIndices = 4096, kSingleMaxLps = kPlanWaves;
+template <int GM, int DM, bool EXACT, int K>
+__global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  __shared__ int rep_of_edge_all[kSingleMaxLps * kWave];
+  __shared__ float share_of[kSingleMaxLps * kWave];
+  const int nl = a.sh.n_logical, R = a.n_rep;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // LDS: the LP waves' areas, the counts as floats, the slice's tables
+  constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
+  const int n_lps = a.solve.n_units;
+  float *staged = reinterpret_cast<float *>(smem_raw + n_lps * kLpArea);
+  const SliceTables t = carve_tables<K>(reinterpret_cast<unsigned char *>(staged + (nl + 3) / 4 * 4), nl, R);
+  const int turn = (wave_s - n_lps) & (kPlanWaves - 1);   // this wave's place in the order of the indices
+  unsigned char *my_records = t.records + (size_t)turn * ((R + 1) * rank_record_bytes_single(K));
+  const PlanTableLoads tl = issue_plan_table_loads(a, tid);
+  const int64_t w0 = (int64_t)turn * (K * kWave);
+  int64_t raw[K];
+  load_chunks<K>(raw, a.idx, w0, a.n, lane);
+  LPLB_PLAN_STAMP(0);
+  uint32_t packed[(K + 1) / 2];
+  // (called by the LP waves once their own table loads are on their way)
+  auto count_the_tokens = [&]() -> bool {
+    build_plan_tables<K>(a, t, tl, tid);
+    SliceTokens<K>::count(a, t, my_records, raw, packed, tid, lane, turn);
+    for (int e = tid; e < nl; e += kPlanThreads) {
+      const int32_t n = t.hist[e];
+      staged[e] = (float)n;
+      a.totals[e] = n;
+    }
+    for (int q = tid; q < R; q += kPlanThreads) {
+      const int le = t.set_expert[q];
+      t.total[q] = le >= 0 && t.route[le].rep == q ? t.hist[le] : 0;
+      set_total(t.reps[q], t.total[q]);
+    }
+    __syncthreads();
+    return true;
+  };
+  if (wave_s < n_lps) {
+    unsigned char *area = smem_raw + wave_s * kLpArea;
+    SolveArgs sa = a.solve;
+    sa.shares_in_lds = share_of;
+    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(sa, wave_s, staged, rep_of_edge_all + wave_s * kWave,
+                                                    reinterpret_cast<double *>(area),
+                                                    reinterpret_cast<float *>(area + lp_pivot_doubles<GM, DM>() * sizeof(double)),
+                                                    count_the_tokens);
+    if (lane == 0 && n_ok > 0)
+      atomicAdd(a.avail, n_ok);
+  } else {
+    count_the_tokens();
+  }
+  const bool has_tokens = w0 < a.n;
+  int32_t h[K];
+  if (has_tokens) {
+    SliceTokens<K>::add_starts(a, t, my_records, lane, turn);
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      h[c] = SliceTokens<K>::hash(t, my_records, packed_expert(packed, c), c);
+  }
+  __syncthreads();
+  LPLB_PLAN_STAMP(2);
+  for (int i = tid; i < R; i += kPlanThreads) {
+    const SetOfPlan s = set_of_plan(a, i);
+    t.reps[R - 1 - i].expected = expected_on_original(share_of[s.ep_rank * a.sh.D + s.d], t.total[R - 1 - i]);
+  }
+  __syncthreads();
+  if (has_tokens) {
+    int32_t o[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const Route rt = t.route[packed_expert(packed, c)];
+      const RepEntry x = t.reps[rt.rep];
+      o[c] = h[c] >= x.expected ? x.replica : rt.original;
+    }
+    store_chunks<K>(o, a.out, w0, a.n, lane);
+  }
+  if (a.physical_counts)
+    plan_physical_counts(a, t, tl.physical_le0, true, tid);
+  LPLB_PLAN_STAMP(7);
+}
+
+// ---- host side: which variant ----
+template <int GM, int DM, bool EXACT, int K>
+static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
+  const size_t lds_slice = plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);
+  // LP workgroups: their waves' working areas, then the counts (one copy per LP if they fit,
+  // else none and the LPs read global memory; own-histogram mode needs one copy in any case)
+  const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
+  const size_t one_copy = (size_t)a.sh.n_logical * sizeof(float);
+  const size_t all_copies = (size_t)min(a.solve.n_units, kLpsPerWorkgroup) * one_copy;
+  size_t lds = max(lds_slice, lp_areas + (a.local_counts ? one_copy : 0));
+  a.solve.staged_stride = 0;
+  if (lp_areas + all_copies <= max(lds, (size_t)16 * 1024)) {   // (a few KiB more are worth one global round trip less)
+    lds = max(lds, lp_areas + all_copies);
+    a.solve.staged_stride = a.sh.n_logical;
+  }
+  if (lds > (size_t)kPlanLdsLimit)
+    return LPLB_OK;
+  static KernelFootprint footprint;
+  return launch_plan(plan_in_one_launch<GM, DM, EXACT, K>, footprint, true, a, lds, s, done);
+}
+template <int GM, int DM, bool EXACT, int K> static int launch_plan_single(PlanArgs &a, hipStream_t s, bool *done) {
+  const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + (a.sh.n_logical + 3) / 4 * 4 * sizeof(float) +
+                     plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);
+  if (lds > (size_t)kPlanLdsLimit)
+    return LPLB_OK;
+  a.solve.staged_stride = a.sh.n_logical;
+  static KernelFootprint footprint;
+  return launch_plan(plan_in_one_workgroup<GM, DM, EXACT, K>, footprint, false, a, lds, s, done);
+}
+template <int GM, int DM, bool EXACT> static int launch_plan_shape(PlanArgs &a, hipStream_t s, bool *done) {
+  if (a.n_lp_workgroups == 0) {   // as few chunks per wave as leave the LP waves without tokens
+    const int64_t per_chunk = (kPlanWaves - min(a.solve.n_units, kPlanWaves - 1)) * kWave;
+    return a.n <= 2 * per_chunk ? launch_plan_single<GM, DM, EXACT, 2>(a, s, done)
+           : a.n <= 4 * per_chunk ? launch_plan_single<GM, DM, EXACT, 4>(a, s, done)
+                                  : launch_plan_single<GM, DM, EXACT, 8>(a, s, done);
+  }
+  return a.per <= 2 * kPlanThreads   ? launch_plan_slices<GM, DM, EXACT, 2>(a, s, done)
+         : a.per <= 4 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 4>(a, s, done)
+         : a.per <= 8 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 8>(a, s, done)
+                                     : launch_plan_slices<GM, DM, EXACT, 16>(a, s, done);
+}
+template <int GM, int DM> static int launch_plan_padded_or_not(PlanArgs &a, hipStream_t s, bool *done) {
+  return a.sh.G == GM && a.sh.D == DM ? launch_plan_shape<GM, DM, true>(a, s, done) : launch_plan_shape<GM, DM, false>(a, s, done);
+}
+
+} // namespace lplb

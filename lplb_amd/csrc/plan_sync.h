@@ -7,8 +7,10 @@
 //     through / miss in the issuing XCD's L2, so the value lives in memory where every
 //     XCD sees it; an agent-scope atomic add is carried out by the atomic unit behind
 //     the caches, so there is no cached copy that could go stale;
+//   * an aligned 8-byte store is one piece: a word whose high half has the launch's tag has its low half too, so
+//     nothing has to be acknowledged or announced before such a word is read;
 //   * s_waitcnt vmcnt(0) after such stores waits for their acknowledgement, i.e. until
-//     they are visible device-wide; the counter that announces them is bumped only
+//     they are visible device-wide; a counter that announces them is bumped only
 //     after that wait and a workgroup barrier;
 //   * everything a workgroup reads of another's is read with such loads, never with plain
 //     loads behind an acquire fence: the fence (buffer_inv sc1) would invalidate this XCD's
@@ -49,7 +51,7 @@ __device__ inline void agent_add(unsigned long long *p, unsigned long long v) {
 // All earlier stores and atomics of this wave have been acknowledged.
 __device__ inline void stores_have_landed() { __builtin_amdgcn_s_waitcnt(0); }
 
-// Counting arrivals.  Updates of one 64-byte line queue up behind each other in memory
+// Counting arrivals, for exchanges whose words do not say themselves that they are complete (the plan's do).  Updates of one 64-byte line queue up behind each other in memory
 // (measured: about 14 ns each, whether or not they hit the same word; 35 ns for one word),
 // so a counter that hundreds of workgroups bump would itself take microseconds.  The count
 // is kept in kArrivalStripes words instead, 256 bytes apart (workgroup i bumps word

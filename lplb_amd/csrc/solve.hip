@@ -20,18 +20,18 @@ __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0)
     atomicAdd(a.avail, a.n_units);
   const int first_unit = blockIdx.x * ROWS;
-  const int n_ok = solve_lps<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_all, rep_of_edge, pivot_rows, tile);
+  const int n_ok = solve_lps<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_all, rep_of_edge, pivot_rows, tile,
+                                                         []() { return true; });
   const int n_mine = min(max(a.n_units - first_unit, 0), ROWS);
   if (threadIdx.x == 0 && n_ok < n_mine)
     atomicAdd(a.avail, n_ok - n_mine);
 }
 
-// One LP per wave has the lowest latency (8 us at (8, 2)) and is the fastest form
-// until the waves outnumber the SIMDs; from kPackFrom LPs on, shapes with G <= 16 and
-// G * D <= 16 put four LPs into each wave (10.4 us per wave, a quarter of the waves).
-// Measured at (8, 2): 1024 LPs 8.8 us unpacked; 2048 LPs 12.9 us unpacked, 11.4 us
-// packed; 16384 LPs 73 us unpacked, 31 us packed.
-constexpr int kPackFrom = 1536;
+// One LP per wave has the lowest latency and is the fastest form as long as no SIMD gets more than three of the
+// waves; with more LPs than that, shapes with G <= 16 and G * D <= 16 put four into each wave.
+// Measured at (8, 2), one per wave / four per wave: 1024 LPs 7.4 / 10.9 us, 2048 8.8 / 10.9, 3072 10.8 / 11.0,
+// 4096 12.9 / 11.3, 16384 39 / 24.
+constexpr int kPackFrom = 3 * 1024 + 1;
 constexpr int kLdsLimit = 64 * 1024 - 2048;
 
 template <int GM, int DM, bool EXACT, int ROWS, int EPL = 1>
@@ -122,7 +122,7 @@ extern "C" int lplb_solve_batched(const int32_t *workloads, float *global_worklo
   a.workload = workloads; a.gw_out = global_workloads; a.r2o = r2o; a.phy2log = phy2log;
   a.avail = avail_num; a.result = results; a.n_group = n_group; a.G = group_size;
   a.D = dup_per_rank; a.C = n_experts_per_var; a.n_fixed = n_experts_fixed;
-  a.n_experts = (int)n_experts; a.step_rule = step_rule; a.n_steps = n_steps; a.tagged_result = nullptr; a.tag_valid = 0; a.tagged_copies = 0; a.tagged_stride = 0; a.counts_ready = nullptr;
+  a.n_experts = (int)n_experts; a.step_rule = step_rule; a.n_steps = n_steps;
 #ifdef LPLB_PHASE_CLOCKS
   a.clocks = g_phase_clocks;
 #else

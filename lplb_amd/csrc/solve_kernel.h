@@ -49,13 +49,13 @@ struct SolveArgs {
   float *result;             // [n_inst][n_group][G][D]
   int n_group, G, D, C, n_fixed, n_experts, step_rule, n_steps, n_units;
   int staged_stride;   // floats of LDS per LP for its counts, 0 = read them from global memory
-  const int *counts_ready;   // or null.  LDS flag: once it is non-zero the caller has put the counts of this
-                             // wave's LP into staged_counts (as floats) and a.workload is not read
-  int counts_wait_polls;     // how many times to look at that flag before giving up on it
+  bool counts_by_caller;   // a.workload is not read: the caller puts the counts into staged_counts (as floats) before its
+                           // `counts_have_come` returns
   unsigned long long *tagged_result;  // or null: a copy of a.result for other workgroups of the same launch,
   uint32_t tag_valid;                 // each value written through to memory as (tag_valid << 32) | its bits
   int tagged_copies, tagged_stride;   // ... tagged_copies times, tagged_stride words apart (the pollers spread over the copies)
                                       // (the caller writes tag_valid + 1 for "no result: use the neutral fallback")
+  float *shares_in_lds;      // or null: another copy of a.result, for the caller's workgroup
   long long *clocks;         // debug builds: wall-clock stamps of wave 0, lane 0 (else null)
 };
 
@@ -186,15 +186,17 @@ template <int ROWS, int W> __device__ inline float lp_max(float v) {
 }
 
 
-// Stores a share, and if asked also the copy other workgroups of the running kernel
-// poll: the high word says "valid, from this launch", so value and flag arrive in one 8-byte store.
-__device__ inline void store_share(float *p, unsigned long long *tagged, uint32_t tag, int copies, int stride,
-                                   int64_t i, float v) {
-  p[i] = v;
-  if (tagged)
-    for (int k = 0; k < copies; ++k)
-      __hip_atomic_store(tagged + (int64_t)k * stride + i, ((unsigned long long)tag << 32) | __builtin_bit_cast(uint32_t, v),
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Stores a share, and if asked also the copies other workgroups of the running kernel poll (the high word says
+// "valid, from this launch", so value and flag arrive in one 8-byte store) and the one in the caller's LDS.
+__device__ inline void store_share(const SolveArgs &a, int64_t i, float v) {
+  if (a.tagged_result)
+    for (int k = 0; k < a.tagged_copies; ++k)
+      __hip_atomic_store(a.tagged_result + (int64_t)k * a.tagged_stride + i,
+                         ((unsigned long long)a.tag_valid << 32) | __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  if (a.shares_in_lds)
+    a.shares_in_lds[i] = v;
+  a.result[i] = v;
 }
 
 // With one LP per wave a lane's row of S is put together in LDS instead of registers: floats the
@@ -219,8 +221,7 @@ constexpr int assembly_tile_floats(int gm, int rows) { return rows == 1 ? gm * (
 //   pivot_rows     LDS, 2 * kWave doubles of this wave, 16-byte aligned
 //   tile           LDS, assembly_tile_floats(GM, ROWS) floats of this wave, 16-byte aligned
 // Returns how many of the wave's LPs passed the feasibility test (same value in
-// every lane); the caller adds it to a.avail.  -1: the counts the caller promised through
-// a.counts_ready never came; nothing was solved or stored.
+// every lane); the caller adds it to a.avail.
 template <int GM, int DM, bool EXACT, int ROWS, int EPL = 1>
 __device__ inline int solve_lp(const SolveArgs &a, int first_unit, float *staged_counts_of_wave,
                                int *rep_of_edge, double *pivot_rows, float *tile) {
@@ -302,45 +303,20 @@ __device__ inline int solve_lp(const SolveArgs &a, int first_unit, float *staged
     r2o_row[d] = k < 0 ? 0 : (k >= G ? G - 1 : k);
   }
   // (d) the counts: the maximum over all experts of all groups, minilp.cu:181-189, and
-  // (e) this group's counts, for the normalised-count output at the end.  A caller
-  // that is still producing the counts hands them over in LDS; the table loads
-  // above are on their way meanwhile.
-  const bool prestaged = a.counts_ready != nullptr;
+  // (e) this group's counts, for the normalised-count output at the end
   float wmax = 0.0f;
   float out_cnt[KG];
-  if (prestaged) {
-    // 1 = the counts are staged, 2 = the caller gave up on them; the wait itself is bounded
-    // as well, so that this wave ends whatever happens to the flag.
-    int ready = 0;
-    for (int polls = 0; polls < a.counts_wait_polls; ++polls) {
-      ready = __hip_atomic_load(a.counts_ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (ready != 0)
-        break;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    if (ready != 1)
-      return -1;   // nothing has been written
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    for (int i = lane; i < a.n_experts; i += WL)
-      wmax = fmaxf(wmax, staged_counts[i]);
-#pragma unroll
-    for (int u = 0; u < KG; ++u) {
-      const int i = lane + u * WL;
-      out_cnt[u] = (a.gw_out && i < G * L) ? staged_counts[grp * G * L + i] : 0.0f;
-    }
-  } else {
 #pragma unroll KG
-    for (int i = lane; i < a.n_experts; i += WL) {
-      const float cnt = (float)wl[i];
-      wmax = fmaxf(wmax, cnt);
-      if (staged)
-        staged_counts[i] = cnt;
-    }
+  for (int i = lane; i < a.n_experts; i += WL) {
+    const float cnt = (float)wl[i];
+    wmax = fmaxf(wmax, cnt);
+    if (staged)
+      staged_counts[i] = cnt;
+  }
 #pragma unroll
-    for (int u = 0; u < KG; ++u) {
-      const int i = lane + u * WL;
-      out_cnt[u] = (a.gw_out && i < G * L) ? (float)wl[grp * G * L + i] : 0.0f;
-    }
+  for (int u = 0; u < KG; ++u) {
+    const int i = lane + u * WL;
+    out_cnt[u] = (a.gw_out && i < G * L) ? (float)wl[grp * G * L + i] : 0.0f;
   }
   __builtin_amdgcn_wave_barrier();   // staged counts are visible to the whole wave
   float w_first[EPL];
@@ -746,8 +722,7 @@ __device__ inline int solve_lp(const SolveArgs &a, int first_unit, float *staged
 #pragma unroll
   for (int p = 0; p < EPL; ++p)
     if (is_edge[p] && unit_on)
-      store_share(a.result, a.tagged_result, a.tag_valid, a.tagged_copies, a.tagged_stride,
-                  (int64_t)unit * n + lane + p * kWave, ok ? xo[p] : 0.5f);
+      a.result[(int64_t)unit * n + lane + p * kWave] = ok ? xo[p] : 0.5f;
   // Normalised counts of this group, for the caller.
   if (a.gw_out && unit_on) {
     float *gw = a.gw_out + (int64_t)inst * a.n_experts + grp * G * L;

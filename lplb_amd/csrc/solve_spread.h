@@ -108,9 +108,11 @@ __device__ inline double step_length(double d_max) {
 // Arguments, LDS contracts and the returned value as for solve_lp; pivot_rows has spread_pivot_doubles(GM)
 // doubles, tile spread_tile_floats(GM, DM) floats, both 16-byte aligned; rep_of_edge kWave ints, or twice
 // that if GM * DM > kWave.
-template <int GM, int DM, bool EXACT>
+// counts_have_come: called once the wave's table loads have been issued if a.counts_by_caller; returns when the
+// counts are in staged_counts (true), or when they will not come: then -1 is returned, nothing solved or stored.
+template <int GM, int DM, bool EXACT, typename Counts>
 __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *staged_counts, int *rep_of_edge,
-                                      double *pivot_rows, float *tile) {
+                                      double *pivot_rows, float *tile, Counts counts_have_come) {
   static_assert(spread_shape(GM, DM) && (GM == 8 || GM == 16 || GM == 32), "a lane holds GM * GM / 64 entries of S");
   constexpr int TS = kWave / GM, KC = GM / TS;
   constexpr int NE = 2 * DM, E = NE > TS ? NE / TS : 1;
@@ -126,7 +128,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
   const int32_t *__restrict__ wl = a.workload + (int64_t)inst * a.n_experts;
   const int32_t *__restrict__ p2l = a.phy2log + (int64_t)grp * G * P;
   const bool is_rank = EXACT || rank < G;
-  const bool staged = a.staged_stride > 0;
+  const bool staged = a.staged_stride > 0 || a.counts_by_caller;
   auto count_of = [&](int e) -> float {
     if (e < 0 || e >= a.n_experts)
       return 0.0f;
@@ -157,20 +159,11 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
     const int j = sub + u * TS;
     fixed_e[u] = (is_rank && j < n_fixed) ? p2l[rank * P + D * C + j] : -1;
   }
-  const bool prestaged = a.counts_ready != nullptr;
   float wmax = 0.0f;
   float out_cnt[KG];
-  if (prestaged) {
-    int ready = 0;
-    for (int polls = 0; polls < a.counts_wait_polls; ++polls) {
-      ready = __hip_atomic_load(a.counts_ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (ready != 0)
-        break;
-      __builtin_amdgcn_s_sleep(1);
-    }
-    if (ready != 1)
-      return -1;   // nothing has been written
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  if (a.counts_by_caller) {
+    if (!counts_have_come())
+      return -1;
     for (int i = lane; i < a.n_experts; i += kWave)
       wmax = fmaxf(wmax, staged_counts[i]);
 #pragma unroll
@@ -583,8 +576,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
 #pragma unroll
   for (int p = 0; p < E; ++p)
     if (on[p] && !is_copy && (NE >= TS || sub < NE))
-      store_share(a.result, a.tagged_result, a.tag_valid, a.tagged_copies, a.tagged_stride,
-                  (int64_t)unit * n + edge[p], ok ? xo[p] : 0.5f);
+      store_share(a, (int64_t)unit * n + edge[p], ok ? xo[p] : 0.5f);
   // Normalised counts of this group, for the caller.
   if (a.gw_out) {
     float *gw = a.gw_out + (int64_t)inst * a.n_experts + grp * G * L;
@@ -609,11 +601,11 @@ template <int GM, int DM, int ROWS = 1, int EPL = 1> constexpr int lp_pivot_doub
 template <int GM, int DM, int ROWS = 1, int EPL = 1> constexpr int lp_tile_floats() {
   return takes_spread_form<GM, DM, ROWS, EPL>() ? spread_tile_floats(GM, DM) : assembly_tile_floats(GM, ROWS);
 }
-template <int GM, int DM, bool EXACT, int ROWS, int EPL>
+template <int GM, int DM, bool EXACT, int ROWS, int EPL, typename Counts>
 __device__ inline int solve_lps(const SolveArgs &a, int first_unit, float *staged_counts, int *rep_of_edge,
-                                double *pivot_rows, float *tile) {
+                                double *pivot_rows, float *tile, Counts counts_have_come) {
   if constexpr (takes_spread_form<GM, DM, ROWS, EPL>())
-    return solve_lp_spread<GM, DM, EXACT>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile);
+    return solve_lp_spread<GM, DM, EXACT>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile, counts_have_come);
   else
     return solve_lp<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile);
 }

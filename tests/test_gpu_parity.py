@@ -939,6 +939,23 @@ def test_plan_one_launch_with_many_groups(cuda, name, use_global):
     np.testing.assert_array_equal(got[0], want)
 
 
+@pytest.mark.parametrize("groups", [1, 8, 9])
+@pytest.mark.parametrize("n,n_sms", [
+    # one workgroup, at the edges of its forms: 2, 4, 8 chunks per wave beside one LP (896, 1792) and beside eight (128, 256)
+    (1, 256), (63, 256), (128, 256), (129, 256), (257, 256), (896, 256), (897, 256), (1793, 256), (4096, 256),
+    # slices: the first size past that, one slice only, full slices of 1024 ... 8192 and one index more, 256 of them
+    (4097, 256), (8192, 1), (8191, 2), (64 * 1024, 64), (64 * 1024 + 1, 64), (9 * 2048 + 1, 9), (3 * 4096 + 1, 3), (256 * 1024, 256)])
+def test_plan_one_launch_at_the_edges_of_its_forms(cuda, groups, n, n_sms):
+    """One workgroup for the whole batch, and slices of every length, against the chain."""
+    cfg = synth.PlanConfig("edges", topology.CUBE_8P2E, 8 * groups, 64 * groups, 2, max(n, 8), 1, 1.0, seed=groups)
+    inp = synth.make_inputs(cfg, mask_fraction=0.02)
+    inp.indices = np.ascontiguousarray(inp.indices.reshape(-1)[:n])
+    # (the ranking tables of slices longer than 2048 indices with over 100 replicated sets do not fit a CU)
+    one_launch = True if groups == 1 or n <= 2048 * n_sms else None
+    for use_global in (False, True):
+        _one_launch_equals_chain(cuda, inp, use_global, n_sms, expect_one_launch=one_launch)
+
+
 def _one_launch_equals_chain(cuda, inp, use_global, n_sms, expect_one_launch=None):
     """Runs the plan as the chain, then twice in the default mode; everything must agree bit for bit.
     expect_one_launch=True additionally requires that the default mode really ran as one kernel launch
