@@ -28,7 +28,8 @@ static std::atomic<int> g_fault_extra_slices{0}, g_fault_max_polls{0};
 struct PlanSlot {
   hipStream_t stream = nullptr;
   int seq = 0;                  // number of the slot's latest launch outside a capture (what it writes when all
-                                // of its workgroups have arrived)
+                                // of its workgroups have arrived); a captured launch carries the number of the one before it
+  int slices = 0, lps = 0;      // of that launch: whose done words the next stream has to see (0: nothing to wait for)
   float cost = 0.0f;            // share of the GPU's resident workgroups its launches take
   bool used = false, captured = false;
   bool maybe_executing = false; // a launch was enqueued and has not been seen to have arrived since
@@ -84,9 +85,35 @@ static bool slot_is_executing(PlanDevice &d, int i) {
   return s.maybe_executing;
 }
 
+// The first thing that a stream runs in a block it has taken over: the launch of the stream before has arrived, but
+// some of its slices may still have to read their shares.  Its workgroups are resident and wait for nothing else, so
+// this ends; should it not, the block is switched off as after any wait that ran out.  (A replay of a captured
+// takeover finds the words at this number or a later one.)
+__global__ void wait_for_last_user(int *sync, int slices, int lps, int seq, int max_polls) {
+  const int i = threadIdx.x;
+  bool done = i >= slices + lps || agent_load(sync + kPoisonAt) != 0;   // (a block that is off is not read)
+  const auto reached = [seq](int number) { return ((number - seq) & 0x3fffffff) <= 0x1fffffff; };
+  for (int polls = 0; polls < max_polls && !done; ++polls) {
+    if (i == 0) {   // its last stores have landed, too
+      const unsigned long long advanced = agent_load(reinterpret_cast<const unsigned long long *>(sync + kAdvancedAt));
+      const int gen = (int)(uint32_t)advanced;
+      done = reached((int)(advanced >> 32)) && agent_load(sync + kGenAt) == gen &&
+             agent_load(reinterpret_cast<const unsigned long long *>(sync + kAvailAt) + (gen & 1)) == 0;
+    } else {
+      done = reached(agent_load(sync + kDoneAt + (i < slices ? i : kMaxSlices + i - slices)));
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  if (!done) {
+    agent_add(sync + kTimeoutsAt, 1);
+    agent_store(sync + kPoisonAt, 1);
+  }
+}
+
 // Admission of one launch that takes `cost` of the GPU's resident workgroups on stream s.
-// Returns the slot, or -1: run the chain.
-static int admit_launch(PlanDevice &d, hipStream_t s, float cost, bool capturing) {
+// Returns the slot, or -1: run the chain.  *taken_over: it was another stream's, whose last launch has arrived but
+// perhaps not ended.
+static int admit_launch(PlanDevice &d, hipStream_t s, float cost, bool capturing, bool *taken_over) {
   int slot = -1;
   for (int i = 0; i < kSyncSlots && slot < 0; ++i)
     if (d.slots[i].used && d.slots[i].stream == s)
@@ -106,6 +133,7 @@ static int admit_launch(PlanDevice &d, hipStream_t s, float cost, bool capturing
   if (executing + cost > kResidencyBudget)
     return -1;
   PlanSlot &ps = d.slots[slot];
+  *taken_over = ps.used && ps.stream != s && ps.slices > 0;
   if (!ps.used || ps.stream != s) {
     ps.stream = s;
     ps.cost = 0.0f;
@@ -165,11 +193,17 @@ int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_ot
     capturing = capture == hipStreamCaptureStatusActive;
     const float cost = (float)n_workgroups / (float)(fit * d->n_cus);
     lock.lock();   // held over the launch: admission and launch order agree
-    const int slot = admit_launch(*d, s, cost, capturing);
+    bool taken_over = false;
+    const int slot = admit_launch(*d, s, cost, capturing, &taken_over);
     if (slot < 0)
       return LPLB_OK;
     ps = &d->slots[slot];
     a.sync = d->sync + (size_t)slot * kSlotInts;
+    if (taken_over) {
+      hipLaunchKernelGGL(wait_for_last_user, dim3(1), dim3(kMaxSlices + kMaxLps), 0, s, a.sync, ps->slices, ps->lps, ps->seq,
+                         kDefaultMaxPolls);
+      LPLB_HIP_TRY(hipGetLastError());
+    }
     a.solve.tagged_result = reinterpret_cast<unsigned long long *>(a.sync + kSharesAt);
     a.solve.tagged_copies = a.n_share_copies;
     a.solve.tagged_stride = kMaxShares;
@@ -177,11 +211,8 @@ int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_ot
     const int fault_polls = g_fault_max_polls.exchange(0);
     a.max_polls = fault_polls > 0 ? fault_polls : kDefaultMaxPolls;
     // (a captured launch keeps its share of the GPU for good and reports nothing)
-    if (!capturing) {
-      ps->seq = (ps->seq + 1) & 0x3fffffff;
-      a.arrived_word = d->arrived + slot;
-      a.arrived_seq = ps->seq;
-    }
+    a.seq = capturing ? ps->seq : (ps->seq + 1) & 0x3fffffff;
+    a.arrived_word = capturing ? nullptr : d->arrived + slot;
   }
   launch(kernel, dim3(n_workgroups), dim3(kPlanThreads), lds, s, a);
   const hipError_t err = hipGetLastError();
@@ -189,6 +220,11 @@ int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_ot
     return fail(LPLB_EHIP, "plan: launch failed: %s", hipGetErrorString(err));
   if (ps)
     ps->maybe_executing = !capturing;
+  if (ps && !capturing) {
+    ps->seq = a.seq;
+    ps->slices = a.n_slices;
+    ps->lps = a.solve.n_units;
+  }
   g_one_launch_plans.fetch_add(1, std::memory_order_relaxed);
   *done = true;
   return LPLB_OK;
@@ -285,6 +321,7 @@ extern "C" int lplb_plan_forget_captured(lplb_stream_t stream) {
       // back to a slot whose stream has nothing pending: it may serve this stream again or pass to another
       ps.captured = ps.maybe_executing = false;
       ps.cost = 0.0f;
+      ps.slices = ps.lps = 0;
     }
   }
   return LPLB_OK;
@@ -316,8 +353,10 @@ extern "C" int lplb_plan_sync_timeouts(int *count) {
   LPLB_HIP_TRY(hipDeviceSynchronize());
   {
     std::lock_guard<std::mutex> lock(g_plan_guard);   // nothing enqueued so far is still running
-    for (int slot = 0; slot < kSyncSlots; ++slot)
+    for (int slot = 0; slot < kSyncSlots; ++slot) {
       d->slots[slot].maybe_executing = false;
+      d->slots[slot].slices = d->slots[slot].lps = 0;
+    }
   }
   return LPLB_OK;
 }

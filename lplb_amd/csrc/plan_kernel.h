@@ -71,15 +71,21 @@ template <int GM, int DM> constexpr size_t plan_lp_area_bytes() {
 //   memory, so slice s polls copy s % copies;
 //   from kSetRowsAt: per slice set_words words with its tokens of the replicated sets, two sets per word;
 //   from kHistRowsAt: per slice hist_words words with its histogram, two experts per word;
-//   from kTotalsAt: one word per expert with the batch's tokens.
-constexpr int kGenAt = 0, kPoisonAt = 1, kTimeoutsAt = 4, kAvailAt = 10;
+//   from kTotalsAt: one word per expert with the batch's tokens;
+//   from kDoneAt: per slice and, behind them, per LP the number (PlanArgs::seq) of the last launch in which it has
+//   read all it reads of this block (the first slice's number is in the high half of [kAdvancedAt], with what
+//   it has set [kGenAt] to in the low half): before the block passes to another stream, whose launches the
+//   device does not order behind this one, wait_for_last_user waits for these.
+constexpr int kGenAt = 0, kPoisonAt = 1, kTimeoutsAt = 4, kAdvancedAt = 6, kAvailAt = 10;
 constexpr unsigned long long kGaveUp = 1ull << 32;
 constexpr int kMaxSlices = 256, kMaxPlanExperts = 1024, kMaxShares = 1024, kShareCopies = 8;
 constexpr int kSharesAt = 16, kMaxSetWords = kMaxPlanExperts / 2, kMaxHistWords = kMaxPlanExperts / 2;
 constexpr int kSetRowsAt = kSharesAt + 2 * kMaxShares * kShareCopies;
 constexpr int kHistRowsAt = kSetRowsAt + 2 * kMaxSlices * kMaxSetWords;
 constexpr int kTotalsAt = kHistRowsAt + 2 * kMaxSlices * kMaxHistWords;
-constexpr int kSlotInts = kTotalsAt + 2 * kMaxPlanExperts, kSyncSlots = 8;
+constexpr int kMaxLps = kLpsPerWorkgroup * kMaxLpWorkgroups;
+constexpr int kDoneAt = kTotalsAt + 2 * kMaxPlanExperts;
+constexpr int kSlotInts = kDoneAt + kMaxSlices + (kMaxLps + 15) / 16 * 16, kSyncSlots = 8;
 static_assert(kSetRowsAt % 16 == 0 && kHistRowsAt % 16 == 0 && kTotalsAt % 16 == 0 && kSlotInts % 16 == 0, "rows start on 64-byte lines");
 
 struct PlanArgs {
@@ -103,8 +109,8 @@ struct PlanArgs {
   SolveArgs solve;   // result = the shares (o_weight); workload is replaced by the batch's own counts if local_counts
   int local_counts;
   int *sync;
-  int *arrived_word;   // pinned host memory, or null: receives arrived_seq once every workgroup of the launch has arrived
-  int arrived_seq;
+  int *arrived_word;   // pinned host memory, or null: receives seq once every workgroup of the launch has arrived
+  int seq;             // number of the launch among those of its block
 };
 
 // plan.hip: admission and launch of one kernel (see there).  lds: dynamic LDS of the launch.
@@ -574,6 +580,8 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
         if (!(before & kGaveUp))
           atomicAdd(a.avail, n_ok);
       }
+      if (lane == 0)
+        agent_store(a.sync + kDoneAt + kMaxSlices + first_lp + wave_s, a.seq);
     } else if (a.local_counts) {
       counts_have_come();
     }
@@ -640,9 +648,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
       t.hist[i] = 0;
     __syncthreads();
     mine_came = add_up_rows(a, hist_rows + first_word, a.hist_words, words, a.adder_words, tag, slice, t.hist, nullptr, tid, lane);
+    if (!mine_came)
+      missing[0] = 1;
     __syncthreads();
     unsigned long long *totals = reinterpret_cast<unsigned long long *>(a.sync + kTotalsAt);
-    if (mine_came)   // (a wave whose words did not come gives the batch up below)
+    if (missing[0] == 0)   // (every wave's words are in the sums; if not, the batch is given up below)
       for (int i = tid; i < 2 * words; i += kPlanThreads)
         if (2 * first_word + i < nl)
           agent_store(totals + 2 * first_word + i, tagged_word(tag, (uint32_t)t.hist[i]));
@@ -701,15 +711,21 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     __syncthreads();
     LPLB_PLAN_STAMP(5);
     ok = missing[1] == 0;
-    if (slice == 0 && tid == 0) {
+    // (By a whole wave: the same word from every lane is one store, and the branch leaves all lanes active.  With the
+    // tokens of 16 chunks live a branch of one lane is not safe here: this compiler has placed the move of a chunk's
+    // register inside it, where the other lanes lose it.)
+    if (slice == 0 && wave_s == 0) {
       // Every slice's counts and every LP's shares carry this launch's tag, so every workgroup has read it: the
       // next launch takes the next one.  From here on no workgroup waits for one that is not resident yet: tell
       // the host, which then stops counting this launch against what the GPU can hold at once (a posted write
       // to host memory).
       agent_store(a.sync + kGenAt, (gen + 1) & 0x3fffffff);
       agent_store(reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (1 - (gen & 1)), 0ull);
+      agent_store(reinterpret_cast<unsigned long long *>(a.sync + kAdvancedAt), tagged_word((uint32_t)a.seq, (gen + 1) & 0x3fffffff));
       if (a.arrived_word)
-        __hip_atomic_store(a.arrived_word, a.arrived_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(a.arrived_word, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    } else if (wave_s == 0) {
+      agent_store(a.sync + kDoneAt + slice, a.seq);
     }
   }
   LPLB_PLAN_STAMP(6);

@@ -939,6 +939,18 @@ def test_plan_one_launch_with_many_groups(cuda, name, use_global):
     np.testing.assert_array_equal(got[0], want)
 
 
+@pytest.mark.parametrize("group,slots", [(8, 1), (8, 2), (8, 4), (7, 2), (16, 1), (16, 2), (13, 2), (32, 1), (32, 2), (29, 2)])
+@pytest.mark.parametrize("n", [2 * 8192 - 3, 3 * 4096 + 1])
+def test_plan_one_launch_longest_slices_of_every_group_size(cuda, group, slots, n):
+    """Slices of 8192 and 6144 indices hold 16 chunks per lane in registers, the form with the least room there:
+    every variant of it against the chain."""
+    r2o = np.stack([(np.arange(group) + 1 + 2 * d) % group for d in range(slots)], axis=1).astype(np.int32)
+    cfg = synth.PlanConfig("longest", r2o, group, 8 * group, slots, n, 1, 1.0, seed=group)
+    inp = synth.make_inputs(cfg, mask_fraction=0.02)
+    for use_global in (False, True):
+        _one_launch_equals_chain(cuda, inp, use_global, 2, expect_one_launch=None if slots > 2 or group > 16 else True)
+
+
 @pytest.mark.parametrize("groups", [1, 8, 9])
 @pytest.mark.parametrize("n,n_sms", [
     # one workgroup, at the edges of its forms: 2, 4, 8 chunks per wave beside one LP (896, 1792) and beside eight (128, 256)
