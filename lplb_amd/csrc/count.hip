@@ -10,7 +10,11 @@
 // (Doing the scan inside the first kernel, by the last workgroup to finish, was
 // measured and rejected: one CU sustains too few outstanding misses to pull the
 // 256 KB table, 20 us against 3 us for this kernel.)
-// HBM-bound: 8 bytes read per index; the [n_blocks, n_experts] table is small.
+// HBM-bound: 8 bytes read per index; the [n_blocks, n_experts] table is small.  The indices are read with ordinary
+// loads because the redirect reads them again: with non-temporal ones, as the redirect's own last read is, that second
+// read came from HBM ([1048576 x 8], 67 MB, whole plan as four kernels: 48.7 us, with ordinary loads 44.7; with the next
+// batch of loads under way while one is counted 44.2; walking a slice backwards, so that its beginning is the
+// part read last, gains nothing).
 // Callers that need only the totals of a short batch get them in one launch: slice_histogram with
 // TOTALS (slices add their counts to one vector) or expert_totals (every workgroup owns four experts).
 #include "common.h"
@@ -57,13 +61,25 @@ __global__ __launch_bounds__(1024) void slice_histogram(
   const int64_t n_pairs = (end - begin - head) >> 1;
   typedef long long i64x2 __attribute__((ext_vector_type(2)));
   const i64x2 *pairs = reinterpret_cast<const i64x2 *>(idx + begin + head);
-  // the first batch of loads is on its way while the histogram is cleared
-  i64x2 first[kLoadsInFlight];
+  // the first batch of loads is on its way while the histogram is cleared, every later one while the batch before it
+  // is counted
+  auto load_batch = [&](i64x2 (&v)[kLoadsInFlight], int64_t i0) {
 #pragma unroll
-  for (int u = 0; u < kLoadsInFlight; ++u) {
-    const int64_t i = tid + (int64_t)u * nt;
-    first[u] = i < n_pairs ? __builtin_nontemporal_load(pairs + i) : i64x2{-1, -1};
-  }
+    for (int u = 0; u < kLoadsInFlight; ++u) {
+      const int64_t i = i0 + tid + (int64_t)u * nt;
+      v[u] = i < n_pairs ? pairs[i] : i64x2{-1, -1};
+    }
+  };
+  auto count_batch = [&](const i64x2 (&v)[kLoadsInFlight]) {
+#pragma unroll
+    for (int u = 0; u < kLoadsInFlight; ++u) {
+      count(v[u].x);
+      count(v[u].y);
+    }
+  };
+  const int64_t batch = (int64_t)nt * kLoadsInFlight;
+  i64x2 even[kLoadsInFlight], odd[kLoadsInFlight];
+  load_batch(even, 0);
   for (int e = tid; e < COPIES * stride; e += nt)
     hist[e] = 0;
   if constexpr (TOTALS)
@@ -71,23 +87,13 @@ __global__ __launch_bounds__(1024) void slice_histogram(
       for (int64_t e = (int64_t)p * nt + tid; e < n_experts; e += (int64_t)gridDim.x * nt)
         clear[e] = 0;
   __syncthreads();
-#pragma unroll
-  for (int u = 0; u < kLoadsInFlight; ++u) {
-    count(first[u].x);
-    count(first[u].y);
-  }
-  for (int64_t i0 = tid + (int64_t)nt * kLoadsInFlight; i0 < n_pairs; i0 += (int64_t)nt * kLoadsInFlight) {
-    i64x2 v[kLoadsInFlight];
-#pragma unroll
-    for (int u = 0; u < kLoadsInFlight; ++u) {
-      const int64_t i = i0 + (int64_t)u * nt;
-      v[u] = i < n_pairs ? __builtin_nontemporal_load(pairs + i) : i64x2{-1, -1};
-    }
-#pragma unroll
-    for (int u = 0; u < kLoadsInFlight; ++u) {
-      count(v[u].x);
-      count(v[u].y);
-    }
+  for (int64_t i0 = 0; i0 < n_pairs; i0 += 2 * batch) {
+    load_batch(odd, i0 + batch);
+    count_batch(even);
+    if (i0 + batch >= n_pairs)
+      break;
+    load_batch(even, i0 + 2 * batch);
+    count_batch(odd);
   }
   if (tid == 0 && head)
     count(idx[begin]);
