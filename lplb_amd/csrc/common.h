@@ -79,6 +79,8 @@ inline void launch(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t
 }
 
 // count.hip: histogram + scan; any_order lets it overlap the kernel enqueued just before it.
+int enqueue_histogram(const int64_t *idx, int64_t n_elements, int n_experts, int n_blocks, int32_t *counts_by_block,
+                      int32_t *no_totals, hipStream_t s);
 int enqueue_count(const int64_t *idx, int64_t n_elements, int n_experts, int n_blocks,
                   int32_t *counts_by_block, hipStream_t s, bool any_order);
 

@@ -17,7 +17,7 @@
 // part read last, gains nothing).
 // Callers that need only the totals of a short batch get them in one launch: slice_histogram with
 // TOTALS (slices add their counts to one vector) or expert_totals (every workgroup owns four experts).
-#include "common.h"
+#include "scan.h"
 
 namespace lplb {
 
@@ -35,8 +35,9 @@ __host__ __device__ constexpr int histogram_stride(int n_experts, int copies) {
 }
 
 // TOTALS: instead of writing its row, a slice adds its counts to the one vector `counts` [n_experts]
-// (device-wide atomic adds, none for an expert the slice has no token of), and the launch sets the
-// vector `clear` (if given) to zero -- a caller that takes two vectors in turn never has to zero one.
+// (device-wide atomic adds, none for an expert the slice has no token of).  The launch sets the vector `clear` [n_experts]
+// (if given) to zero -- a caller that takes two vectors in turn never has to zero one --, or without TOTALS to kNoTotal,
+// for scan_and_solve.
 template <int COPIES, bool TOTALS>
 __global__ __launch_bounds__(1024) void slice_histogram(
     const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per,
@@ -82,10 +83,9 @@ __global__ __launch_bounds__(1024) void slice_histogram(
   load_batch(even, 0);
   for (int e = tid; e < COPIES * stride; e += nt)
     hist[e] = 0;
-  if constexpr (TOTALS)
-    if (clear)
-      for (int64_t e = (int64_t)p * nt + tid; e < n_experts; e += (int64_t)gridDim.x * nt)
-        clear[e] = 0;
+  if (clear)
+    for (int64_t e = (int64_t)p * nt + tid; e < n_experts; e += (int64_t)gridDim.x * nt)
+      clear[e] = TOTALS ? 0 : kNoTotal;
   __syncthreads();
   for (int64_t i0 = 0; i0 < n_pairs; i0 += 2 * batch) {
     load_batch(odd, i0 + batch);
@@ -155,54 +155,10 @@ static int launch_slice_histogram(const int64_t *idx, int64_t n_elements, int n_
   return LPLB_OK;
 }
 
-constexpr int kScanBands = 16;      // bands of rows, one per group of kScanCols lanes
-constexpr int kScanRows = 16;       // rows of a band a thread keeps in registers
-constexpr int kScanCols = 16;       // experts per workgroup: many small workgroups pull the
-                                    // table through many CUs (one CU sustains few misses)
-
-// counts[p][e] <- sum_{p' <= p} counts[p'][e].  A workgroup owns kScanCols experts;
-// thread = (band of rows, expert).  All loads of a band are in flight at once
-// (clamped addresses, masked values); band sums meet in LDS; tables with more than
-// 256 slices take several sweeps with a running carry.
-__global__ __launch_bounds__(kScanBands *kScanCols) void prefix_over_slices(
-    int32_t *__restrict__ counts, int n_blocks, int n_experts) {
-  __shared__ int32_t part[kScanBands][kScanCols];
-  __shared__ int32_t carry[kScanCols];
+__global__ __launch_bounds__(kScanThreads) void prefix_over_slices(int32_t *__restrict__ counts, int n_blocks, int n_experts) {
+  __shared__ ScanLds lds;
   fetch_arguments_now(counts, n_blocks, n_experts);
-  const int col = threadIdx.x % kScanCols, band = threadIdx.x / kScanCols;
-  const int e = blockIdx.x * kScanCols + col;
-  const bool live = e < n_experts;
-  int32_t *column = counts + (live ? e : 0);
-  if (band == 0)
-    carry[col] = 0;
-  __syncthreads();
-  for (int row0 = 0; row0 < n_blocks; row0 += kScanBands * kScanRows) {
-    const int r0 = row0 + band * kScanRows;
-    int32_t v[kScanRows];
-#pragma unroll
-    for (int k = 0; k < kScanRows; ++k)
-      v[k] = column[(int64_t)min(r0 + k, n_blocks - 1) * n_experts];
-#pragma unroll
-    for (int k = 0; k < kScanRows; ++k)
-      v[k] = (live && r0 + k < n_blocks) ? v[k] : 0;
-#pragma unroll
-    for (int k = 1; k < kScanRows; ++k)
-      v[k] += v[k - 1];
-    part[band][col] = v[kScanRows - 1];
-    __syncthreads();
-    int32_t offset = carry[col];
-#pragma unroll
-    for (int b = 0; b < kScanBands; ++b)
-      offset += b < band ? part[b][col] : 0;
-#pragma unroll
-    for (int k = 0; k < kScanRows; ++k)
-      if (live && r0 + k < n_blocks)
-        column[(int64_t)(r0 + k) * n_experts] = v[k] + offset;
-    __syncthreads();
-    if (band == kScanBands - 1)
-      carry[col] = offset + v[kScanRows - 1];
-    __syncthreads();
-  }
+  scan_columns(counts, n_blocks, n_experts, blockIdx.x, lds, [](int, int32_t) {});
 }
 
 // ---- totals only, for short batches: one launch, nothing shared between workgroups ----
@@ -278,6 +234,11 @@ __global__ __launch_bounds__(1024) void expert_totals(const int64_t *__restrict_
   }
 }
 
+// Enqueues the histogram alone: rows of counts that are not summed over the slices yet, and kNoTotal into no_totals.
+int enqueue_histogram(const int64_t *idx, int64_t n_elements, int n_experts, int n_blocks, int32_t *counts_by_block,
+                      int32_t *no_totals, hipStream_t s) {
+  return launch_slice_histogram<false>(idx, n_elements, n_experts, n_blocks, counts_by_block, no_totals, s, 0u);
+}
 // Enqueues histogram and prefix.  any_order: the histogram launch does not wait for
 // the kernel enqueued just before it on the stream (it still starts after everything
 // that kernel waited for); the prefix launch is ordered after both.
@@ -287,7 +248,7 @@ int enqueue_count(const int64_t *idx, int64_t n_elements, int n_experts, int n_b
                                                any_order ? hipExtAnyOrderLaunch : 0u);
   if (rc != LPLB_OK)
     return rc;
-  launch(prefix_over_slices, dim3((n_experts + kScanCols - 1) / kScanCols), dim3(kScanBands * kScanCols), 0, s,
+  launch(prefix_over_slices, dim3((n_experts + kScanCols - 1) / kScanCols), dim3(kScanThreads), 0, s,
          counts_by_block, n_blocks, n_experts);
   LPLB_HIP_TRY(hipGetLastError());
   return LPLB_OK;

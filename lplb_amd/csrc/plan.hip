@@ -230,6 +230,9 @@ int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_ot
   return LPLB_OK;
 }
 
+// LP shapes that are built here: (8, 1) (8, 2) (8, 4) (16, 1) (16, 2) (32, 1) (32, 2) and what pads into them
+static bool lp_shape_is_built(int G, int D) { return G <= 8 ? D <= 4 : G <= 32 && D <= 2; }
+
 // Tries the one-launch plan.  *done = false: shape or size outside what it covers, or no
 // room on the GPU right now; nothing was enqueued.
 static int try_one_launch(const int64_t *idx, int64_t n_elements, const int32_t *counts, const int32_t *r2o,
@@ -242,9 +245,7 @@ static int try_one_launch(const int64_t *idx, int64_t n_elements, const int32_t 
   const int n_logical = n_group * G * L, n_rep = n_group * G * C * D;
   if (!g_cooperative || n_elements <= 0 || n_rep == 0)
     return LPLB_OK;
-  // LP shapes that are built: (8, 1) (8, 2) (8, 4) (16, 1) (16, 2) (32, 1) (32, 2) and what pads into them
-  const bool lp_shape = G <= 8 ? D <= 4 : G <= 32 && D <= 2;
-  if (!lp_shape || n_group > kLpsPerWorkgroup * kMaxLpWorkgroups || n_group * G * D > kMaxShares || global_workload == nullptr ||
+  if (!lp_shape_is_built(G, D) || n_group > kLpsPerWorkgroup * kMaxLpWorkgroups || n_group * G * D > kMaxShares || global_workload == nullptr ||
       n_logical > kMaxPlanExperts || n_group * G * P >= 65536)
     return LPLB_OK;
   PlanArgs a{};   // every field the host does not set below is zero
@@ -443,6 +444,24 @@ static int plan_checked(const int64_t *idx, int64_t n_elements, const int32_t *g
     if (rc != LPLB_OK)
       return rc;
     rc = enqueue_count(idx, n_elements, n_logical, n_blocks, counts_by_block, s, /*any_order=*/true);
+    if (rc != LPLB_OK)
+      return rc;
+  } else if (g_cooperative && lp_shape_is_built(group_size, dup_per_rank) && n_group <= kScanSolveLps &&
+             n_logical <= kMaxPlanExperts && n_elements > 0 && global_workload != nullptr) {
+    ScanSolveArgs a{};
+    a.counts = counts_by_block;
+    a.totals = reinterpret_cast<int32_t *>(global_workload);
+    a.n_blocks = n_blocks;
+    a.max_polls = kDefaultMaxPolls;
+    SolveArgs &sa = a.solve;
+    sa.gw_out = global_workload; sa.r2o = r2o; sa.phy2log = phy2log; sa.avail = avail_num; sa.result = o_weight;
+    sa.n_group = sa.n_units = n_group; sa.G = group_size; sa.D = dup_per_rank; sa.C = n_combined_experts;
+    sa.n_fixed = n_fixed; sa.n_experts = n_logical; sa.step_rule = step_rule; sa.n_steps = n_steps;
+    sa.counts_by_caller = true;
+    rc = enqueue_histogram(idx, n_elements, n_logical, n_blocks, counts_by_block, a.totals, s);
+    if (rc != LPLB_OK)
+      return rc;
+    rc = group_size <= 8 ? scan_and_solve_up_to_8(a, s) : group_size <= 16 ? scan_and_solve_up_to_16(a, s) : scan_and_solve_up_to_32(a, s);
     if (rc != LPLB_OK)
       return rc;
   } else {

@@ -11,4 +11,8 @@ int launch_plan_up_to_32(PlanArgs &a, hipStream_t s, bool *done) {
   return LPLB_OK;
 }
 
+int scan_and_solve_up_to_32(const ScanSolveArgs &a, hipStream_t s) {
+  return a.solve.D <= 1 ? launch_scan_and_solve<32, 1>(a, s) : launch_scan_and_solve<32, 2>(a, s);
+}
+
 } // namespace lplb

@@ -13,4 +13,8 @@ int launch_plan_up_to_8(PlanArgs &a, hipStream_t s, bool *done) {
   return LPLB_OK;
 }
 
+int scan_and_solve_up_to_8(const ScanSolveArgs &a, hipStream_t s) {
+  return a.solve.D <= 1 ? launch_scan_and_solve<8, 1>(a, s) : a.solve.D <= 2 ? launch_scan_and_solve<8, 2>(a, s) : launch_scan_and_solve<8, 4>(a, s);
+}
+
 } // namespace lplb

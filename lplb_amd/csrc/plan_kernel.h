@@ -38,6 +38,7 @@
 #pragma once
 #include "map_kernel.h"
 #include "plan_sync.h"
+#include "scan.h"
 #include "solve_spread.h"
 
 namespace lplb {
@@ -122,6 +123,10 @@ typedef void (*PlanKernel)(PlanArgs);
 int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_others, PlanArgs &a, size_t lds, hipStream_t s,
                 bool *done);
 // plan_8.hip, plan_16.hip, plan_32.hip: the variants for group sizes up to 8, 16, 32.
+struct ScanSolveArgs;
+int scan_and_solve_up_to_8(const ScanSolveArgs &a, hipStream_t s);
+int scan_and_solve_up_to_16(const ScanSolveArgs &a, hipStream_t s);
+int scan_and_solve_up_to_32(const ScanSolveArgs &a, hipStream_t s);
 int launch_plan_up_to_8(PlanArgs &a, hipStream_t s, bool *done);
 int launch_plan_up_to_16(PlanArgs &a, hipStream_t s, bool *done);
 int launch_plan_up_to_32(PlanArgs &a, hipStream_t s, bool *done);
@@ -838,7 +843,76 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   LPLB_PLAN_STAMP(7);
 }
 
+// ---- long batches that feed the LPs themselves: scan over the slices and LPs as one launch behind the histogram ----
+// The first workgroup solves up to four LPs; the others turn the histogram's rows into running sums, as
+// prefix_over_slices does, and hand every expert's total over in the vector that will hold the normalised counts
+// (kNoTotal until then: set by the histogram's launch, so nothing outlives the plan).  Against two launches the LP's
+// table loads and the second launch's start are off the path: [1048576 x 8] 44.2 -> 42.3 us for the whole
+// plan.  The waiting workgroup is one in a grid of a few, and those it waits for wait for nobody.
+struct ScanSolveArgs {
+  SolveArgs solve;
+  int32_t *counts;   // [n_blocks][n_experts]
+  int32_t *totals;   // the words of solve.gw_out
+  int n_blocks, max_polls;
+};
+constexpr int kScanSolveLps = kScanThreads / kWave;
+template <int GM, int DM, bool EXACT> __global__ __launch_bounds__(kScanThreads) void scan_and_solve(ScanSolveArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  __shared__ int rep_of_edge_all[kScanSolveLps * kWave];
+  __shared__ int missing;
+  __shared__ ScanLds scan_lds;
+  const int nl = a.solve.n_experts;
+  if (blockIdx.x > 0) {
+    scan_columns(a.counts, a.n_blocks, nl, blockIdx.x - 1, scan_lds, [&](int e, int32_t sum) { agent_store(a.totals + e, sum); });
+    return;
+  }
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
+  constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
+  float *staged = reinterpret_cast<float *>(smem_raw + a.solve.n_units * kLpArea);
+  if (tid == 0)
+    missing = 0;
+  __syncthreads();
+  auto counts_have_come = [&]() -> bool {
+    for (int e = tid; e < nl; e += kScanThreads) {
+      int32_t sum = kNoTotal;
+      for (int polls = 0; polls < a.max_polls && (sum = agent_load(a.totals + e)) == kNoTotal; ++polls)
+        __builtin_amdgcn_s_sleep(1);
+      if (sum == kNoTotal)
+        missing = 1;
+      staged[e] = (float)sum;
+    }
+    __syncthreads();   // (from here on the totals may be overwritten by the normalised counts)
+    return missing == 0;
+  };
+  if (wave_s >= a.solve.n_units) {
+    counts_have_come();
+    return;
+  }
+  unsigned char *area = smem_raw + wave_s * kLpArea;
+  const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(a.solve, wave_s, staged, rep_of_edge_all + wave_s * kWave,
+                                                  reinterpret_cast<double *>(area),
+                                                  reinterpret_cast<float *>(area + lp_pivot_doubles<GM, DM>() * sizeof(double)),
+                                                  counts_have_come);
+  if (n_ok > 0 && lane == 0)
+    atomicAdd(a.solve.avail, n_ok);
+  if (n_ok < 0)   // (the wait ran out: the shares of an LP without a solution)
+    for (int j = lane; j < a.solve.G * a.solve.D; j += kWave)
+      a.solve.result[wave_s * a.solve.G * a.solve.D + j] = 0.5f;
+}
+
 // ---- host side: which variant ----
+template <int GM, int DM> static int launch_scan_and_solve(const ScanSolveArgs &a, hipStream_t s) {
+  const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + a.solve.n_experts * sizeof(float);
+  static_assert(kScanSolveLps * plan_lp_area_bytes<GM, DM>() + kMaxPlanExperts * sizeof(float) <= 60 * 1024, "LDS of a kernel without asking for more");
+  const dim3 grid(1 + (a.solve.n_experts + kScanCols - 1) / kScanCols), block(kScanThreads);
+  if (a.solve.G == GM && a.solve.D == DM)
+    launch(scan_and_solve<GM, DM, true>, grid, block, lds, s, a);
+  else
+    launch(scan_and_solve<GM, DM, false>, grid, block, lds, s, a);
+  LPLB_HIP_TRY(hipGetLastError());
+  return LPLB_OK;
+}
 template <int GM, int DM, bool EXACT, int K>
 static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   const size_t lds_slice = plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);

@@ -939,6 +939,19 @@ def test_plan_one_launch_with_many_groups(cuda, name, use_global):
     np.testing.assert_array_equal(got[0], want)
 
 
+@pytest.mark.parametrize("group,slots,groups,n,n_sms", [
+    (*shape, 8192 * n_sms + 1, n_sms) for n_sms in (1, 3, 17)
+    for shape in [(8, 1, 1), (8, 2, 4), (8, 2, 5), (8, 4, 1), (7, 2, 3), (16, 1, 2), (16, 2, 1), (13, 2, 4), (32, 1, 1),
+                  (32, 2, 4), (29, 2, 1)]] + [(8, 2, 4, 256 * 8192 + 1, 300)])
+def test_plan_of_a_long_batch_scans_and_solves_in_one_launch(cuda, group, slots, groups, n, n_sms):
+    """Batches past what one launch covers, fed by their own counts: scan and LPs as one launch (up to four groups)
+    against the chain; tables of less and of more than the 256 rows of one sweep, odd numbers of experts."""
+    r2o = np.stack([(np.arange(group) + 1 + 2 * d) % group for d in range(slots)], axis=1).astype(np.int32)
+    cfg = synth.PlanConfig("long", r2o, group * groups, 7 * group * groups, slots, n, 1, 1.0, seed=group)
+    inp = synth.make_inputs(cfg, mask_fraction=0.02)
+    _one_launch_equals_chain(cuda, inp, False, n_sms, expect_one_launch=False)
+
+
 @pytest.mark.parametrize("group,slots", [(8, 1), (8, 2), (8, 4), (7, 2), (16, 1), (16, 2), (13, 2), (32, 1), (32, 2), (29, 2)])
 @pytest.mark.parametrize("n", [2 * 8192 - 3, 3 * 4096 + 1])
 def test_plan_one_launch_longest_slices_of_every_group_size(cuda, group, slots, n):
