@@ -397,7 +397,8 @@ int lplb_build_mapping(const float *weight, const double *history, const int32_t
  * No counterpart in the reference.  enabled = 0 makes lplb_plan always run the
  * chain of kernels (for callers that replay captured plans concurrently on
  * several streams, that let four or more plans execute at once, or that keep the
- * GPU full of kernels which themselves wait for a plan); 1 (the default) lets it use the one-launch form where that applies.
+ * GPU full of kernels which themselves wait for a plan); 1 (the default) lets it use the one-launch form where that applies,
+ * and for longer batches that feed the LPs themselves one launch for the scan over the slices and the LPs.
  * Process-wide.
  */
 int lplb_plan_set_cooperative(int enabled);
