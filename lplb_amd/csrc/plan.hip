@@ -100,7 +100,7 @@ __global__ void wait_for_last_user(int *sync, int slices, int lps, int seq, int 
       done = reached((int)(advanced >> 32)) && agent_load(sync + kGenAt) == gen &&
              agent_load(reinterpret_cast<const unsigned long long *>(sync + kAvailAt) + (gen & 1)) == 0;
     } else {
-      done = reached(agent_load(sync + kDoneAt + (i < slices ? i : kMaxSlices + i - slices)));
+      done = reached(agent_load(sync + kDoneAt + (i < slices ? i : kMaxSlices + i - slices) * kDoneStride));
     }
     __builtin_amdgcn_s_sleep(1);
   }

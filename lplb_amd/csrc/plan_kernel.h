@@ -86,7 +86,8 @@ constexpr int kHistRowsAt = kSetRowsAt + 2 * kMaxSlices * kMaxSetWords;
 constexpr int kTotalsAt = kHistRowsAt + 2 * kMaxSlices * kMaxHistWords;
 constexpr int kMaxLps = kLpsPerWorkgroup * kMaxLpWorkgroups;
 constexpr int kDoneAt = kTotalsAt + 2 * kMaxPlanExperts;
-constexpr int kSlotInts = kDoneAt + kMaxSlices + (kMaxLps + 15) / 16 * 16, kSyncSlots = 8;
+constexpr int kDoneStride = 16;   // ints from word to word: stores to one 64-byte line queue up (16 in a line: plan [8192 x 8] 8.35 -> 8.6 us)
+constexpr int kSlotInts = kDoneAt + (kMaxSlices + kMaxLps) * kDoneStride, kSyncSlots = 8;
 static_assert(kSetRowsAt % 16 == 0 && kHistRowsAt % 16 == 0 && kTotalsAt % 16 == 0 && kSlotInts % 16 == 0, "rows start on 64-byte lines");
 
 struct PlanArgs {
@@ -586,7 +587,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
           atomicAdd(a.avail, n_ok);
       }
       if (lane == 0)
-        agent_store(a.sync + kDoneAt + kMaxSlices + first_lp + wave_s, a.seq);
+        agent_store(a.sync + kDoneAt + (kMaxSlices + first_lp + wave_s) * kDoneStride, a.seq);
     } else if (a.local_counts) {
       counts_have_come();
     }
@@ -730,7 +731,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
       if (a.arrived_word)
         __hip_atomic_store(a.arrived_word, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     } else if (wave_s == 0) {
-      agent_store(a.sync + kDoneAt + slice, a.seq);
+      agent_store(a.sync + kDoneAt + slice * kDoneStride, a.seq);
     }
   }
   LPLB_PLAN_STAMP(6);
