@@ -2,9 +2,9 @@
 // lanes.  Same problem, method and arithmetic as solve_kernel.h (read that first); what differs is who
 // holds what.
 //
-// A lone wave issues one instruction every 2.3 ns (3.5 ns if it needs the one before), whatever the
-// instruction does for how many lanes, so the time of an LP is the number of instructions on its path
-// and the round trips through LDS in it.
+// A lone wave issues one instruction every 2.3 ns (4.4 ns if it is an fp64 one that needs the one before), whatever the
+// instruction does for how many lanes, a reciprocal takes 9 ns, what goes through LDS 30 ns and 3 more for every further
+// read: the time of an LP is the number of instructions on its path and the round trips through LDS in it.
 // With one lane per rank and one lane per edge (solve_kernel.h) 48 or 56 of the 64 lanes idle, every
 // lane carries a whole row of S through assembly and elimination, and what goes from edges to ranks and
 // back goes through ten ds_bpermute per step.  Here
@@ -14,10 +14,12 @@
 //     copy it hosts ("edge ends": end e = 2 d is the rank's own edge in slot d, e = 2 d + 1 the edge
 //     copied into slot d; lane l holds ends l % TS + TS * p).  Every edge lives twice, at its two ends,
 //     with the same values computed twice; a rank's sums over its edges are DPP adds inside its lanes,
-//     and the only value that has to travel is the solution y of the other end's rank.
-// Measured per affine-scaling step (in-kernel clock; one lane per rank and edge before): (8, 2) 1.15 -> 0.70 us,
-// of which the elimination is 0.48 (a pivot is one round trip through LDS), assembly 0.15 and the rest 0.2;
-// (16, 2) 1.8 -> 1.3 us; (32, 2) 3.1 -> 2.9 us, nearly all of it elimination.
+//     and the only value that has to travel is the solution y of the other end's rank;
+//   * pivots are taken two at a time, so that there is one round trip through LDS and one reciprocal for two.
+// Measured per affine-scaling step, one wave on the GPU, pivots one by one -> two at a time (and sums without
+// wait states, moves folded into them, no sum over the edges between solution and step length):
+// (8, 2) 0.66 -> 0.52 us, of which the elimination is 0.26 (73 ns a pair); (16, 2) 1.21 -> 1.05; (32, 2) 2.87 -> 2.35,
+// bound by the number of instructions (212, 390 and 974 a step).  With one lane per rank and edge (8, 2) took 1.15 us.
 // (A form in which rank i is lane i of every 16-lane row and holds its whole row, the elimination made of
 // fp64 multiply-adds with a row_newbcast operand, has pivots of 40 instead of 60 ns and no LDS in them; but
 // getting the rows into that shape costs 0.25 us a step more than it gains at 8 ranks.)
@@ -29,45 +31,80 @@ namespace lplb {
 // Which instantiations take this form (one LP per wave, one edge per lane in the other form).
 constexpr bool spread_shape(int gm, int dm) { return gm <= 32 && gm * dm <= 128 && dm <= 8; }
 
-// LDS per wave: the pivot columns in flight (two buffers) and, except at 8 ranks with at most two slots,
-// the tile in which the rows of S are put together, followed by a copy of v.
-constexpr int spread_row_doubles = 9;   // 8 ranks: rows of S, padded so that a column is in distinct banks
-constexpr int spread_pivot_doubles(int gm) { return gm <= 8 ? 2 * 8 * spread_row_doubles : 2 * kWave; }
+// LDS per wave: what the elimination passes between lanes (8 ranks: the rows of S and the right-hand side, and the
+// constants of the pivot rows; else an area per pair of pivots, with the pairs of entries of all rows, zeros and, with four
+// lanes per rank, a place for those lanes that hold none, then the right-hand sides) and, except at 8 ranks with at most
+// two slots, the tile in which the rows of S are put together, followed by a copy of v.
+constexpr int kRow8 = 10;   // 8 ranks: doubles from row to row (pairs on 16-byte boundaries, a column's in distinct banks)
+constexpr int spread_part_doubles(int gm) { return 2 * (gm * gm / kWave) + 2; }   // the rows of equal number modulo TS (parts in distinct banks)
+constexpr int spread_pair_area(int gm) { return kWave / gm * spread_part_doubles(gm) + 4; }
+constexpr int spread_pivot_doubles(int gm) { return gm <= 8 ? 9 * kRow8 + 16 : gm / 2 * spread_pair_area(gm) + gm; }
 constexpr bool spread_uses_tile(int gm, int dm) { return gm > 8 || dm > 2; }
 constexpr int spread_tile_floats(int gm, int dm) { return spread_uses_tile(gm, dm) ? gm * (gm + 4) + 2 * gm : 4; }
 
 // v of the lane that CTRL names, for controls in which every lane has a source.
 template <int CTRL> __device__ inline float dpp_all(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+  // (zeros for lanes without a source, of which there are none, let the compiler fold the move into its user)
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 constexpr int kRowRor8 = 0x128;
 template <int LANE> __device__ inline float quad_bcast(float v) { return dpp_all<LANE * 0x55>(v); }
 
 // Sums and maxima across the four 16-lane rows (complete in the last row) and, for maxima, inside them.
 // Written out because the compiler splits a DPP operand with a row mask, or one of a maximum, into two to
-// four instructions.  (A DPP operand must be two wait states old.)
-#define LPLB_DPP(OP, CTRL, ROWS) "s_nop 1\n\t" OP "_dpp %0, %0, %0 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"
-#define LPLB_ROWS(OP) LPLB_DPP(OP, "row_bcast:15", "0xa") LPLB_DPP(OP, "row_bcast:31", "0xc")
+// four instructions, and does not fill the two wait states that a DPP operand needs with another sum's instructions.
+#define LPLB_DPP(OP, REG, CTRL, ROWS) OP "_dpp " REG ", " REG ", " REG " " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"
+#define LPLB_WAIT_DPP(OP, CTRL, ROWS) "s_nop 1\n\t" LPLB_DPP(OP, "%0", CTRL, ROWS)
+#define LPLB_ROWS(OP) LPLB_WAIT_DPP(OP, "row_bcast:15", "0xa") LPLB_WAIT_DPP(OP, "row_bcast:31", "0xc")
+#define LPLB_MAX(CTRL) LPLB_WAIT_DPP("v_max_f32", CTRL, "0xf")
+#define LPLB_MAX_ROWS LPLB_MAX("row_ror:8") LPLB_ROWS("v_max_f32")
 __device__ inline float rows_sum(float v) {
   asm(LPLB_ROWS("v_add_f32") : "+v"(v));
   return readlane(v, kWave - 1);
 }
-template <bool Q1, bool Q2, bool H> __device__ inline float wave_max_of_groups(float v) {
-  if (Q1) asm(LPLB_DPP("v_max_f32", "quad_perm:[1,0,3,2]", "0xf") : "+v"(v));
-  if (Q2) asm(LPLB_DPP("v_max_f32", "quad_perm:[2,3,0,1]", "0xf") : "+v"(v));
-  if (H) asm(LPLB_DPP("v_max_f32", "row_half_mirror", "0xf") : "+v"(v));
-  asm(LPLB_DPP("v_max_f32", "row_ror:8", "0xf") LPLB_ROWS("v_max_f32") : "+v"(v));
+__device__ inline void rows_sums(float &v, float &w) {
+  asm("s_nop 1\n\t" LPLB_DPP("v_add_f32", "%0", "row_bcast:15", "0xa") LPLB_DPP("v_add_f32", "%1", "row_bcast:15", "0xa")
+      "s_nop 0\n\t" LPLB_DPP("v_add_f32", "%0", "row_bcast:31", "0xc") LPLB_DPP("v_add_f32", "%1", "row_bcast:31", "0xc")
+      : "+v"(v), "+v"(w));
+  v = readlane(v, kWave - 1);
+  w = readlane(w, kWave - 1);
+}
+template <bool Q2, bool H> __device__ inline float wave_max_of_groups(float v) {
+  if constexpr (Q2 && H)
+    asm(LPLB_MAX("quad_perm:[1,0,3,2]") LPLB_MAX("quad_perm:[2,3,0,1]") LPLB_MAX("row_half_mirror") LPLB_MAX_ROWS : "+v"(v));
+  else if constexpr (Q2)
+    asm(LPLB_MAX("quad_perm:[1,0,3,2]") LPLB_MAX("quad_perm:[2,3,0,1]") LPLB_MAX_ROWS : "+v"(v));
+  else if constexpr (H)
+    asm(LPLB_MAX("quad_perm:[1,0,3,2]") LPLB_MAX("row_half_mirror") LPLB_MAX_ROWS : "+v"(v));
+  else
+    asm(LPLB_MAX("quad_perm:[1,0,3,2]") LPLB_MAX_ROWS : "+v"(v));
   return readlane(v, kWave - 1);
 }
+#undef LPLB_MAX_ROWS
+#undef LPLB_MAX
 #undef LPLB_ROWS
+#undef LPLB_WAIT_DPP
 #undef LPLB_DPP
 
+// %0 += SEL times %1 of lane N of every four
+#define LPLB_FMAC(SEL, N) "v_fmac_f32_dpp %0, %1, " SEL " quad_perm:[" #N "," #N "," #N "," #N "] row_mask:0xf bank_mask:0xf\n\t"
+// The value is formed here: a product is not contracted with an addition whose operand comes by DPP (two instructions then).
+__device__ inline float formed_here(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 // Over the ranks: v is the same in the TS lanes of each rank; the result is wave-uniform.
-template <int TS> __device__ inline float over_ranks_sum(float v) {
+template <int TS> __device__ inline float over_ranks_in_row(float v) {
   if (TS <= 2) v += dpp_all<kQuadSwap2>(v);
   if (TS <= 4) v += dpp_all<kHalfMirror>(v);
-  v += dpp_all<kRowRor8>(v);
-  return rows_sum(v);
+  return v + dpp_all<kRowRor8>(v);
+}
+template <int TS> __device__ inline float over_ranks_sum(float v) { return rows_sum(over_ranks_in_row<TS>(v)); }
+template <int TS> __device__ inline void over_ranks_sums(float &v, float &w) {
+  v = over_ranks_in_row<TS>(v);
+  w = over_ranks_in_row<TS>(w);
+  rows_sums(v, w);
 }
 // Over a rank's edge ends (NE of them, E per lane); every lane of the rank gets the result.
 template <int TS, int NE, int E> __device__ inline float over_ends_sum(const float (&v)[E]) {
@@ -81,26 +118,45 @@ template <int TS, int NE, int E> __device__ inline float over_ends_sum(const flo
 }
 // Maximum over the wave (a NaN operand is ignored); lanes that only repeat other lanes' edge ends are skipped.
 template <int TS, int NE> __device__ inline float over_all_max(float v) {
-  return wave_max_of_groups<true, (TS <= 2 || NE > 2), (TS <= 4 || NE > 4)>(v);
+  return wave_max_of_groups<(TS <= 2 || NE > 2), (TS <= 4 || NE > 4)>(v);
 }
 
-// `old` with the lanes of rank RANK replaced by those of v, which is the same in all lanes of a 16-lane row:
-// one instruction (DPP row_newbcast with row and bank masks; a bank is four lanes).  With two lanes per rank
-// the other rank of the bank is overwritten as well.
-template <int TS, int RANK> __device__ inline double set_rank(double old, double v) {
-  constexpr int row = RANK * TS / 16, bank = RANK * TS % 16 / 4, banks = TS == 8 ? 3 << bank : 1 << bank;
-  const long long o = __builtin_bit_cast(long long, old), w = __builtin_bit_cast(long long, v);
-  const long long r = __builtin_amdgcn_update_dpp(o, w, 0x150, 1 << row, banks, false);
-  return __builtin_bit_cast(double, r);
+// LDS by its own addresses (32 bits), so that an address can be chosen lane by lane with one move.
+typedef __attribute__((address_space(3))) double lds_double;
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f64x2 lds_f64x2;
+__device__ inline double2 lds_pair(const lds_double *base, int at) {
+  const f64x2 v = *reinterpret_cast<const lds_f64x2 *>(base + at);
+  return double2{v.x, v.y};
+}
+// v of the first of every eight lanes.
+__device__ inline float bcast_in_eight(float v) {
+  const int q = __builtin_bit_cast(int, quad_bcast<0>(v));
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(q, q, 0x114 /* row_shr:4 */, 0xF, 0xA, false));
+}
+constexpr int kIdentityPerm = 0xE4;   // quad_perm [0,1,2,3]
+// v with the 16-lane row ROW made zero, through its high word only (what is left of a number is a denormal below 2^-1022).
+template <int ROW> __device__ inline double clear_dpp_row(double v) {
+  int2 q = __builtin_bit_cast(int2, v);
+  q.y = __builtin_amdgcn_update_dpp(q.y, 0, kIdentityPerm, 1 << ROW, 0xF, false);
+  return __builtin_bit_cast(double, q);
+}
+// v of the other rank of the pair (2 p, 2 p + 1); v is the same in the TS lanes of each rank.
+template <int TS> __device__ inline double rank_partner(double v) {
+  constexpr int ctrl = TS == 2 ? kQuadSwap2 : kHalfMirror;
+  int2 q = __builtin_bit_cast(int2, v);
+  q.x = __builtin_amdgcn_mov_dpp(q.x, ctrl, 0xF, 0xF, false);
+  q.y = __builtin_amdgcn_mov_dpp(q.y, ctrl, 0xF, 0xF, false);
+  return __builtin_bit_cast(double, q);
 }
 
-// 0.999 / d_max in fp64, rounded to fp32 by the caller: estimate, Newton step, one correction of the
-// quotient (error below one fp64 ulp; the compiler's full division takes twice the instructions, all of
+// 0.999 / d_max in fp64, rounded to fp32 by the caller: quotient by the estimated reciprocal and one correction of it
+// (error about 2^-46, far below the rounding to fp32; the compiler's full division takes four times the instructions, all of
 // them in the chain from one step to the next).  d_max = 0 or infinite gives NaN where the division gives
 // infinity or 0: either way the step leaves the artificial variable without a number below the
 // feasibility limit, so the LP is reported infeasible and its shares are the neutral ones.
 __device__ inline double step_length(double d_max) {
-  const double r = rcp_f64(d_max);
+  const double r = __builtin_amdgcn_rcp(d_max);
   const double q = 0.999 * r;
   return __builtin_fma(__builtin_fma(-d_max, q, 0.999), r, q);
 }
@@ -297,7 +353,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
   float d_max = 0.0f;
   const int NV = 2 * n + G + 2;
   const int win_lo = a.step_rule == LPLB_STEP_REFERENCE_WINDOW ? (NV > 32 ? NV - 32 : 0) : 0;
-  const bool with_zero = a.step_rule != LPLB_STEP_REFERENCE_WINDOW || NV < 32;
+  const float at_least = a.step_rule != LPLB_STEP_REFERENCE_WINDOW || NV < 32 ? 0.0f : __builtin_nanf("");
   bool win_o[E], win_r[E];
 #pragma unroll
   for (int p = 0; p < E; ++p) {
@@ -306,6 +362,44 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
     win_r[p] = on[p] && n + edge[p] >= win_lo;
   }
   const bool win_s = is_rank && 2 * n + rank >= win_lo;
+
+  // ---- where the elimination's entries are in LDS ----
+  lds_double *const pivot_at = (lds_double *)pivot_rows;
+  constexpr int kPartDoubles = spread_part_doubles(GM), kPairArea = spread_pair_area(GM);
+  lds_double *my_rhs, *my_entry = nullptr, *put_pair[2] = {};
+  const lds_double *row_of_pair[GM / 2] = {};   // where a lane finds its row's entries in the pivot columns
+  const lds_double *my_column = nullptr;                         // 8 ranks
+  const lds_double *my_part = nullptr, *all_rhs = nullptr;   // 16 and 32
+  const lds_double *my_diagonal = nullptr, *partners_diagonal = nullptr, *my_off_diagonal = nullptr;
+  if constexpr (KC == 1) {
+    my_entry = pivot_at + rank * kRow8 + sub;
+    my_rhs = pivot_at + 8 * kRow8 + rank;
+    my_column = pivot_at + (sub == 0 ? 8 : sub) * kRow8;
+    lds_double *constants = pivot_at + 9 * kRow8;   // (-1, 0) four times, (0, -1) four times
+    if (lane < 16)
+      constants[lane] = lane % 2 == lane / 8 ? -1.0 : 0.0;
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      row_of_pair[p] = rank / 2 == p ? constants + rank % 2 * 8 : pivot_at + rank * kRow8;
+  } else {
+    const int at = (rank % TS) * kPartDoubles + rank / TS * 2;
+    constexpr int zeros = TS * kPartDoubles, nowhere = zeros + 2;
+    put_pair[0] = pivot_at + (sub < 2 ? at + sub : nowhere);
+    put_pair[1] = pivot_at + (sub < 2 ? nowhere : at + sub - 2);
+#pragma unroll
+    for (int p = 0; p < GM / 2; ++p)
+      row_of_pair[p] = pivot_at + (rank / 2 == p ? zeros : at);
+    my_part = pivot_at + sub * kPartDoubles;
+    all_rhs = pivot_at + GM / 2 * kPairArea;
+    my_rhs = pivot_at + GM / 2 * kPairArea + rank;
+    if (lane < GM)
+      pivot_at[lane / 2 * kPairArea + zeros + lane % 2] = 0.0;
+    const lds_double *area = pivot_at + rank / 2 * kPairArea;
+    const int partner = rank ^ 1;
+    my_diagonal = area + at + rank % 2;
+    my_off_diagonal = area + at + 1 - rank % 2;
+    partners_diagonal = area + (partner % TS) * kPartDoubles + partner / TS * 2 + partner % 2;
+  }
 
   for (int step = 0; step < a.n_steps; ++step) {
     const float ss = xs * xs, st = xt * xt, sM = xM * xM;
@@ -317,44 +411,34 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
       u[p] = on[p] ? __builtin_amdgcn_rcpf(so[p] + sr[p]) : 0.0f;
       const float wu = w[p] * u[p];
       const float ao = wu * so[p], ar = wu * sr[p];
-      lam[p] = w_lap[p] * ao * sr[p];            // w^2 so sr / (so + sr)
+      lam[p] = formed_here(w_lap[p] * ao * sr[p]);   // w^2 so sr / (so + sr)
       mine[p] = is_copy ? ar : ao;               // what the edge adds to q of this end's rank
       u_own[p] = is_copy ? 0.0f : u[p];          // every edge once
     }
-    const float sigma = over_ranks_sum<TS>(over_ends_sum<TS, NE, E>(u_own));
-    const float kappa = sM * __builtin_amdgcn_rcpf(1.0f + sM * sigma);
-    const float v = is_rank ? m + over_ends_sum<TS, NE, E>(mine) : 0.0f;
-    // the Laplacian's diagonal, added up slot by slot
-    float lam_sum = ss;
-    if constexpr (TS >= 4 && NE == 4) {
-      const float pair = lam[0] + dpp_all<kQuadSwap1>(lam[0]);
-      lam_sum += quad_bcast<0>(pair);
-      lam_sum += quad_bcast<2>(pair);
-    } else if constexpr (TS == 2 || NE == 2) {
-#pragma unroll
-      for (int p = 0; p < E; ++p)
-        lam_sum += lam[p] + dpp_all<kQuadSwap1>(lam[p]);
-    } else {
-      lam_sum += over_ends_sum<TS, NE, E>(lam);
+    const float sum_mine = over_ends_sum<TS, NE, E>(mine), sum_u = over_ends_sum<TS, NE, E>(u_own);
+    const float v = is_rank ? m + sum_mine : 0.0f;
+    float v_col = 0.0f;
+    if constexpr (!kTile) {
+      v_col = bpermute(v, sub * TS);
+      __builtin_amdgcn_sched_barrier(0);   // (on its way while the sum over the edges is formed)
     }
+    const float sigma = over_ranks_sum<TS>(sum_u);
+    const float kappa = sM * __builtin_amdgcn_rcpf(1.0f + sM * sigma);
+    // the Laplacian's diagonal
+    const float lam_sum = ss + over_ends_sum<TS, NE, E>(lam);
 
     if (step == 0) LPLB_STAMP(5);
     double S[KC];
-    const double dst = (double)st, dkv = (double)kappa * (double)v;
+    const double dst = (double)st, dk = (double)kappa, dv = (double)v, dkv = dk * dv;
     if constexpr (!kTile) {
-      const float v_col = bpermute(v, sub * TS);
       float t = diagonal ? lam_sum : 0.0f;
-      if constexpr (DM == 2) {
-        t = __builtin_fmaf(sel[0], quad_bcast<0>(lam[0]), t);
-        t = __builtin_fmaf(sel[2], quad_bcast<2>(lam[0]), t);
-        t = __builtin_fmaf(sel[1], quad_bcast<1>(lam[0]), t);
-        t = __builtin_fmaf(sel[3], quad_bcast<3>(lam[0]), t);
-      } else {
-        t = __builtin_fmaf(sel[0], quad_bcast<0>(lam[0]), t);
-        t = __builtin_fmaf(sel[1], quad_bcast<1>(lam[0]), t);
-      }
+      if constexpr (DM == 2)
+        asm("s_nop 1\n\t" LPLB_FMAC("%2", 0) LPLB_FMAC("%4", 2) LPLB_FMAC("%3", 1) LPLB_FMAC("%5", 3)
+            : "+v"(t) : "v"(lam[0]), "v"(sel[0]), "v"(sel[1]), "v"(sel[2]), "v"(sel[3]));
+      else
+        asm("s_nop 1\n\t" LPLB_FMAC("%2", 0) LPLB_FMAC("%3", 1) : "+v"(t) : "v"(lam[0]), "v"(sel[0]), "v"(sel[1]));
       const double base = (EXACT || (rank < G && sub < G)) ? dst : 0.0;
-      S[0] = __builtin_fma(dkv, (double)v_col, base) + (double)t;
+      S[0] = __builtin_fma(dk, dv * (double)v_col, base + (double)t);
     } else {
       // (LDS float adds without a return value, to my own rank's row; the row was cleared when it was
       // last read)
@@ -388,146 +472,133 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
       __builtin_amdgcn_wave_barrier();
       clear_my_tile();
     }
-    double rhs = (EXACT || rank < G) ? 1000.0 * dkv - dst : 0.0;
+    double rhs = (EXACT || rank < G) ? __builtin_fma(dk, 1000.0 * dv, -dst) : 0.0;
 
     if (step == 0) LPLB_STAMP(6);
-    // Gauss-Jordan elimination of [S | rhs] by columns, as in solve_kernel.h: the pivot's entry is
-    // cleared as soon as it has been read as the pivot (so the multiple of the pivot row itself is zero),
-    // column c + 1 goes through LDS right after its first update, and the next reciprocal is worked out
-    // while that is on its way.  The right-hand side is kept by every lane of a rank.
+    // Gauss-Jordan elimination of [S | rhs], two pivots at a time.  Columns c and c + 1 of the rows that are left go
+    // through LDS once; from there every lane has its row's entries in them (the multiples before division by the pivot
+    // block), the two pivot rows' entries above its own columns (by symmetry those columns' entries of the row of that
+    // number), the pivot block [a b; b d] and the pivot rows' right-hand sides.  With e = entries * adj(block) the row's
+    // multiples are e / det: e needs no reciprocal, so the chain from pair to pair is update -> LDS -> det -> reciprocal ->
+    // multiply -> two updates, once for two pivots.  Lanes also update columns left of the pivots that share a register
+    // index with live ones; nothing reads those again.  The right-hand side is kept by every lane of a rank.
     float y;
+    struct Multiples {
+      double e0, e1, rinv;
+    };
+    auto multiples = [](const double2 &in_row, const double2 &ab, double d) {
+      Multiples m;
+      m.rinv = rcp_f64(__builtin_fma(ab.x, d, -(ab.y * ab.y)));
+      m.e0 = __builtin_fma(in_row.x, d, -(in_row.y * ab.y));
+      m.e1 = __builtin_fma(in_row.y, ab.x, -(in_row.x * ab.y));
+      return m;
+    };
     if constexpr (KC == 1) {
-      // One entry per lane: both the multiple f of the lane's row (entry (rank, c)) and the pivot row's
-      // entry above the lane's column (entry (sub, c), by symmetry) come from column c in LDS, from
-      // rows 9 doubles apart.  The chain from pivot to pivot is update -> LDS -> multiply -> update; the
-      // next reciprocal is worked out meanwhile, and is set to zero in the pivot's own row.
-      double *put = pivot_rows + rank * spread_row_doubles + sub;
-      const double *get_row = pivot_rows + rank * spread_row_doubles, *get_col = pivot_rows + sub * spread_row_doubles;
-      constexpr int kBuffer = 8 * spread_row_doubles;
-      double rinv_of_row = 1.0, rinv = 0.0;
-      static_for<GM>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        constexpr int at = (c % 2) * kBuffer + c;
-        put[(c % 2) * kBuffer] = S[0];
+      // One entry per lane.  The pivot rows themselves are replaced by the rows divided by the block: as if they were
+      // zero and had the entries (-1, 0) and (0, -1), which their lanes read from constants instead.  Column 0 is not used
+      // any more once it has been published: its lanes go on with the right-hand side (row 8 in LDS).
+      static_for<GM / 2>([&](auto pc) {
+        constexpr int p = decltype(pc)::value, c = 2 * p;
+        *(p == 0 || sub > 0 ? my_entry : my_rhs) = S[0];
+        if constexpr (p == 0) {
+          *my_rhs = rhs;
+          S[0] = sub == 0 ? rhs : S[0];
+        }
         __builtin_amdgcn_wave_barrier();
-        const double in_row = get_row[at], in_col = get_col[at];
-        __builtin_amdgcn_sched_barrier(0);   // the reads stay here, ahead of their use
-        rinv = rcp_f64(readlane(S[0], c * TS + c));
-        rinv_of_row = set_rank<TS, c>(rinv_of_row, rinv);
-        const double f = in_row * set_rank<TS, c>(rinv, 0.0);
-        S[0] = __builtin_fma(-f, in_col, S[0]);
-        rhs = __builtin_fma(-f, readlane(rhs, c * TS), rhs);
+        __builtin_amdgcn_sched_barrier(0);
+        const double2 ab = lds_pair(pivot_at, c * kRow8 + c);
+        const double d = pivot_at[(c + 1) * kRow8 + c + 1];
+        __builtin_amdgcn_sched_barrier(0);   // the reads stay here, ahead of their use, those of the longest chain first
+        const double2 in_row = lds_pair(row_of_pair[p], c);
+        __builtin_amdgcn_sched_barrier(0);
+        const double2 above = lds_pair(my_column, c);
+        __builtin_amdgcn_sched_barrier(0);
+        S[0] = clear_dpp_row<p>(S[0]);
+        const Multiples m = multiples(in_row, ab, d);
+        S[0] = __builtin_fma(-__builtin_fma(m.e1, above.y, m.e0 * above.x), m.rinv, S[0]);
       });
-      y = (float)(rhs * rinv_of_row);
+      y = bcast_in_eight((float)S[0]);
     } else {
-      // Several entries per lane.  The TS lanes of row i all need f_i = S[i][c] / pivot: the lane that
-      // holds column c hands its entry round with one quad-permute DPP move per half.  That value is also
-      // what the row adds to the pivot row in LDS (S[c][i] = S[i][c]), stored part by part, so a lane
-      // reads the entries above its own columns, two per 16-byte read, from one of TS addresses.  A lane
-      // also updates columns left of the pivot that share a register index with live ones; nothing reads
-      // those again.
-      constexpr int kStride = KC + 2;                 // doubles between the parts of a pivot row (distinct banks)
-      constexpr int kPart = KC < 8 ? KC : 8;          // columns per batch of LDS reads
-      constexpr int kParts = KC / kPart;
-      static_assert(kParts <= 2 && TS * kStride <= kWave, "pivot rows are fetched in at most two batches");
-      const int publish_at = (rank % TS) * kStride + rank / TS;
-      const double *my_part = pivot_rows + sub * kStride;
-      auto share = [](auto jc, double val) {     // val of lane j of every group of TS lanes
-        constexpr int j = decltype(jc)::value;
-        constexpr int ctrl = TS == 4 ? j * 0x55 : (j == 0 ? 0xA0 : 0xF5);
-        int2 q = __builtin_bit_cast(int2, val);
-        q.x = __builtin_amdgcn_mov_dpp(q.x, ctrl, 0xF, 0xF, false);   // (every lane has a source: no old value)
-        q.y = __builtin_amdgcn_mov_dpp(q.y, ctrl, 0xF, 0xF, false);
-        return __builtin_bit_cast(double, q);
+      // Several entries per lane.  Every pair has an area of its own in LDS: the pairs of entries of all rows, part by
+      // part (rows of equal number modulo TS), so that a lane reads those above its own columns from one of TS addresses.
+      // The lanes of the pivot rows read zeros for their own row, which leaves it alone; what it takes to divide the
+      // right-hand side by the block at the end is still there then.  The next pair's columns are updated first and
+      // published, and the rest of the update runs while they are on their way.
+      double2 in_row[2], ab[2], r[2], above[2][KC];
+      double d[2];
+      auto publish = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        put_pair[TS == 2 ? 0 : p % 2][p * kPairArea] = S[2 * p / TS];
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);
       };
-      // columns [q * kPart, (q + 1) * kPart) of the pivot row in buffer `parity`, those from k_from on
-      auto load_part = [&](int parity, int q, int k_from, double (&buf)[kPart]) {
-        const double2 *src = reinterpret_cast<const double2 *>(my_part + parity * kWave + q * kPart);
+      auto fetch = [&](auto pc) {
+        constexpr int p = decltype(pc)::value, c = 2 * p, first_live = (c + 2) / TS;
+        auto area_of = [](int row) { return (row % TS) * kPartDoubles + row / TS * 2; };
+        ab[p % 2] = lds_pair(pivot_at, p * kPairArea + area_of(c));
+        d[p % 2] = pivot_at[p * kPairArea + area_of(c + 1) + 1];
+        __builtin_amdgcn_sched_barrier(0);   // the reads stay here, ahead of their use, those of the longest chain first
+        in_row[p % 2] = lds_pair(row_of_pair[p], p * kPairArea);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < kPart / 2; ++j)
-          if (q * kPart + 2 * j + 1 >= k_from) {
-            const double2 both = src[j];
-            buf[2 * j] = both.x;
-            buf[2 * j + 1] = both.y;
-          }
-        __builtin_amdgcn_sched_barrier(0);   // the reads stay here, ahead of their use
+        for (int k = first_live; k < KC; ++k)
+          above[p % 2][k] = lds_pair(my_part, p * kPairArea + 2 * k);
+        __builtin_amdgcn_sched_barrier(0);
       };
-      double head[2][kPart];
-      double rinv_even = 1.0, rinv_odd = 1.0;   // (four lanes per rank: one of them serves all ranks)
-      double rinv = rcp_f64(readlane(S[0], 0));
-      S[0] = lp_clear_lane<1, 0>(S[0], 0);
-      double col = share(std::integral_constant<int, 0>{}, S[0]);
-      pivot_rows[publish_at] = col;
-      __builtin_amdgcn_wave_barrier();
-      load_part(0, 0, 0, head[0]);
-      static_for<GM>([&](auto cc) {
-        constexpr int c = decltype(cc)::value;
-        constexpr int k1 = (c + 1) / TS;              // register of column c + 1, the first one still live
-        constexpr int q0 = k1 / kPart;
-        double body[kPart];
-        auto clear = [&](auto kc, double f) {
-          constexpr int k = decltype(kc)::value;
-          if constexpr (k < KC) {
-            if constexpr (k / kPart == q0)
-              S[k] = __builtin_fma(-f, head[c % 2][k % kPart], S[k]);
-            else
-              S[k] = __builtin_fma(-f, body[k % kPart], S[k]);
-          }
+      auto exchange_rhs = [&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        *my_rhs = rhs;
+        __builtin_amdgcn_wave_barrier();
+        r[p % 2] = lds_pair(all_rhs, 2 * p);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      publish(std::integral_constant<int, 0>{});
+      fetch(std::integral_constant<int, 0>{});
+      exchange_rhs(std::integral_constant<int, 0>{});
+      static_for<GM / 2>([&](auto pc) {
+        constexpr int p = decltype(pc)::value, first_live = (2 * p + 2) / TS;
+        const Multiples m = multiples(in_row[p % 2], ab[p % 2], d[p % 2]);
+        const double f0 = m.e0 * m.rinv, f1 = m.e1 * m.rinv;
+        auto update = [&](int k) {
+          S[k] = __builtin_fma(-f1, above[p % 2][k].y, __builtin_fma(-f0, above[p % 2][k].x, S[k]));
         };
-        if constexpr (TS == 2 && c % 2)
-          rinv_odd = set_rank<TS, c>(rinv_odd, rinv);
-        else
-          rinv_even = set_rank<TS, c>(rinv_even, rinv);
-        const double f = col * rinv;   // multiple of row c to subtract from my row (0 in row c)
-        double next_pivot = 1.0, estimate = 1.0, error = 0.0, next_col = 0.0;
-        if constexpr (q0 + 1 < kParts)
-          load_part(c % 2, q0 + 1, 0, body);
-        clear(std::integral_constant<int, k1>{}, f);
-        if constexpr (c + 1 < GM) {
-          constexpr int holder = (c + 1) * TS + (c + 1) % TS;   // lane with entry (c + 1, c + 1)
-          next_pivot = readlane(S[k1], holder);
-          estimate = __builtin_amdgcn_rcp(next_pivot);
-          S[k1] = lp_clear_lane<1, holder>(S[k1], 0);
-          next_col = share(std::integral_constant<int, (c + 1) % TS>{}, S[k1]);
-          pivot_rows[((c + 1) % 2) * kWave + publish_at] = next_col;
-          __builtin_amdgcn_wave_barrier();
-          constexpr int k1_next = (c + 2) / TS;
-          if constexpr (k1_next < KC)
-            load_part((c + 1) % 2, k1_next / kPart, k1_next, head[(c + 1) % 2]);
+        auto update_rhs = [&]() { rhs = __builtin_fma(-f1, r[p % 2].y, __builtin_fma(-f0, r[p % 2].x, rhs)); };
+        if constexpr (p + 1 < GM / 2) {
+          update(first_live);
+          publish(std::integral_constant<int, p + 1>{});
+          fetch(std::integral_constant<int, p + 1>{});
+          update_rhs();
+          exchange_rhs(std::integral_constant<int, p + 1>{});
+#pragma unroll
+          for (int k = first_live + 1; k < KC; ++k)
+            update(k);
+        } else {
+          update_rhs();
         }
-        rhs = __builtin_fma(-f, readlane(rhs, c * TS), rhs);
-        clear(std::integral_constant<int, k1 + 1>{}, f);
-        if constexpr (c + 1 < GM)
-          error = __builtin_fma(-next_pivot, estimate, 1.0);
-        clear(std::integral_constant<int, k1 + 2>{}, f);
-        clear(std::integral_constant<int, k1 + 3>{}, f);
-        if constexpr (c + 1 < GM) {
-          rinv = __builtin_fma(error, estimate, estimate);   // = rcp_f64(next_pivot)
-        }
-        static_for<(KC > k1 + 4 ? KC - k1 - 4 : 0)>([&](auto kk) {
-          clear(std::integral_constant<int, k1 + 4 + decltype(kk)::value>{}, f);
-        });
-        col = next_col;
       });
-      y = (float)(rhs * (TS == 2 && rank % 2 ? rinv_odd : rinv_even));
+      const double b = *my_off_diagonal, partner = *partners_diagonal;
+      const double rinv = rcp_f64(__builtin_fma(*my_diagonal, partner, -(b * b)));
+      y = (float)(__builtin_fma(partner, rhs, -(b * rank_partner<TS>(rhs))) * rinv);
     }
     y = is_rank ? y : 0.0f;
     if (step == 0) LPLB_STAMP(7);
 
     // r = A^T w and the direction d = x (c - r); the edge part of w is
-    // z = u (h + kappa (m.y - u.h - 1000)), h = -B^T y.
-    float yk[E], yrep[E], hp[E], uhp[E];
+    // z = u (h + kappa (m.y - u.h - 1000)), h = -B^T y; m.y - u.h = v.y, because q = B u.
+    float y_other[E];
+#pragma unroll
+    for (int p = 0; p < E; ++p)
+      y_other[p] = bpermute(y, other[p] * TS);
+    float sumy = y, vy = formed_here(v * y);
+    over_ranks_sums<TS>(vy, sumy);
+    float yk[E], yrep[E], hp[E];
 #pragma unroll
     for (int p = 0; p < E; ++p) {
-      const float y_other = bpermute(y, other[p] * TS);
-      yk[p] = is_copy ? y_other : y;
-      yrep[p] = is_copy ? y : y_other;
+      yk[p] = is_copy ? y_other[p] : y;
+      yrep[p] = is_copy ? y : y_other[p];
       hp[p] = -w[p] * (so[p] * yk[p] + sr[p] * yrep[p]);
-      uhp[p] = u_own[p] * hp[p];
     }
-    const float sumy = over_ranks_sum<TS>(y);
-    const float my_uh = over_ranks_sum<TS>(m * y - over_ends_sum<TS, NE, E>(uhp));   // m.y - u.h
-    const float from_M = my_uh - 1000.0f;
+    const float from_M = vy - 1000.0f;
     const float shift = kappa * from_M;
     const float d_s = -xs * y;
     const float d_t = xt * (1.0f + sumy);
@@ -544,9 +615,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
       cand = fmaxf(cand, win_o[p] ? d_o[p] : none);
       cand = fmaxf(cand, win_r[p] ? d_r[p] : none);
     }
-    d_max = over_all_max<TS, NE>(fmaxf(cand, fmaxf(d_t, d_M)));
-    if (with_zero)
-      d_max = fmaxf(d_max, 0.0f);
+    d_max = over_all_max<TS, NE>(fmaxf(cand, fmaxf(fmaxf(d_t, d_M), at_least)));
     const float alpha = (float)step_length((double)d_max);
 #pragma unroll
     for (int p = 0; p < E; ++p) {
@@ -610,4 +679,5 @@ __device__ inline int solve_lps(const SolveArgs &a, int first_unit, float *stage
     return solve_lp<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile);
 }
 
+#undef LPLB_FMAC
 } // namespace lplb
