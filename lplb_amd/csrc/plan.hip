@@ -245,6 +245,10 @@ static int try_one_launch(const int64_t *idx, int64_t n_elements, const int32_t 
   a.n_share_copies = 1;
   while (a.n_share_copies < kShareCopies && a.n_share_copies * 8 < a.n_slices)
     a.n_share_copies *= 2;
+  const int n = a.n_slices;
+  a.unit_lanes_log2 = n > 32 ? 2 : n > 16 ? 3 : n > 8 ? 4 : n > 4 ? 5 : 6;
+  a.unit_blocks = (n + kUnitSlices - 1) / kUnitSlices;
+  a.unit_block_bits = a.unit_blocks > 2 ? 2 : a.unit_blocks - 1;
   return launch_variant(a, s, done);
 }
 

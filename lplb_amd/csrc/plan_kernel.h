@@ -16,17 +16,20 @@
 // counter of arrivals between a slice's counts and their readers and no acknowledgement to wait for:
 // every word carries the launch's tag in its high half, and a launch overwrites the words of the launch before it
 // (which has ended; so nothing has to be cleared either).
-//   * A slice publishes its counts, two of 16 bits per word: those of the replicated sets for every other slice, the
-//     whole histogram for the slices that add up the batch's totals.
+//   * A slice publishes its counts, two of 16 bits per word, as soon as its tokens are in the histogram (one barrier): those of
+//     the replicated sets for every other slice, the whole histogram for the slices that add up the batch's totals.
 //   * The totals are added up by up to 64 of the slices, each for eight words of every slice's histogram, and
-//     published once more; the LP workgroups and the first slice collect those.  (One CU reads such words past the
-//     caches at 25 bytes per ns: collecting 64 whole rows takes an LP workgroup 2.8 us, 256 rows 8 us.  As atomic
+//     published once more; the LP workgroups and the first slice collect those.  (Whole rows of 64 slices would be 64 KiB for an
+//     LP workgroup, 1 us at the 68 bytes per ns that one CU reads past the caches with 16-byte loads.  As atomic
 //     adds to shared totals they run into the rate of the atomic units, about 5 per ns over the whole GPU: 1.6 us
 //     for 64 slices, 6.6 us for 256.)
-// Measured per call, own histogram, against rows read once a counter of arrivals said that everybody's were there:
-// [8192 x 8] 12.0 -> 11.6 us, [16384 x 8] at 32 ranks 25.3 -> 24.1, [262144 x 8] 22.8 -> 19.6.  What bounds it at
-// [8192 x 8]: 3.7 us until the last slice's counts are out (1.0 of them until the last workgroup has started), 2.6 us
-// until the LP has the totals, 4.6 us of LP, 0.9 us until the last index is stored.
+// A word takes 0.3-0.5 us from one CU to another; what the hops cost beyond that is the waves' own instructions, so whatever
+// the counts do not wait for (ordinals inside a slice, the LP's topology) is done while they are on their way.
+// Per call, own histogram, before / after the counts went out ahead of the ordinals, units of 16-byte loads instead of sums by
+// the whole workgroup, and one batch of arguments: [8192 x 8] 10.9 -> 10.2 us, [262144 x 8] 19.3 -> 17.7, counts supplied
+// [8192 x 8] 8.1 -> 7.7.  What bounds it at [8192 x 8]: 2.7 us until the last slice's counts are out (0.9 of them until the last
+// workgroup has started), 2.0 until the LP has the totals, 4.1 of LP, 0.9 until its shares are seen, 0.6 until the last index
+// is stored.
 // Words are written and read with agent-scope atomics (plan_sync.h).
 // The workgroups wait for each other, so the whole grid has to be resident: its size is bounded by what fits
 // the GPU, and the host admits a launch only while the plans still executing leave room for it.
@@ -56,6 +59,9 @@ constexpr int kLpsPerWorkgroup = 4, kMaxLpWorkgroups = 8;
 template <int GM, int DM> constexpr size_t plan_lp_area_bytes() {
   return lp_pivot_doubles<GM, DM>() * sizeof(double) + lp_tile_floats<GM, DM>() * sizeof(float);
 }
+
+// The counts an LP works on, in LDS, with the zeros behind them.
+constexpr size_t counts_bytes(int n_logical) { return (size_t)(n_logical / 4 * 4 + 8) * sizeof(int32_t); }
 
 // One block of these per stream that plans (kSyncSlots of them per device), offsets in ints:
 //   [kGenAt] launches that have used the block; (value + 1) tags what a launch publishes;
@@ -98,6 +104,7 @@ struct PlanArgs {
   int n_slices, n_lp_workgroups;
   int n_share_copies;    // copies of the LP's shares: a power of two, at most kShareCopies
   int set_words;         // words per slice for its counts of the replicated sets: a power of two >= 8
+  int unit_lanes_log2, unit_blocks, unit_block_bits;   // how what slices add up is cut into units: lanes of a slice, blocks of slices, bits that number those
   int hist_words;        // ... for its histogram: a multiple of 8 that holds n_logical counts
   int adders, adder_words;     // slices that add up the totals, for adder_words words (a power of two >= 8) of every histogram each
   int expected_slices;   // = n_slices unless a fault is injected
@@ -168,29 +175,28 @@ __device__ inline void give_up(const PlanArgs &a, unsigned long long *avail_stat
 constexpr int64_t kLongestSlice = 16 * kPlanThreads;   // 16 chunks per wave
 template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
   return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * rank_record_bytes_single(K) +
-         (size_t)(n_logical + 1) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
-         (size_t)(3 + kPlanWaves) * (n_rep + 1) * sizeof(int32_t) + 32;
+         (size_t)(n_logical + 2) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
+         (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t);
 }
 struct SliceTables {
   RepEntry *reps;           // [R + 1]
   unsigned char *records;   // [waves][R + 1][record bytes]
   Route *route;             // [n_logical + 1]
-  int32_t *set_expert;      // [R] the set's expert, -1: none
+  int32_t *set_expert;      // [R] the expert whose tokens the set has; n_logical (which has none): it has none
   int32_t *before, *total;  // [R] tokens of the set before this slice, in the whole batch
-  int32_t *wave_total;      // [waves][R] ... in the chunks of the waves before each wave (one pass)
-  int32_t *hist;            // [n_logical up to a multiple of 16, + 1] the slice's histogram; once that is published, what it adds up of the
-                            // batch's; in the first slice at last the whole of the batch's
+  int32_t *wave_total;      // [waves][R] ... in each wave
+  int32_t *hist;            // [more than n_logical, a multiple of 16] the slice's histogram, then zeros; in the first slice at last the batch's
 };
 template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, int nl, int R) {
   SliceTables t;
   t.reps = reinterpret_cast<RepEntry *>(lds);
   t.records = lds + (size_t)(R + 1) * sizeof(RepEntry);
   t.route = reinterpret_cast<Route *>(t.records + (size_t)kPlanWaves * (R + 1) * rank_record_bytes_single(K));
-  t.set_expert = reinterpret_cast<int32_t *>(t.route + nl + 1);
+  t.hist = reinterpret_cast<int32_t *>(t.route + ((nl + 2) & ~1));   // (16-byte aligned, as what lies before it is)
+  t.set_expert = t.hist + nl / 16 * 16 + 16;
   t.before = t.set_expert + R;
   t.total = t.before + R;
   t.wave_total = t.total + R;
-  t.hist = t.wave_total + kPlanWaves * R;
   return t;
 }
 
@@ -229,14 +235,15 @@ __device__ inline PlanTableLoads issue_plan_table_loads(const PlanArgs &a, int t
   return t;
 }
 // Where an expert's tokens go when nothing is redirected and which replicated set (if any) it belongs to
-// (minilp.cu:466-496); everything else empty.  Ends with a workgroup barrier.
+// (minilp.cu:466-496); everything else empty.  The routes are there when it ends (a workgroup barrier), the sets' experts
+// behind the next one.
 template <int K>
 __device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t, const PlanTableLoads &l, int tid) {
   constexpr int nt = kPlanThreads;
   const int nl = a.sh.n_logical, R = a.n_rep, cd = a.sh.C * a.sh.D;
   for (int e = tid; e <= nl; e += nt)
     t.route[e] = Route{-1, R};
-  for (int e = tid; e <= nl; e += nt)
+  for (int e = tid; e < nl / 16 * 16 + 16; e += nt)
     t.hist[e] = 0;
   {
     const i32x4 zero{0, 0, 0, 0};
@@ -265,7 +272,7 @@ __device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t
     if (ok)
       atomicMin(&t.route[le].rep, R - 1 - i);
     t.reps[R - 1 - i] = RepEntry{0, 0u, 0, ((s.ep_rank - s.group_rank) + host + 1) * a.sh.P - cd + s.place};
-    t.set_expert[R - 1 - i] = ok ? le : -1;
+    t.set_expert[R - 1 - i] = ok ? le : nl;
   };
   if (l.set0)
     enter_set(tid, l.s0, l.rle0, l.host0);
@@ -274,6 +281,10 @@ __device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t
     enter_set(i, s, a.phy2log[s.ep_rank * a.sh.P + s.place], a.o2r[s.group_rank * a.sh.D + s.d]);
   }
   __syncthreads();
+  // (of two sets that name the same expert only one has the tokens; read behind the next barrier)
+  for (int q = tid; q < R; q += nt)
+    if (t.route[t.set_expert[q]].rep != q)
+      t.set_expert[q] = nl;
 }
 
 // K chunks of 64 indices from w0 on (uniform), those before `end`.
@@ -313,16 +324,16 @@ template <int N> __device__ inline void pack_expert(uint32_t (&packed)[N], int c
   packed[c / 2] = (c % 2) ? packed[c / 2] | ((uint32_t)e << 16) : (uint32_t)e;
 }
 
-// ---- a slice's tokens: bitmaps and histogram, the tokens of the earlier chunks and waves ----
+// ---- a slice's tokens: histogram and bitmaps, the tokens of the earlier chunks and waves ----
 template <int K> struct SliceTokens {
   static constexpr int kRec = rank_record_bytes_single(K);
   __device__ static ChunkSlot *slot(unsigned char *my_records, int set, int c) {
     return reinterpret_cast<ChunkSlot *>(my_records + __umul24((uint32_t)set, (uint32_t)kRec)) + c;
   }
-  // Enters the wave's tokens; afterwards t.hist is the slice's histogram, a slot's start the tokens of its set
-  // in the wave's earlier chunks, t.wave_total those in the earlier waves.  Ends with a workgroup barrier.
+  // Enters the wave's tokens; afterwards t.hist is the slice's histogram and a slot's bits are the chunk's tokens of its
+  // set.  Ends with a workgroup barrier, the only one between the tokens and the counts that others wait for.
   __device__ static void count(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, const int64_t (&raw)[K],
-                               uint32_t (&packed)[(K + 1) / 2], int tid, int lane, int wave_s) {
+                               uint32_t (&packed)[(K + 1) / 2], int lane) {
     const int nl = a.sh.n_logical, R = a.n_rep;
     const unsigned long long my_bit = 1ull << lane;
 #pragma unroll
@@ -331,18 +342,19 @@ template <int K> struct SliceTokens {
       const int e = valid ? (int)raw[c] : nl;
       pack_expert(packed, c, e);
       const int set = t.route[e].rep;
-      // a token of a replicated set is counted through the set's bitmaps (the sets hold the hot
-      // experts, whose tokens would queue up at one histogram counter), any other one here
+      if (valid)
+        atomicAdd(&t.hist[e], 1);
       if (set < R)
         atomicOr(reinterpret_cast<unsigned long long *>(slot(my_records, set, c)), my_bit);
-      else if (valid)
-        atomicAdd(&t.hist[e], 1);
     }
     __syncthreads();
     LPLB_PLAN_STAMP(8);
     LPLB_SLICE_STAMP(1);
-    // inside the wave: lane = (set, chunk), chunk fastest
-    const int c = lane % K;
+  }
+  // The tokens of each set in the wave's earlier chunks into the slots, those in the whole wave into t.wave_total.
+  // lane = (set, chunk), chunk fastest.
+  __device__ static void starts_in_wave(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, int lane, int wave_s) {
+    const int R = a.n_rep, c = lane % K;
     for (int p0 = 0; p0 < R * K; p0 += kWave) {
       const bool live = p0 + lane < R * K;
       const int q = live ? (p0 + lane) / K : R;   // lanes past the end read the stand-in record (zeros)
@@ -356,22 +368,6 @@ template <int K> struct SliceTokens {
           t.wave_total[wave_s * R + q] = in_my_wave;
       }
     }
-    __syncthreads();
-    for (int q = tid; q < R; q += kPlanThreads) {   // the sets' tokens in this slice, into the histogram
-      int32_t n = 0, of_wave[kPlanWaves];
-#pragma unroll
-      for (int w = 0; w < kPlanWaves; ++w)
-        of_wave[w] = t.wave_total[w * R + q];
-#pragma unroll
-      for (int w = 0; w < kPlanWaves; ++w) {   // (each wave's count becomes the count of the waves before it)
-        t.wave_total[w * R + q] = n;
-        n += of_wave[w];
-      }
-      const int le = t.set_expert[q];
-      if (le >= 0 && t.route[le].rep == q)   // (of two sets that name the same expert only one has the tokens)
-        t.hist[le] = n;
-    }
-    __syncthreads();
   }
   // Ordinal of the first token of every chunk: what is there already plus the tokens before this slice and in
   // the waves before this one.  The wave's own slots only: no barrier.
@@ -380,10 +376,34 @@ template <int K> struct SliceTokens {
     for (int p0 = 0; p0 < R * K; p0 += kWave) {
       const bool live = p0 + lane < R * K;
       const int q = live ? (p0 + lane) / K : 0;
-      const int32_t base = t.before[q] + t.wave_total[wave_s * R + q];
+      int32_t base = t.before[q];
+      for (int w = 0; w < wave_s; ++w)
+        base += t.wave_total[w * R + q];
       if (live)
         atomicAdd(&slot(my_records, q, c)->start, base);
     }
+    own_slots_are_written();
+  }
+  // The same where the workgroup holds the whole batch: from the bitmaps of the `turn` waves before this one, records_of(w)
+  // their records.
+  template <typename Records>
+  __device__ static void starts_of_batch(const PlanArgs &a, unsigned char *my_records, int lane, int turn, Records records_of) {
+    const int R = a.n_rep, c = lane % K;
+    for (int p0 = 0; p0 < R * K; p0 += kWave) {
+      const bool live = p0 + lane < R * K;
+      const int q = live ? (p0 + lane) / K : R;
+      int earlier = 0;
+      for (int w = 0; w < turn; ++w)
+        earlier += __popcll(*reinterpret_cast<const unsigned long long *>(slot(records_of(w), q, c)));
+      ChunkSlot *mine = slot(my_records, q, c);
+      const int own = __popcll(*reinterpret_cast<const unsigned long long *>(mine));
+      const int start = group_sum<K>(earlier) + group_exclusive_scan<K>(own, c);
+      if (live)
+        mine->start = start;
+    }
+    own_slots_are_written();
+  }
+  __device__ static void own_slots_are_written() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -425,85 +445,109 @@ __device__ inline void set_total(RepEntry &x, int32_t total) {
 
 // ---- collecting words ----
 __device__ inline unsigned long long tagged_word(uint32_t tag, uint32_t v) { return ((unsigned long long)tag << 32) | v; }
-// Up to N words per lane (its first `mine`), all with the launch's tag: polls until they are or max_polls polls have
-// passed; words past `mine` are 0.  Whole waves; false: the wait ran out.
+// Up to N words per lane (its first `mine`), all with the launch's tag: polls those that are not in yet until they are or
+// max_polls polls have passed; words past `mine` are 0.  Whole waves; false: the wait ran out.
 template <int N, typename Address>
 __device__ inline bool collect_words(uint32_t (&words)[N], uint32_t tag, int mine, int max_polls, Address address) {
+  unsigned long long v[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    v[k] = k < mine ? ~(unsigned long long)tag << 32 : (unsigned long long)tag << 32;
   for (int polls = 0; polls < max_polls; ++polls) {
-    unsigned long long v[N];
 #pragma unroll
     for (int k = 0; k < N; ++k)
-      v[k] = k < mine ? agent_load(address(k)) : (unsigned long long)tag << 32;
+      if ((uint32_t)(v[k] >> 32) != tag)
+        v[k] = agent_load(address(k));
     bool all_in = true;
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
+    for (int k = 0; k < N; ++k)
       all_in = all_in && (uint32_t)(v[k] >> 32) == tag;
-      words[k] = (uint32_t)v[k];
-    }
-    if (__all(all_in))
+    if (__all(all_in)) {
+#pragma unroll
+      for (int k = 0; k < N; ++k)
+        words[k] = (uint32_t)v[k];
       return true;
+    }
     __builtin_amdgcn_s_sleep(1);
   }
   return false;
 }
-// Adds up `words` words (two counts each) of every slice's row over the slices, into total[] and, over the slices
-// before this one, into before[] (LDS, zeroed; before may be null).  row_words: a power of two >= words; stride:
-// words from row to row.  By the whole workgroup: a thread takes one word of every (threads / row_words)-th slice,
-// IN_FLIGHT of them at a time.  Returns whether this wave's words all came.
-template <int IN_FLIGHT>
-__device__ inline bool add_up_rows_n(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int row_words,
-                                     uint32_t tag, int slice, int32_t *total, int32_t *before, int tid, int lane) {
-  const bool can_come = a.expected_slices == a.n_slices;   // (an injected fault: one slice never comes)
-  const int max_polls = can_come ? a.max_polls : 1;
-  const int q_lanes = min(row_words, kPlanThreads), p_lanes = kPlanThreads / q_lanes;   // powers of two
-  const int p_first = tid / q_lanes;
-  bool came = can_come;
-  for (int q0 = 0; q0 < words; q0 += q_lanes) {
-    const int q = q0 + tid % q_lanes;
-    const bool in_row = q < words;
-    int32_t sum[2] = {0, 0}, earlier[2] = {0, 0};
-    for (int p0 = 0; p0 < a.n_slices; p0 += IN_FLIGHT * p_lanes) {
-      const unsigned long long *at = rows + (int64_t)(p0 + p_first) * stride + q;
-      const int left = in_row ? (a.n_slices - p0 - p_first + p_lanes - 1) / p_lanes : 0;   // words of this thread, at most IN_FLIGHT now
-      uint32_t counts[IN_FLIGHT];
-      came = collect_words<IN_FLIGHT>(counts, tag, left, max_polls, [&](int k) { return at + (int64_t)k * p_lanes * stride; }) && came;
+// What slices add up of each other's rows is cut into units, one wave's work each: kUnitSlices slices' words at eight adjacent
+// places (more if there are fewer slices).  lane = (slice, pair of words); a lane loads the pairs of four slices at once.
+// No barrier, and nothing to clear first.  (One CU reads such words at 25 bytes per ns with 8-byte loads, one a lane, and at 68
+// with four and more 16-byte loads a lane on their way.)
+constexpr int kUnitSlices = 64, kUnitLoads = 4;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// The sum over the slices of a unit, for N values of every lane; lanes_log2: of a slice.
+template <int N> __device__ inline void over_slices_of_unit(uint32_t (&v)[N], int lanes_log2) {
+  if (lanes_log2 == 2)
 #pragma unroll
-      for (int k = 0; k < IN_FLIGHT; ++k) {
-        const bool is_before = p0 + k * p_lanes + p_first < slice;
-        const int32_t lo = (int32_t)(counts[k] & 0xffffu), hi = (int32_t)(counts[k] >> 16);
-        sum[0] += lo;
-        sum[1] += hi;
-        earlier[0] += is_before ? lo : 0;
-        earlier[1] += is_before ? hi : 0;
-      }
+    for (int j = 0; j < N; ++j)
+      v[j] += (uint32_t)dpp_int<0x124>((int)v[j]);   // row_ror:4
+  if (lanes_log2 <= 3)
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      v[j] += (uint32_t)dpp_int<0x128>((int)v[j]);   // row_ror:8
+  if (lanes_log2 <= 4)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const u32x2 s = __builtin_amdgcn_permlane16_swap(v[j], v[j], false, false);
+      v[j] = s.x + s.y;
     }
-    // lanes of a wave that hold the same word add up first (updates of one LDS word queue up)
-    for (int m = q_lanes; m < kWave; m <<= 1)
+  if (lanes_log2 <= 5)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        sum[h] += __shfl_xor(sum[h], m);
-        earlier[h] += before ? __shfl_xor(earlier[h], m) : 0;
-      }
-    if (in_row && lane < q_lanes)
+    for (int j = 0; j < N; ++j) {
+      const u32x2 s = __builtin_amdgcn_permlane32_swap(v[j], v[j], false, false);
+      v[j] = s.x + s.y;
+    }
+}
+// Words 2 (lane % lanes of a slice) and the next of the rows from `rows` on (16-byte aligned; lanes past the last of `words` words,
+// an even number, repeat that), over the slices of block `block`: the four counts added up over the slices into sums[0..3]
+// and, if BEFORE, over the slices before `slice` into sums[4..7].  Whole waves; false: some never came.
+template <bool BEFORE>
+__device__ inline bool add_up_unit(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int block, uint32_t tag,
+                                   int slice, int lane, uint32_t (&sums)[BEFORE ? 8 : 4]) {
+  if (a.expected_slices != a.n_slices)   // (an injected fault: one slice never comes)
+    return false;
+  const int per_round = kWave >> a.unit_lanes_log2, p0 = block * kUnitSlices + (lane >> a.unit_lanes_log2);
+  const unsigned long long *mine = rows + min(2 * (lane & ((1 << a.unit_lanes_log2) - 1)), words - 2);
+  const unsigned long long *at[kUnitLoads];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        atomicAdd(&total[2 * q + h], sum[h]);
-        if (before)
-          atomicAdd(&before[2 * q + h], earlier[h]);
-      }
+  for (int k = 0; k < kUnitLoads; ++k)   // (past the last slice: that one again, not counted)
+    at[k] = mine + min(p0 + k * per_round, a.n_slices - 1) * stride;
+  u32x4 v[kUnitLoads];
+  bool all_in = false;
+  for (int polls = 0; polls < a.max_polls; ++polls) {
+    if (!all_in) {
+      agent_load_pairs(v, at);
+      uint32_t off = 0;
+#pragma unroll
+      for (int k = 0; k < kUnitLoads; ++k)
+        off |= (v[k].y ^ tag) | (v[k].w ^ tag);
+      all_in = off == 0;
+    }
+    if (__all(all_in))
+      break;
+    __builtin_amdgcn_s_sleep(1);
   }
-  return came;
+  // (two counts to a word: of four slices they stay below 2^16)
+  static_assert(kUnitLoads * kLongestSlice < 65536, "sums of two 16-bit counts side by side");
+  u32x2 total{0, 0}, before{0, 0};
+#pragma unroll
+  for (int k = 0; k < kUnitLoads; ++k) {
+    const int p = p0 + k * per_round;
+    const u32x2 counts{v[k].x, v[k].z};
+    total += p < a.n_slices ? counts : u32x2{0, 0};
+    before += BEFORE && p < slice ? counts : u32x2{0, 0};
+  }
+  sums[0] = total.x & 0xffffu, sums[1] = total.x >> 16, sums[2] = total.y & 0xffffu, sums[3] = total.y >> 16;
+  if constexpr (BEFORE)
+    sums[4] = before.x & 0xffffu, sums[5] = before.x >> 16, sums[6] = before.y & 0xffffu, sums[7] = before.y >> 16;
+  over_slices_of_unit(sums, a.unit_lanes_log2);
+  return __all(all_in);
 }
-__device__ inline bool add_up_rows(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int row_words,
-                                   uint32_t tag, int slice, int32_t *total, int32_t *before, int tid, int lane) {
-  return a.n_slices * min(row_words, kPlanThreads) <= kPlanThreads
-             ? add_up_rows_n<1>(a, rows, stride, words, row_words, tag, slice, total, before, tid, lane)
-             : add_up_rows_n<4>(a, rows, stride, words, row_words, tag, slice, total, before, tid, lane);
-}
-// The batch's totals into `counts` (LDS, floats or ints; below 2^24 a count is exact as a float), by every wave of
-// the workgroup.  Returns whether this wave's have come.
-template <typename T>
-__device__ inline bool collect_totals(const PlanArgs &a, T *counts, uint32_t tag, int tid, int wave_s) {
+// The batch's totals into `counts` (LDS), by every wave of the workgroup.  Returns whether this wave's have come.
+__device__ inline bool collect_totals(const PlanArgs &a, int32_t *counts, uint32_t tag, int tid, int wave_s) {
   const unsigned long long *totals = reinterpret_cast<const unsigned long long *>(a.sync + kTotalsAt);
   const int nl = a.sh.n_logical;
   if (a.expected_slices != a.n_slices)   // (an injected fault: one slice never comes)
@@ -514,7 +558,7 @@ __device__ inline bool collect_totals(const PlanArgs &a, T *counts, uint32_t tag
     if (!collect_words<1>(count, tag, e < nl, a.max_polls, [&](int) { return totals + e; }))
       return false;
     if (e < nl)
-      counts[e] = (T)count[0];
+      counts[e] = (int32_t)count[0];
   }
   return true;
 }
@@ -528,18 +572,19 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
   __shared__ int missing[2];   // LP workgroup: [0] some counts did not come; slice: [0] the same, [1] some share will not come
+  __shared__ int block_sums[17];   // slice: what its units have added up of the totals, [16] how many of them have
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
   const int pid = blockIdx.x;
+  // (one argument of every 64 bytes of them: the others then come out of the scalar cache)
+  fetch_arguments_now(a.idx, a.unit_blocks, a.sh.G, a.solve.workload, a.solve.n_group, a.solve.tagged_result, a.sync);
   // Which launch of this block of words this is (the same value in every workgroup: it is advanced only once
-  // all of them have read it), and whether the block is switched off.
-  const int gen = agent_load(a.sync + kGenAt);
-  const bool poisoned = agent_load(a.sync + kPoisonAt) != 0;
-  const uint32_t tag = (uint32_t)gen + 1u;
-  const uint32_t tag_valid = (tag << 2) | 1u, tag_none = tag_valid + 1u;
+  // all of them have read it), and whether the block is switched off.  Both are looked at once the loads behind this one
+  // are on their way.
+  static_assert(kGenAt == 0 && kPoisonAt == 1, "one word");
+  unsigned long long gen_and_poison = agent_load(reinterpret_cast<const unsigned long long *>(a.sync));
   unsigned long long *shares = reinterpret_cast<unsigned long long *>(a.sync + kSharesAt);
-  unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen & 1);
 
   if (pid < a.n_lp_workgroups) {
     // ------------------------------------------------------------ the LPs
@@ -548,17 +593,21 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     const int n_lps = min(kLpsPerWorkgroup, sa.n_units - first_lp);
     LPLB_PLAN_STAMP(0);
     if (tid == kPlanThreads - kWave)   // (a wave without an LP)
-      agent_store(reinterpret_cast<unsigned long long *>(a.sync + kLpHereAt) + pid, tagged_word(tag, 0));
+      agent_store(reinterpret_cast<unsigned long long *>(a.sync + kLpHereAt) + pid, tagged_word((uint32_t)gen_and_poison + 1u, 0));
     // dynamic LDS of an LP workgroup: [LP wave][pivot rows | assembly tile], then the counts
     constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
     static_assert(kLpArea % 16 == 0, "the LP waves' areas keep 16-byte alignment");
     unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
     float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
-    sa.tag_valid = tag_valid;
+    sa.launch = (uint32_t)gen_and_poison;
+    auto switched_off = [&]() { return (gen_and_poison >> 32) != 0; };
     // Own-histogram mode: the LP waves' table loads are on their way when they and the other waves turn to the
     // batch's histogram.  (Switched off: no slice will publish.)
     auto counts_have_come = [&]() -> bool {
-      const bool mine = !poisoned && collect_totals(a, staged, tag, tid, wave_s);
+      if (tid >= kPlanThreads - 4)   // the zeros behind the counts
+        reinterpret_cast<int32_t *>(staged)[nl + tid - (kPlanThreads - 4)] = 0;
+      worked_out_here(gen_and_poison);
+      const bool mine = !switched_off() && collect_totals(a, reinterpret_cast<int32_t *>(staged), (uint32_t)gen_and_poison + 1u, tid, wave_s);
       if (!mine && lane == 0)
         missing[0] = 1;
       __syncthreads();
@@ -576,16 +625,18 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
       const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
           sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave, reinterpret_cast<double *>(my_area),
           reinterpret_cast<float *>(my_area + lp_pivot_doubles<GM, DM>() * sizeof(double)), counts_have_come);
+      worked_out_here(gen_and_poison);
+      unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen_and_poison & 1);
       if (n_ok < 0) {
         // no counts, no solution: tell the slices not to wait for this LP's shares
-        if (wave_s == 0 && lane == 0 && !poisoned)
+        if (wave_s == 0 && lane == 0 && !switched_off())
           give_up(a, avail_state);
         const int n_edges = sa.G * sa.D;
         for (int j = lane; j < n_edges; j += kWave)
           for (int k = 0; k < a.n_share_copies; ++k)
             agent_store(shares + (int64_t)k * kMaxShares + (int64_t)(first_lp + wave_s) * n_edges + j,
-                        (unsigned long long)tag_none << 32);
-      } else if (lane == 0 && n_ok > 0 && !poisoned) {
+                        (unsigned long long)(share_tag(sa.launch) + 1u) << 32);
+      } else if (lane == 0 && n_ok > 0 && !switched_off()) {
         // feasible: count it for the caller unless some workgroup has already given up on this batch
         const unsigned long long before = __hip_atomic_fetch_or(avail_state, 1ull << (first_lp + wave_s), __ATOMIC_RELAXED,
                                                                  __HIP_MEMORY_SCOPE_AGENT);
@@ -624,56 +675,109 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     missing[0] = 0;
     missing[1] = 0;
   }
+  if (tid < 17)
+    block_sums[tid] = 0;
   build_plan_tables<K>(a, t, tl, tid);
   LPLB_PLAN_STAMP(10);
 
   // ---- the tokens ----
   uint32_t packed[(K + 1) / 2];
-  SliceTokens<K>::count(a, t, my_records, raw, packed, tid, lane, wave_s);
-  LPLB_PLAN_STAMP(9);
-  // ---- this slice's counts, for every workgroup ----
+  SliceTokens<K>::count(a, t, my_records, raw, packed, lane);
+  // ---- this slice's counts, for every workgroup: the histogram by the first half of the waves, the sets by the others ----
+  worked_out_here(gen_and_poison);
+  const int gen = (int)(uint32_t)gen_and_poison;
+  const bool poisoned = (gen_and_poison >> 32) != 0;
+  const uint32_t tag = (uint32_t)gen + 1u;
+  unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen & 1);
   unsigned long long *set_rows = reinterpret_cast<unsigned long long *>(a.sync + kSetRowsAt);
   unsigned long long *hist_rows = reinterpret_cast<unsigned long long *>(a.sync + kHistRowsAt);
-  const int real_set_words = (R + 1) / 2;
+  const int set_lanes = a.set_words;
   if (!poisoned) {
-    auto count_of_set = [&](int q) {
-      const int le = q < R ? t.set_expert[q] : -1;
-      return le >= 0 && t.route[le].rep == q ? (uint32_t)t.hist[le] : 0u;
-    };
-    auto count_of = [&](int e) { return e < nl ? (uint32_t)t.hist[e] : 0u; };
-    for (int e2 = tid; e2 < a.hist_words; e2 += kPlanThreads)
-      agent_store(hist_rows + (int64_t)slice * a.hist_words + e2, tagged_word(tag, count_of(2 * e2) | count_of(2 * e2 + 1) << 16));
-    for (int q2 = tid; q2 < real_set_words; q2 += kPlanThreads)
-      agent_store(set_rows + (int64_t)slice * a.set_words + q2, tagged_word(tag, count_of_set(2 * q2) | count_of_set(2 * q2 + 1) << 16));
+    constexpr int kHalf = kPlanThreads / 2;
+    if (tid < kHalf) {
+      for (int e2 = tid; e2 < a.hist_words; e2 += kHalf) {
+        const int2 both = reinterpret_cast<const int2 *>(t.hist)[e2];
+        agent_store(hist_rows + slice * a.hist_words + e2, tagged_word(tag, (uint32_t)both.x | (uint32_t)both.y << 16));
+      }
+    } else {
+      for (int q2 = tid - kHalf; q2 < set_lanes; q2 += kHalf) {
+        const int first = t.hist[2 * q2 < R ? t.set_expert[2 * q2] : nl], second = t.hist[2 * q2 + 1 < R ? t.set_expert[2 * q2 + 1] : nl];
+        agent_store(set_rows + slice * a.set_words + q2, tagged_word(tag, (uint32_t)first | (uint32_t)second << 16));
+      }
+    }
   } else if (slice == 0 && tid == 0) {
     agent_add(a.sync + kTimeoutsAt, 1);   // one more plan that this block of words could not serve
   }
   LPLB_PLAN_STAMP(1);
   LPLB_SLICE_STAMP(2);
-  // ---- the batch's totals of eight words' experts (more if there are fewer slices than that takes), if this slice
-  //      is one that adds them up ----
-  bool mine_came = !poisoned;
-  if (!poisoned && slice < a.adders) {
-    const int first_word = slice * a.adder_words, words = min(a.adder_words, a.hist_words - first_word);
-    __syncthreads();   // (the histogram has been read)
-    for (int i = tid; i < 2 * words; i += kPlanThreads)
-      t.hist[i] = 0;
-    __syncthreads();
-    mine_came = add_up_rows(a, hist_rows + first_word, a.hist_words, words, a.adder_words, tag, slice, t.hist, nullptr, tid, lane);
-    if (!mine_came)
-      missing[0] = 1;
-    __syncthreads();
+  // ---- while the others' words are on their way: the tokens of each set in this slice's earlier chunks (a wave that adds
+  //      up totals, which the LP waits for, does that first) ----
+  const bool adds_totals = slice < a.adders && wave_s >= kPlanWaves - a.unit_blocks;
+  if (!adds_totals)
+    SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
+  // ---- what others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
+  //      those that add them up; the tokens of each replicated set before this slice and in the whole batch ----
+  if (!poisoned) {
+    const int unit_lanes = 1 << a.unit_lanes_log2, unit_words_log2 = a.unit_lanes_log2 + 1, block_bits = a.unit_block_bits;
+    const int first_word = slice * a.adder_words, my_words = slice < a.adders ? min(a.adder_words, a.hist_words - first_word) : 0;
+    const int adder_units = ((my_words + (1 << unit_words_log2) - 1) >> unit_words_log2) << block_bits;
+    const int units = adder_units + (((set_lanes + (1 << unit_words_log2) - 1) >> unit_words_log2) << block_bits);
     unsigned long long *totals = reinterpret_cast<unsigned long long *>(a.sync + kTotalsAt);
-    if (missing[0] == 0)   // (every wave's words are in the sums; if not, the batch is given up below)
-      for (int i = tid; i < 2 * words; i += kPlanThreads)
-        if (2 * first_word + i < nl)
-          agent_store(totals + 2 * first_word + i, tagged_word(tag, (uint32_t)t.hist[i]));
+    for (int unit = kPlanWaves - 1 - wave_s; unit < units; unit += kPlanWaves) {   // the last waves first: the others have published
+      const int block = unit & ((1 << block_bits) - 1);
+      if (block >= a.unit_blocks)
+        continue;
+      if (unit >= adder_units) {
+        const int word0 = (unit - adder_units) >> block_bits << unit_words_log2;
+        uint32_t sums[8];
+        if (add_up_unit<true>(a, set_rows + word0, a.set_words, set_lanes - word0, block, tag, slice, lane, sums)) {
+          const int first_set = 2 * word0 + 4 * lane;
+          if (lane < unit_lanes)   // (words past set_lanes have no sets)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (first_set + j < R) {
+                atomicAdd(&t.total[first_set + j], (int32_t)sums[j]);
+                atomicAdd(&t.before[first_set + j], (int32_t)sums[4 + j]);
+              }
+        } else {
+          missing[0] = 1;
+        }
+      } else {
+        const int at = unit >> block_bits << unit_words_log2, word0 = first_word + at;
+        uint32_t sums[4];
+        if (add_up_unit<false>(a, hist_rows + word0, a.hist_words, my_words - at, block, tag, slice, lane, sums)) {
+          bool all_in = true;
+          if (a.unit_blocks > 1) {   // (eight words then, in one unit per block: the wave that comes last publishes)
+            if (lane < 4)
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                atomicAdd(&block_sums[4 * lane + j], (int32_t)sums[j]);
+            int arrived = 0;
+            if (lane == 0)
+              arrived = atomicAdd(&block_sums[16], 1);
+            all_in = __builtin_amdgcn_readfirstlane(arrived) == a.unit_blocks - 1;
+            if (all_in && lane < 4)
+#pragma unroll
+              for (int j = 0; j < 4; ++j)
+                sums[j] = (uint32_t)block_sums[4 * lane + j];
+          }
+          if (all_in && lane < unit_lanes && 2 * lane < my_words - at)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const int e = 2 * word0 + 4 * lane + j;
+              if (e < nl)
+                agent_store(totals + e, tagged_word(tag, sums[j]));
+            }
+        } else {
+          missing[0] = 1;
+        }
+      }
+    }
   }
+  if (adds_totals)
+    SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
   LPLB_PLAN_STAMP(11);
-  // ---- tokens of each replicated set before this slice and in the whole batch ----
-  if (!poisoned)
-    mine_came = add_up_rows(a, set_rows, a.set_words, real_set_words, a.set_words, tag, slice, t.total, t.before, tid, lane) && mine_came;
-  if (!mine_came)
+  if (poisoned)
     missing[0] = 1;
   __syncthreads();
   LPLB_PLAN_STAMP(2);
@@ -724,6 +828,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     }
     LPLB_PLAN_STAMP(4);
     // ---- the LP's shares: every set's thread polls its own; value and tag arrive in the same word ----
+    const uint32_t tag_valid = share_tag((uint32_t)gen), tag_none = tag_valid + 1u;
     for (int i = tid; i < R; i += kPlanThreads) {
       const SetOfPlan s = set_of_plan(a, i);
       const unsigned long long *word_at = shares + (slice & (a.n_share_copies - 1)) * kMaxShares + s.ep_rank * a.sh.D + s.d;
@@ -778,10 +883,10 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 }
 
 // A short batch that feeds the LP itself, as one workgroup: the LPs are solved by its first waves between the
-// histogram and the choice.  Bound by the chain table loads -> indices -> histogram -> LP (4 us of 7.7) -> choice,
-// of which the slices' form above adds two round trips through memory between slices and LP: [7 x 8] indices 11.3 ->
-// 9.0 us per call, [128 x 8] 11.6 -> 9.5 us, where the calling thread needs 8 us for a call.  Up to
-// kSingleMaxIndices, eight per lane: past that a wave's chunks take longer than the exchange.  The LP waves come last
+// histogram and the choice.  Bound by the chain table loads -> indices -> histogram (1.3 us) -> LP -> choice,
+// of which the slices' form above adds two round trips through memory between slices and LP.  The LP reads the histogram
+// where the tokens were counted, behind the one barrier that it takes; the ordinals are worked out by the other waves while it runs.
+// Up to kSingleMaxIndices, eight per lane: past that a wave's chunks take longer than the exchange.  The LP waves come last
 // in the order of the indices, so that they have none unless the batch fills all eight waves.
 constexpr int kSingleMaxIndices = 4096, kSingleMaxLps = kPlanWaves;
 template <int GM, int DM, bool EXACT, int K>
@@ -792,13 +897,13 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
-  // LDS: the LP waves' areas, the counts as floats, the slice's tables
+  // LDS: the LP waves' areas, the slice's tables
   constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
   const int n_lps = a.solve.n_units;
-  float *staged = reinterpret_cast<float *>(smem_raw + n_lps * kLpArea);
-  const SliceTables t = carve_tables<K>(reinterpret_cast<unsigned char *>(staged + (nl + 3) / 4 * 4), nl, R);
+  const SliceTables t = carve_tables<K>(smem_raw + n_lps * kLpArea, nl, R);
   const int turn = (wave_s - n_lps) & (kPlanWaves - 1);   // this wave's place in the order of the indices
-  unsigned char *my_records = t.records + (size_t)turn * ((R + 1) * rank_record_bytes_single(K));
+  auto records_of = [&](int place) { return t.records + (size_t)place * ((R + 1) * rank_record_bytes_single(K)); };
+  unsigned char *my_records = records_of(turn);
   const PlanTableLoads tl = issue_plan_table_loads(a, tid);
   const int64_t w0 = (int64_t)turn * (K * kWave);
   int64_t raw[K];
@@ -808,25 +913,15 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   // (called by the LP waves once their own table loads are on their way)
   auto count_the_tokens = [&]() -> bool {
     build_plan_tables<K>(a, t, tl, tid);
-    SliceTokens<K>::count(a, t, my_records, raw, packed, tid, lane, turn);
-    for (int e = tid; e < nl; e += kPlanThreads) {
-      const int32_t n = t.hist[e];
-      staged[e] = (float)n;
-      a.totals[e] = n;
-    }
-    for (int q = tid; q < R; q += kPlanThreads) {
-      const int le = t.set_expert[q];
-      t.total[q] = le >= 0 && t.route[le].rep == q ? t.hist[le] : 0;
-      set_total(t.reps[q], t.total[q]);
-    }
-    __syncthreads();
+    SliceTokens<K>::count(a, t, my_records, raw, packed, lane);
     return true;
   };
   if (wave_s < n_lps) {
     unsigned char *area = smem_raw + wave_s * kLpArea;
     SolveArgs sa = a.solve;
     sa.shares_in_lds = share_of;
-    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(sa, wave_s, staged, rep_of_edge_all + wave_s * kWave,
+    sa.gw_out = nullptr;   // (written below, by waves that do not solve)
+    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(sa, wave_s, reinterpret_cast<float *>(t.hist), rep_of_edge_all + wave_s * kWave,
                                                     reinterpret_cast<double *>(area),
                                                     reinterpret_cast<float *>(area + lp_pivot_doubles<GM, DM>() * sizeof(double)),
                                                     count_the_tokens);
@@ -835,21 +930,43 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   } else {
     count_the_tokens();
   }
+  auto tokens_of = [&](int q) { return t.hist[t.set_expert[q]]; };   // of a set, in the batch
+  // The totals and the normalised counts go out while the LPs are solved.
+  if (wave_s >= n_lps || n_lps == kPlanWaves) {
+    const int first = n_lps == kPlanWaves ? 0 : n_lps * kWave;
+    int32_t most = 0;
+    for (int i = 4 * lane; i < nl; i += 4 * kWave) {
+      const i32x4 c = *reinterpret_cast<const i32x4 *>(t.hist + i);
+      most = max(max(most, max(c.x, c.y)), max(c.z, c.w));
+    }
+    const float wmax = wave_max_of_groups<true, true>((float)most);
+    for (int e = tid - first; e < nl; e += kPlanThreads - first) {
+      const int32_t n = t.hist[e];
+      a.totals[e] = n;
+      a.solve.gw_out[e] = (float)n / wmax;
+    }
+  }
   const bool has_tokens = w0 < a.n;
   int32_t h[K];
   if (has_tokens) {
-    SliceTokens<K>::add_starts(a, t, my_records, lane, turn);
+    for (int q = lane; q < R; q += kWave)   // (every wave enters the same values: none has to wait for another)
+      set_total(t.reps[q], tokens_of(q));
+    SliceTokens<K>::starts_of_batch(a, my_records, lane, turn, records_of);
 #pragma unroll
     for (int c = 0; c < K; ++c)
       h[c] = SliceTokens<K>::hash(t, my_records, packed_expert(packed, c), c);
   }
-  __syncthreads();
-  LPLB_PLAN_STAMP(2);
-  for (int i = tid; i < R; i += kPlanThreads) {
-    const SetOfPlan s = set_of_plan(a, i);
-    t.reps[R - 1 - i].expected = expected_on_original(share_of[s.ep_rank * a.sh.D + s.d], t.total[R - 1 - i]);
+  if (wave_s < n_lps) {
+    __builtin_amdgcn_wave_barrier();   // (its shares have been stored)
+    const int per_group = a.sh.G * a.sh.C * a.sh.D;
+    for (int i = lane; i < per_group; i += kWave) {
+      const int set = wave_s * per_group + i;
+      const SetOfPlan s = set_of_plan(a, set);
+      t.reps[R - 1 - set].expected = expected_on_original(share_of[s.ep_rank * a.sh.D + s.d], tokens_of(R - 1 - set));
+    }
   }
   __syncthreads();
+  LPLB_PLAN_STAMP(2);
   if (has_tokens) {
     int32_t o[K];
 #pragma unroll
@@ -902,13 +1019,15 @@ template <int GM, int DM, bool EXACT> __global__ __launch_bounds__(kScanThreads)
   __syncthreads();
   const bool can_come = a.expected_blocks == a.n_blocks;   // (an injected fault: one slice never comes)
   auto counts_have_come = [&]() -> bool {
+    if (tid < 4)   // the zeros behind the counts
+      reinterpret_cast<int32_t *>(staged)[nl + tid] = 0;
     for (int e = tid; e < nl; e += kScanThreads) {
       int32_t sum = kNoTotal;
       for (int polls = 0; polls < a.max_polls && (sum = agent_load(a.totals + e)) == kNoTotal; ++polls)
         __builtin_amdgcn_s_sleep(1);
       if (sum == kNoTotal || !can_come)
         missing = 1;
-      staged[e] = (float)sum;
+      reinterpret_cast<int32_t *>(staged)[e] = sum;
     }
     __syncthreads();   // (from here on the totals may be overwritten by the normalised counts)
     return missing == 0;
@@ -938,8 +1057,8 @@ template <int GM, int DM, bool EXACT> __global__ __launch_bounds__(kScanThreads)
 
 // ---- host side: which variant ----
 template <int GM, int DM> static int launch_scan_and_solve(const ScanSolveArgs &a, hipStream_t s) {
-  const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + a.solve.n_experts * sizeof(float);
-  static_assert(kScanSolveLps * plan_lp_area_bytes<GM, DM>() + kMaxPlanExperts * sizeof(float) <= 60 * 1024, "LDS of a kernel without asking for more");
+  const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + counts_bytes(a.solve.n_experts);
+  static_assert(kScanSolveLps * plan_lp_area_bytes<GM, DM>() + counts_bytes(kMaxPlanExperts) <= 62 * 1024, "LDS of a kernel without asking for more");
   const dim3 grid(1 + (a.solve.n_experts + kScanCols - 1) / kScanCols), block(kScanThreads);
   if (a.solve.G == GM && a.solve.D == DM)
     launch(scan_and_solve<GM, DM, true>, grid, block, lds, s, a);
@@ -954,13 +1073,13 @@ static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   // LP workgroups: their waves' working areas, then the counts (one copy per LP if they fit,
   // else none and the LPs read global memory; own-histogram mode needs one copy in any case)
   const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
-  const size_t one_copy = (size_t)a.sh.n_logical * sizeof(float);
+  const size_t one_copy = counts_bytes(a.sh.n_logical);
   const size_t all_copies = (size_t)min(a.solve.n_units, kLpsPerWorkgroup) * one_copy;
   size_t lds = max(lds_slice, lp_areas + (a.local_counts ? one_copy : 0));
   a.solve.staged_stride = 0;
   if (lp_areas + all_copies <= max(lds, (size_t)16 * 1024)) {   // (a few KiB more are worth one global round trip less)
     lds = max(lds, lp_areas + all_copies);
-    a.solve.staged_stride = a.sh.n_logical;
+    a.solve.staged_stride = (int)(one_copy / sizeof(int32_t));
   }
   if (lds > (size_t)kPlanLdsLimit)
     return LPLB_OK;
@@ -968,8 +1087,7 @@ static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   return launch_plan(plan_in_one_launch<GM, DM, EXACT, K>, footprint, true, a, lds, s, done);
 }
 template <int GM, int DM, bool EXACT, int K> static int launch_plan_single(PlanArgs &a, hipStream_t s, bool *done) {
-  const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + (a.sh.n_logical + 3) / 4 * 4 * sizeof(float) +
-                     plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);
+  const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);
   if (lds > (size_t)kPlanLdsLimit)
     return LPLB_OK;
   a.solve.staged_stride = a.sh.n_logical;

@@ -28,6 +28,19 @@ __device__ inline int agent_load(const int *p) {
 __device__ inline unsigned long long agent_load(const unsigned long long *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Four pairs of words, each 16-byte aligned, with one load past the caches for both (there is no 16-byte atomic to
+// ask the compiler for; each of the two words arrives in one piece).  Returns when they are there.
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ inline void agent_load_pairs(u32x4 (&v)[4], const unsigned long long *const (&p)[4]) {
+  asm volatile("global_load_dwordx4 %0, %4, off sc1\n\t"
+               "global_load_dwordx4 %1, %5, off sc1\n\t"
+               "global_load_dwordx4 %2, %6, off sc1\n\t"
+               "global_load_dwordx4 %3, %7, off sc1\n\t"
+               "s_waitcnt vmcnt(0)"
+               : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+               : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3])
+               : "memory");
+}
 __device__ inline void agent_store(int *p, int v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

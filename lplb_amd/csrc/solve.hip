@@ -49,8 +49,8 @@ constexpr int kLdsLimit = 64 * 1024 - 2048;
 
 template <int GM, int DM, bool EXACT, int ROWS, int EPL = 1>
 static void launch_variant(SolveArgs a, hipStream_t s) {
-  const size_t lds = (size_t)ROWS * a.n_experts * sizeof(float);
-  a.staged_stride = lds <= kLdsLimit ? a.n_experts : 0;
+  const size_t lds = (size_t)ROWS * (a.n_experts + 1) * sizeof(float);   // (one LP per wave has a zero behind its counts)
+  a.staged_stride = lds <= kLdsLimit ? a.n_experts + 1 : 0;
   launch(solve_groups<GM, DM, EXACT, ROWS, EPL>, dim3((a.n_units + ROWS - 1) / ROWS), dim3(kWave),
          a.staged_stride ? lds : 0, s, a);
 }

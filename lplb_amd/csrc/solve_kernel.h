@@ -49,12 +49,12 @@ struct SolveArgs {
   float *result;             // [n_inst][n_group][G][D]
   int n_group, G, D, C, n_fixed, n_experts, step_rule, n_steps, n_units;
   int staged_stride;   // floats of LDS per LP for its counts, 0 = read them from global memory
-  bool counts_by_caller;   // a.workload is not read: the caller puts the counts into staged_counts (as floats) before its
+  bool counts_by_caller;   // a.workload is not read: the caller puts the counts into staged_counts (as int32) before its
                            // `counts_have_come` returns
   unsigned long long *tagged_result;  // or null: a copy of a.result for other workgroups of the same launch,
-  uint32_t tag_valid;                 // each value written through to memory as (tag_valid << 32) | its bits
+  uint32_t launch;                    // each value written through to memory as (share_tag(launch) << 32) | its bits
   int tagged_copies, tagged_stride;   // ... tagged_copies times, tagged_stride words apart (the pollers spread over the copies)
-                                      // (the caller writes tag_valid + 1 for "no result: use the neutral fallback")
+                                      // (the caller writes share_tag(launch) + 1 for "no result: use the neutral fallback")
   float *shares_in_lds;      // or null: another copy of a.result, for the caller's workgroup
   long long *clocks;         // debug builds: wall-clock stamps of wave 0, lane 0 (else null)
 };
@@ -186,13 +186,16 @@ template <int ROWS, int W> __device__ inline float lp_max(float v) {
 }
 
 
+// What says that a share is there, from the launch that found `launch` in its block's counter (formed where it is stored: that
+// counter may still be on its way when the LP begins).
+__host__ __device__ inline uint32_t share_tag(uint32_t launch) { return ((launch + 1u) << 2) | 1u; }
 // Stores a share, and if asked also the copies other workgroups of the running kernel poll (the high word says
 // "valid, from this launch", so value and flag arrive in one 8-byte store) and the one in the caller's LDS.
 __device__ inline void store_share(const SolveArgs &a, int64_t i, float v) {
   if (a.tagged_result)
     for (int k = 0; k < a.tagged_copies; ++k)
       __hip_atomic_store(a.tagged_result + (int64_t)k * a.tagged_stride + i,
-                         ((unsigned long long)a.tag_valid << 32) | __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
+                         ((unsigned long long)share_tag(a.launch) << 32) | __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
   if (a.shares_in_lds)
     a.shares_in_lds[i] = v;
