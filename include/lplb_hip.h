@@ -37,6 +37,12 @@ extern "C" {
 #define LPLB_STEP_REFERENCE_WINDOW 0 /* max over the last 32 columns, as minilp.cu:355-359 does */
 #define LPLB_STEP_FULL_MAX 1         /* max over all columns (and 0) */
 
+/* Types of a load history (lplb_place_experts). */
+#define LPLB_INT32 0
+#define LPLB_INT64 1
+#define LPLB_FLOAT32 2
+#define LPLB_FLOAT64 3
+
 typedef void *lplb_stream_t;
 
 int lplb_abi_version(void);
@@ -398,6 +404,21 @@ int lplb_build_mapping(const float *weight, const double *history, const int32_t
                        int group_size, int dup_per_rank, int ep_size, int n_logical,
                        int n_physical, int n_nodes, int32_t *phy2log, int32_t *log2phy,
                        int32_t *logcnt);
+
+/*
+ * lplb_build_mapping for a load history that is on the GPU: one kernel on the stream, the same result bit for bit
+ * (the history rounded to fp32 for the packing, to fp64 for the order inside a rank).  All pointers are
+ * device pointers; returns when the tables are there.
+ *
+ *   history, history_type  [n_logical] of one of the types above
+ *   r2o                    int32 [group_size, dup_per_rank], every column a permutation
+ *
+ * LPLB_EUNSUPPORTED (use lplb_build_mapping) beyond 1024 logical experts, 128 of them (unless a rank has one only) or 64
+ * ranks to be packed at once, and where several groups share a node.
+ */
+int lplb_place_experts(const void *history, int history_type, const int32_t *r2o, int group_size,
+                       int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
+                       int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream);
 
 /*
  * No counterpart in the reference.  enabled = 0 makes lplb_plan always run the

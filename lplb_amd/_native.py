@@ -66,6 +66,7 @@ _SIGNATURES = {
     "lplb_replicate_experts": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp]),
     "lplb_rebalance_experts": (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "lplb_build_mapping": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
+    "lplb_place_experts": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "lplb_plan_noalloc": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
 }
 
@@ -163,6 +164,28 @@ def plan_one_launch_count() -> int:
     count = ctypes.c_longlong(-1)
     _check(load().lplb_plan_one_launch_count(ctypes.byref(count)))
     return count.value
+
+
+# LPLB_INT32 ... LPLB_FLOAT64 of include/lplb_hip.h
+_HISTORY_TYPES = {torch.int32: 0, torch.int64: 1, torch.float32: 2, torch.float64: 3}
+
+
+def place_experts(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_physical: int, n_nodes: int) -> torch.Tensor | None:
+    """build_redundancy_mapping for a history on the current device, by a kernel there: its three arrays as parts of
+    one int32 tensor [n_physical + 3 * n_logical] on that device, complete on return; None if the kernel does not cover it."""
+    kind = _HISTORY_TYPES.get(history.dtype)
+    if kind is None or not history.is_contiguous() or _device_index(history) != torch.cuda.current_device():
+        return None
+    n_logical = history.numel()
+    table = torch.empty(n_physical + 3 * n_logical, dtype=torch.int32, device=history.device)
+    at = table.data_ptr()
+    rc = load().lplb_place_experts(history.data_ptr(), kind, r2o.data_ptr(), r2o.shape[0], r2o.shape[1], ep_size, n_logical,
+                                   n_physical, n_nodes, at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical),
+                                   _stream(history))
+    if rc == 2:
+        return None
+    _check(rc)
+    return table
 
 
 class UnsupportedShape(RuntimeError):

@@ -78,7 +78,9 @@ class Planner:
         self.gpus_per_node = gpus_per_node
 
         self.phy2log: torch.Tensor
+        self._r2o_placed: torch.Tensor | None = None
         self.update_redundancy_mapping()
+        self._r2o_placed = self.r2o.clone()   # what the mapping above was made for
 
         self.ep_group = group
         self.deep_ep_initialized = False
@@ -115,15 +117,26 @@ class Planner:
         :param workload: per-logical-expert history; ``None`` keeps experts in index order.
         :return: ``(phy2log [n_routed], log2phy [n_logical, 2], logcnt [n_logical])``, int32.
         """
-        host = None if workload is None else workload.detach().cpu().numpy()
-        # the three arrays are parts of one buffer, which goes to the GPU in one copy
-        n_phy, n_log = self.n_routed_experts, self.n_logical_routed_experts
-        staged = torch.empty(n_phy + 3 * n_log, dtype=torch.int32, pin_memory=self.device.type == "cuda")
-        build_redundancy_mapping(self._r2o_host, self.ep_size, n_log, n_phy, host,
-                                 n_nodes=max(1, self.ep_size // self.gpus_per_node), out=staged.numpy())
-        table = staged.to(self.device)
+        # the three arrays are parts of one buffer
+        n_phy, n_log, n_nodes = self.n_routed_experts, self.n_logical_routed_experts, max(1, self.ep_size // self.gpus_per_node)
+        table = self._mapping_where_the_history_is(workload, n_nodes)
+        if table is None:
+            host = None if workload is None else workload.detach().cpu().numpy()
+            staged = torch.empty(n_phy + 3 * n_log, dtype=torch.int32, pin_memory=self.device.type == "cuda")
+            build_redundancy_mapping(self._r2o_host, self.ep_size, n_log, n_phy, host, n_nodes=n_nodes, out=staged.numpy())
+            table = staged.to(self.device)
         self.phy2log = table[:n_phy]
         return self.phy2log, table[n_phy:n_phy + 2 * n_log].view(n_log, 2), table[n_phy + 2 * n_log:]
+
+    def _mapping_where_the_history_is(self, workload: torch.Tensor | None, n_nodes: int) -> torch.Tensor | None:
+        """The mapping's tables made on the GPU, if the history is on the planner's and one kernel covers the deployment:
+        the history need not come to the host and the tables need not go back (the shape itself was checked when the planner
+        was built).  Not inside a capture, where reading the history on the host is refused and this would wait."""
+        if (workload is None or not workload.is_cuda or self.device.type != "cuda" or self._r2o_placed is None
+                or workload.numel() != self.n_logical_routed_experts or workload.device != self._r2o_placed.device
+                or torch.cuda.is_current_stream_capturing()):
+            return None
+        return _native.place_experts(workload, self._r2o_placed, self.ep_size, self.n_routed_experts, n_nodes)
 
     def count_workload(self, idx: torch.Tensor, n_sms: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Histogram of ``idx`` (values in [-1, n_logical), -1 ignored) over ``n_sms`` slices.
