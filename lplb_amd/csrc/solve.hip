@@ -30,20 +30,20 @@ __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
 // One LP per wave has the lowest latency; shapes with G <= 16 and G * D <= 16 can put four into each wave, which takes
 // longer but needs a quarter of the waves.  Alone on its SIMD a lone LP is the faster one throughout.  Up to 8 ranks its
 // lanes are busy less than half the time, and it still is with three on a SIMD; four packed ones fill one wave of every SIMD
-// and take no longer, then a second packed wave is behind until there are more than six LPs per SIMD.
+// and take no longer, then a second packed wave is behind until there are six LPs per SIMD.
 // From 9 ranks on (16 pivots a step instead of 8) the second is already too many.  Measured, one per wave / four per wave:
 //                    1024         2048         3072         4096         5120         6144         8192 LPs
-//   (8, 2)      6.7 / 10.2   7.8 / 10.7   9.3 / 10.7  10.8 / 10.9  12.4 / 14.4  13.9 / 15.0  17.0 / 15.4 us
-//   (8, 1)      6.5 /  9.6   7.4 /  9.9   9.0 / 10.0  10.4 / 10.3  11.9 / 13.2  13.4 / 13.9  16.5 / 14.4
-//   (7, 2)      7.3 / 10.8   8.5 / 11.2  10.3 / 11.2  11.7 / 11.3  13.5 / 14.9  15.1 / 15.2  18.5 / 15.8   (padded)
-//   (4, 2)      7.4 / 12.4   8.5 / 12.7  10.1 / 12.8  11.8 / 13.1  13.6 / 16.4  15.4 / 16.6  18.7 / 16.9   (padded)
-//   (16, 1)    12.0 / 13.3  18.5 / 14.1  25.3 / 14.4  31.9 / 14.9  38.8 / 19.6  45.9 / 20.2  59.6 / 21.1
-//   (10, 1)    13.4 / 16.7  19.9 / 17.5  26.8 / 17.6  33.5 / 18.1  41.1 / 22.9  48.2 / 23.6  62.2 / 24.4   (padded)
+//   (8, 2)      6.7 / 10.2   7.7 / 10.7   9.6 / 10.7  10.9 / 10.9  12.7 / 14.4  14.3 / 14.9  17.5 / 15.4 us
+//   (8, 1)      6.5 /  9.5   7.7 / 10.0   9.1 / 10.0  10.7 / 10.2  12.2 / 13.2  13.7 / 13.8  17.1 / 14.4
+//   (7, 2)      7.6 / 10.7   8.7 / 11.2  10.4 / 11.1  12.2 / 11.3  13.7 / 14.8  15.6 / 15.2  19.0 / 15.9   (padded)
+//   (4, 2)      7.6 / 12.5   8.6 / 12.7  10.4 / 12.8  12.0 / 13.1  13.7 / 16.3  15.6 / 16.6  18.8 / 16.9   (padded)
+//   (16, 1)    12.4 / 13.2  18.8 / 14.1  25.5 / 14.4  32.2 / 14.5  38.9 / 19.3  45.8 / 19.8  59.5 / 20.4
+//   (10, 1)    13.6 / 16.4  20.3 / 17.3  27.0 / 17.3  33.9 / 17.6  40.7 / 22.3  48.1 / 22.8  62.3 / 23.5   (padded)
 static bool packing_pays(int G, int n_units) {
   const int n_cus = current_device_cu_count();
   const int n_simds = 4 * (n_cus > 0 ? n_cus : 256);
   const int per_simd = n_units / n_simds + (n_units % n_simds != 0);
-  return G <= 8 ? per_simd == 4 || per_simd > 6 : per_simd > 1;
+  return G <= 8 ? per_simd == 4 || per_simd > 5 : per_simd > 1;
 }
 constexpr int kLdsLimit = 64 * 1024 - 2048;
 

@@ -130,10 +130,10 @@ __device__ inline double2 lds_pair(const lds_double *base, int at) {
   const f64x2 v = *reinterpret_cast<const lds_f64x2 *>(base + at);
   return double2{v.x, v.y};
 }
-// v of the first of every eight lanes.
-__device__ inline float bcast_in_eight(float v) {
-  const int q = __builtin_bit_cast(int, quad_bcast<0>(v));
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(q, q, 0x114 /* row_shr:4 */, 0xF, 0xA, false));
+// v of the last of every eight lanes.
+__device__ inline float last_of_eight(float v) {
+  const int q = __builtin_bit_cast(int, quad_bcast<3>(v));
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(q, q, 0x104 /* row_shl:4 */, 0xF, 0x5, false));
 }
 constexpr int kIdentityPerm = 0xE4;   // quad_perm [0,1,2,3]
 // v with the 16-lane row ROW made zero, through its high word only (what is left of a number is a denormal below 2^-1022).
@@ -293,7 +293,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
   if constexpr (KC == 1) {
     my_entry = pivot_at + rank * kRow8 + sub;
     my_rhs = pivot_at + 8 * kRow8 + rank;
-    my_column = pivot_at + (sub == 0 ? 8 : sub) * kRow8;
+    my_column = pivot_at + (sub == 7 ? 8 : sub) * kRow8;
     lds_double *constants = pivot_at + 9 * kRow8;   // (-1, 0) four times, (0, -1) four times
     if (lane < 16)
       constants[lane] = lane % 2 == lane / 8 ? -1.0 : 0.0;
@@ -386,7 +386,8 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
   float d_max = 0.0f;
   const int NV = 2 * n + G + 2;
   const int win_lo = a.step_rule == LPLB_STEP_REFERENCE_WINDOW ? (NV > 32 ? NV - 32 : 0) : 0;
-  const float at_least = a.step_rule != LPLB_STEP_REFERENCE_WINDOW || NV < 32 ? 0.0f : __builtin_nanf("");
+  float at_least = a.step_rule != LPLB_STEP_REFERENCE_WINDOW || NV < 32 ? 0.0f : __builtin_nanf("");
+  asm("" : "+v"(at_least));   // (one operand of a maximum; known to be one of the two, it becomes a select behind one)
   bool win_o[E], win_r[E];
 #pragma unroll
   for (int p = 0; p < E; ++p) {
@@ -494,14 +495,15 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
     };
     if constexpr (KC == 1) {
       // One entry per lane.  The pivot rows themselves are replaced by the rows divided by the block: as if they were
-      // zero and had the entries (-1, 0) and (0, -1), which their lanes read from constants instead.  Column 0 is not used
-      // any more once it has been published: its lanes go on with the right-hand side (row 8 in LDS).
+      // zero and had the entries (-1, 0) and (0, -1), which their lanes read from constants instead.  The last pair comes first:
+      // column 7 is not used any more once it has been published, and its lanes go on with the right-hand side (row 8 in LDS),
+      // which so ends up in the lanes that sums over the ranks are taken from.
       static_for<GM / 2>([&](auto pc) {
-        constexpr int p = decltype(pc)::value, c = 2 * p;
-        *(p == 0 || sub > 0 ? my_entry : my_rhs) = S[0];
-        if constexpr (p == 0) {
+        constexpr int p = GM / 2 - 1 - decltype(pc)::value, c = 2 * p;
+        *(p == GM / 2 - 1 || sub < 7 ? my_entry : my_rhs) = S[0];
+        if constexpr (p == GM / 2 - 1) {
           *my_rhs = rhs;
-          S[0] = sub == 0 ? rhs : S[0];
+          S[0] = sub == 7 ? rhs : S[0];
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_sched_barrier(0);
@@ -518,7 +520,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
         const double second = __builtin_fma(-in_row.x, v.l, in_row.y) * __builtin_fma(-above.x, v.l, above.y);
         S[0] = __builtin_fma(-second, v.inv_second, S[0]);
       });
-      y = bcast_in_eight((float)S[0]);
+      y = (float)S[0];   // (in the last lane of every rank)
     } else {
       // Several entries per lane.  Every pair has an area of its own in LDS: the pairs of entries of all rows, part by
       // part (rows of equal number modulo TS), so that a lane reads those above its own columns from one of TS addresses.
@@ -595,9 +597,11 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
     float y_other[E];
 #pragma unroll
     for (int p = 0; p < E; ++p)
-      y_other[p] = bpermute(y, other[p] * TS);
+      y_other[p] = bpermute(y, other[p] * TS + (KC == 1 ? TS - 1 : 0));
     float sumy = y, vy = formed_here(v * y);
     over_ranks_sums<TS>(vy, sumy);
+    if constexpr (KC == 1)
+      y = is_rank ? last_of_eight(y) : 0.0f;
     float yk[E], yrep[E], hp[E];
 #pragma unroll
     for (int p = 0; p < E; ++p) {
