@@ -173,10 +173,28 @@ __device__ inline void give_up(const PlanArgs &a, unsigned long long *avail_stat
 // ---- a slice's tables in LDS ----
 // One ranking slot per (wave, replicated set, chunk of 64 indices), K chunks per wave.
 constexpr int64_t kLongestSlice = 16 * kPlanThreads;   // 16 chunks per wave
+constexpr int kLongChunks = 8, kLongPasses = 8;        // of a long slice: chunks per wave and pass, passes
+constexpr int kFewestLongSlices = 64;
+constexpr int64_t kLongestOfLongSlices = kLongPasses * kLongChunks * kPlanThreads;
+// (K = 0: a long slice, without its records, which lie behind the rest)
+constexpr int slice_record_bytes(int k) { return k > 0 ? rank_record_bytes_single(k) : 0; }
 template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
-  return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * rank_record_bytes_single(K) +
+  return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * slice_record_bytes(K) +
          (size_t)(n_logical + 2) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
          (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t);
+}
+// A long slice's records per (wave, replicated set): the bitmaps of a pass's chunks, and what a token's ordinal is made of (a
+// bitmap and the tokens before it), both padded for the LDS banks; sixteen sets are worked on at once.
+constexpr int kLongBitsBytes = kLongChunks * 8 + 8, kLongRanksBytes = kLongChunks * 16 + 16;
+__host__ __device__ constexpr int long_slice_padded_sets(int n_rep) { return n_rep / 16 * 16 + 16; }   // at least one more: of tokens without a set
+__host__ __device__ constexpr size_t long_slice_records_at(int n_logical, int n_rep) {
+  return ((size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)(n_logical + 2) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
+          (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t) + 15) / 16 * 16;
+}
+inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
+  return long_slice_records_at(n_logical, n_rep) +
+         (size_t)kPlanWaves * (long_slice_padded_sets(n_rep) * (kLongBitsBytes + kLongRanksBytes + sizeof(int32_t)) + 2 * hist_words * sizeof(int32_t)) +
+         (size_t)(n_logical + 16) / 16 * 16;
 }
 struct SliceTables {
   RepEntry *reps;           // [R + 1]
@@ -191,12 +209,14 @@ template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, 
   SliceTables t;
   t.reps = reinterpret_cast<RepEntry *>(lds);
   t.records = lds + (size_t)(R + 1) * sizeof(RepEntry);
-  t.route = reinterpret_cast<Route *>(t.records + (size_t)kPlanWaves * (R + 1) * rank_record_bytes_single(K));
+  t.route = reinterpret_cast<Route *>(t.records + (size_t)kPlanWaves * (R + 1) * slice_record_bytes(K));
   t.hist = reinterpret_cast<int32_t *>(t.route + ((nl + 2) & ~1));   // (16-byte aligned, as what lies before it is)
   t.set_expert = t.hist + nl / 16 * 16 + 16;
   t.before = t.set_expert + R;
   t.total = t.before + R;
   t.wave_total = t.total + R;
+  if (K == 0)
+    t.records = lds + long_slice_records_at(nl, R);
   return t;
 }
 
@@ -248,7 +268,7 @@ __device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t
   {
     const i32x4 zero{0, 0, 0, 0};
     i32x4 *z = reinterpret_cast<i32x4 *>(t.records);
-    for (int i = tid; i < kPlanWaves * (R + 1) * rank_record_bytes_single(K) / 16; i += nt)
+    for (int i = tid; i < kPlanWaves * (R + 1) * slice_record_bytes(K) / 16; i += nt)
       z[i] = zero;
   }
   for (int q = tid; q < R; q += nt) {
@@ -504,7 +524,8 @@ template <int N> __device__ inline void over_slices_of_unit(uint32_t (&v)[N], in
 // Words 2 (lane % lanes of a slice) and the next of the rows from `rows` on (16-byte aligned; lanes past the last of `words` words,
 // an even number, repeat that), over the slices of block `block`: the four counts added up over the slices into sums[0..3]
 // and, if BEFORE, over the slices before `slice` into sums[4..7].  Whole waves; false: some never came.
-template <bool BEFORE>
+// LONG: slices of up to kLongestOfLongSlices indices.
+template <bool BEFORE, bool LONG>
 __device__ inline bool add_up_unit(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int block, uint32_t tag,
                                    int slice, int lane, uint32_t (&sums)[BEFORE ? 8 : 4]) {
   if (a.expected_slices != a.n_slices)   // (an injected fault: one slice never comes)
@@ -530,19 +551,37 @@ __device__ inline bool add_up_unit(const PlanArgs &a, const unsigned long long *
       break;
     __builtin_amdgcn_s_sleep(1);
   }
-  // (two counts to a word: of four slices they stay below 2^16)
-  static_assert(kUnitLoads * kLongestSlice < 65536, "sums of two 16-bit counts side by side");
-  u32x2 total{0, 0}, before{0, 0};
+  if constexpr (LONG) {
+    static_assert(kLongestOfLongSlices < 65536, "two counts to a word");
 #pragma unroll
-  for (int k = 0; k < kUnitLoads; ++k) {
-    const int p = p0 + k * per_round;
-    const u32x2 counts{v[k].x, v[k].z};
-    total += p < a.n_slices ? counts : u32x2{0, 0};
-    before += BEFORE && p < slice ? counts : u32x2{0, 0};
+    for (int j = 0; j < (BEFORE ? 8 : 4); ++j)
+      sums[j] = 0;
+#pragma unroll
+    for (int k = 0; k < kUnitLoads; ++k) {
+      const int p = p0 + k * per_round;
+      const uint32_t counts[4] = {v[k].x & 0xffffu, v[k].x >> 16, v[k].z & 0xffffu, v[k].z >> 16};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        sums[j] += p < a.n_slices ? counts[j] : 0u;
+        if constexpr (BEFORE)
+          sums[4 + j] += p < slice ? counts[j] : 0u;
+      }
+    }
+  } else {
+    // (two counts to a word: of four slices they stay below 2^16)
+    static_assert(kUnitLoads * kLongestSlice < 65536, "sums of two 16-bit counts side by side");
+    u32x2 total{0, 0}, before{0, 0};
+#pragma unroll
+    for (int k = 0; k < kUnitLoads; ++k) {
+      const int p = p0 + k * per_round;
+      const u32x2 counts{v[k].x, v[k].z};
+      total += p < a.n_slices ? counts : u32x2{0, 0};
+      before += BEFORE && p < slice ? counts : u32x2{0, 0};
+    }
+    sums[0] = total.x & 0xffffu, sums[1] = total.x >> 16, sums[2] = total.y & 0xffffu, sums[3] = total.y >> 16;
+    if constexpr (BEFORE)
+      sums[4] = before.x & 0xffffu, sums[5] = before.x >> 16, sums[6] = before.y & 0xffffu, sums[7] = before.y >> 16;
   }
-  sums[0] = total.x & 0xffffu, sums[1] = total.x >> 16, sums[2] = total.y & 0xffffu, sums[3] = total.y >> 16;
-  if constexpr (BEFORE)
-    sums[4] = before.x & 0xffffu, sums[5] = before.x >> 16, sums[6] = before.y & 0xffffu, sums[7] = before.y >> 16;
   over_slices_of_unit(sums, a.unit_lanes_log2);
   return __all(all_in);
 }
@@ -561,6 +600,192 @@ __device__ inline bool collect_totals(const PlanArgs &a, int32_t *counts, uint32
       counts[e] = (int32_t)count[0];
   }
   return true;
+}
+
+// What others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
+// those that add them up; the tokens of each replicated set before this slice and in the whole batch.
+// (long slices take the two apart)
+enum class Units { kAll, kTotals, kSets };
+template <bool LONG, Units WHICH>
+__device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceTables &t, int slice, uint32_t tag, int lane, int wave_s,
+                                                 int *missing, int *block_sums) {
+  const int nl = a.sh.n_logical, R = a.n_rep, set_lanes = a.set_words;
+  unsigned long long *set_rows = reinterpret_cast<unsigned long long *>(a.sync + kSetRowsAt);
+  unsigned long long *hist_rows = reinterpret_cast<unsigned long long *>(a.sync + kHistRowsAt);
+  const int unit_lanes = 1 << a.unit_lanes_log2, unit_words_log2 = a.unit_lanes_log2 + 1, block_bits = a.unit_block_bits;
+  const int first_word = slice * a.adder_words, my_words = slice < a.adders ? min(a.adder_words, a.hist_words - first_word) : 0;
+  const int adder_units = ((my_words + (1 << unit_words_log2) - 1) >> unit_words_log2) << block_bits;
+  const int units = adder_units + (((set_lanes + (1 << unit_words_log2) - 1) >> unit_words_log2) << block_bits);
+  unsigned long long *totals = reinterpret_cast<unsigned long long *>(a.sync + kTotalsAt);
+  for (int unit = kPlanWaves - 1 - wave_s; unit < units; unit += kPlanWaves) {   // the last waves first: the others have published
+    const int block = unit & ((1 << block_bits) - 1);
+    if (block >= a.unit_blocks || (WHICH == Units::kSets && unit < adder_units))
+      continue;
+    if (unit >= adder_units) {
+      if (WHICH == Units::kTotals)
+        break;
+      const int word0 = (unit - adder_units) >> block_bits << unit_words_log2;
+      uint32_t sums[8];
+      if (add_up_unit<true, LONG>(a, set_rows + word0, a.set_words, set_lanes - word0, block, tag, slice, lane, sums)) {
+        const int first_set = 2 * word0 + 4 * lane;
+        if (lane < unit_lanes)   // (words past set_lanes have no sets)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (first_set + j < R) {
+              atomicAdd(&t.total[first_set + j], (int32_t)sums[j]);
+              atomicAdd(&t.before[first_set + j], (int32_t)sums[4 + j]);
+            }
+      } else {
+        missing[0] = 1;
+      }
+    } else {
+      const int at = unit >> block_bits << unit_words_log2, word0 = first_word + at;
+      uint32_t sums[4];
+      if (add_up_unit<false, LONG>(a, hist_rows + word0, a.hist_words, my_words - at, block, tag, slice, lane, sums)) {
+        bool all_in = true;
+        if (a.unit_blocks > 1) {   // (eight words then, in one unit per block: the wave that comes last publishes)
+          if (lane < 4)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              atomicAdd(&block_sums[4 * lane + j], (int32_t)sums[j]);
+          int arrived = 0;
+          if (lane == 0)
+            arrived = atomicAdd(&block_sums[16], 1);
+          all_in = __builtin_amdgcn_readfirstlane(arrived) == a.unit_blocks - 1;
+          if (all_in && lane < 4)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              sums[j] = (uint32_t)block_sums[4 * lane + j];
+        }
+        if (all_in && lane < unit_lanes && 2 * lane < my_words - at)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int e = 2 * word0 + 4 * lane + j;
+            if (e < nl)
+              agent_store(totals + e, tagged_word(tag, sums[j]));
+          }
+      } else {
+        missing[0] = 1;
+      }
+    }
+  }
+}
+
+// By one wave of a slice that has every slice's counts.
+__device__ __forceinline__ void say_that_all_arrived(const PlanArgs &a, uint32_t tag, int lane) {
+  // Every slice has published its counts; once the LP workgroups have shown up too, no workgroup waits for one that is
+  // not resident yet.  Tell the host, which then stops counting this launch against what the GPU can hold at
+  // once (a posted write to host memory).  Told at the end, behind the LP, plans on several streams found the GPU
+  // full more often and ran as the chain: [16384 x 8] at 32 ranks in turn on 4 streams 11.0 us a plan, 0.34 of them
+  // as one launch; told here 9.9 us, 0.50.
+  uint32_t here[1];
+  if (collect_words<1>(here, tag, lane < a.n_lp_workgroups, a.max_polls,
+                       [&](int) { return reinterpret_cast<const unsigned long long *>(a.sync + kLpHereAt) + lane; }))
+    __hip_atomic_store(a.arrived_word, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// The LP's shares: every set's thread polls its own; value and tag arrive in the same word.  missing[1]: some will not come.
+__device__ __forceinline__ void collect_shares(const PlanArgs &a, const SliceTables &t, int slice, int gen, unsigned long long *avail_state,
+                                               int *missing, int tid) {
+  const int R = a.n_rep;
+  const unsigned long long *shares = reinterpret_cast<const unsigned long long *>(a.sync + kSharesAt);
+  const uint32_t tag_valid = share_tag((uint32_t)gen), tag_none = tag_valid + 1u;
+  for (int i = tid; i < R; i += kPlanThreads) {
+    const SetOfPlan s = set_of_plan(a, i);
+    const unsigned long long *word_at = shares + (slice & (a.n_share_copies - 1)) * kMaxShares + s.ep_rank * a.sh.D + s.d;
+    unsigned long long word = 0;
+    int polls = 0;
+    uint32_t got = 0;
+    while ((got = (uint32_t)((word = agent_load(word_at)) >> 32)) != tag_valid && got != tag_none && ++polls < a.max_polls)
+      __builtin_amdgcn_s_sleep(1);
+    if (got == tag_valid) {
+      t.reps[R - 1 - i].expected = expected_on_original(__builtin_bit_cast(float, (uint32_t)word), t.total[R - 1 - i]);
+    } else {
+      if (got != tag_none)
+        give_up(a, avail_state);
+      missing[1] = 1;
+    }
+  }
+}
+// The slice has read all it reads of this block of words.  (By a whole wave: the same word from every lane is one store.)
+__device__ __forceinline__ void slice_has_read_all(const PlanArgs &a, int slice, int gen, int wave_s) {
+  if (slice == 0 && wave_s == 0) {
+    // Every slice's counts and every LP's shares carry this launch's tag, so every workgroup has read it: the
+    // next launch takes the next one.
+    agent_store(a.sync + kGenAt, (gen + 1) & 0x3fffffff);
+    agent_store(reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (1 - (gen & 1)), 0ull);
+    unsigned long long *advanced = reinterpret_cast<unsigned long long *>(a.sync + kAdvancedAt);
+    agent_store(advanced, tagged_word(a.seq >= 0 ? (uint32_t)a.seq : (uint32_t)(agent_load(advanced) >> 32), (gen + 1) & 0x3fffffff));
+  } else if (wave_s == 0 && a.seq >= 0) {
+    agent_store(a.sync + kDoneAt + slice * kDoneStride, a.seq);
+  }
+}
+
+// An LP workgroup of a plan: one wave per LP, the others help to collect the counts.
+template <int GM, int DM, bool EXACT>
+__device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *smem_raw, int *rep_of_edge_all, int *missing,
+                                             unsigned long long gen_and_poison, int tid, int lane, int wave_s) {
+  const int nl = a.sh.n_logical, pid = blockIdx.x;
+  unsigned long long *shares = reinterpret_cast<unsigned long long *>(a.sync + kSharesAt);
+  SolveArgs sa = a.solve;
+  const int first_lp = pid * kLpsPerWorkgroup;          // of this workgroup
+  const int n_lps = min(kLpsPerWorkgroup, sa.n_units - first_lp);
+  LPLB_PLAN_STAMP(0);
+  if (tid == kPlanThreads - kWave)   // (a wave without an LP)
+    agent_store(reinterpret_cast<unsigned long long *>(a.sync + kLpHereAt) + pid, tagged_word((uint32_t)gen_and_poison + 1u, 0));
+  // dynamic LDS of an LP workgroup: [LP wave][pivot rows | assembly tile], then the counts
+  constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
+  static_assert(kLpArea % 16 == 0, "the LP waves' areas keep 16-byte alignment");
+  unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
+  float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
+  sa.launch = (uint32_t)gen_and_poison;
+  auto switched_off = [&]() { return (gen_and_poison >> 32) != 0; };
+  // Own-histogram mode: the LP waves' table loads are on their way when they and the other waves turn to the
+  // batch's histogram.  (Switched off: no slice will publish.)
+  auto counts_have_come = [&]() -> bool {
+    if (tid >= kPlanThreads - 4)   // the zeros behind the counts
+      reinterpret_cast<int32_t *>(staged)[nl + tid - (kPlanThreads - 4)] = 0;
+    worked_out_here(gen_and_poison);
+    const bool mine = !switched_off() && collect_totals(a, reinterpret_cast<int32_t *>(staged), (uint32_t)gen_and_poison + 1u, tid, wave_s);
+    if (!mine && lane == 0)
+      missing[0] = 1;
+    __syncthreads();
+    return missing[0] == 0;
+  };
+  if (a.local_counts) {
+    if (tid == 0)
+      missing[0] = 0;
+    __syncthreads();
+  }
+  LPLB_PLAN_STAMP(1);
+  if (wave_s < n_lps) {
+    // (own-histogram mode: every LP of the batch reads the one staged copy)
+    float *mine = a.local_counts ? staged : staged + (size_t)wave_s * sa.staged_stride;
+    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
+        sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave, reinterpret_cast<double *>(my_area),
+        reinterpret_cast<float *>(my_area + lp_pivot_doubles<GM, DM>() * sizeof(double)), counts_have_come);
+    worked_out_here(gen_and_poison);
+    unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen_and_poison & 1);
+    if (n_ok < 0) {
+      // no counts, no solution: tell the slices not to wait for this LP's shares
+      if (wave_s == 0 && lane == 0 && !switched_off())
+        give_up(a, avail_state);
+      const int n_edges = sa.G * sa.D;
+      for (int j = lane; j < n_edges; j += kWave)
+        for (int k = 0; k < a.n_share_copies; ++k)
+          agent_store(shares + (int64_t)k * kMaxShares + (int64_t)(first_lp + wave_s) * n_edges + j,
+                      (unsigned long long)(share_tag(sa.launch) + 1u) << 32);
+    } else if (lane == 0 && n_ok > 0 && !switched_off()) {
+      // feasible: count it for the caller unless some workgroup has already given up on this batch
+      const unsigned long long before = __hip_atomic_fetch_or(avail_state, 1ull << (first_lp + wave_s), __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT);
+      if (!(before & kGaveUp))
+        atomicAdd(a.avail, n_ok);
+    }
+    if (lane == 0 && a.seq >= 0)
+      agent_store(a.sync + kDoneAt + (kMaxSlices + first_lp + wave_s) * kDoneStride, a.seq);
+  } else if (a.local_counts) {
+    counts_have_come();
+  }
 }
 
 // K: 64-index chunks per wave.
@@ -584,70 +809,10 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   // are on their way.
   static_assert(kGenAt == 0 && kPoisonAt == 1, "one word");
   unsigned long long gen_and_poison = agent_load(reinterpret_cast<const unsigned long long *>(a.sync));
-  unsigned long long *shares = reinterpret_cast<unsigned long long *>(a.sync + kSharesAt);
 
   if (pid < a.n_lp_workgroups) {
     // ------------------------------------------------------------ the LPs
-    SolveArgs sa = a.solve;
-    const int first_lp = pid * kLpsPerWorkgroup;          // of this workgroup
-    const int n_lps = min(kLpsPerWorkgroup, sa.n_units - first_lp);
-    LPLB_PLAN_STAMP(0);
-    if (tid == kPlanThreads - kWave)   // (a wave without an LP)
-      agent_store(reinterpret_cast<unsigned long long *>(a.sync + kLpHereAt) + pid, tagged_word((uint32_t)gen_and_poison + 1u, 0));
-    // dynamic LDS of an LP workgroup: [LP wave][pivot rows | assembly tile], then the counts
-    constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
-    static_assert(kLpArea % 16 == 0, "the LP waves' areas keep 16-byte alignment");
-    unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
-    float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
-    sa.launch = (uint32_t)gen_and_poison;
-    auto switched_off = [&]() { return (gen_and_poison >> 32) != 0; };
-    // Own-histogram mode: the LP waves' table loads are on their way when they and the other waves turn to the
-    // batch's histogram.  (Switched off: no slice will publish.)
-    auto counts_have_come = [&]() -> bool {
-      if (tid >= kPlanThreads - 4)   // the zeros behind the counts
-        reinterpret_cast<int32_t *>(staged)[nl + tid - (kPlanThreads - 4)] = 0;
-      worked_out_here(gen_and_poison);
-      const bool mine = !switched_off() && collect_totals(a, reinterpret_cast<int32_t *>(staged), (uint32_t)gen_and_poison + 1u, tid, wave_s);
-      if (!mine && lane == 0)
-        missing[0] = 1;
-      __syncthreads();
-      return missing[0] == 0;
-    };
-    if (a.local_counts) {
-      if (tid == 0)
-        missing[0] = 0;
-      __syncthreads();
-    }
-    LPLB_PLAN_STAMP(1);
-    if (wave_s < n_lps) {
-      // (own-histogram mode: every LP of the batch reads the one staged copy)
-      float *mine = a.local_counts ? staged : staged + (size_t)wave_s * sa.staged_stride;
-      const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
-          sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave, reinterpret_cast<double *>(my_area),
-          reinterpret_cast<float *>(my_area + lp_pivot_doubles<GM, DM>() * sizeof(double)), counts_have_come);
-      worked_out_here(gen_and_poison);
-      unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen_and_poison & 1);
-      if (n_ok < 0) {
-        // no counts, no solution: tell the slices not to wait for this LP's shares
-        if (wave_s == 0 && lane == 0 && !switched_off())
-          give_up(a, avail_state);
-        const int n_edges = sa.G * sa.D;
-        for (int j = lane; j < n_edges; j += kWave)
-          for (int k = 0; k < a.n_share_copies; ++k)
-            agent_store(shares + (int64_t)k * kMaxShares + (int64_t)(first_lp + wave_s) * n_edges + j,
-                        (unsigned long long)(share_tag(sa.launch) + 1u) << 32);
-      } else if (lane == 0 && n_ok > 0 && !switched_off()) {
-        // feasible: count it for the caller unless some workgroup has already given up on this batch
-        const unsigned long long before = __hip_atomic_fetch_or(avail_state, 1ull << (first_lp + wave_s), __ATOMIC_RELAXED,
-                                                                 __HIP_MEMORY_SCOPE_AGENT);
-        if (!(before & kGaveUp))
-          atomicAdd(a.avail, n_ok);
-      }
-      if (lane == 0 && a.seq >= 0)
-        agent_store(a.sync + kDoneAt + (kMaxSlices + first_lp + wave_s) * kDoneStride, a.seq);
-    } else if (a.local_counts) {
-      counts_have_come();
-    }
+    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, missing, gen_and_poison, tid, lane, wave_s);
     LPLB_PLAN_STAMP(2);
     return;
   }
@@ -718,61 +883,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   // ---- what others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
   //      those that add them up; the tokens of each replicated set before this slice and in the whole batch ----
   if (!poisoned) {
-    const int unit_lanes = 1 << a.unit_lanes_log2, unit_words_log2 = a.unit_lanes_log2 + 1, block_bits = a.unit_block_bits;
-    const int first_word = slice * a.adder_words, my_words = slice < a.adders ? min(a.adder_words, a.hist_words - first_word) : 0;
-    const int adder_units = ((my_words + (1 << unit_words_log2) - 1) >> unit_words_log2) << block_bits;
-    const int units = adder_units + (((set_lanes + (1 << unit_words_log2) - 1) >> unit_words_log2) << block_bits);
-    unsigned long long *totals = reinterpret_cast<unsigned long long *>(a.sync + kTotalsAt);
-    for (int unit = kPlanWaves - 1 - wave_s; unit < units; unit += kPlanWaves) {   // the last waves first: the others have published
-      const int block = unit & ((1 << block_bits) - 1);
-      if (block >= a.unit_blocks)
-        continue;
-      if (unit >= adder_units) {
-        const int word0 = (unit - adder_units) >> block_bits << unit_words_log2;
-        uint32_t sums[8];
-        if (add_up_unit<true>(a, set_rows + word0, a.set_words, set_lanes - word0, block, tag, slice, lane, sums)) {
-          const int first_set = 2 * word0 + 4 * lane;
-          if (lane < unit_lanes)   // (words past set_lanes have no sets)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (first_set + j < R) {
-                atomicAdd(&t.total[first_set + j], (int32_t)sums[j]);
-                atomicAdd(&t.before[first_set + j], (int32_t)sums[4 + j]);
-              }
-        } else {
-          missing[0] = 1;
-        }
-      } else {
-        const int at = unit >> block_bits << unit_words_log2, word0 = first_word + at;
-        uint32_t sums[4];
-        if (add_up_unit<false>(a, hist_rows + word0, a.hist_words, my_words - at, block, tag, slice, lane, sums)) {
-          bool all_in = true;
-          if (a.unit_blocks > 1) {   // (eight words then, in one unit per block: the wave that comes last publishes)
-            if (lane < 4)
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                atomicAdd(&block_sums[4 * lane + j], (int32_t)sums[j]);
-            int arrived = 0;
-            if (lane == 0)
-              arrived = atomicAdd(&block_sums[16], 1);
-            all_in = __builtin_amdgcn_readfirstlane(arrived) == a.unit_blocks - 1;
-            if (all_in && lane < 4)
-#pragma unroll
-              for (int j = 0; j < 4; ++j)
-                sums[j] = (uint32_t)block_sums[4 * lane + j];
-          }
-          if (all_in && lane < unit_lanes && 2 * lane < my_words - at)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const int e = 2 * word0 + 4 * lane + j;
-              if (e < nl)
-                agent_store(totals + e, tagged_word(tag, sums[j]));
-            }
-        } else {
-          missing[0] = 1;
-        }
-      }
-    }
+    add_up_published<false, Units::kAll>(a, t, slice, tag, lane, wave_s, missing, block_sums);
   }
   if (adds_totals)
     SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
@@ -790,17 +901,8 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     for (int q = tid; q < R; q += kPlanThreads)
       set_total(t.reps[q], t.total[q]);
     SliceTokens<K>::add_starts(a, t, my_records, lane, wave_s);
-    if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word) {
-      // Every slice has published its counts; once the LP workgroups have shown up too, no workgroup waits for one that is
-      // not resident yet.  Tell the host, which then stops counting this launch against what the GPU can hold at
-      // once (a posted write to host memory).  Told at the end, behind the LP, plans on several streams found the GPU
-      // full more often and ran as the chain: [16384 x 8] at 32 ranks in turn on 4 streams 11.0 us a plan, 0.34 of them
-      // as one launch; told here 9.9 us, 0.50.
-      uint32_t here[1];
-      if (collect_words<1>(here, tag, lane < a.n_lp_workgroups, a.max_polls,
-                           [&](int) { return reinterpret_cast<const unsigned long long *>(a.sync + kLpHereAt) + lane; }))
-        __hip_atomic_store(a.arrived_word, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word)
+      say_that_all_arrived(a, tag, lane);
     if (slice == 0 && !collect_totals(a, t.hist, tag, tid, wave_s)) {   // for the caller (and for the counts below)
       if (lane == 0)
         give_up(a, avail_state);
@@ -828,37 +930,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     }
     LPLB_PLAN_STAMP(4);
     // ---- the LP's shares: every set's thread polls its own; value and tag arrive in the same word ----
-    const uint32_t tag_valid = share_tag((uint32_t)gen), tag_none = tag_valid + 1u;
-    for (int i = tid; i < R; i += kPlanThreads) {
-      const SetOfPlan s = set_of_plan(a, i);
-      const unsigned long long *word_at = shares + (slice & (a.n_share_copies - 1)) * kMaxShares + s.ep_rank * a.sh.D + s.d;
-      unsigned long long word = 0;
-      int polls = 0;
-      uint32_t got = 0;
-      while ((got = (uint32_t)((word = agent_load(word_at)) >> 32)) != tag_valid && got != tag_none && ++polls < a.max_polls)
-        __builtin_amdgcn_s_sleep(1);
-      if (got == tag_valid) {
-        t.reps[R - 1 - i].expected = expected_on_original(__builtin_bit_cast(float, (uint32_t)word), t.total[R - 1 - i]);
-      } else {
-        if (got != tag_none)
-          give_up(a, avail_state);
-        missing[1] = 1;
-      }
-    }
+    collect_shares(a, t, slice, gen, avail_state, missing, tid);
     __syncthreads();
     LPLB_PLAN_STAMP(5);
     ok = missing[1] == 0;
-    // (by a whole wave: the same word from every lane is one store)
-    if (slice == 0 && wave_s == 0) {
-      // Every slice's counts and every LP's shares carry this launch's tag, so every workgroup has read it: the
-      // next launch takes the next one.
-      agent_store(a.sync + kGenAt, (gen + 1) & 0x3fffffff);
-      agent_store(reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (1 - (gen & 1)), 0ull);
-      unsigned long long *advanced = reinterpret_cast<unsigned long long *>(a.sync + kAdvancedAt);
-      agent_store(advanced, tagged_word(a.seq >= 0 ? (uint32_t)a.seq : (uint32_t)(agent_load(advanced) >> 32), (gen + 1) & 0x3fffffff));
-    } else if (wave_s == 0 && a.seq >= 0) {
-      agent_store(a.sync + kDoneAt + slice * kDoneStride, a.seq);
-    }
+    slice_has_read_all(a, slice, gen, wave_s);
   }
   LPLB_PLAN_STAMP(6);
   // ---- choose and store; if a wait ran out, every token goes to its original slot ----
@@ -878,6 +954,279 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   if (slice == 0 && a.physical_counts)
     plan_physical_counts(a, t, tl.physical_le0, ok, tid);
   store_chunks<K>(o, a.out, w0, end, lane);
+  LPLB_PLAN_STAMP(7);
+  LPLB_SLICE_STAMP(3);
+}
+
+// Slices of more than kLongestSlice indices (batches of more than 256 x 8192 on 256 CUs): the same exchange, with the tokens of
+// a wave in passes of eight chunks.  The chain reads the indices twice and leaves the memory idle while its LP runs; here they
+// are read once and stay in registers (11 bits of expert, 12 of ordinal among the wave's tokens of the set), and the ordinals
+// are worked out while the LP is running.  At 8 ranks, as the chain and so: [1048576 x 8] 41.7 and 33.5 us; 2097153 indices in 256
+// slices 22.7 and 17.3, 4200000 30.5 and 23.3; 524289 in 64 slices 21.8 and 16.6, 1280000 27.9 and 22.4.  Read 9.3 and written 11.2 us
+// by kernels that do nothing else.  What bounds it: 10.5 us until the last index is
+// counted, 4 until the LP has the totals, 5 until its shares are seen, then the choice and the stores (9) with the second half
+// of the ordinals between them: a pass of those is about 1 us a wave, waits for the LDS and instructions in
+// turn.  With every pass unrolled, for the registers' sake, the code is 58 KiB, nearly the instruction cache of two CUs.
+// The histogram is per wave: what is in the waves before then costs nothing more than the sums, and
+// a lookup of the set beside the histogram's update made the counting twice as long (the LDS serves them in turn).
+template <int GM, int DM, bool EXACT>
+__global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void plan_of_long_slices(PlanArgs a) {
+  constexpr int K = kLongChunks;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
+  __shared__ int missing[2];
+  __shared__ int block_sums[17];
+  const int nl = a.sh.n_logical, R = a.n_rep;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
+  const int pid = blockIdx.x;
+  fetch_arguments_now(a.idx, a.unit_blocks, a.sh.G, a.solve.workload, a.solve.n_group, a.solve.tagged_result, a.sync);
+  unsigned long long gen_and_poison = agent_load(reinterpret_cast<const unsigned long long *>(a.sync));
+  if (pid < a.n_lp_workgroups) {
+    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, missing, gen_and_poison, tid, lane, wave_s);
+    return;
+  }
+  const int slice = pid - a.n_lp_workgroups;
+  const SliceTables t = carve_tables<0>(smem_raw, nl, R);
+  const int hist_len = 2 * a.hist_words, padded_sets = long_slice_padded_sets(R);
+  // [waves][padded_sets][kLongBitsBytes], [waves][padded_sets][kLongRanksBytes], [waves][padded_sets], [waves][hist_len], [n_logical + 1]
+  unsigned char *my_bits = t.records + wave_s * padded_sets * kLongBitsBytes;
+  unsigned char *my_ranks = t.records + kPlanWaves * padded_sets * kLongBitsBytes + wave_s * padded_sets * kLongRanksBytes;
+  int32_t *my_so_far = reinterpret_cast<int32_t *>(t.records + kPlanWaves * padded_sets * (kLongBitsBytes + kLongRanksBytes)) + wave_s * padded_sets;
+  int32_t *wave_hists = my_so_far + (kPlanWaves - wave_s) * padded_sets;
+  int32_t *my_hist = wave_hists + wave_s * hist_len;
+  unsigned char *set_of_expert = reinterpret_cast<unsigned char *>(wave_hists + kPlanWaves * hist_len);   // four to a word: lanes rarely meet in a bank
+  const int64_t begin = slice_begin(a.n, a.per, slice);
+  const int64_t end = slice_begin(a.n, a.per, slice + 1);
+  const int wave_len = (int)(a.per + kPlanThreads - 1) / kPlanThreads * kWave;   // this wave's indices, whole chunks
+  const int64_t w0 = begin + (int64_t)wave_s * wave_len;
+  const int last = (int)(min(end, w0 + wave_len) - 1 - w0);   // place of its last index; -1 and less: it has none
+  const int passes = (wave_len + K * kWave - 1) / (K * kWave);
+  LPLB_PLAN_STAMP(0);
+  LPLB_SLICE_STAMP(0);
+  __builtin_amdgcn_s_setprio(2);
+
+  const PlanTableLoads tl = issue_plan_table_loads(a, tid);
+  // (places past the last repeat it: without a branch the loads of the next pass stay on their way while one is counted)
+  const int64_t *mine = a.idx + w0;
+  auto load_pass = [&](int64_t (&v)[K], int p) {
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      v[c] = __builtin_nontemporal_load(mine + min((p * K + c) * kWave + lane, last));
+  };
+  int64_t raw[2][K];
+  load_pass(raw[0], 0);
+  if (tid == 0) {
+    missing[0] = 0;
+    missing[1] = 0;
+  }
+  if (tid < 17)
+    block_sums[tid] = 0;
+  for (int q = lane; q < padded_sets; q += kWave)
+    my_so_far[q] = 0;
+  for (int e = lane; e < hist_len; e += kWave)
+    my_hist[e] = 0;
+  for (int i = lane; i < padded_sets * kLongBitsBytes / 8; i += kWave)
+    reinterpret_cast<unsigned long long *>(my_bits)[i] = 0ull;
+  build_plan_tables<0>(a, t, tl, tid);
+  for (int e = tid; e <= nl; e += kPlanThreads)   // (read behind the next barrier)
+    set_of_expert[e] = (unsigned char)t.route[e].rep;
+  LPLB_PLAN_STAMP(10);
+
+  // ---- the tokens: every wave counts its own ----
+  uint32_t token[kLongPasses * K];   // expert; later with the token's ordinal among the wave's tokens of its set in the high half
+#pragma unroll
+  for (int p = 0; p < kLongPasses; ++p) {
+    load_pass(raw[(p + 1) & 1], min(p + 1, passes - 1));
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const int64_t v = raw[p & 1][c];
+      const bool valid = (uint64_t)v < (uint64_t)nl && (p * K + c) * kWave + lane <= last;   // -1, other negatives and too large ids fail
+      token[p * K + c] = valid ? (uint32_t)v : (uint32_t)nl;
+      if (valid)
+        atomicAdd(&my_hist[token[p * K + c]], 1);
+    }
+    if (p + 1 >= passes)
+      break;
+  }
+  __syncthreads();
+  LPLB_PLAN_STAMP(8);
+  LPLB_SLICE_STAMP(1);
+  worked_out_here(gen_and_poison);
+  const int gen = (int)(uint32_t)gen_and_poison;
+  const bool poisoned = (gen_and_poison >> 32) != 0;
+  const uint32_t tag = (uint32_t)gen + 1u;
+  unsigned long long *avail_state = reinterpret_cast<unsigned long long *>(a.sync + kAvailAt) + (gen & 1);
+  if (wave_s >= kPlanWaves / 2)   // (they publish sets and add up totals while the others are at their ordinals already)
+    __builtin_amdgcn_s_setprio(3);
+  if (!poisoned) {
+    unsigned long long *set_rows = reinterpret_cast<unsigned long long *>(a.sync + kSetRowsAt);
+    unsigned long long *hist_rows = reinterpret_cast<unsigned long long *>(a.sync + kHistRowsAt);
+    constexpr int kHalf = kPlanThreads / 2;
+    if (tid < kHalf) {
+      for (int e2 = tid; e2 < a.hist_words; e2 += kHalf) {
+        int2 both{0, 0};
+#pragma unroll
+        for (int w = 0; w < kPlanWaves; ++w) {
+          const int2 of_wave = reinterpret_cast<const int2 *>(wave_hists + w * hist_len)[e2];
+          both.x += of_wave.x;
+          both.y += of_wave.y;
+        }
+        agent_store(hist_rows + slice * a.hist_words + e2, tagged_word(tag, (uint32_t)both.x | (uint32_t)both.y << 16));
+      }
+    } else {
+      // lane = (word, set of its two, wave): what is in the waves before, and the word from the lane that has the last wave's
+      for (int i = tid - kHalf; i < 16 * a.set_words; i += kHalf) {
+        const int w = i % kPlanWaves, q = i / kPlanWaves, x = q < R ? t.set_expert[q] : nl;
+        const int own = x < nl ? wave_hists[w * hist_len + x] : 0;
+        const int before = group_exclusive_scan<kPlanWaves>(own, w);
+        if (q < R)
+          t.wave_total[w * R + q] = before;   // (in a long slice: in the waves before)
+        const int first = row_shr<8>(before + own);
+        if (i % 16 == 15)
+          agent_store(set_rows + slice * a.set_words + i / 16, tagged_word(tag, (uint32_t)first | (uint32_t)(before + own) << 16));
+      }
+    }
+  } else if (slice == 0 && tid == 0) {
+    agent_add(a.sync + kTimeoutsAt, 1);   // one more plan that this block of words could not serve
+  }
+  LPLB_PLAN_STAMP(1);
+  LPLB_SLICE_STAMP(2);
+  if (!poisoned)
+    add_up_published<true, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+  // ---- while the others' words are on their way: ordinals among the wave's tokens, pass by pass (the wave's own records: no barrier) ----
+  __builtin_amdgcn_s_setprio(2);
+  const uint32_t my_bit = 1u << lane % 32;
+  unsigned char *my_half_of_bits = my_bits + lane / 32 * 4;
+  const int c_of_lane = lane % K;
+  auto rank_pass = [&](int p) {
+    uint32_t set[K];
+    // (all reads ahead of the first update: the compiler keeps their order, and each would be waited for)
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      set[c] = set_of_expert[token[p * K + c]];
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      if (set[c] < (uint32_t)R)
+        atomicOr(reinterpret_cast<uint32_t *>(my_half_of_bits + __umul24(set[c], (uint32_t)kLongBitsBytes) + c * 8), my_bit);
+    }
+    SliceTokens<K>::own_slots_are_written();
+    // lane = (set, chunk), chunk fastest, two sets side by side; the bitmaps are empty again behind it
+    unsigned char *bits_at = my_bits + (lane / K) * kLongBitsBytes + c_of_lane * 8;
+    unsigned char *ranks_at = my_ranks + (lane / K) * kLongRanksBytes + c_of_lane * 16;
+    int32_t *so_far = my_so_far + lane / K;
+    constexpr int kSets = kWave / K;   // at once
+    for (int q0 = 0; q0 < R; q0 += 2 * kSets) {
+      unsigned long long bits[2];
+      int earlier[2], start[2], own[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        bits[j] = *reinterpret_cast<const unsigned long long *>(bits_at + j * kSets * kLongBitsBytes);
+        earlier[j] = so_far[j * kSets];
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        own[j] = __popcll(bits[j]);
+        start[j] = earlier[j] + group_exclusive_scan<K>(own[j], c_of_lane);
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        *reinterpret_cast<unsigned long long *>(bits_at + j * kSets * kLongBitsBytes) = 0ull;
+        *reinterpret_cast<i32x4 *>(ranks_at + j * kSets * kLongRanksBytes) = i32x4{(int)(uint32_t)bits[j], (int)(uint32_t)(bits[j] >> 32), start[j], 0};
+        if (c_of_lane == K - 1)
+          so_far[j * kSets] = start[j] + own[j];
+      }
+      bits_at += 2 * kSets * kLongBitsBytes;
+      ranks_at += 2 * kSets * kLongRanksBytes;
+      so_far += 2 * kSets;
+    }
+    SliceTokens<K>::own_slots_are_written();
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const i32x4 x = *reinterpret_cast<const i32x4 *>(my_ranks + __umul24(set[c], (uint32_t)kLongRanksBytes) + c * 16);
+      const uint32_t k = (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)x.y, __builtin_amdgcn_mbcnt_lo((uint32_t)x.x, (uint32_t)x.z));
+      token[p * K + c] |= k << 16;   // (without a set: whatever is there)
+      worked_out_here(token[p * K + c]);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < kLongPasses / 2; ++p)
+    if (p < passes)
+      rank_pass(p);
+  if (!poisoned)
+    add_up_published<true, Units::kSets>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+  LPLB_PLAN_STAMP(11);
+  if (poisoned)
+    missing[0] = 1;
+  __syncthreads();
+  LPLB_PLAN_STAMP(2);
+  LPLB_SLICE_STAMP(4);
+  bool ok = missing[0] == 0;   // (the same in every thread)
+  if (!ok && !poisoned && tid == 0)
+    give_up(a, avail_state);
+  int32_t *my_bases = t.wave_total + wave_s * R;
+  if (ok) {
+    for (int q = tid; q < R; q += kPlanThreads)
+      set_total(t.reps[q], t.total[q]);
+    for (int q = lane; q < R; q += kWave)
+      my_bases[q] += t.before[q];
+    if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word)
+      say_that_all_arrived(a, tag, lane);
+    if (slice == 0) {   // for the caller (and for the counts below)
+      if (!collect_totals(a, t.hist, tag, tid, wave_s)) {
+        if (lane == 0)
+          give_up(a, avail_state);
+        missing[1] = 1;
+      }
+      __syncthreads();
+      for (int e = tid; e < nl; e += kPlanThreads)
+        a.totals[e] = t.hist[e];
+    }
+    LPLB_PLAN_STAMP(3);
+    LPLB_PLAN_STAMP(4);
+    collect_shares(a, t, slice, gen, avail_state, missing, tid);
+    __syncthreads();
+    LPLB_PLAN_STAMP(5);
+    ok = missing[1] == 0;
+    slice_has_read_all(a, slice, gen, wave_s);
+  }
+  LPLB_PLAN_STAMP(6);
+  // ---- choose and store; if a wait ran out, every token goes to its original slot ----
+  if (slice == 0 && a.physical_counts)
+    plan_physical_counts(a, t, tl.physical_le0, ok, tid);
+  int64_t *out = a.out + w0;
+  auto store_pass = [&](int p) {
+    int32_t o[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const uint32_t e = token[p * K + c] & 0xffffu, k = token[p * K + c] >> 16;
+      const Route rt = t.route[e];
+      o[c] = rt.original;
+      if (ok) {
+        const RepEntry x = t.reps[rt.rep];   // (without a replica: stays whatever the hash)
+        const int32_t h = ordinal_hash<true>(my_bases[min(rt.rep, R - 1)] + (int32_t)k, x.total, x.magic);
+        o[c] = h >= x.expected ? x.replica : rt.original;
+      }
+    }
+    if ((p + 1) * K * kWave - 1 <= last) {
+#pragma unroll
+      for (int c = 0; c < K; ++c)
+        __builtin_nontemporal_store((int64_t)o[c], out + (p * K + c) * kWave + lane);
+    } else {
+#pragma unroll
+      for (int c = 0; c < K; ++c)
+        if ((p * K + c) * kWave + lane <= last)
+          __builtin_nontemporal_store((int64_t)o[c], out + (p * K + c) * kWave + lane);
+    }
+  };
+  // (the second half's ordinals between the first half's stores, which take longer)
+#pragma unroll
+  for (int p = 0; p < kLongPasses; ++p) {
+    if (p < passes)
+      store_pass(p);
+    if (p < kLongPasses / 2 && p + kLongPasses / 2 < passes)
+      rank_pass(p + kLongPasses / 2);
+  }
   LPLB_PLAN_STAMP(7);
   LPLB_SLICE_STAMP(3);
 }
@@ -1067,9 +1416,11 @@ template <int GM, int DM> static int launch_scan_and_solve(const ScanSolveArgs &
   LPLB_HIP_TRY(hipGetLastError());
   return LPLB_OK;
 }
+// K: as in plan_in_one_launch; 0: long slices.
 template <int GM, int DM, bool EXACT, int K>
 static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
-  const size_t lds_slice = plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);
+  const size_t lds_slice = K > 0 ? plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep)
+                                 : long_slice_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words);
   // LP workgroups: their waves' working areas, then the counts (one copy per LP if they fit,
   // else none and the LPs read global memory; own-histogram mode needs one copy in any case)
   const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
@@ -1084,7 +1435,10 @@ static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   if (lds > (size_t)kPlanLdsLimit)
     return LPLB_OK;
   static KernelFootprint footprint;
-  return launch_plan(plan_in_one_launch<GM, DM, EXACT, K>, footprint, true, a, lds, s, done);
+  if constexpr (K > 0)
+    return launch_plan(plan_in_one_launch<GM, DM, EXACT, K>, footprint, true, a, lds, s, done);
+  else
+    return launch_plan(plan_of_long_slices<GM, DM, EXACT>, footprint, true, a, lds, s, done);
 }
 template <int GM, int DM, bool EXACT, int K> static int launch_plan_single(PlanArgs &a, hipStream_t s, bool *done) {
   const size_t lds = a.solve.n_units * plan_lp_area_bytes<GM, DM>() + plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep);
@@ -1104,7 +1458,8 @@ template <int GM, int DM, bool EXACT> static int launch_plan_shape(PlanArgs &a, 
   return a.per <= 2 * kPlanThreads   ? launch_plan_slices<GM, DM, EXACT, 2>(a, s, done)
          : a.per <= 4 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 4>(a, s, done)
          : a.per <= 8 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 8>(a, s, done)
-                                     : launch_plan_slices<GM, DM, EXACT, 16>(a, s, done);
+         : a.per <= kLongestSlice    ? launch_plan_slices<GM, DM, EXACT, 16>(a, s, done)
+                                     : launch_plan_slices<GM, DM, EXACT, 0>(a, s, done);
 }
 template <int GM, int DM> static int launch_plan_padded_or_not(PlanArgs &a, hipStream_t s, bool *done) {
   return a.sh.G == GM && a.sh.D == DM ? launch_plan_shape<GM, DM, true>(a, s, done) : launch_plan_shape<GM, DM, false>(a, s, done);
