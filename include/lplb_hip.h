@@ -282,8 +282,8 @@ int lplb_map_idx_prepared(const int64_t *idx, const float *o_weight,
  * One batch's whole plan in a single call: what Planner.run does with three
  * extension calls (lplb/planner.py:245-266), with the same results as
  * lplb_count_idx, lplb_solve and lplb_map_idx chained on `stream`.  Batches of up
- * to about two million indices (slices of at most 8192 indices, as many of them as
- * fit the GPU together) with LP shapes up to 32 x 2, up to 32 EP groups and up to 1024
+ * to about eight million indices (slices of at most 8192 indices, of at most 32768 where
+ * n_blocks is at least 64, as many of them as fit the GPU together) with LP shapes up to 32 x 2, up to 32 EP groups and up to 1024
  * logical experts run as ONE kernel launch in which the workgroups exchange their
  * counts and the LP's result through memory; everything else runs as the chain of
  * the three entry points' kernels.

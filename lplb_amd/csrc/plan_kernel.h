@@ -961,7 +961,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 // Slices of more than kLongestSlice indices (batches of more than 256 x 8192 on 256 CUs): the same exchange, with the tokens of
 // a wave in passes of eight chunks.  The chain reads the indices twice and leaves the memory idle while its LP runs; here they
 // are read once and stay in registers (11 bits of expert, 12 of ordinal among the wave's tokens of the set), and the ordinals
-// are worked out while the LP is running.  At 8 ranks, as the chain and so: [1048576 x 8] 41.7 and 33.5 us; 2097153 indices in 256
+// are worked out while the LP is running.  At 8 ranks, as the chain and so: [1048576 x 8] 42 and 33.5-35.1 us; 2097153 indices in 256
 // slices 22.7 and 17.3, 4200000 30.5 and 23.3; 524289 in 64 slices 21.8 and 16.6, 1280000 27.9 and 22.4.  Read 9.3 and written 11.2 us
 // by kernels that do nothing else.  What bounds it: 10.5 us until the last index is
 // counted, 4 until the LP has the totals, 5 until its shares are seen, then the choice and the stores (9) with the second half
