@@ -36,6 +36,7 @@
 // solve_spread.h, in which a rank's row and edges are spread over its 8, 4 or 2 lanes.
 #pragma once
 #include "common.h"
+#include "reciprocal.h"
 
 namespace lplb {
 
@@ -100,12 +101,6 @@ template <int W> __device__ inline float reduce_max(float v) {
   if (W <= 32)
     return fmaxf(readlane(v, 0), readlane(v, 16));
   return fmaxf(fmaxf(readlane(v, 0), readlane(v, 16)), fmaxf(readlane(v, 32), readlane(v, 48)));
-}
-
-// 1/a in fp64: hardware estimate (about 2^-23) + one Newton step.
-__device__ inline double rcp_f64(double a) {
-  double r = __builtin_amdgcn_rcp(a);
-  return __builtin_fma(__builtin_fma(-a, r, 1.0), r, r);
 }
 
 // ---- one LP per wave (ROWS == 1) or one LP per 16-lane DPP row (ROWS == 4) ----

@@ -18,7 +18,7 @@
 //   * pivots are taken two at a time, so that there is one round trip through LDS for two.
 // Measured per affine-scaling step, one wave on the GPU, pivots one by one -> two at a time (and sums without
 // wait states, moves folded into them, no sum over the edges between solution and step length):
-// (8, 2) 0.66 -> 0.54 us, half of it elimination; (16, 2) 1.21 -> 1.15; (32, 2) 2.87 -> 2.53, bound by the number of
+// (8, 2) 0.66 -> 0.55 us, half of it elimination; (16, 2) 1.21 -> 1.13; (32, 2) 2.87 -> 2.54, bound by the number of
 // instructions.  With one lane per rank and edge (8, 2) took 1.15 us.
 // (A form in which rank i is lane i of every 16-lane row and holds its whole row, the elimination made of
 // fp64 multiply-adds with a row_newbcast operand, has pivots of 40 instead of 60 ns and no LDS in them; but
@@ -149,17 +149,6 @@ template <int TS> __device__ inline double rank_partner(double v) {
   q.x = __builtin_amdgcn_mov_dpp(q.x, ctrl, 0xF, 0xF, false);
   q.y = __builtin_amdgcn_mov_dpp(q.y, ctrl, 0xF, 0xF, false);
   return __builtin_bit_cast(double, q);
-}
-
-// 0.999 / d_max in fp64, rounded to fp32 by the caller: quotient by the estimated reciprocal and one correction of it
-// (error about 2^-46, far below the rounding to fp32; the compiler's full division takes four times the instructions, all of
-// them in the chain from one step to the next).  d_max = 0 or infinite gives NaN where the division gives
-// infinity or 0: either way the step leaves the artificial variable without a number below the
-// feasibility limit, so the LP is reported infeasible and its shares are the neutral ones.
-__device__ inline double step_length(double d_max) {
-  const double r = __builtin_amdgcn_rcp(d_max);
-  const double q = 0.999 * r;
-  return __builtin_fma(__builtin_fma(-d_max, q, 0.999), r, q);
 }
 
 // Arguments, LDS contracts and the returned value as for solve_lp; pivot_rows has spread_pivot_doubles(GM)

@@ -361,6 +361,39 @@ extern "C" __global__ void collect(const unsigned long long *words, unsigned tag
     assert kernels >= 14 * 4 + 14 + 1, kernels
 
 
+def test_the_lp_s_reciprocals_have_all_of_fp64(tmp_path):
+    """An LP's step length is rounded to fp32 only at its end (minilp.cu:361 divides in fp64): with the hardware's estimate off by
+    up to 2^-23 either way (v_rcp_f64's bound), the reciprocal keeps an error of that squared and the last roundings,
+    and the quotient, corrected once more, one rounding only.  lplb_amd/csrc/reciprocal.h on the host, against long double."""
+    import subprocess
+    (tmp_path / "reciprocal.cpp").write_text('''
+#define __device__
+static double relative_error;
+static double __builtin_amdgcn_rcp(double a) { return 1.0 / a * (1.0 + relative_error); }
+#include "reciprocal.h"
+extern "C" double step_length_error(double d, double estimate_error) {
+  relative_error = estimate_error;
+  const long double exact = (long double)0.999 / (long double)d;
+  return (double)(((long double)lplb::step_length(d) - exact) / exact);
+}
+extern "C" double reciprocal_error(double d, double estimate_error) {
+  relative_error = estimate_error;
+  return (double)((long double)lplb::rcp_f64(d) * (long double)d - 1.0L);
+}
+''')
+    subprocess.run(["g++", "-O1", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC", f"-I{ROOT / 'lplb_amd' / 'csrc'}",
+                    str(tmp_path / "reciprocal.cpp"), "-o", str(tmp_path / "reciprocal.so")], check=True, capture_output=True)
+    lib = ctypes.CDLL(str(tmp_path / "reciprocal.so"))
+    for fn in (lib.step_length_error, lib.reciprocal_error):
+        fn.restype, fn.argtypes = ctypes.c_double, [ctypes.c_double, ctypes.c_double]
+    rng = np.random.default_rng(0)
+    for d in np.exp(rng.uniform(np.log(1e-30), np.log(1e30), 5000)):
+        off = float(rng.choice([-1, 1, rng.uniform(-1, 1)])) * 2.0 ** -23
+        assert abs(lib.step_length_error(d, off)) <= 1.001 * 2.0 ** -53, (d, off)
+        # the estimate's error squared; one rounding each of the residual (at most 2^-23 of the result) and of the sum
+        assert abs(lib.reciprocal_error(d, off)) <= 1.01 * 2.0 ** -46 + 1.001 * 2.0 ** -53, (d, off)
+
+
 @pytest.fixture(scope="module")
 def admission(tmp_path_factory):
     """lplb_amd/csrc/plan_admit.h with eight blocks, driven from the host: (admit, launched, forget, idle, arrived)."""
