@@ -602,6 +602,17 @@ __device__ inline bool collect_totals(const PlanArgs &a, int32_t *counts, uint32
   return true;
 }
 
+// By whole waves of a workgroup that have added to words in LDS: true for the wave that comes last, which sees what all `waves`
+// of them have added.  (On either side of the count a wait for the LDS and no more; only with more than 64 slices.)
+__device__ inline bool last_wave_to_arrive(int *arrived, int waves, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  int before = 0;
+  if (lane == 0)
+    before = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  const bool last = __builtin_amdgcn_readfirstlane(before) == waves - 1;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  return last;
+}
 // What others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
 // those that add them up; the tokens of each replicated set before this slice and in the whole batch.
 // (long slices take the two apart)
@@ -648,10 +659,7 @@ __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceT
 #pragma unroll
             for (int j = 0; j < 4; ++j)
               atomicAdd(&block_sums[4 * lane + j], (int32_t)sums[j]);
-          int arrived = 0;
-          if (lane == 0)
-            arrived = atomicAdd(&block_sums[16], 1);
-          all_in = __builtin_amdgcn_readfirstlane(arrived) == a.unit_blocks - 1;
+          all_in = last_wave_to_arrive(&block_sums[16], a.unit_blocks, lane);
           if (all_in && lane < 4)
 #pragma unroll
             for (int j = 0; j < 4; ++j)

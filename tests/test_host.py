@@ -361,6 +361,48 @@ extern "C" __global__ void collect(const unsigned long long *words, unsigned tag
     assert kernels >= 14 * 4 + 14 + 1, kernels
 
 
+def test_the_last_wave_to_add_up_totals_sees_what_the_others_have_added(tmp_path):
+    """With more than 64 slices several waves of a workgroup add to the same sums in LDS, count themselves, and the one that comes
+    last reads the sums.  Nothing but fences keeps the compiler from moving the count ahead of a wave's own additions, or the
+    reads ahead of the count: look for both, and for the waits that they become, where the waves do this."""
+    import shutil
+    import subprocess
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("no hipcc")
+    probe = tmp_path / "probe.hip"
+    probe.write_text('''
+#include "plan_kernel.h"
+using namespace lplb;
+extern "C" __global__ void add_up(PlanArgs a, SliceTables t, uint32_t tag) {
+  __shared__ int missing[2], block_sums[17];
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  add_up_published<LONG_SLICES, Units::kTotals>(a, t, blockIdx.x, tag, lane, wave, missing, block_sums);
+}
+''')
+
+    def compiled(form, *flags):
+        out = tmp_path / "probe.out"
+        subprocess.run([hipcc, "-O3", "-std=c++17", "--offload-arch=gfx950", "--cuda-device-only", "-S", *flags,
+                        f"-I{ROOT / 'lplb_amd' / 'csrc'}", f"-DLONG_SLICES={form}", str(probe), "-o", str(out)], check=True, capture_output=True)
+        return out.read_text()
+
+    for form in ("false", "true"):
+        steps = ""
+        for line in compiled(form, "-emit-llvm").split("define ")[1].splitlines():
+            if "fence" in line:
+                steps += "R" if "release" in line else "A"
+            elif re.search(r"atomicrmw .*addrspace\(3\)", line):
+                steps += "c" if "block_sums, i32 64)" in line else "+"
+            elif re.search(r"= load .*addrspace\(3\)", line):
+                steps += "l"
+        assert re.fullmatch(r"\++RcAl+", steps), steps
+        order = [m.group(1) for m in re.finditer(r"^\s+(ds_add_u32|ds_add_rtn_u32|ds_read\w+|s_waitcnt .*lgkmcnt\(0\))",
+                                                 compiled(form), flags=re.M)]
+        steps = "".join({"ds_add_u32": "+", "ds_add_rtn_u32": "c"}.get(o, "l" if o.startswith("ds_read") else "w") for o in order)
+        assert re.search(r"\++w+cw+l", steps), steps
+
+
 def test_the_lp_s_reciprocals_have_all_of_fp64(tmp_path):
     """An LP's step length is rounded to fp32 only at its end (minilp.cu:361 divides in fp64): with the hardware's estimate off by
     up to 2^-23 either way (v_rcp_f64's bound), the reciprocal keeps an error of that squared and the last roundings,
