@@ -1,5 +1,6 @@
 // LP solver entry points: batches of LPs, one per wave or four per wave.
 // The device code and the description of the method are in solve_kernel.h and solve_spread.h.
+#include "solve_pack.h"
 #include "solve_spread.h"
 
 namespace lplb {
@@ -27,23 +28,11 @@ __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
     atomicAdd(a.avail, n_ok - n_mine);
 }
 
-// One LP per wave has the lowest latency; shapes with G <= 16 and G * D <= 16 can put four into each wave, which takes
-// longer but needs a quarter of the waves.  Alone on its SIMD a lone LP is the faster one throughout.  Up to 8 ranks its
-// lanes are busy less than half the time, and it still is with three on a SIMD; four packed ones fill one wave of every SIMD
-// and take no longer, then a second packed wave is behind until there are six LPs per SIMD.
-// From 9 ranks on (16 pivots a step instead of 8) the second is already too many.  Measured, one per wave / four per wave:
-//                    1024         2048         3072         4096         5120         6144         8192 LPs
-//   (8, 2)      6.7 / 10.2   7.7 / 10.7   9.6 / 10.7  10.9 / 10.9  12.7 / 14.4  14.3 / 14.9  17.5 / 15.4 us
-//   (8, 1)      6.5 /  9.5   7.7 / 10.0   9.1 / 10.0  10.7 / 10.2  12.2 / 13.2  13.7 / 13.8  17.1 / 14.4
-//   (7, 2)      7.6 / 10.7   8.7 / 11.2  10.4 / 11.1  12.2 / 11.3  13.7 / 14.8  15.6 / 15.2  19.0 / 15.9   (padded)
-//   (4, 2)      7.6 / 12.5   8.6 / 12.7  10.4 / 12.8  12.0 / 13.1  13.7 / 16.3  15.6 / 16.6  18.8 / 16.9   (padded)
-//   (16, 1)    12.4 / 13.2  18.8 / 14.1  25.5 / 14.4  32.2 / 14.5  38.9 / 19.3  45.8 / 19.8  59.5 / 20.4
-//   (10, 1)    13.6 / 16.4  20.3 / 17.3  27.0 / 17.3  33.9 / 17.6  40.7 / 22.3  48.1 / 22.8  62.3 / 23.5   (padded)
-static bool packing_pays(int G, int n_units) {
+// Shapes with G <= 16 and G * D <= 16 can put four LPs into each wave: solve_pack.h says when.
+static bool packing_pays(const SolveArgs &a) {
   const int n_cus = current_device_cu_count();
   const int n_simds = 4 * (n_cus > 0 ? n_cus : 256);
-  const int per_simd = n_units / n_simds + (n_units % n_simds != 0);
-  return G <= 8 ? per_simd == 4 || per_simd > 5 : per_simd > 1;
+  return packing_pays(a.G, a.D * a.C + a.n_fixed, a.n_experts, a.n_units / n_simds + (a.n_units % n_simds != 0));
 }
 constexpr int kLdsLimit = 64 * 1024 - 2048;
 
@@ -57,7 +46,7 @@ static void launch_variant(SolveArgs a, hipStream_t s) {
 
 template <int GM, int DM, bool EXACT> static void launch_exactness(const SolveArgs &a, hipStream_t s) {
   if constexpr (GM <= kRowLanes && GM * DM <= kRowLanes) {
-    if (packing_pays(a.G, a.n_units))
+    if (packing_pays(a))
       return launch_variant<GM, DM, EXACT, 4>(a, s);
   }
   launch_variant<GM, DM, EXACT, 1>(a, s);

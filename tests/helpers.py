@@ -28,6 +28,38 @@ CASE_SEED = {"cube8_ep32": 42, "cube8_ep32_c2": 42, "cube8_ep64": 42, "ring8_ep3
              "hypercube16": 42, "torus8x4": 42}
 
 
+def shifted_ring(g, shifts):
+    return np.array([[(i + s) % g for s in shifts] for i in range(g)], np.int32)
+
+
+# Batches of LPs around the places where the number of LPs to a wave changes (on 1024 SIMDs):
+# (name, r2o, ep_size, n_logical, LP instances, four to a wave?)
+BATCHED_LPS = [
+    ("cube8x2", topology.CUBE_8P2E, 8, 256, 1541, False),
+    ("ring8x1", shifted_ring(8, [1]), 8, 128, 1538, False),
+    ("ring6x2_padded", shifted_ring(6, [1, 2]), 6, 60, 1537, False),  # rounded up to the 8 x 2 instantiation
+    ("ring16x1", shifted_ring(16, [1]), 32, 256, 771, True),         # two groups per instance
+    # exact and padded instantiations packed from more than three LPs per SIMD on, last wave part full
+    ("cube8x2_packed", topology.CUBE_8P2E, 8, 256, 3077, True),
+    ("ring8x1_packed", shifted_ring(8, [1]), 8, 128, 3074, True),
+    ("ring6x2_packed", shifted_ring(6, [1, 2]), 6, 60, 3073, True),
+    ("ring8x1_last_lone", shifted_ring(8, [1]), 8, 128, 3072, False),
+    # beyond 8 ranks from more than one
+    ("ring16x1_packed", shifted_ring(16, [1]), 16, 128, 1025, True),
+    ("ring13x1_packed", shifted_ring(13, [1]), 13, 104, 1026, True),
+    ("ring16x1_last_lone", shifted_ring(16, [1]), 16, 128, 1024, False),
+    ("cube8x2_three_per_simd", topology.CUBE_8P2E, 8, 256, 3072, False),
+    ("ring6x2_four_per_simd", shifted_ring(6, [1, 2]), 6, 60, 4096, True),
+    ("cube8x2_five_per_simd", topology.CUBE_8P2E, 8, 256, 4097, False),
+    ("ring8x1_six_per_simd", shifted_ring(8, [1]), 8, 128, 5123, True),
+    # as many experts as make the sixth per SIMD, or the fourth, too much for packing; two groups per instance packed
+    ("cube8x2_six_per_simd", topology.CUBE_8P2E, 8, 256, 5121, False),
+    ("cube8x2_seven_per_simd", topology.CUBE_8P2E, 8, 256, 6147, True),
+    ("cube8x2_512_experts_four_per_simd", topology.CUBE_8P2E, 8, 512, 3077, False),
+    ("cube8x2_two_groups", topology.CUBE_8P2E, 16, 256, 1539, True),
+]
+
+
 @dataclass
 class Shape:
     r2o: np.ndarray

@@ -13,7 +13,7 @@ import torch
 
 from lplb_amd import Planner, _native, eplb, synth, topology
 from lplb_amd.mapping import build_redundancy_mapping
-from tests.helpers import REFERENCE_SOLVE_CASES
+from tests.helpers import BATCHED_LPS, REFERENCE_SOLVE_CASES
 
 ROOT = Path(__file__).resolve().parent.parent
 GOLDEN = ROOT / "tests" / "golden"
@@ -359,6 +359,39 @@ extern "C" __global__ void collect(const unsigned long long *words, unsigned tag
             kernels += 1
             assert not any(op.startswith(("buffer_inv", "buffer_wbl2")) for _, op, _ in code), name
     assert kernels >= 14 * 4 + 14 + 1, kernels
+
+
+def test_lps_are_packed_where_that_was_measured_to_pay(tmp_path):
+    """Four LPs to a wave or one: the rule (lplb_amd/csrc/solve_pack.h) against the measurements that stand above it.  Nowhere may it choose
+    the form that was slower by more than 3 % (two runs of one form differ by up to that)."""
+    import subprocess
+    (tmp_path / "pack.cpp").write_text('''
+#include "solve_pack.h"
+extern "C" int pays(int G, int per_rank, int n_experts, int per_simd) { return lplb::packing_pays(G, per_rank, n_experts, per_simd); }
+''')
+    header = ROOT / "lplb_amd" / "csrc" / "solve_pack.h"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{header.parent}",
+                    str(tmp_path / "pack.cpp"), "-o", str(tmp_path / "pack.so")], check=True, capture_output=True)
+    pays = ctypes.CDLL(str(tmp_path / "pack.so")).pays
+    text = header.read_text()
+    counts = [int(n) for n in re.search(r"of a rank, in all((?: +\d+)+) LPs", text).group(1).split()]
+    rows = re.findall(r"^//   \((\d+), \d+\) +(\d+) +(\d+) +((?:[\d.]+ / *[\d.]+ *)+)", text, flags=re.M)
+    assert len(rows) >= 10 and counts[0] == 2048
+    chosen = set()
+    for G, per_rank, n_experts, times in rows:
+        both = [(float(lone), float(packed)) for lone, packed in re.findall(r"([\d.]+) / *([\d.]+)", times)]
+        assert len(both) == len(counts)
+        for n, (lone, packed) in zip(counts, both):
+            packs = pays(int(G), int(per_rank), int(n_experts), -(-n // 1024))
+            chosen.add(packs)
+            slower, faster = (packed, lone) if packs else (lone, packed)
+            assert slower <= 1.03 * faster, (G, per_rank, n_experts, n, lone, packed)
+    assert chosen == {0, 1}
+    assert not any(pays(G, per_rank, per_rank * G, 1) for G in range(1, 17) for per_rank in (1, 32, 1024))   # alone on its SIMD
+    # the batches that the GPU's test takes for packed ones and for lone ones are
+    for name, r2o, ep, n_logical, n_inst, packed in BATCHED_LPS:
+        n_lps = n_inst * (ep // len(r2o))
+        assert pays(len(r2o), n_logical // ep, n_logical, -(-n_lps // 1024)) == packed, name
 
 
 def test_the_last_wave_to_add_up_totals_sees_what_the_others_have_added(tmp_path):
