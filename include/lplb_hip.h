@@ -414,8 +414,11 @@ int lplb_build_mapping(const float *weight, const double *history, const int32_t
  *   r2o                    int32 [group_size, dup_per_rank], every column a permutation
  *
  * LPLB_EUNSUPPORTED (use lplb_build_mapping) beyond 1024 logical experts, 128 of them (unless a rank has one only) or 64
- * ranks to be packed at once, and where several groups share a node.
+ * ranks to be packed at once, and where several groups share a node.  lplb_place_experts_covers says so beforehand: 1 if it
+ * places the experts of this deployment, 0 if not (or if it is none).
  */
+int lplb_place_experts_covers(int group_size, int dup_per_rank, int ep_size, int n_logical, int n_physical,
+                              int n_nodes);
 int lplb_place_experts(const void *history, int history_type, const int32_t *r2o, int group_size,
                        int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
                        int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream);

@@ -196,26 +196,43 @@ template <typename T> __global__ __launch_bounds__(kPlaceMaxExperts) void place_
   }
 }
 
+static bool is_a_deployment(int G, int D, int ep_size, int n_logical, int n_physical, int n_nodes) {
+  if (G <= 0 || D <= 0 || ep_size <= 0 || n_nodes <= 0 || n_logical <= 0 || ep_size % G != 0 || n_logical % ep_size != 0)
+    return false;
+  const int L = n_logical / ep_size, P = n_physical / ep_size, C = (P - L) / D;
+  return P > L && C > 0 && C * D <= L && (int64_t)ep_size * (L + C * D) == n_physical;
+}
+// Groups go onto nodes only where every node takes one, so that no group has to be weighed; else all ranks are one node.
+static int packed_nodes(int G, int ep_size, int n_nodes) { return ep_size / G % n_nodes == 0 ? n_nodes : 1; }
+static bool is_placed_here(int G, int D, int ep_size, int n_logical, int n_physical, int n_nodes) {
+  const int n_group = ep_size / G, nodes = packed_nodes(G, ep_size, n_nodes);
+  return (nodes == 1 ? n_group % n_nodes != 0 || n_group == 1 : n_group == nodes) && ep_size % nodes == 0 &&
+         n_logical <= kPlaceMaxExperts && (n_logical / nodes <= kPlaceMaxPerNode || n_logical == ep_size) &&
+         ep_size / nodes <= kPlaceMaxPacks && G * D <= kPlaceMaxEdges && n_physical < 65536;
+}
+
 } // namespace lplb
+
+extern "C" int lplb_place_experts_covers(int group_size, int dup_per_rank, int ep_size, int n_logical, int n_physical,
+                                         int n_nodes) {
+  using namespace lplb;
+  return is_a_deployment(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes) &&
+         is_placed_here(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes);
+}
 
 extern "C" int lplb_place_experts(const void *history, int history_type, const int32_t *r2o, int group_size,
                                   int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
                                   int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream) {
   using namespace lplb;
   LPLB_REQUIRE(history && r2o && phy2log && log2phy && logcnt, LPLB_EINVAL, "place_experts: null pointer");
-  LPLB_REQUIRE(group_size > 0 && dup_per_rank > 0 && ep_size > 0 && n_nodes > 0 && n_logical > 0 && ep_size % group_size == 0 &&
-                   n_logical % ep_size == 0,
-               LPLB_EINVAL, "place_experts: %d logical experts on %d ranks in groups of %d", n_logical, ep_size, group_size);
-  const int G = group_size, D = dup_per_rank, L = n_logical / ep_size, P = n_physical / ep_size, C = (P - L) / D;
-  LPLB_REQUIRE(P > L && C > 0 && C * D <= L && (int64_t)ep_size * (L + C * D) == n_physical, LPLB_EINVAL,
-               "place_experts: %d physical experts do not lay out %d logical ones on %d ranks with %d slots for replicas",
-               n_physical, n_logical, ep_size, D);
-  // (groups onto nodes only where every node takes one, so that no group has to be weighed)
-  const int n_group = ep_size / G, nodes = n_group % n_nodes == 0 ? n_nodes : 1;
-  LPLB_REQUIRE((nodes == 1 ? n_group % n_nodes != 0 || n_group == 1 : n_group == nodes) && ep_size % nodes == 0 &&
-                   n_logical <= kPlaceMaxExperts && (n_logical / nodes <= kPlaceMaxPerNode || L == 1) && ep_size / nodes <= kPlaceMaxPacks && G * D <= kPlaceMaxEdges && n_physical < 65536,
-               LPLB_EUNSUPPORTED, "place_experts: %d groups on %d nodes, %d experts on %d ranks are placed on the host only",
-               n_group, n_nodes, n_logical, ep_size);
+  LPLB_REQUIRE(is_a_deployment(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes), LPLB_EINVAL,
+               "place_experts: %d logical and %d physical experts on %d ranks in groups of %d with %d slots for replicas",
+               n_logical, n_physical, ep_size, group_size, dup_per_rank);
+  LPLB_REQUIRE(is_placed_here(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes), LPLB_EUNSUPPORTED,
+               "place_experts: %d groups on %d nodes, %d experts on %d ranks are placed on the host only",
+               ep_size / group_size, n_nodes, n_logical, ep_size);
+  const int G = group_size, D = dup_per_rank, L = n_logical / ep_size, P = n_physical / ep_size;
+  const int nodes = packed_nodes(G, ep_size, n_nodes);
   const auto magic = [](int d) { return fast_div_magic((uint32_t)d); };
   const PlaceArgs a{history, r2o, phy2log, log2phy, logcnt, G, D, L, P, ep_size, n_logical, n_logical / nodes, nodes, ep_size / nodes,
                     magic(G), magic(D), magic(L), magic(P), magic(n_logical / nodes)};

@@ -60,6 +60,18 @@ BATCHED_LPS = [
 ]
 
 
+RING_64 = shifted_ring(64, [1])
+# Deployments around what is placed on the GPU: (r2o, ep_size, n_logical, replicas per rank, covered?)
+PLACEMENTS = {
+    "ring8_8": (topology.RING_8P, 8, 8, 1, True), "cube8_128": (topology.CUBE_8P2E, 8, 128, 2, True),
+    "cube8_136": (topology.CUBE_8P2E, 8, 136, 2, False), "cube8x2_256": (topology.CUBE_8P2E, 16, 256, 4, True),
+    "cube8x8_512": (topology.CUBE_8P2E, 64, 512, 2, True), "ring8x4_256": (topology.RING_8P, 32, 256, 1, True),
+    "hyper16_96": (topology.HYPERCUBE_16P2E, 16, 96, 2, True), "torus32_128": (topology.torus_2d(8, 4), 32, 128, 2, True),
+    "torus32x2_256": (topology.torus_2d(8, 4), 64, 256, 2, False), "ring64_128": (RING_64, 64, 128, 1, True),
+    "ring64_64": (RING_64, 64, 64, 1, True),
+}
+
+
 @dataclass
 class Shape:
     r2o: np.ndarray

@@ -13,7 +13,7 @@ import torch
 
 from lplb_amd import Planner, _native, eplb, synth, topology
 from lplb_amd.mapping import build_redundancy_mapping
-from tests.helpers import BATCHED_LPS, REFERENCE_SOLVE_CASES
+from tests.helpers import BATCHED_LPS, PLACEMENTS, REFERENCE_SOLVE_CASES
 
 ROOT = Path(__file__).resolve().parent.parent
 GOLDEN = ROOT / "tests" / "golden"
@@ -786,6 +786,36 @@ print("placed")
 """
     got = subprocess.run([sys.executable, "-c", program], cwd=tmp_path, capture_output=True, text=True)
     assert got.returncode == 0 and got.stdout.strip() == "placed", got.stderr[-2000:]
+
+
+def test_a_deployment_that_the_gpu_does_not_place_allocates_nothing_there(monkeypatch):
+    """Whether the placement kernel covers a deployment is asked before its tables are allocated, once per deployment; and the
+    question refuses what is no deployment at all."""
+    lib = _native.load()
+    for name, (r2o, ep, n_logical, replicas, covered) in PLACEMENTS.items():
+        assert lib.lplb_place_experts_covers(*r2o.shape, ep, n_logical, n_logical + replicas * ep, ep // 8) == covered, name
+    assert lib.lplb_place_experts_covers(8, 2, 8, 128, 144, 1) == 1
+    for wrong in ((0, 2, 8, 128, 144, 1), (8, 0, 8, 128, 144, 1), (8, 2, 12, 128, 144, 1), (8, 2, 8, 129, 144, 1), (8, 2, 8, 128, 128, 1),
+                  (8, 2, 8, 128, 145, 1), (8, 2, 8, 128, 144, 0), (8, 2, 8, -128, 144, 1), (8, 2, 8, 128, 136, 1), (8, 2, 8, 8, 24, 1)):
+        assert lib.lplb_place_experts_covers(*wrong) == 0, wrong
+
+    class History:
+        dtype, device = torch.int64, torch.device("cuda", 0)
+        is_contiguous, numel, data_ptr = staticmethod(lambda: True), staticmethod(lambda: 136), staticmethod(lambda: 0)
+    asked = []
+
+    class Library:
+        lplb_place_experts_covers = staticmethod(lambda *shape: asked.append(shape) or lib.lplb_place_experts_covers(*shape))
+
+    def no_tables(*args, **kwargs):
+        raise AssertionError("a table was allocated")
+    monkeypatch.setattr(_native, "load", lambda: Library)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch, "empty", no_tables)
+    _native.placement_covers.cache_clear()
+    for _ in range(3):
+        assert _native.place_experts(History, torch.from_numpy(topology.CUBE_8P2E), 8, 152, 1) is None
+    assert asked == [(8, 2, 8, 136, 152, 1)]
 
 
 def test_placement_reports_memory_that_runs_out():
