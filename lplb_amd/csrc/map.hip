@@ -43,7 +43,9 @@ struct MapArgs {
   long long *clocks;   // debug builds: stamps of the first and the last workgroup (else null)
 };
 #define LPLB_MAP_STAMP(k)                                                                      \
-  LPLB_STAMP_AT(blockIdx.x == 0 ? a.clocks + 32 : (blockIdx.x == gridDim.x - 1 ? a.clocks + 48 : nullptr), k)
+  LPLB_STAMP_AT(a.clocks == nullptr           ? nullptr                                        \
+                : blockIdx.x == 0             ? a.clocks + 32                                  \
+                : blockIdx.x == gridDim.x - 1 ? a.clocks + 48 : nullptr, k)
 
 __global__ void zero_ints(int32_t *p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;

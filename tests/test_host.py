@@ -361,6 +361,39 @@ extern "C" __global__ void collect(const unsigned long long *words, unsigned tag
     assert kernels >= 14 * 4 + 14 + 1, kernels
 
 
+def test_a_debug_build_without_a_buffer_stamps_nothing(tmp_path):
+    """Builds with phase clocks write them to a buffer that the caller sets; until one is set no kernel may take a place in it
+    for an address.  The kernels' stamp macros on the host, with and without a buffer, in the first, a middle and the last workgroup."""
+    import subprocess
+    csrc = ROOT / "lplb_amd" / "csrc"
+    macros = [re.search(rf"#define {name}\(k\)(?:.*\\\n)*.*\n", (csrc / source).read_text()).group()
+              for name, source in (("LPLB_STAMP", "solve_kernel.h"), ("LPLB_PLAN_STAMP", "plan_kernel.h"), ("LPLB_MAP_STAMP", "map.hip"))]
+    (tmp_path / "stamps.cpp").write_text('''
+#include <cstdint>
+struct { unsigned x; } blockIdx, gridDim;
+struct Solve { long long *clocks; };
+struct Args { long long *clocks; int n_lp_workgroups; Solve solve; };
+static long long *seen;
+#define LPLB_STAMP_AT(ptr, k) seen = (ptr)
+''' + "".join(macros) + '''
+extern "C" long stamped(int which, unsigned block, unsigned blocks, int lps, long long *clocks) {
+  blockIdx.x = block; gridDim.x = blocks;
+  Args a{clocks, lps, {clocks}};
+  if (which == 0) LPLB_STAMP(3); else if (which == 1) LPLB_PLAN_STAMP(3); else LPLB_MAP_STAMP(3);
+  return reinterpret_cast<intptr_t>(seen);
+}
+''')
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", str(tmp_path / "stamps.cpp"), "-o", str(tmp_path / "stamps.so")],
+                   check=True, capture_output=True)
+    stamped = ctypes.CDLL(str(tmp_path / "stamps.so")).stamped
+    stamped.restype, stamped.argtypes = ctypes.c_long, [ctypes.c_int, ctypes.c_uint, ctypes.c_uint, ctypes.c_int, ctypes.c_void_p]
+    for which in range(3):
+        for blocks in (1, 2, 7):
+            places = [stamped(which, block, blocks, 1, 4096) for block in range(blocks)]
+            assert all(p == 0 or p >= 4096 for p in places) and any(places)
+            assert [stamped(which, block, blocks, 1, None) for block in range(blocks)] == [0] * blocks, which
+
+
 def test_lps_are_packed_where_that_was_measured_to_pay(tmp_path):
     """Four LPs to a wave or one: the rule (lplb_amd/csrc/solve_pack.h) against the measurements that stand above it.  Nowhere may it choose
     the form that was slower by more than 3 % (two runs of one form differ by up to that)."""
