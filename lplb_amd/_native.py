@@ -186,11 +186,12 @@ def place_experts(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_phys
     if kind is None or not history.is_contiguous() or _device_index(history) != torch.cuda.current_device():
         return None
     n_logical = history.numel()
-    if not placement_covers(r2o.shape[0], r2o.shape[1], ep_size, n_logical, n_physical, n_nodes):
+    group_size, dup_per_rank = r2o.shape
+    if not placement_covers(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes):
         return None
     table = torch.empty(n_physical + 3 * n_logical, dtype=torch.int32, device=history.device)
     at = table.data_ptr()
-    _check(load().lplb_place_experts(history.data_ptr(), kind, r2o.data_ptr(), r2o.shape[0], r2o.shape[1], ep_size, n_logical,
+    _check(load().lplb_place_experts(history.data_ptr(), kind, r2o.data_ptr(), group_size, dup_per_rank, ep_size, n_logical,
                                      n_physical, n_nodes, at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical),
                                      _stream(history)))
     return table
