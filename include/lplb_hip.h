@@ -282,11 +282,15 @@ int lplb_map_idx_prepared(const int64_t *idx, const float *o_weight,
  * One batch's whole plan in a single call: what Planner.run does with three
  * extension calls (lplb/planner.py:245-266), with the same results as
  * lplb_count_idx, lplb_solve and lplb_map_idx chained on `stream`.  Batches of up
- * to about eight million indices (slices of at most 8192 indices, of at most 32768 where
- * n_blocks is at least 64, as many of them as fit the GPU together) with LP shapes up to 32 x 2, up to 32 EP groups and up to 1024
- * logical experts run as ONE kernel launch in which the workgroups exchange their
- * counts and the LP's result through memory; everything else runs as the chain of
- * the three entry points' kernels.
+ * to about two million indices (slices of at most 8192 indices, as many of them as n_blocks
+ * and the GPU allow; 1.6 million with groups of more than 16 ranks) with LP shapes up to 8 x 4 or 32 x 2, up to 32 EP
+ * groups, up to 1024 logical experts and tables that fit a compute unit run as ONE kernel launch in which the workgroups
+ * exchange their counts and the LP's result through memory; everything else runs as the chain of
+ * the three entry points' kernels.  Longer batches are one launch of slices of up to 32768 indices where n_blocks is
+ * at least 64 and the slices' tables, which take 1.7 KiB of LDS per replicated expert set (in sixteens), leave room
+ * for all of them at once: on 256 compute units and at 256 logical experts, with n_blocks = 256 and groups of up to 16 ranks up
+ * to eight million indices with up to 31 sets; with n_blocks of at most 203, or groups of more than 16 ranks, up to 6.6 million
+ * with up to 63 sets.
  *
  *   global_counts    int32 [n_logical] or NULL.  NULL: the LP is fed this GPU's
  *                    own histogram, as Planner.run does without a process

@@ -236,6 +236,8 @@ static int try_one_launch(const int64_t *idx, int64_t n_elements, const int32_t 
     len *= 2;
   a.per = slice_len(n_elements, (int)min((n_elements + len - 1) / len, (int64_t)most));
   // Past that as many long slices as there may be, unless these are few: a caller that allows few workgroups keeps the chain.
+  // (So many may turn out not to be resident at once: up to 16 ranks `most` is for two per CU, and the tables of 32 sets and more
+  // leave room for one.  launch_plan refuses those.)
   if (a.per > kLongestSlice && (a.per > kLongestOfLongSlices || most < kFewestLongSlices))
     return LPLB_OK;
   a.n_slices = (int)((n_elements + a.per - 1) / a.per);   // (rounding the length up may have emptied the last ones)
