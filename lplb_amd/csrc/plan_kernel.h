@@ -181,7 +181,7 @@ constexpr int slice_record_bytes(int k) { return k > 0 ? rank_record_bytes_singl
 template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
   return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * slice_record_bytes(K) +
          (size_t)(n_logical + 2) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
-         (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t);
+         (size_t)(3 + 2 * kPlanWaves) * n_rep * sizeof(int32_t);
 }
 // A long slice's records per (wave, replicated set): the bitmaps of a pass's chunks, and what a token's ordinal is made of (a
 // bitmap and the tokens before it), both padded for the LDS banks; sixteen sets are worked on at once.
@@ -203,6 +203,7 @@ struct SliceTables {
   int32_t *set_expert;      // [R] the expert whose tokens the set has; n_logical (which has none): it has none
   int32_t *before, *total;  // [R] tokens of the set before this slice, in the whole batch
   int32_t *wave_total;      // [waves][R] ... in each wave
+  int32_t *base;            // [waves][R] ... before each wave (not for long slices)
   int32_t *hist;            // [more than n_logical, a multiple of 16] the slice's histogram, then zeros; in the first slice at last the batch's
 };
 template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, int nl, int R) {
@@ -215,6 +216,7 @@ template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, 
   t.before = t.set_expert + R;
   t.total = t.before + R;
   t.wave_total = t.total + R;
+  t.base = t.wave_total + kPlanWaves * R;
   if (K == 0)
     t.records = lds + long_slice_records_at(nl, R);
   return t;
@@ -371,36 +373,35 @@ template <int K> struct SliceTokens {
     LPLB_PLAN_STAMP(8);
     LPLB_SLICE_STAMP(1);
   }
-  // The tokens of each set in the wave's earlier chunks into the slots, those in the whole wave into t.wave_total.
-  // lane = (set, chunk), chunk fastest.
+  // The tokens of each set in the wave's earlier chunks into the slots, those in the whole wave into t.wave_total.  lane = set:
+  // the chunks' pop-counts add up as they are read.  (lane = (set, chunk) with a scan over the lanes of a set takes as many instructions
+  // at 16 sets and eight times as many at 128.  Counts supplied, [100000 x 8]: 64 sets 15.2 -> 12.8 us, 32 sets 12.1 -> 11.3; [16384 x 8]
+  // with 128 sets 11.0 -> 10.2; [262144 x 8] with 16 sets 18.0 -> 17.9.)
   __device__ static void starts_in_wave(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, int lane, int wave_s) {
-    const int R = a.n_rep, c = lane % K;
-    for (int p0 = 0; p0 < R * K; p0 += kWave) {
-      const bool live = p0 + lane < R * K;
-      const int q = live ? (p0 + lane) / K : R;   // lanes past the end read the stand-in record (zeros)
-      ChunkSlot *mine = slot(my_records, q, c);
-      const int own = __popcll(*reinterpret_cast<const unsigned long long *>(mine));
-      const int in_my_wave = group_sum<K>(own);
-      const int in_earlier_chunks = group_exclusive_scan<K>(own, c);
-      if (live) {
-        mine->start = in_earlier_chunks;
-        if (c == 0)
-          t.wave_total[wave_s * R + q] = in_my_wave;
+    const int R = a.n_rep;
+    for (int q = lane; q < R; q += kWave) {
+      unsigned long long bits[K];
+#pragma unroll
+      for (int c = 0; c < K; ++c)
+        bits[c] = *reinterpret_cast<const unsigned long long *>(slot(my_records, q, c));
+      int before = 0;
+#pragma unroll
+      for (int c = 0; c < K; ++c) {
+        slot(my_records, q, c)->start = before;
+        before += __popcll(bits[c]);
       }
+      t.wave_total[wave_s * R + q] = before;
     }
   }
-  // Ordinal of the first token of every chunk: what is there already plus the tokens before this slice and in
-  // the waves before this one.  The wave's own slots only: no barrier.
-  __device__ static void add_starts(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, int lane, int wave_s) {
-    const int R = a.n_rep, c = lane % K;
-    for (int p0 = 0; p0 < R * K; p0 += kWave) {
-      const bool live = p0 + lane < R * K;
-      const int q = live ? (p0 + lane) / K : 0;
+  // The tokens of each set before this wave's first into t.base.  The wave's own entries only: no barrier.
+  __device__ static void bases(const PlanArgs &a, const SliceTables &t, int lane, int wave_s) {
+    const int R = a.n_rep;
+    for (int q = lane; q < R; q += kWave) {
       int32_t base = t.before[q];
-      for (int w = 0; w < wave_s; ++w)
-        base += t.wave_total[w * R + q];
-      if (live)
-        atomicAdd(&slot(my_records, q, c)->start, base);
+#pragma unroll
+      for (int w = 0; w < kPlanWaves - 1; ++w)
+        base += w < wave_s ? t.wave_total[w * R + q] : 0;
+      t.base[wave_s * R + q] = base;
     }
     own_slots_are_written();
   }
@@ -428,12 +429,14 @@ template <int K> struct SliceTokens {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  __device__ static int32_t hash(const SliceTables &t, unsigned char *my_records, int e, int c) {
+  // base: of the wave's sets, or null: part of the starts.
+  __device__ static int32_t hash(const SliceTables &t, unsigned char *my_records, const int32_t *base, int R, int e, int c) {
     const int set = t.route[e].rep;
+    const int32_t before = base ? base[min(set, R - 1)] : 0;
     const i32x4 s = *reinterpret_cast<const i32x4 *>(slot(my_records, set, c));   // bits_lo, bits_hi, start
     const i32x4 x = *reinterpret_cast<const i32x4 *>(&t.reps[set]);               // total, magic, -, -
     const int32_t k =
-        __builtin_amdgcn_mbcnt_hi((uint32_t)s.y, __builtin_amdgcn_mbcnt_lo((uint32_t)s.x, (uint32_t)s.z));
+        __builtin_amdgcn_mbcnt_hi((uint32_t)s.y, __builtin_amdgcn_mbcnt_lo((uint32_t)s.x, (uint32_t)(s.z + before)));
     return ordinal_hash<false>(k, x.x, (uint32_t)x.y);
   }
 };
@@ -908,7 +911,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   if (ok) {
     for (int q = tid; q < R; q += kPlanThreads)
       set_total(t.reps[q], t.total[q]);
-    SliceTokens<K>::add_starts(a, t, my_records, lane, wave_s);
+    SliceTokens<K>::bases(a, t, lane, wave_s);
     if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word)
       say_that_all_arrived(a, tag, lane);
     if (slice == 0 && !collect_totals(a, t.hist, tag, tid, wave_s)) {   // for the caller (and for the counts below)
@@ -928,7 +931,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     // lanes on again: copied in no lane, lost in all.  97 registers this way at 8 ranks.  tests/test_host.py looks for such copies in the built library.
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      h[c] = SliceTokens<K>::hash(t, my_records, packed_expert(packed, c), c);
+      h[c] = SliceTokens<K>::hash(t, my_records, t.base + wave_s * R, R, packed_expert(packed, c), c);
       if (K > 8 && c % 8 == 7) {
 #pragma unroll
         for (int j = c - 7; j <= c; ++j)
@@ -1311,7 +1314,7 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
     SliceTokens<K>::starts_of_batch(a, my_records, lane, turn, records_of);
 #pragma unroll
     for (int c = 0; c < K; ++c)
-      h[c] = SliceTokens<K>::hash(t, my_records, packed_expert(packed, c), c);
+      h[c] = SliceTokens<K>::hash(t, my_records, nullptr, R, packed_expert(packed, c), c);
   }
   if (wave_s < n_lps) {
     __builtin_amdgcn_wave_barrier();   // (its shares have been stored)
