@@ -769,6 +769,7 @@ __device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *s
   }
   LPLB_PLAN_STAMP(1);
   if (wave_s < n_lps) {
+    __builtin_amdgcn_s_setprio(1);
     // (own-histogram mode: every LP of the batch reads the one staged copy)
     float *mine = a.local_counts ? staged : staged + (size_t)wave_s * sa.staged_stride;
     const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
@@ -907,6 +908,9 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   bool ok = missing[0] == 0;   // (the same in every thread)
   if (!ok && !poisoned && tid == 0)
     give_up(a, avail_state);
+  // From here on it is the slice that has time.  (At 2 for its whole length, the one that shares a CU with the LP slowed its first step
+  // from 0.6 to 1.7 us while it hashed: [262144 x 8] 17.5 -> 16.7 us.)
+  __builtin_amdgcn_s_setprio(0);
   int32_t h[K];   // hashes of this thread's tokens: worked out while the LP is still running
   if (ok) {
     for (int q = tid; q < R; q += kPlanThreads)
