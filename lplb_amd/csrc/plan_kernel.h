@@ -731,7 +731,18 @@ __device__ __forceinline__ void slice_has_read_all(const PlanArgs &a, int slice,
   }
 }
 
-// An LP workgroup of a plan: one wave per LP, the others help to collect the counts.
+// Normalised counts of the experts from `first` on, `n` of them, for the caller, by nt threads (whole waves): each count over the
+// largest of all.
+__device__ inline void write_normalised_counts(const PlanArgs &a, const int32_t *counts, int first, int n, int thread, int nt, int lane) {
+  int32_t most = 0;
+  for (int e = lane; e < a.sh.n_logical; e += kWave)
+    most = max(most, counts[e]);
+  const float wmax = wave_max_of_groups<true, true>((float)most);
+  for (int i = thread; i < n; i += nt)
+    a.solve.gw_out[first + i] = (float)counts[first + i] / wmax;
+}
+// An LP workgroup of a plan: one wave per LP, the others help to collect the counts and write the normalised ones (by the LP waves
+// themselves, at their end, those took 0.8 us, and what is counted for the caller behind them came as much later).
 template <int GM, int DM, bool EXACT>
 __device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *smem_raw, int *rep_of_edge_all, int *missing,
                                              unsigned long long gen_and_poison, int tid, int lane, int wave_s) {
@@ -749,6 +760,7 @@ __device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *s
   unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
   float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
   sa.launch = (uint32_t)gen_and_poison;
+  sa.gw_out = nullptr;   // (written by the waves without an LP)
   auto switched_off = [&]() { return (gen_and_poison >> 32) != 0; };
   // Own-histogram mode: the LP waves' table loads are on their way when they and the other waves turn to the
   // batch's histogram.  (Switched off: no slice will publish.)
@@ -772,7 +784,7 @@ __device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *s
     __builtin_amdgcn_s_setprio(1);
     // (own-histogram mode: every LP of the batch reads the one staged copy)
     float *mine = a.local_counts ? staged : staged + (size_t)wave_s * sa.staged_stride;
-    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(
+    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1, true>(
         sa, first_lp + wave_s, mine, rep_of_edge_all + wave_s * kWave, reinterpret_cast<double *>(my_area),
         reinterpret_cast<float *>(my_area + lp_pivot_doubles<GM, DM>() * sizeof(double)), counts_have_come);
     worked_out_here(gen_and_poison);
@@ -795,8 +807,11 @@ __device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *s
     }
     if (lane == 0 && a.seq >= 0)
       agent_store(a.sync + kDoneAt + (kMaxSlices + first_lp + wave_s) * kDoneStride, a.seq);
-  } else if (a.local_counts) {
-    counts_have_come();
+  } else if (!a.local_counts || counts_have_come()) {
+    const int helper = kLpsPerWorkgroup * kWave, per_lp = sa.G * (sa.D * sa.C + sa.n_fixed);
+    if (tid >= helper)
+      write_normalised_counts(a, a.local_counts ? reinterpret_cast<const int32_t *>(staged) : sa.workload, first_lp * per_lp, n_lps * per_lp,
+                              tid - helper, kPlanThreads - helper, lane);
   }
 }
 
@@ -1285,7 +1300,7 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
     SolveArgs sa = a.solve;
     sa.shares_in_lds = share_of;
     sa.gw_out = nullptr;   // (written below, by waves that do not solve)
-    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(sa, wave_s, reinterpret_cast<float *>(t.hist), rep_of_edge_all + wave_s * kWave,
+    const int n_ok = solve_lps<GM, DM, EXACT, 1, 1, true>(sa, wave_s, reinterpret_cast<float *>(t.hist), rep_of_edge_all + wave_s * kWave,
                                                     reinterpret_cast<double *>(area),
                                                     reinterpret_cast<float *>(area + lp_pivot_doubles<GM, DM>() * sizeof(double)),
                                                     count_the_tokens);
@@ -1401,7 +1416,7 @@ template <int GM, int DM, bool EXACT> __global__ __launch_bounds__(kScanThreads)
     return;
   }
   unsigned char *area = smem_raw + wave_s * kLpArea;
-  const int n_ok = solve_lps<GM, DM, EXACT, 1, 1>(a.solve, wave_s, staged, rep_of_edge_all + wave_s * kWave,
+  const int n_ok = solve_lps<GM, DM, EXACT, 1, 1, true>(a.solve, wave_s, staged, rep_of_edge_all + wave_s * kWave,
                                                   reinterpret_cast<double *>(area),
                                                   reinterpret_cast<float *>(area + lp_pivot_doubles<GM, DM>() * sizeof(double)),
                                                   counts_have_come);
@@ -1436,17 +1451,12 @@ template <int GM, int DM, bool EXACT, int K>
 static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   const size_t lds_slice = K > 0 ? plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep)
                                  : long_slice_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words);
-  // LP workgroups: their waves' working areas, then the counts (one copy per LP if they fit,
-  // else none and the LPs read global memory; own-histogram mode needs one copy in any case)
+  // LP workgroups: their waves' working areas, then the counts (one copy per LP, or one for all of the batch's own)
   const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
   const size_t one_copy = counts_bytes(a.sh.n_logical);
   const size_t all_copies = (size_t)min(a.solve.n_units, kLpsPerWorkgroup) * one_copy;
-  size_t lds = max(lds_slice, lp_areas + (a.local_counts ? one_copy : 0));
-  a.solve.staged_stride = 0;
-  if (lp_areas + all_copies <= max(lds, (size_t)16 * 1024)) {   // (a few KiB more are worth one global round trip less)
-    lds = max(lds, lp_areas + all_copies);
-    a.solve.staged_stride = (int)(one_copy / sizeof(int32_t));
-  }
+  const size_t lds = max(lds_slice, lp_areas + (a.local_counts ? one_copy : all_copies));
+  a.solve.staged_stride = (int)(one_copy / sizeof(int32_t));
   if (lds > (size_t)kPlanLdsLimit)
     return LPLB_OK;
   static KernelFootprint footprint;

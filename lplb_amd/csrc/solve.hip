@@ -12,7 +12,8 @@ namespace lplb {
 // the arithmetic).  So the first thread of the grid counts every LP of the launch as
 // feasible with one add, and a wave takes back the LPs of its own that failed -- rare,
 // and the sum is the same.
-template <int GM, int DM, bool EXACT, int ROWS, int EPL>
+// STAGED: the counts fit in LDS.
+template <int GM, int DM, bool EXACT, int ROWS, int EPL, bool STAGED>
 __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
   extern __shared__ float staged_all[];   // a.staged_stride floats per LP of this wave
   __shared__ int rep_of_edge[EPL * kWave];
@@ -21,7 +22,7 @@ __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0)
     atomicAdd(a.avail, a.n_units);
   const int first_unit = blockIdx.x * ROWS;
-  const int n_ok = solve_lps<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_all, rep_of_edge, pivot_rows, tile,
+  const int n_ok = solve_lps<GM, DM, EXACT, ROWS, EPL, STAGED>(a, first_unit, staged_all, rep_of_edge, pivot_rows, tile,
                                                          []() { return true; });
   const int n_mine = min(max(a.n_units - first_unit, 0), ROWS);
   if (threadIdx.x == 0 && n_ok < n_mine)
@@ -32,7 +33,7 @@ __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
 static bool packing_pays(const SolveArgs &a) {
   const int n_cus = current_device_cu_count();
   const int n_simds = 4 * (n_cus > 0 ? n_cus : 256);
-  return packing_pays(a.G, a.D * a.C + a.n_fixed, a.n_experts, a.n_units / n_simds + (a.n_units % n_simds != 0));
+  return packing_pays(a.G, a.D * a.C + a.n_fixed, a.n_experts, a.n_units / n_simds + (a.n_units % n_simds != 0), a.D);
 }
 constexpr int kLdsLimit = 64 * 1024 - 2048;
 
@@ -40,8 +41,12 @@ template <int GM, int DM, bool EXACT, int ROWS, int EPL = 1>
 static void launch_variant(SolveArgs a, hipStream_t s) {
   const size_t lds = (size_t)ROWS * (a.n_experts + 1) * sizeof(float);   // (one LP per wave has a zero behind its counts)
   a.staged_stride = lds <= kLdsLimit ? a.n_experts + 1 : 0;
-  launch(solve_groups<GM, DM, EXACT, ROWS, EPL>, dim3((a.n_units + ROWS - 1) / ROWS), dim3(kWave),
-         a.staged_stride ? lds : 0, s, a);
+  const dim3 grid((a.n_units + ROWS - 1) / ROWS), block(kWave);
+  constexpr bool kKnown = takes_spread_form<GM, DM, ROWS, EPL>() || ROWS > 1;   // whether the kernel is built for either case
+  if (a.staged_stride)
+    launch(solve_groups<GM, DM, EXACT, ROWS, EPL, kKnown>, grid, block, lds, s, a);
+  else   // (more than 15 thousand experts, 3900 with four LPs per wave: one kernel, the padded one, serves every group that it holds)
+    launch(solve_groups<GM, DM, EXACT && !kKnown, ROWS, EPL, false>, grid, block, 0, s, a);
 }
 
 template <int GM, int DM, bool EXACT> static void launch_exactness(const SolveArgs &a, hipStream_t s) {

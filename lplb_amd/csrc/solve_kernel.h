@@ -214,13 +214,13 @@ constexpr int assembly_tile_floats(int gm, int rows) { return rows == 1 ? gm * (
 //
 // Called by all 64 lanes of a wave; waves share nothing and never synchronise.
 //   first_unit     LP (instance * n_group + group) of the wave's first row
-//   staged_counts  LDS, ROWS * a.staged_stride floats (unused if the stride is 0)
+//   staged_counts  LDS, ROWS * a.staged_stride floats (unused if the stride is 0; STAGED: it is not)
 //   rep_of_edge    LDS, EPL * kWave ints
 //   pivot_rows     LDS, 2 * kWave doubles of this wave, 16-byte aligned
 //   tile           LDS, assembly_tile_floats(GM, ROWS) floats of this wave, 16-byte aligned
 // Returns how many of the wave's LPs passed the feasibility test (same value in
 // every lane); the caller adds it to a.avail.
-template <int GM, int DM, bool EXACT, int ROWS, int EPL = 1>
+template <int GM, int DM, bool EXACT, int ROWS, int EPL, bool STAGED>
 __device__ inline int solve_lp(const SolveArgs &a, int first_unit, float *staged_counts_of_wave,
                                int *rep_of_edge, double *pivot_rows, float *tile) {
   constexpr int WL = Layout<ROWS>::kWidth;   // lanes of one LP
@@ -271,7 +271,7 @@ __device__ inline int solve_lp(const SolveArgs &a, int first_unit, float *staged
   }
   // When they fit, the counts are staged in LDS as floats, so that the gathers
   // through phy2log do not need a second round trip to global memory.
-  const bool staged = a.staged_stride > 0;
+  const bool staged = STAGED || a.staged_stride > 0;
   auto count_of = [&](int e) -> float {
     if (e < 0 || e >= a.n_experts)
       return 0.0f;

@@ -156,7 +156,10 @@ template <int TS> __device__ inline double rank_partner(double v) {
 // that if GM * DM > kWave.
 // counts_have_come: called once what does not depend on the counts is done if a.counts_by_caller; returns when the
 // counts are in staged_counts (as int32, 16-byte aligned, with a zero behind the last and up to a multiple of four: true), or when they will not come: then -1 is returned, nothing solved or stored.
-template <int GM, int DM, bool EXACT, typename Counts>
+// STAGED: the counts fit in LDS (a.staged_stride > 0, or they are the caller's).  Known here, a count is an LDS read; else it is
+// a load that finds out where its address is and waits for both kinds of memory, one after the other: 0.55 us from the counts' arrival
+// until the LP has its weights, 0.25 this way (8 ranks, 256 experts), and as much again at the end for the normalised counts.
+template <int GM, int DM, bool EXACT, bool STAGED, typename Counts>
 __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *staged_counts, int *rep_of_edge,
                                       double *pivot_rows, float *tile, Counts counts_have_come) {
   static_assert(spread_shape(GM, DM) && (GM == 8 || GM == 16 || GM == 32), "a lane holds GM * GM / 64 entries of S");
@@ -174,7 +177,7 @@ __device__ inline int solve_lp_spread(const SolveArgs &a, int unit, float *stage
   const int32_t *__restrict__ p2l = a.phy2log + (int64_t)grp * G * P;
   const bool is_rank = EXACT || rank < G;
   // The counts, as int32: in LDS if they fit there (entry n_experts is a zero), else in global memory.
-  const bool staged = a.staged_stride > 0 || a.counts_by_caller;
+  const bool staged = STAGED || a.staged_stride > 0 || a.counts_by_caller;
   int32_t *const counts_in_lds = reinterpret_cast<int32_t *>(staged_counts);
   auto index_of = [&](int e) { return e < 0 || e > a.n_experts ? a.n_experts : e; };   // of an expert; no expert: of a zero
   auto count_at = [&](int i) -> float {
@@ -669,13 +672,13 @@ template <int GM, int DM, int ROWS = 1, int EPL = 1> constexpr int lp_pivot_doub
 template <int GM, int DM, int ROWS = 1, int EPL = 1> constexpr int lp_tile_floats() {
   return takes_spread_form<GM, DM, ROWS, EPL>() ? spread_tile_floats(GM, DM) : assembly_tile_floats(GM, ROWS);
 }
-template <int GM, int DM, bool EXACT, int ROWS, int EPL, typename Counts>
+template <int GM, int DM, bool EXACT, int ROWS, int EPL, bool STAGED, typename Counts>
 __device__ inline int solve_lps(const SolveArgs &a, int first_unit, float *staged_counts, int *rep_of_edge,
                                 double *pivot_rows, float *tile, Counts counts_have_come) {
   if constexpr (takes_spread_form<GM, DM, ROWS, EPL>())
-    return solve_lp_spread<GM, DM, EXACT>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile, counts_have_come);
+    return solve_lp_spread<GM, DM, EXACT, STAGED>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile, counts_have_come);
   else
-    return solve_lp<GM, DM, EXACT, ROWS, EPL>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile);
+    return solve_lp<GM, DM, EXACT, ROWS, EPL, STAGED>(a, first_unit, staged_counts, rep_of_edge, pivot_rows, tile);
 }
 
 #undef LPLB_FMAC
