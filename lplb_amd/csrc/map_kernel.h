@@ -102,7 +102,9 @@ template <bool WRAP> __device__ inline int32_t ordinal_hash(int32_t k, int32_t t
 __host__ __device__ inline uint32_t fast_div_magic(uint32_t d) {
   return d <= 1 ? 0u : (uint32_t)(0x100000000ull / d) + 1u;
 }
-__device__ inline uint32_t fast_div(uint32_t n, uint32_t m) { return m ? __umulhi(n, m) : n; }
+__device__ inline uint32_t fast_div(uint32_t n, uint32_t m) {
+  return __umulhi(n, m) | (n & (m ? 0u : ~0u));   // (m ? ... : n becomes a branch each time)
+}
 
 // DPP row shift right by N lanes inside a row of 16 (lanes without a source get 0).
 template <int N> __device__ inline int row_shr(int v) {

@@ -6,8 +6,8 @@
 // kernels have 1-8 us of work.  Here the LP workgroups (one per four LPs, first in the grid) and one
 // workgroup per slice of the indices run side by side in a single grid:
 //   slice workgroup: load the indices once (they stay in registers as 16-bit expert ids) -> histogram of the
-//     slice in LDS, bitmaps of the replicated sets -> publish both -> collect the other slices' counts of the
-//     replicated sets -> ordinals and hashes -> wait for the LP's shares -> choose original or replica, store;
+//     slice in LDS -> publish it and the replicated sets' part of it -> bitmaps of the replicated sets, the other slices' counts
+//     of those -> ordinals and hashes -> wait for the LP's shares -> choose original or replica, store;
 //   LP workgroup: (own-histogram mode: collect the slices' histograms ->) solve -> publish the shares.
 // A batch of up to 4096 indices that feeds the LP itself is one workgroup that does both (plan_in_one_workgroup):
 // nothing is exchanged and nothing has to be resident beside it.
@@ -209,13 +209,13 @@ struct SliceTables {
 template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, int nl, int R) {
   SliceTables t;
   t.reps = reinterpret_cast<RepEntry *>(lds);
-  t.records = lds + (size_t)(R + 1) * sizeof(RepEntry);
-  t.route = reinterpret_cast<Route *>(t.records + (size_t)kPlanWaves * (R + 1) * slice_record_bytes(K));
-  t.hist = reinterpret_cast<int32_t *>(t.route + ((nl + 2) & ~1));   // (16-byte aligned, as what lies before it is)
-  t.set_expert = t.hist + nl / 16 * 16 + 16;
-  t.before = t.set_expert + R;
+  t.route = reinterpret_cast<Route *>(t.reps + R + 1);
+  t.records = reinterpret_cast<unsigned char *>(t.route + ((nl + 2) & ~1));   // (16-byte aligned, as what lies before it is)
+  t.hist = reinterpret_cast<int32_t *>(t.records + (size_t)kPlanWaves * (R + 1) * slice_record_bytes(K));
+  t.before = t.hist + nl / 16 * 16 + 16;
   t.total = t.before + R;
-  t.wave_total = t.total + R;
+  t.set_expert = t.total + R;
+  t.wave_total = t.set_expert + R;
   t.base = t.wave_total + kPlanWaves * R;
   if (K == 0)
     t.records = lds + long_slice_records_at(nl, R);
@@ -256,30 +256,34 @@ __device__ inline PlanTableLoads issue_plan_table_loads(const PlanArgs &a, int t
   t.physical_le0 = a.phy2log[min(tid, a.sh.n_ranks * a.sh.P - 1)];
   return t;
 }
-// Where an expert's tokens go when nothing is redirected and which replicated set (if any) it belongs to
-// (minilp.cu:466-496); everything else empty.  The routes are there when it ends (a workgroup barrier), the sets' experts
-// behind the next one.
-template <int K>
-__device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t, const PlanTableLoads &l, int tid) {
+// What a slice does before its counts are out is what the LP waits for, and it is bound by instructions: the loads
+// have come 0.9 us after the workgroup started, when the LDS has just been cleared (a launch begins with an empty instruction cache:
+// an instruction that runs once costs three times what it does in a loop).  So tokens are counted without a look at the mapping, the
+// mapping is entered in the same interval between two barriers, and the bitmaps are marked behind the publishing.  Per call,
+// against tables first and a route looked up for every token that is counted: run [8192 x 8] 9.55 -> 9.3 us, [32768 x 8] 10.45 -> 9.9,
+// [100000 x 8] 12.6 -> 11.7, [262144 x 8] 16.85 -> 15.4, [16384 x 8] at 32 ranks 20.85 -> 20.25; in one workgroup [128 x 8] 7.2 -> 7.05.
+// (Beyond that, the sets' totals and the waves' bases worked out ahead of the barrier instead of behind it: no faster.)
+
+// Everything empty: routes to nowhere, zeros from the records to the totals (which lie side by side, so that this is one loop,
+// of one turn for most).  A workgroup barrier has to follow.
+template <int K> __device__ inline void clear_plan_tables(const PlanArgs &a, const SliceTables &t, int tid) {
   constexpr int nt = kPlanThreads;
-  const int nl = a.sh.n_logical, R = a.n_rep, cd = a.sh.C * a.sh.D;
+  const int nl = a.sh.n_logical, R = a.n_rep;
   for (int e = tid; e <= nl; e += nt)
     t.route[e] = Route{-1, R};
-  for (int e = tid; e < nl / 16 * 16 + 16; e += nt)
-    t.hist[e] = 0;
-  {
-    const i32x4 zero{0, 0, 0, 0};
-    i32x4 *z = reinterpret_cast<i32x4 *>(t.records);
-    for (int i = tid; i < kPlanWaves * (R + 1) * slice_record_bytes(K) / 16; i += nt)
-      z[i] = zero;
-  }
-  for (int q = tid; q < R; q += nt) {
-    t.before[q] = 0;
-    t.total[q] = 0;
-  }
+  unsigned char *from = K > 0 ? t.records : reinterpret_cast<unsigned char *>(t.hist);
+  const int n16 = (int)(reinterpret_cast<unsigned char *>(t.set_expert) - from + 15) / 16;   // (the end may reach into set_expert)
+  const i32x4 zero{0, 0, 0, 0};
+  for (int i = tid; i < n16; i += nt)
+    reinterpret_cast<i32x4 *>(from)[i] = zero;
   if (tid == 0)
     t.reps[R] = RepEntry{1, 0xffffffffu, INT32_MAX, -1};   // "no replica": every token stays
-  __syncthreads();
+}
+// Where an expert's tokens go when nothing is redirected and which replicated set (if any) it belongs to
+// (minilp.cu:466-496).  A workgroup barrier has to follow.
+__device__ inline void enter_plan_tables(const PlanArgs &a, const SliceTables &t, const PlanTableLoads &l, int tid) {
+  constexpr int nt = kPlanThreads;
+  const int nl = a.sh.n_logical, R = a.n_rep, cd = a.sh.C * a.sh.D;
   if (tid < nl && l.le0 >= 0 && l.le0 < nl)
     t.route[l.le0].original = l.slot0;
   for (int e = tid + nt; e < nl; e += nt) {
@@ -302,11 +306,12 @@ __device__ inline void build_plan_tables(const PlanArgs &a, const SliceTables &t
     const SetOfPlan s = set_of_plan(a, i);
     enter_set(i, s, a.phy2log[s.ep_rank * a.sh.P + s.place], a.o2r[s.group_rank * a.sh.D + s.d]);
   }
-  __syncthreads();
-  // (of two sets that name the same expert only one has the tokens; read behind the next barrier)
-  for (int q = tid; q < R; q += nt)
-    if (t.route[t.set_expert[q]].rep != q)
-      t.set_expert[q] = nl;
+}
+// The expert whose tokens set q has, once the routes are there; n_logical: none (of two sets that name the same expert only one
+// has the tokens).
+__device__ inline int expert_of_set(const PlanArgs &a, const SliceTables &t, int q) {
+  const int e = t.set_expert[q];
+  return t.route[e].rep == q ? e : a.sh.n_logical;
 }
 
 // K chunks of 64 indices from w0 on (uniform), those before `end`.
@@ -352,26 +357,33 @@ template <int K> struct SliceTokens {
   __device__ static ChunkSlot *slot(unsigned char *my_records, int set, int c) {
     return reinterpret_cast<ChunkSlot *>(my_records + __umul24((uint32_t)set, (uint32_t)kRec)) + c;
   }
-  // Enters the wave's tokens; afterwards t.hist is the slice's histogram and a slot's bits are the chunk's tokens of its
-  // set.  Ends with a workgroup barrier, the only one between the tokens and the counts that others wait for.
-  __device__ static void count(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, const int64_t (&raw)[K],
-                               uint32_t (&packed)[(K + 1) / 2], int lane) {
-    const int nl = a.sh.n_logical, R = a.n_rep;
-    const unsigned long long my_bit = 1ull << lane;
+  // Counts the wave's tokens in t.hist; needs nothing of the mapping.
+  __device__ static void count(const PlanArgs &a, const SliceTables &t, const int64_t (&raw)[K], uint32_t (&packed)[(K + 1) / 2]) {
+    const int nl = a.sh.n_logical;
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const bool valid = (uint64_t)raw[c] < (uint64_t)nl;   // -1, other negatives and too large ids fail
-      const int e = valid ? (int)raw[c] : nl;
-      pack_expert(packed, c, e);
-      const int set = t.route[e].rep;
+      pack_expert(packed, c, valid ? (int)raw[c] : nl);
       if (valid)
-        atomicAdd(&t.hist[e], 1);
-      if (set < R)
-        atomicOr(reinterpret_cast<unsigned long long *>(slot(my_records, set, c)), my_bit);
+        atomicAdd(&t.hist[(int)raw[c]], 1);
     }
-    __syncthreads();
-    LPLB_PLAN_STAMP(8);
-    LPLB_SLICE_STAMP(1);
+  }
+  // A slot's bits become the chunk's tokens of its set.  The wave's own slots: no barrier.
+  __device__ static void mark(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, const uint32_t (&packed)[(K + 1) / 2], int lane) {
+    constexpr int N = K < 8 ? K : 8;   // (reads ahead of the first update: the compiler keeps their order, and each would be waited for)
+    const unsigned long long my_bit = 1ull << lane;
+#pragma unroll
+    for (int c0 = 0; c0 < K; c0 += N) {
+      int set[N];
+#pragma unroll
+      for (int c = 0; c < N; ++c)
+        set[c] = t.route[packed_expert(packed, c0 + c)].rep;
+#pragma unroll
+      for (int c = 0; c < N; ++c)
+        if (set[c] < a.n_rep)
+          atomicOr(reinterpret_cast<unsigned long long *>(slot(my_records, set[c], c0 + c)), my_bit);
+    }
+    own_slots_are_written();
   }
   // The tokens of each set in the wave's earlier chunks into the slots, those in the whole wave into t.wave_total.  lane = set:
   // the chunks' pop-counts add up as they are read.  (lane = (set, chunk) with a scan over the lanes of a set takes as many instructions
@@ -618,8 +630,7 @@ __device__ inline bool last_wave_to_arrive(int *arrived, int waves, int lane) {
 }
 // What others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
 // those that add them up; the tokens of each replicated set before this slice and in the whole batch.
-// (long slices take the two apart)
-enum class Units { kAll, kTotals, kSets };
+enum class Units { kTotals, kSets };
 template <bool LONG, Units WHICH>
 __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceTables &t, int slice, uint32_t tag, int lane, int wave_s,
                                                  int *missing, int *block_sums) {
@@ -869,12 +880,16 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   }
   if (tid < 17)
     block_sums[tid] = 0;
-  build_plan_tables<K>(a, t, tl, tid);
+  clear_plan_tables<K>(a, t, tid);
+  __syncthreads();
   LPLB_PLAN_STAMP(10);
-
+  enter_plan_tables(a, t, tl, tid);
   // ---- the tokens ----
   uint32_t packed[(K + 1) / 2];
-  SliceTokens<K>::count(a, t, my_records, raw, packed, lane);
+  SliceTokens<K>::count(a, t, raw, packed);
+  __syncthreads();
+  LPLB_PLAN_STAMP(8);
+  LPLB_SLICE_STAMP(1);
   // ---- this slice's counts, for every workgroup: the histogram by the first half of the waves, the sets by the others ----
   worked_out_here(gen_and_poison);
   const int gen = (int)(uint32_t)gen_and_poison;
@@ -893,7 +908,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
       }
     } else {
       for (int q2 = tid - kHalf; q2 < set_lanes; q2 += kHalf) {
-        const int first = t.hist[2 * q2 < R ? t.set_expert[2 * q2] : nl], second = t.hist[2 * q2 + 1 < R ? t.set_expert[2 * q2 + 1] : nl];
+        const int first = t.hist[2 * q2 < R ? expert_of_set(a, t, 2 * q2) : nl], second = t.hist[2 * q2 + 1 < R ? expert_of_set(a, t, 2 * q2 + 1) : nl];
         agent_store(set_rows + slice * a.set_words + q2, tagged_word(tag, (uint32_t)first | (uint32_t)second << 16));
       }
     }
@@ -902,18 +917,15 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   }
   LPLB_PLAN_STAMP(1);
   LPLB_SLICE_STAMP(2);
-  // ---- while the others' words are on their way: the tokens of each set in this slice's earlier chunks (a wave that adds
-  //      up totals, which the LP waits for, does that first) ----
-  const bool adds_totals = slice < a.adders && wave_s >= kPlanWaves - a.unit_blocks;
-  if (!adds_totals)
-    SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
   // ---- what others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
-  //      those that add them up; the tokens of each replicated set before this slice and in the whole batch ----
-  if (!poisoned) {
-    add_up_published<false, Units::kAll>(a, t, slice, tag, lane, wave_s, missing, block_sums);
-  }
-  if (adds_totals)
-    SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
+  //      those that add them up and the LP waits for them; the tokens of each replicated set before this slice and in the whole batch.
+  //      In between, while words are on their way, the tokens of each set in this slice's earlier chunks ----
+  if (!poisoned)
+    add_up_published<false, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+  SliceTokens<K>::mark(a, t, my_records, packed, lane);
+  SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
+  if (!poisoned)
+    add_up_published<false, Units::kSets>(a, t, slice, tag, lane, wave_s, missing, block_sums);
   LPLB_PLAN_STAMP(11);
   if (poisoned)
     missing[0] = 1;
@@ -1058,7 +1070,10 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     my_hist[e] = 0;
   for (int i = lane; i < padded_sets * kLongBitsBytes / 8; i += kWave)
     reinterpret_cast<unsigned long long *>(my_bits)[i] = 0ull;
-  build_plan_tables<0>(a, t, tl, tid);
+  clear_plan_tables<0>(a, t, tid);
+  __syncthreads();
+  enter_plan_tables(a, t, tl, tid);
+  __syncthreads();
   for (int e = tid; e <= nl; e += kPlanThreads)   // (read behind the next barrier)
     set_of_expert[e] = (unsigned char)t.route[e].rep;
   LPLB_PLAN_STAMP(10);
@@ -1107,7 +1122,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     } else {
       // lane = (word, set of its two, wave): what is in the waves before, and the word from the lane that has the last wave's
       for (int i = tid - kHalf; i < 16 * a.set_words; i += kHalf) {
-        const int w = i % kPlanWaves, q = i / kPlanWaves, x = q < R ? t.set_expert[q] : nl;
+        const int w = i % kPlanWaves, q = i / kPlanWaves, x = q < R ? expert_of_set(a, t, q) : nl;
         const int own = x < nl ? wave_hists[w * hist_len + x] : 0;
         const int before = group_exclusive_scan<kPlanWaves>(own, w);
         if (q < R)
@@ -1291,8 +1306,14 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   uint32_t packed[(K + 1) / 2];
   // (called by the LP waves once their own table loads are on their way)
   auto count_the_tokens = [&]() -> bool {
-    build_plan_tables<K>(a, t, tl, tid);
-    SliceTokens<K>::count(a, t, my_records, raw, packed, lane);
+    clear_plan_tables<K>(a, t, tid);
+    __syncthreads();
+    enter_plan_tables(a, t, tl, tid);
+    SliceTokens<K>::count(a, t, raw, packed);
+    __syncthreads();
+    SliceTokens<K>::mark(a, t, my_records, packed, lane);
+    __syncthreads();
+    LPLB_PLAN_STAMP(8);
     return true;
   };
   if (wave_s < n_lps) {
@@ -1309,7 +1330,7 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   } else {
     count_the_tokens();
   }
-  auto tokens_of = [&](int q) { return t.hist[t.set_expert[q]]; };   // of a set, in the batch
+  auto tokens_of = [&](int q) { return t.hist[expert_of_set(a, t, q)]; };   // of a set, in the batch
   // The totals and the normalised counts go out while the LPs are solved.
   if (wave_s >= n_lps || n_lps == kPlanWaves) {
     const int first = n_lps == kPlanWaves ? 0 : n_lps * kWave;
