@@ -217,7 +217,7 @@ static int try_one_launch(const int64_t *idx, int64_t n_elements, const int32_t 
   const auto launch_variant = G <= 8 ? launch_plan_up_to_8 : G <= 16 ? launch_plan_up_to_16 : launch_plan_up_to_32;
   // A short batch that feeds the LPs itself is one workgroup, unless its tables do not fit a CU (or a fault is to be
   // injected, which needs workgroups that wait).
-  if (counts == nullptr && n_elements <= kSingleMaxIndices && n_group <= kSingleMaxLps && g_fault_extra_slices == 0) {
+  if (counts == nullptr && n_group <= kSingleMaxLps && n_elements <= single_max_indices(n_group) && g_fault_extra_slices == 0) {
     a.n_slices = 1;
     a.per = slice_len(n_elements, 1);
     const int rc = launch_variant(a, s, done);

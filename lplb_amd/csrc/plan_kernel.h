@@ -9,7 +9,7 @@
 //     slice in LDS -> publish it and the replicated sets' part of it -> bitmaps of the replicated sets, the other slices' counts
 //     of those -> ordinals and hashes -> wait for the LP's shares -> choose original or replica, store;
 //   LP workgroup: (own-histogram mode: collect the slices' histograms ->) solve -> publish the shares.
-// A batch of up to 4096 indices that feeds the LP itself is one workgroup that does both (plan_in_one_workgroup):
+// A batch of up to 3584 indices that feeds the LP itself is one workgroup that does both (plan_in_one_workgroup):
 // nothing is exchanged and nothing has to be resident beside it.
 //
 // What crosses workgroups are 8-byte words that say themselves whether they are complete, so that there is no
@@ -314,17 +314,27 @@ __device__ inline int expert_of_set(const PlanArgs &a, const SliceTables &t, int
   return t.route[e].rep == q ? e : a.sh.n_logical;
 }
 
-// K chunks of 64 indices from w0 on (uniform), those before `end`.
+// K chunks of 64 indices from w0 on (uniform); places past the last before `end` (not 0) repeat that, until mask_chunks is called
+// once something else has been done.  (Loads that some lanes leave out, or a look at what was loaded, wait for all loads before.)
 template <int K> __device__ inline void load_chunks(int64_t (&raw)[K], const int64_t *idx, int64_t w0, int64_t end, int lane) {
-  const int64_t *src = idx + w0 + lane;
+  const int64_t *src = idx + w0;
   if (w0 + K * kWave <= end) {
 #pragma unroll
     for (int c = 0; c < K; ++c)
-      raw[c] = __builtin_nontemporal_load(src + c * kWave);
+      raw[c] = __builtin_nontemporal_load(src + lane + c * kWave);
   } else {
+    const int last = (int)(end - 1 - w0);
 #pragma unroll
     for (int c = 0; c < K; ++c)
-      raw[c] = w0 + c * kWave + lane < end ? __builtin_nontemporal_load(src + c * kWave) : -1;
+      raw[c] = __builtin_nontemporal_load(src + min(c * kWave + lane, last));
+  }
+}
+template <int K> __device__ inline void mask_chunks(int64_t (&raw)[K], int64_t w0, int64_t end, int lane) {
+  if (w0 + K * kWave > end) {
+    const int last = (int)(end - 1 - w0);
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      raw[c] = c * kWave + lane <= last ? raw[c] : -1;
   }
 }
 template <int K> __device__ inline void store_chunks(const int32_t (&o)[K], int64_t *out, int64_t w0, int64_t end, int lane) {
@@ -617,6 +627,18 @@ __device__ inline bool collect_totals(const PlanArgs &a, int32_t *counts, uint32
   return true;
 }
 
+// Waves of a workgroup that wait for some of the others without a barrier for all: what one has done to the LDS before it arrives
+// is there for those that have waited.  (Whoever is waited for arrives before it waits itself, so every wait ends.)
+__device__ inline void wave_arrives(int *arrived, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  if (lane == 0)
+    __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline void wait_for_waves(const int *arrived, int waves) {
+  while (__hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < waves)
+    __builtin_amdgcn_s_sleep(1);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 // By whole waves of a workgroup that have added to words in LDS: true for the wave that comes last, which sees what all `waves`
 // of them have added.  (On either side of the count a wait for the LDS and no more; only with more than 64 slices.)
 __device__ inline bool last_wave_to_arrive(int *arrived, int waves, int lane) {
@@ -886,6 +908,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   enter_plan_tables(a, t, tl, tid);
   // ---- the tokens ----
   uint32_t packed[(K + 1) / 2];
+  mask_chunks<K>(raw, w0, end, lane);
   SliceTokens<K>::count(a, t, raw, packed);
   __syncthreads();
   LPLB_PLAN_STAMP(8);
@@ -1277,17 +1300,23 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 }
 
 // A short batch that feeds the LP itself, as one workgroup: the LPs are solved by its first waves between the
-// histogram and the choice.  Bound by the chain table loads -> indices -> histogram (1.3 us) -> LP -> choice,
-// of which the slices' form above adds two round trips through memory between slices and LP.  The LP reads the histogram
-// where the tokens were counted, behind the one barrier that it takes; the ordinals are worked out by the other waves while it runs.
-// Up to kSingleMaxIndices, eight per lane: past that a wave's chunks take longer than the exchange.  The LP waves come last
-// in the order of the indices, so that they have none unless the batch fills all eight waves.
-constexpr int kSingleMaxIndices = 4096, kSingleMaxLps = kPlanWaves;
+// histogram and the choice.  Bound by the chain indices -> histogram (1.1 us) -> LP -> choice, of which the slices' form above adds
+// two round trips through memory between slices and LP.  The LP reads the histogram where the tokens were counted; bitmaps, ordinals
+// and where each set's share will be are worked out by the other waves while it runs, and those wait for each other by a count in
+// LDS, since a barrier would wait for the LP.  (With the bitmaps marked by all waves ahead of the LP: [7 x 8] 6.75 instead of 6.4 us,
+// [128 x 8] 7.0 and 6.7.)
+// Up to as many indices as leave the LP waves, which come last in the order of the indices, without any at eight chunks a wave.
+// One LP, in one workgroup / as slices: 3584 indices 7.6 / 8.9 us, 4096 9.7 / 8.9; two LPs, 3072 7.8 / 9.1, 3584 10.3 / 9.2; four, 2048
+// 8.4 / 9.25, 2560 11.0 / 9.25; (16, 2) 3584 10.9 / 12.1, 4096 13.9 / 12.1; (32, 2) 3584 18.3 / 19.4, 4096 22.7 / 19.4.  With eight LPs
+// every wave has one: 128 indices (two chunks in one wave) 8.5 / 9.2, 192 9.45 / 9.25.
+constexpr int kSingleMaxLps = kPlanWaves;
+constexpr int64_t single_max_indices(int n_lps) { return (n_lps < kPlanWaves ? 8 * (kPlanWaves - n_lps) : 2) * kWave; }
 template <int GM, int DM, bool EXACT, int K>
 __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __shared__ int rep_of_edge_all[kSingleMaxLps * kWave];
   __shared__ float share_of[kSingleMaxLps * kWave];
+  __shared__ int marked;   // waves whose tokens are in their bitmaps
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -1300,6 +1329,8 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   unsigned char *my_records = records_of(turn);
   const PlanTableLoads tl = issue_plan_table_loads(a, tid);
   const int64_t w0 = (int64_t)turn * (K * kWave);
+  const bool has_tokens = w0 < a.n;
+  const int waves_with_tokens = (int)((a.n + K * kWave - 1) / (K * kWave));
   int64_t raw[K];
   load_chunks<K>(raw, a.idx, w0, a.n, lane);
   LPLB_PLAN_STAMP(0);
@@ -1307,12 +1338,22 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   // (called by the LP waves once their own table loads are on their way)
   auto count_the_tokens = [&]() -> bool {
     clear_plan_tables<K>(a, t, tid);
+    if (tid == 0)
+      marked = 0;
     __syncthreads();
     enter_plan_tables(a, t, tl, tid);
+    mask_chunks<K>(raw, w0, a.n, lane);
     SliceTokens<K>::count(a, t, raw, packed);
     __syncthreads();
-    SliceTokens<K>::mark(a, t, my_records, packed, lane);
-    __syncthreads();
+    if (has_tokens) {
+      SliceTokens<K>::mark(a, t, my_records, packed, lane);
+      for (int q = lane; q < R; q += kWave) {   // (every wave enters the same values)
+        const SetOfPlan s = set_of_plan(a, R - 1 - q);
+        set_total(t.reps[q], t.hist[expert_of_set(a, t, q)]);
+        t.reps[q].expected = s.ep_rank * a.sh.D + s.d;   // until the shares are there: where its share will be
+      }
+      wave_arrives(&marked, lane);
+    }
     LPLB_PLAN_STAMP(8);
     return true;
   };
@@ -1330,7 +1371,6 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   } else {
     count_the_tokens();
   }
-  auto tokens_of = [&](int q) { return t.hist[expert_of_set(a, t, q)]; };   // of a set, in the batch
   // The totals and the normalised counts go out while the LPs are solved.
   if (wave_s >= n_lps || n_lps == kPlanWaves) {
     const int first = n_lps == kPlanWaves ? 0 : n_lps * kWave;
@@ -1346,23 +1386,20 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
       a.solve.gw_out[e] = (float)n / wmax;
     }
   }
-  const bool has_tokens = w0 < a.n;
   int32_t h[K];
   if (has_tokens) {
-    for (int q = lane; q < R; q += kWave)   // (every wave enters the same values: none has to wait for another)
-      set_total(t.reps[q], tokens_of(q));
+    wait_for_waves(&marked, waves_with_tokens);
     SliceTokens<K>::starts_of_batch(a, my_records, lane, turn, records_of);
 #pragma unroll
     for (int c = 0; c < K; ++c)
       h[c] = SliceTokens<K>::hash(t, my_records, nullptr, R, packed_expert(packed, c), c);
   }
   if (wave_s < n_lps) {
-    __builtin_amdgcn_wave_barrier();   // (its shares have been stored)
+    wait_for_waves(&marked, waves_with_tokens);   // (and its own shares have been stored)
     const int per_group = a.sh.G * a.sh.C * a.sh.D;
     for (int i = lane; i < per_group; i += kWave) {
-      const int set = wave_s * per_group + i;
-      const SetOfPlan s = set_of_plan(a, set);
-      t.reps[R - 1 - set].expected = expected_on_original(share_of[s.ep_rank * a.sh.D + s.d], tokens_of(R - 1 - set));
+      RepEntry &x = t.reps[R - 1 - (wave_s * per_group + i)];
+      x.expected = expected_on_original(share_of[x.expected], x.total);
     }
   }
   __syncthreads();
