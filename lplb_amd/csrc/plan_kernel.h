@@ -171,6 +171,13 @@ __device__ inline void give_up(const PlanArgs &a, unsigned long long *avail_stat
 #endif
 
 // ---- a slice's tables in LDS ----
+// Per logical expert; all zeros: no slot and no set, as for masked and out-of-range tokens (entry n_logical).
+// Sets are numbered from 1 in the order of minilp.cu:478-495, 0 is no set, so that what is empty is zero throughout.
+struct __attribute__((aligned(8))) PlanRoute {
+  int32_t not_original;   // complement of the original's physical slot
+  int32_t set;
+  __device__ int32_t original() const { return ~not_original; }
+};
 // One ranking slot per (wave, replicated set, chunk of 64 indices), K chunks per wave.
 constexpr int64_t kLongestSlice = 16 * kPlanThreads;   // 16 chunks per wave
 constexpr int kLongChunks = 8, kLongPasses = 8;        // of a long slice: chunks per wave and pass, passes
@@ -178,18 +185,20 @@ constexpr int kFewestLongSlices = 64;
 constexpr int64_t kLongestOfLongSlices = kLongPasses * kLongChunks * kPlanThreads;
 // (K = 0: a long slice, without its records, which lie behind the rest)
 constexpr int slice_record_bytes(int k) { return k > 0 ? rank_record_bytes_single(k) : 0; }
+// (what a slice's workgroup keeps beside its tables: missing, block_sums)
+constexpr int kBlockSums = 17, kSliceFlags = 2 + kBlockSums;
 template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
   return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * slice_record_bytes(K) +
-         (size_t)(n_logical + 2) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
-         (size_t)(3 + 2 * kPlanWaves) * n_rep * sizeof(int32_t);
+         (size_t)(n_logical + 2) * sizeof(PlanRoute) + (size_t)(n_logical + 16 + kSliceFlags) * sizeof(int32_t) +
+         (size_t)(3 + 2 * kPlanWaves) * (n_rep + 1) * sizeof(int32_t);
 }
 // A long slice's records per (wave, replicated set): the bitmaps of a pass's chunks, and what a token's ordinal is made of (a
 // bitmap and the tokens before it), both padded for the LDS banks; sixteen sets are worked on at once.
 constexpr int kLongBitsBytes = kLongChunks * 8 + 8, kLongRanksBytes = kLongChunks * 16 + 16;
 __host__ __device__ constexpr int long_slice_padded_sets(int n_rep) { return n_rep / 16 * 16 + 16; }   // at least one more: of tokens without a set
 __host__ __device__ constexpr size_t long_slice_records_at(int n_logical, int n_rep) {
-  return ((size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)(n_logical + 2) * sizeof(Route) + (size_t)(n_logical + 16) * sizeof(int32_t) +
-          (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t) + 15) / 16 * 16;
+  return ((size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)(n_logical + 2) * sizeof(PlanRoute) + (size_t)(n_logical + 16 + kSliceFlags) * sizeof(int32_t) +
+          (size_t)(3 + kPlanWaves) * (n_rep + 1) * sizeof(int32_t) + 15) / 16 * 16;
 }
 inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
   return long_slice_records_at(n_logical, n_rep) +
@@ -197,26 +206,30 @@ inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
          (size_t)(n_logical + 16) / 16 * 16;
 }
 struct SliceTables {
-  RepEntry *reps;           // [R + 1]
+  RepEntry *reps;           // [R + 1] by set; of set 0: a test that never sends a token away
+  PlanRoute *route;         // [n_logical + 1]
   unsigned char *records;   // [waves][R + 1][record bytes]
-  Route *route;             // [n_logical + 1]
-  int32_t *set_expert;      // [R] the expert whose tokens the set has; n_logical (which has none): it has none
-  int32_t *before, *total;  // [R] tokens of the set before this slice, in the whole batch
-  int32_t *wave_total;      // [waves][R] ... in each wave
-  int32_t *base;            // [waves][R] ... before each wave (not for long slices)
   int32_t *hist;            // [more than n_logical, a multiple of 16] the slice's histogram, then zeros; in the first slice at last the batch's
+  int32_t *missing;         // [2] [0] some counts did not come, [1] some share will not come
+  int32_t *block_sums;      // [kBlockSums] what the workgroup's units have added up of the totals, the last: how many of them have
+  int32_t *before, *total;  // [R + 1] tokens of the set before this slice, in the whole batch
+  int32_t *set_expert;      // [R + 1] the expert whose tokens the set has; n_logical (which has none): it has none
+  int32_t *wave_total;      // [waves][R + 1] ... in each wave
+  int32_t *base;            // [waves][R + 1] ... before each wave (not for long slices)
 };
 template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, int nl, int R) {
   SliceTables t;
   t.reps = reinterpret_cast<RepEntry *>(lds);
-  t.route = reinterpret_cast<Route *>(t.reps + R + 1);
+  t.route = reinterpret_cast<PlanRoute *>(t.reps + R + 1);
   t.records = reinterpret_cast<unsigned char *>(t.route + ((nl + 2) & ~1));   // (16-byte aligned, as what lies before it is)
   t.hist = reinterpret_cast<int32_t *>(t.records + (size_t)kPlanWaves * (R + 1) * slice_record_bytes(K));
-  t.before = t.hist + nl / 16 * 16 + 16;
-  t.total = t.before + R;
-  t.set_expert = t.total + R;
-  t.wave_total = t.set_expert + R;
-  t.base = t.wave_total + kPlanWaves * R;
+  t.missing = t.hist + nl / 16 * 16 + 16;
+  t.block_sums = t.missing + 2;
+  t.before = t.missing + kSliceFlags;
+  t.total = t.before + R + 1;
+  t.set_expert = t.total + R + 1;
+  t.wave_total = t.set_expert + R + 1;
+  t.base = t.wave_total + kPlanWaves * (R + 1);
   if (K == 0)
     t.records = lds + long_slice_records_at(nl, R);
   return t;
@@ -239,21 +252,31 @@ __device__ inline SetOfPlan set_of_plan(const PlanArgs &a, int i) {
 __device__ inline int slot_of_plan(const PlanArgs &a, int e) {
   return e + (int)fast_div((uint32_t)e, a.magic_L) * (a.sh.P - a.sh.L);
 }
+// Half of the waves look after the experts, the others after the sets: the fewer instructions a wave has in front of its counts,
+// the better (below).  With that, empty entries that are all zeros (one loop clears everything) and places of 32 bits, counts are out
+// 1.4 instead of 1.6 us after the start: plan [8192 x 8] 7.0 -> 6.85 us, run [262144 x 8] 15.45 -> 15.25, [1048576 x 8] 34.7 -> 33.4.
+constexpr int kPlanHalf = kPlanThreads / 2;
 struct PlanTableLoads {
-  int slot0, le0, rle0, host0;
-  int physical_le0;   // phy2log of physical slot tid
-  bool set0;
-  SetOfPlan s0;
+  int slot, expert, second;   // an original's slot and its expert, that of the next kPlanHalf; or a set's replica and its expert
+  int physical_le0;           // phy2log of physical slot tid, where it is asked for
 };
-__device__ inline PlanTableLoads issue_plan_table_loads(const PlanArgs &a, int tid) {
-  PlanTableLoads t;
-  t.slot0 = slot_of_plan(a, min(tid, a.sh.n_logical - 1));
-  t.le0 = a.phy2log[t.slot0];
-  t.set0 = tid < a.n_rep;
-  t.s0 = set_of_plan(a, t.set0 ? tid : 0);
-  t.rle0 = a.phy2log[t.s0.ep_rank * a.sh.P + t.s0.place];
-  t.host0 = a.o2r[t.s0.group_rank * a.sh.D + t.s0.d];
-  t.physical_le0 = a.phy2log[min(tid, a.sh.n_ranks * a.sh.P - 1)];
+__device__ inline PlanTableLoads issue_plan_table_loads(const PlanArgs &a, int tid, int wave_s, bool with_physical) {
+  PlanTableLoads t{};
+  if (wave_s < kPlanWaves / 2) {
+    const int nl = a.sh.n_logical;
+    t.slot = slot_of_plan(a, min(tid, nl - 1));
+    t.expert = a.phy2log[t.slot];
+    if (nl > kPlanHalf)
+      t.second = a.phy2log[slot_of_plan(a, min(tid + kPlanHalf, nl - 1))];
+  } else {
+    const int i = min(tid - kPlanHalf, a.n_rep - 1);
+    const SetOfPlan s = set_of_plan(a, i);
+    t.expert = a.phy2log[s.ep_rank * a.sh.P + s.place];
+    t.second = a.o2r[s.group_rank * a.sh.D + s.d];
+    t.slot = (s.ep_rank - s.group_rank + 1) * a.sh.P - a.sh.C * a.sh.D + s.place;   // (on the group's first rank)
+  }
+  if (with_physical)
+    t.physical_le0 = a.phy2log[min(tid, a.sh.n_ranks * a.sh.P - 1)];
   return t;
 }
 // What a slice does before its counts are out is what the LP waits for, and it is bound by instructions: the loads
@@ -262,61 +285,72 @@ __device__ inline PlanTableLoads issue_plan_table_loads(const PlanArgs &a, int t
 // mapping is entered in the same interval between two barriers, and the bitmaps are marked behind the publishing.  Per call,
 // against tables first and a route looked up for every token that is counted: run [8192 x 8] 9.55 -> 9.3 us, [32768 x 8] 10.45 -> 9.9,
 // [100000 x 8] 12.6 -> 11.7, [262144 x 8] 16.85 -> 15.4, [16384 x 8] at 32 ranks 20.85 -> 20.25; in one workgroup [128 x 8] 7.2 -> 7.05.
-// (Beyond that, the sets' totals and the waves' bases worked out ahead of the barrier instead of behind it: no faster.)
+// (Beyond that, the sets' totals and the waves' bases worked out ahead of the barrier instead of behind it: no faster; the places of
+// the first totals to add up worked out while the loads are on their way: 0.3 us slower.)
 
-// Everything empty: routes to nowhere, zeros from the records to the totals (which lie side by side, so that this is one loop,
-// of one turn for most).  A workgroup barrier has to follow.
-template <int K> __device__ inline void clear_plan_tables(const PlanArgs &a, const SliceTables &t, int tid) {
-  constexpr int nt = kPlanThreads;
-  const int nl = a.sh.n_logical, R = a.n_rep;
-  for (int e = tid; e <= nl; e += nt)
-    t.route[e] = Route{-1, R};
-  unsigned char *from = K > 0 ? t.records : reinterpret_cast<unsigned char *>(t.hist);
-  const int n16 = (int)(reinterpret_cast<unsigned char *>(t.set_expert) - from + 15) / 16;   // (the end may reach into set_expert)
-  const i32x4 zero{0, 0, 0, 0};
-  for (int i = tid; i < n16; i += nt)
-    reinterpret_cast<i32x4 *>(from)[i] = zero;
-  if (tid == 0)
-    t.reps[R] = RepEntry{1, 0xffffffffu, INT32_MAX, -1};   // "no replica": every token stays
+// Everything empty: zeros from the routes to the totals (which lie side by side, so that this is one loop, of one turn for most).  A
+// workgroup barrier has to follow.
+template <int K> __device__ inline void clear_plan_tables(const SliceTables &t, int tid) {
+  auto clear = [&](void *from, void *to) {   // (the end may reach into what is written behind the barrier)
+    const int n16 = (int)(reinterpret_cast<unsigned char *>(to) - reinterpret_cast<unsigned char *>(from) + 15) / 16;
+    const i32x4 zero{0, 0, 0, 0};
+    for (int i = tid; i < n16; i += kPlanThreads)
+      reinterpret_cast<i32x4 *>(from)[i] = zero;
+  };
+  clear(t.route, t.set_expert);   // (in a long slice the records, which lie elsewhere, are the waves' own)
 }
 // Where an expert's tokens go when nothing is redirected and which replicated set (if any) it belongs to
 // (minilp.cu:466-496).  A workgroup barrier has to follow.
-__device__ inline void enter_plan_tables(const PlanArgs &a, const SliceTables &t, const PlanTableLoads &l, int tid) {
-  constexpr int nt = kPlanThreads;
-  const int nl = a.sh.n_logical, R = a.n_rep, cd = a.sh.C * a.sh.D;
-  if (tid < nl && l.le0 >= 0 && l.le0 < nl)
-    t.route[l.le0].original = l.slot0;
-  for (int e = tid + nt; e < nl; e += nt) {
-    const int s = slot_of_plan(a, e), le = a.phy2log[s];
-    if (le >= 0 && le < nl)
-      t.route[le].original = s;
-  }
-  // A set's key is R - 1 - i, so that of two sets that name the same expert the later one
-  // wins (as a sequential pass over the sets would have it) with an atomic min.
-  auto enter_set = [&](int i, const SetOfPlan &s, int le, int host) {
-    const bool ok = le >= 0 && le < nl;
-    if (ok)
-      atomicMin(&t.route[le].rep, R - 1 - i);
-    t.reps[R - 1 - i] = RepEntry{0, 0u, 0, ((s.ep_rank - s.group_rank) + host + 1) * a.sh.P - cd + s.place};
-    t.set_expert[R - 1 - i] = ok ? le : nl;
-  };
-  if (l.set0)
-    enter_set(tid, l.s0, l.rle0, l.host0);
-  for (int i = tid + nt; i < R; i += nt) {
-    const SetOfPlan s = set_of_plan(a, i);
-    enter_set(i, s, a.phy2log[s.ep_rank * a.sh.P + s.place], a.o2r[s.group_rank * a.sh.D + s.d]);
+__device__ inline void enter_plan_tables(const PlanArgs &a, const SliceTables &t, const PlanTableLoads &l, int tid, int wave_s) {
+  const int nl = a.sh.n_logical, R = a.n_rep;
+  if (wave_s < kPlanWaves / 2) {
+    auto enter_expert = [&](int slot, int le) {
+      if ((uint32_t)le < (uint32_t)nl)
+        t.route[le].not_original = ~slot;
+    };
+    if (tid < nl)
+      enter_expert(l.slot, l.expert);
+    if (nl > kPlanHalf) {
+      if (tid + kPlanHalf < nl)
+        enter_expert(slot_of_plan(a, tid + kPlanHalf), l.second);
+      for (int e = tid + 2 * kPlanHalf; e < nl; e += kPlanHalf) {
+        const int s = slot_of_plan(a, e);
+        enter_expert(s, a.phy2log[s]);
+      }
+    }
+  } else {
+    // (of two sets that name the same expert the later one wins, as a sequential pass over the sets would have it)
+    auto enter_set = [&](int i, int slot, int le, int host) {
+      const bool ok = (uint32_t)le < (uint32_t)nl;
+      if (ok)
+        atomicMax(&t.route[le].set, i + 1);
+      t.reps[i + 1] = RepEntry{0, 0u, 0, slot + host * a.sh.P};
+      t.set_expert[i + 1] = ok ? le : nl;
+    };
+    const int i0 = tid - kPlanHalf;
+    if (i0 < R)
+      enter_set(i0, l.slot, l.expert, l.second);
+    if (i0 == kPlanHalf - 1)
+      t.reps[0] = RepEntry{1, 0xffffffffu, INT32_MAX, -1};   // "no replica": every token stays
+    if (R > kPlanHalf)
+      for (int i = i0 + kPlanHalf; i < R; i += kPlanHalf) {
+        const SetOfPlan s = set_of_plan(a, i);
+        enter_set(i, (s.ep_rank - s.group_rank + 1) * a.sh.P - a.sh.C * a.sh.D + s.place, a.phy2log[s.ep_rank * a.sh.P + s.place],
+                  a.o2r[s.group_rank * a.sh.D + s.d]);
+      }
   }
 }
-// The expert whose tokens set q has, once the routes are there; n_logical: none (of two sets that name the same expert only one
+// The expert whose tokens a set has, once the routes are there; n_logical: none (of two sets that name the same expert only one
 // has the tokens).
-__device__ inline int expert_of_set(const PlanArgs &a, const SliceTables &t, int q) {
-  const int e = t.set_expert[q];
-  return t.route[e].rep == q ? e : a.sh.n_logical;
+__device__ inline int expert_of_set(const PlanArgs &a, const SliceTables &t, int set) {
+  const int e = t.set_expert[set];
+  return t.route[e].set == set ? e : a.sh.n_logical;
 }
 
 // K chunks of 64 indices from w0 on (uniform); places past the last before `end` (not 0) repeat that, until mask_chunks is called
 // once something else has been done.  (Loads that some lanes leave out, or a look at what was loaded, wait for all loads before.)
-template <int K> __device__ inline void load_chunks(int64_t (&raw)[K], const int64_t *idx, int64_t w0, int64_t end, int lane) {
+// Places are below 2^32: a batch has fewer than 2^31 indices.
+template <int K> __device__ inline void load_chunks(int64_t (&raw)[K], const int64_t *idx, uint32_t w0, uint32_t end, int lane) {
   const int64_t *src = idx + w0;
   if (w0 + K * kWave <= end) {
 #pragma unroll
@@ -329,7 +363,7 @@ template <int K> __device__ inline void load_chunks(int64_t (&raw)[K], const int
       raw[c] = __builtin_nontemporal_load(src + min(c * kWave + lane, last));
   }
 }
-template <int K> __device__ inline void mask_chunks(int64_t (&raw)[K], int64_t w0, int64_t end, int lane) {
+template <int K> __device__ inline void mask_chunks(int64_t (&raw)[K], uint32_t w0, uint32_t end, int lane) {
   if (w0 + K * kWave > end) {
     const int last = (int)(end - 1 - w0);
 #pragma unroll
@@ -337,16 +371,17 @@ template <int K> __device__ inline void mask_chunks(int64_t (&raw)[K], int64_t w
       raw[c] = c * kWave + lane <= last ? raw[c] : -1;
   }
 }
-template <int K> __device__ inline void store_chunks(const int32_t (&o)[K], int64_t *out, int64_t w0, int64_t end, int lane) {
+template <int K> __device__ inline void store_chunks(const int32_t (&o)[K], int64_t *out, uint32_t w0, uint32_t end, int lane) {
   int64_t *dst = out + w0 + lane;
   if (w0 + K * kWave <= end) {
 #pragma unroll
     for (int c = 0; c < K; ++c)
       __builtin_nontemporal_store((int64_t)o[c], dst + c * kWave);
   } else {
+    const int last = (int)(end - 1 - w0);
 #pragma unroll
     for (int c = 0; c < K; ++c)
-      if (w0 + c * kWave + lane < end)
+      if (c * kWave + lane <= last)
         __builtin_nontemporal_store((int64_t)o[c], dst + c * kWave);
   }
 }
@@ -387,10 +422,10 @@ template <int K> struct SliceTokens {
       int set[N];
 #pragma unroll
       for (int c = 0; c < N; ++c)
-        set[c] = t.route[packed_expert(packed, c0 + c)].rep;
+        set[c] = t.route[packed_expert(packed, c0 + c)].set;
 #pragma unroll
       for (int c = 0; c < N; ++c)
-        if (set[c] < a.n_rep)
+        if (set[c] != 0)
           atomicOr(reinterpret_cast<unsigned long long *>(slot(my_records, set[c], c0 + c)), my_bit);
     }
     own_slots_are_written();
@@ -401,7 +436,7 @@ template <int K> struct SliceTokens {
   // with 128 sets 11.0 -> 10.2; [262144 x 8] with 16 sets 18.0 -> 17.9.)
   __device__ static void starts_in_wave(const PlanArgs &a, const SliceTables &t, unsigned char *my_records, int lane, int wave_s) {
     const int R = a.n_rep;
-    for (int q = lane; q < R; q += kWave) {
+    for (int q = lane + 1; q <= R; q += kWave) {
       unsigned long long bits[K];
 #pragma unroll
       for (int c = 0; c < K; ++c)
@@ -412,18 +447,18 @@ template <int K> struct SliceTokens {
         slot(my_records, q, c)->start = before;
         before += __popcll(bits[c]);
       }
-      t.wave_total[wave_s * R + q] = before;
+      t.wave_total[wave_s * (R + 1) + q] = before;
     }
   }
   // The tokens of each set before this wave's first into t.base.  The wave's own entries only: no barrier.
   __device__ static void bases(const PlanArgs &a, const SliceTables &t, int lane, int wave_s) {
     const int R = a.n_rep;
-    for (int q = lane; q < R; q += kWave) {
+    for (int q = lane + 1; q <= R; q += kWave) {
       int32_t base = t.before[q];
 #pragma unroll
       for (int w = 0; w < kPlanWaves - 1; ++w)
-        base += w < wave_s ? t.wave_total[w * R + q] : 0;
-      t.base[wave_s * R + q] = base;
+        base += w < wave_s ? t.wave_total[w * (R + 1) + q] : 0;
+      t.base[wave_s * (R + 1) + q] = base;
     }
     own_slots_are_written();
   }
@@ -434,7 +469,7 @@ template <int K> struct SliceTokens {
     const int R = a.n_rep, c = lane % K;
     for (int p0 = 0; p0 < R * K; p0 += kWave) {
       const bool live = p0 + lane < R * K;
-      const int q = live ? (p0 + lane) / K : R;
+      const int q = live ? (p0 + lane) / K + 1 : 0;
       int earlier = 0;
       for (int w = 0; w < turn; ++w)
         earlier += __popcll(*reinterpret_cast<const unsigned long long *>(slot(records_of(w), q, c)));
@@ -452,9 +487,9 @@ template <int K> struct SliceTokens {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   // base: of the wave's sets, or null: part of the starts.
-  __device__ static int32_t hash(const SliceTables &t, unsigned char *my_records, const int32_t *base, int R, int e, int c) {
-    const int set = t.route[e].rep;
-    const int32_t before = base ? base[min(set, R - 1)] : 0;
+  __device__ static int32_t hash(const SliceTables &t, unsigned char *my_records, const int32_t *base, int e, int c) {
+    const int set = t.route[e].set;
+    const int32_t before = base ? base[set] : 0;   // (of no set: whatever is there)
     const i32x4 s = *reinterpret_cast<const i32x4 *>(slot(my_records, set, c));   // bits_lo, bits_hi, start
     const i32x4 x = *reinterpret_cast<const i32x4 *>(&t.reps[set]);               // total, magic, -, -
     const int32_t k =
@@ -466,18 +501,18 @@ template <int K> struct SliceTokens {
 // Tokens per physical expert (= bincount of the output) from a slice's tables; hist: of the batch.
 // le0: phy2log of slot tid (or of any slot if there is none), read ahead of time.
 __device__ inline void plan_physical_counts(const PlanArgs &a, const SliceTables &t, int le0, bool ok, int tid) {
-  const int nl = a.sh.n_logical, R = a.n_rep;
+  const int nl = a.sh.n_logical;
   for (int i = tid; i < a.sh.n_ranks * a.sh.P; i += kPlanThreads) {
     const int le = !ok ? -1 : i == tid ? le0 : a.phy2log[i];
     int32_t v = ok ? 0 : -1;
     if (le >= 0 && le < nl) {
-      const Route rt = t.route[le];
-      if (rt.rep >= R) {
-        v = rt.original == i ? t.hist[le] : 0;
+      const PlanRoute rt = t.route[le];
+      if (rt.set == 0) {
+        v = rt.original() == i ? t.hist[le] : 0;
       } else {
-        const RepEntry x = t.reps[rt.rep];
+        const RepEntry x = t.reps[rt.set];
         const int32_t kept = kept_on_original(x.total, x.expected);
-        v = rt.original == i ? kept : (x.replica == i ? x.total - kept : 0);
+        v = rt.original() == i ? kept : (x.replica == i ? x.total - kept : 0);
       }
     }
     a.physical_counts[i] = v;
@@ -546,26 +581,35 @@ template <int N> __device__ inline void over_slices_of_unit(uint32_t (&v)[N], in
       v[j] = s.x + s.y;
     }
 }
-// Words 2 (lane % lanes of a slice) and the next of the rows from `rows` on (16-byte aligned; lanes past the last of `words` words,
-// an even number, repeat that), over the slices of block `block`: the four counts added up over the slices into sums[0..3]
-// and, if BEFORE, over the slices before `slice` into sums[4..7].  Whole waves; false: some never came.
+// Where a lane finds its pairs of words of a unit: words 2 (lane % lanes of a slice) and the next of the rows from `rows` on (16-byte
+// aligned; lanes past the last of `words` words, an even number, repeat that), of the slices of block `block` (past the last
+// slice: that one again).
+struct UnitAt {
+  const unsigned long long *at[kUnitLoads];
+};
+__device__ inline UnitAt unit_at(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int block, int lane) {
+  const int per_round = kWave >> a.unit_lanes_log2, p0 = block * kUnitSlices + (lane >> a.unit_lanes_log2);
+  const unsigned long long *mine = rows + min(2 * (lane & ((1 << a.unit_lanes_log2) - 1)), words - 2);
+  UnitAt u;
+#pragma unroll
+  for (int k = 0; k < kUnitLoads; ++k)
+    u.at[k] = mine + min(p0 + k * per_round, a.n_slices - 1) * stride;
+  return u;
+}
+// Adds a unit up: the four counts of a lane's words over the slices into sums[0..3] and, if BEFORE, over the slices before `slice`
+// into sums[4..7].  Whole waves; false: some never came.
 // LONG: slices of up to kLongestOfLongSlices indices.
 template <bool BEFORE, bool LONG>
-__device__ inline bool add_up_unit(const PlanArgs &a, const unsigned long long *rows, int stride, int words, int block, uint32_t tag,
-                                   int slice, int lane, uint32_t (&sums)[BEFORE ? 8 : 4]) {
+__device__ inline bool add_up_unit(const PlanArgs &a, const UnitAt &u, int block, uint32_t tag, int slice, int lane,
+                                   uint32_t (&sums)[BEFORE ? 8 : 4]) {
   if (a.expected_slices != a.n_slices)   // (an injected fault: one slice never comes)
     return false;
   const int per_round = kWave >> a.unit_lanes_log2, p0 = block * kUnitSlices + (lane >> a.unit_lanes_log2);
-  const unsigned long long *mine = rows + min(2 * (lane & ((1 << a.unit_lanes_log2) - 1)), words - 2);
-  const unsigned long long *at[kUnitLoads];
-#pragma unroll
-  for (int k = 0; k < kUnitLoads; ++k)   // (past the last slice: that one again, not counted)
-    at[k] = mine + min(p0 + k * per_round, a.n_slices - 1) * stride;
   u32x4 v[kUnitLoads];
   bool all_in = false;
   for (int polls = 0; polls < a.max_polls; ++polls) {
     if (!all_in) {
-      agent_load_pairs(v, at);
+      agent_load_pairs(v, u.at);
       uint32_t off = 0;
 #pragma unroll
       for (int k = 0; k < kUnitLoads; ++k)
@@ -656,7 +700,7 @@ enum class Units { kTotals, kSets };
 template <bool LONG, Units WHICH>
 __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceTables &t, int slice, uint32_t tag, int lane, int wave_s,
                                                  int *missing, int *block_sums) {
-  const int nl = a.sh.n_logical, R = a.n_rep, set_lanes = a.set_words;
+  const int R = a.n_rep, set_lanes = a.set_words;
   unsigned long long *set_rows = reinterpret_cast<unsigned long long *>(a.sync + kSetRowsAt);
   unsigned long long *hist_rows = reinterpret_cast<unsigned long long *>(a.sync + kHistRowsAt);
   const int unit_lanes = 1 << a.unit_lanes_log2, unit_words_log2 = a.unit_lanes_log2 + 1, block_bits = a.unit_block_bits;
@@ -673,14 +717,14 @@ __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceT
         break;
       const int word0 = (unit - adder_units) >> block_bits << unit_words_log2;
       uint32_t sums[8];
-      if (add_up_unit<true, LONG>(a, set_rows + word0, a.set_words, set_lanes - word0, block, tag, slice, lane, sums)) {
+      if (add_up_unit<true, LONG>(a, unit_at(a, set_rows + word0, a.set_words, set_lanes - word0, block, lane), block, tag, slice, lane, sums)) {
         const int first_set = 2 * word0 + 4 * lane;
         if (lane < unit_lanes)   // (words past set_lanes have no sets)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             if (first_set + j < R) {
-              atomicAdd(&t.total[first_set + j], (int32_t)sums[j]);
-              atomicAdd(&t.before[first_set + j], (int32_t)sums[4 + j]);
+              atomicAdd(&t.total[first_set + j + 1], (int32_t)sums[j]);
+              atomicAdd(&t.before[first_set + j + 1], (int32_t)sums[4 + j]);
             }
       } else {
         missing[0] = 1;
@@ -688,7 +732,8 @@ __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceT
     } else {
       const int at = unit >> block_bits << unit_words_log2, word0 = first_word + at;
       uint32_t sums[4];
-      if (add_up_unit<false, LONG>(a, hist_rows + word0, a.hist_words, my_words - at, block, tag, slice, lane, sums)) {
+      if (add_up_unit<false, LONG>(a, unit_at(a, hist_rows + word0, a.hist_words, my_words - at, block, lane), block, tag,
+                                   slice, lane, sums)) {
         bool all_in = true;
         if (a.unit_blocks > 1) {   // (eight words then, in one unit per block: the wave that comes last publishes)
           if (lane < 4)
@@ -701,13 +746,11 @@ __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceT
             for (int j = 0; j < 4; ++j)
               sums[j] = (uint32_t)block_sums[4 * lane + j];
         }
-        if (all_in && lane < unit_lanes && 2 * lane < my_words - at)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int e = 2 * word0 + 4 * lane + j;
-            if (e < nl)
-              agent_store(totals + e, tagged_word(tag, sums[j]));
-          }
+        if (all_in && lane < unit_lanes && 2 * lane < my_words - at) {   // (words behind the last expert's have zeros and are not read)
+          unsigned long long *to = totals + 2 * word0 + 4 * lane;
+          agent_store_pair(to, u32x4{sums[0], tag, sums[1], tag});
+          agent_store_pair(to + 2, u32x4{sums[2], tag, sums[3], tag});
+        }
       } else {
         missing[0] = 1;
       }
@@ -729,7 +772,7 @@ __device__ __forceinline__ void say_that_all_arrived(const PlanArgs &a, uint32_t
 }
 // The LP's shares: every set's thread polls its own; value and tag arrive in the same word.  missing[1]: some will not come.
 __device__ __forceinline__ void collect_shares(const PlanArgs &a, const SliceTables &t, int slice, int gen, unsigned long long *avail_state,
-                                               int *missing, int tid) {
+                                               int tid) {
   const int R = a.n_rep;
   const unsigned long long *shares = reinterpret_cast<const unsigned long long *>(a.sync + kSharesAt);
   const uint32_t tag_valid = share_tag((uint32_t)gen), tag_none = tag_valid + 1u;
@@ -742,11 +785,11 @@ __device__ __forceinline__ void collect_shares(const PlanArgs &a, const SliceTab
     while ((got = (uint32_t)((word = agent_load(word_at)) >> 32)) != tag_valid && got != tag_none && ++polls < a.max_polls)
       __builtin_amdgcn_s_sleep(1);
     if (got == tag_valid) {
-      t.reps[R - 1 - i].expected = expected_on_original(__builtin_bit_cast(float, (uint32_t)word), t.total[R - 1 - i]);
+      t.reps[i + 1].expected = expected_on_original(__builtin_bit_cast(float, (uint32_t)word), t.total[i + 1]);
     } else {
       if (got != tag_none)
         give_up(a, avail_state);
-      missing[1] = 1;
+      t.missing[1] = 1;
     }
   }
 }
@@ -856,8 +899,7 @@ template <int GM, int DM, bool EXACT, int K>
 __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void plan_in_one_launch(PlanArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
-  __shared__ int missing[2];   // LP workgroup: [0] some counts did not come; slice: [0] the same, [1] some share will not come
-  __shared__ int block_sums[17];   // slice: what its units have added up of the totals, [16] how many of them have
+  __shared__ int lp_missing[1];   // LP workgroup: some counts did not come
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
@@ -872,7 +914,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 
   if (pid < a.n_lp_workgroups) {
     // ------------------------------------------------------------ the LPs
-    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, missing, gen_and_poison, tid, lane, wave_s);
+    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, lp_missing, gen_and_poison, tid, lane, wave_s);
     LPLB_PLAN_STAMP(2);
     return;
   }
@@ -881,8 +923,8 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   const int slice = pid - a.n_lp_workgroups;
   const SliceTables t = carve_tables<K>(smem_raw, nl, R);
   unsigned char *my_records = t.records + (size_t)wave_s * ((R + 1) * rank_record_bytes_single(K));
-  const int64_t begin = slice_begin(a.n, a.per, slice);
-  const int64_t end = slice_begin(a.n, a.per, slice + 1);
+  int *const missing = t.missing;
+  const uint32_t end = (uint32_t)min(a.n, a.per * (slice + 1)), w0 = (uint32_t)a.per * (uint32_t)slice + wave_s * (K * kWave);   // this wave's first index (uniform)
   LPLB_PLAN_STAMP(0);
   LPLB_SLICE_STAMP(0);
   // Where a slice shares a CU with an LP workgroup (grids with more workgroups than CUs), its
@@ -892,20 +934,13 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   __builtin_amdgcn_s_setprio(2);
 
   // ---- small table reads, the index loads right behind them, the tables while they are on their way ----
-  const PlanTableLoads tl = issue_plan_table_loads(a, tid);
-  const int64_t w0 = begin + (int64_t)wave_s * (K * kWave);   // first index of this wave's chunks (uniform)
+  const PlanTableLoads tl = issue_plan_table_loads(a, tid, wave_s, slice == 0 && a.physical_counts);
   int64_t raw[K];
   load_chunks<K>(raw, a.idx, w0, end, lane);
-  if (tid == 0) {
-    missing[0] = 0;
-    missing[1] = 0;
-  }
-  if (tid < 17)
-    block_sums[tid] = 0;
-  clear_plan_tables<K>(a, t, tid);
+  clear_plan_tables<K>(t, tid);
   __syncthreads();
   LPLB_PLAN_STAMP(10);
-  enter_plan_tables(a, t, tl, tid);
+  enter_plan_tables(a, t, tl, tid, wave_s);
   // ---- the tokens ----
   uint32_t packed[(K + 1) / 2];
   mask_chunks<K>(raw, w0, end, lane);
@@ -931,7 +966,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
       }
     } else {
       for (int q2 = tid - kHalf; q2 < set_lanes; q2 += kHalf) {
-        const int first = t.hist[2 * q2 < R ? expert_of_set(a, t, 2 * q2) : nl], second = t.hist[2 * q2 + 1 < R ? expert_of_set(a, t, 2 * q2 + 1) : nl];
+        const int first = t.hist[2 * q2 < R ? expert_of_set(a, t, 2 * q2 + 1) : nl], second = t.hist[2 * q2 + 1 < R ? expert_of_set(a, t, 2 * q2 + 2) : nl];
         agent_store(set_rows + slice * a.set_words + q2, tagged_word(tag, (uint32_t)first | (uint32_t)second << 16));
       }
     }
@@ -944,11 +979,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   //      those that add them up and the LP waits for them; the tokens of each replicated set before this slice and in the whole batch.
   //      In between, while words are on their way, the tokens of each set in this slice's earlier chunks ----
   if (!poisoned)
-    add_up_published<false, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+    add_up_published<false, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, t.block_sums);
   SliceTokens<K>::mark(a, t, my_records, packed, lane);
   SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
   if (!poisoned)
-    add_up_published<false, Units::kSets>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+    add_up_published<false, Units::kSets>(a, t, slice, tag, lane, wave_s, missing, t.block_sums);
   LPLB_PLAN_STAMP(11);
   if (poisoned)
     missing[0] = 1;
@@ -963,7 +998,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   __builtin_amdgcn_s_setprio(0);
   int32_t h[K];   // hashes of this thread's tokens: worked out while the LP is still running
   if (ok) {
-    for (int q = tid; q < R; q += kPlanThreads)
+    for (int q = tid + 1; q <= R; q += kPlanThreads)
       set_total(t.reps[q], t.total[q]);
     SliceTokens<K>::bases(a, t, lane, wave_s);
     if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word)
@@ -985,7 +1020,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     // lanes on again: copied in no lane, lost in all.  97 registers this way at 8 ranks.  tests/test_host.py looks for such copies in the built library.
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      h[c] = SliceTokens<K>::hash(t, my_records, t.base + wave_s * R, R, packed_expert(packed, c), c);
+      h[c] = SliceTokens<K>::hash(t, my_records, t.base + wave_s * (R + 1), packed_expert(packed, c), c);
       if (K > 8 && c % 8 == 7) {
 #pragma unroll
         for (int j = c - 7; j <= c; ++j)
@@ -995,7 +1030,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     }
     LPLB_PLAN_STAMP(4);
     // ---- the LP's shares: every set's thread polls its own; value and tag arrive in the same word ----
-    collect_shares(a, t, slice, gen, avail_state, missing, tid);
+    collect_shares(a, t, slice, gen, avail_state, tid);
     __syncthreads();
     LPLB_PLAN_STAMP(5);
     ok = missing[1] == 0;
@@ -1007,11 +1042,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 #pragma unroll
   for (int c = 0; c < K; ++c) {
     const int e = packed_expert(packed, c);
-    const Route rt = t.route[e];
-    o[c] = rt.original;
+    const PlanRoute rt = t.route[e];
+    o[c] = rt.original();
     if (ok) {
-      const RepEntry x = t.reps[rt.rep];
-      o[c] = h[c] >= x.expected ? x.replica : rt.original;
+      const RepEntry x = t.reps[rt.set];
+      o[c] = h[c] >= x.expected ? x.replica : rt.original();
     }
     if (K > 8 && c % 8 == 7)
       __builtin_amdgcn_sched_barrier(0);
@@ -1039,8 +1074,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   constexpr int K = kLongChunks;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
-  __shared__ int missing[2];
-  __shared__ int block_sums[17];
+  __shared__ int lp_missing[1];
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
@@ -1048,11 +1082,12 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   fetch_arguments_now(a.idx, a.unit_blocks, a.sh.G, a.solve.workload, a.solve.n_group, a.solve.tagged_result, a.sync);
   unsigned long long gen_and_poison = agent_load(reinterpret_cast<const unsigned long long *>(a.sync));
   if (pid < a.n_lp_workgroups) {
-    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, missing, gen_and_poison, tid, lane, wave_s);
+    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, lp_missing, gen_and_poison, tid, lane, wave_s);
     return;
   }
   const int slice = pid - a.n_lp_workgroups;
   const SliceTables t = carve_tables<0>(smem_raw, nl, R);
+  int *const missing = t.missing;
   const int hist_len = 2 * a.hist_words, padded_sets = long_slice_padded_sets(R);
   // [waves][padded_sets][kLongBitsBytes], [waves][padded_sets][kLongRanksBytes], [waves][padded_sets], [waves][hist_len], [n_logical + 1]
   unsigned char *my_bits = t.records + wave_s * padded_sets * kLongBitsBytes;
@@ -1071,7 +1106,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   LPLB_SLICE_STAMP(0);
   __builtin_amdgcn_s_setprio(2);
 
-  const PlanTableLoads tl = issue_plan_table_loads(a, tid);
+  const PlanTableLoads tl = issue_plan_table_loads(a, tid, wave_s, slice == 0 && a.physical_counts);
   // (places past the last repeat it: without a branch the loads of the next pass stay on their way while one is counted)
   const int64_t *mine = a.idx + w0;
   auto load_pass = [&](int64_t (&v)[K], int p) {
@@ -1081,24 +1116,18 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   };
   int64_t raw[2][K];
   load_pass(raw[0], 0);
-  if (tid == 0) {
-    missing[0] = 0;
-    missing[1] = 0;
-  }
-  if (tid < 17)
-    block_sums[tid] = 0;
   for (int q = lane; q < padded_sets; q += kWave)
     my_so_far[q] = 0;
   for (int e = lane; e < hist_len; e += kWave)
     my_hist[e] = 0;
   for (int i = lane; i < padded_sets * kLongBitsBytes / 8; i += kWave)
     reinterpret_cast<unsigned long long *>(my_bits)[i] = 0ull;
-  clear_plan_tables<0>(a, t, tid);
+  clear_plan_tables<0>(t, tid);
   __syncthreads();
-  enter_plan_tables(a, t, tl, tid);
+  enter_plan_tables(a, t, tl, tid, wave_s);
   __syncthreads();
   for (int e = tid; e <= nl; e += kPlanThreads)   // (read behind the next barrier)
-    set_of_expert[e] = (unsigned char)t.route[e].rep;
+    set_of_expert[e] = (unsigned char)(t.route[e].set ? t.route[e].set - 1 : R);   // (from 0 on here; of no set: R)
   LPLB_PLAN_STAMP(10);
 
   // ---- the tokens: every wave counts its own ----
@@ -1145,11 +1174,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     } else {
       // lane = (word, set of its two, wave): what is in the waves before, and the word from the lane that has the last wave's
       for (int i = tid - kHalf; i < 16 * a.set_words; i += kHalf) {
-        const int w = i % kPlanWaves, q = i / kPlanWaves, x = q < R ? expert_of_set(a, t, q) : nl;
+        const int w = i % kPlanWaves, q = i / kPlanWaves, x = q < R ? expert_of_set(a, t, q + 1) : nl;
         const int own = x < nl ? wave_hists[w * hist_len + x] : 0;
         const int before = group_exclusive_scan<kPlanWaves>(own, w);
         if (q < R)
-          t.wave_total[w * R + q] = before;   // (in a long slice: in the waves before)
+          t.wave_total[w * (R + 1) + q + 1] = before;   // (in a long slice: in the waves before)
         const int first = row_shr<8>(before + own);
         if (i % 16 == 15)
           agent_store(set_rows + slice * a.set_words + i / 16, tagged_word(tag, (uint32_t)first | (uint32_t)(before + own) << 16));
@@ -1161,7 +1190,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   LPLB_PLAN_STAMP(1);
   LPLB_SLICE_STAMP(2);
   if (!poisoned)
-    add_up_published<true, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+    add_up_published<true, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, t.block_sums);
   // ---- while the others' words are on their way: ordinals among the wave's tokens, pass by pass (the wave's own records: no barrier) ----
   __builtin_amdgcn_s_setprio(2);
   const uint32_t my_bit = 1u << lane % 32;
@@ -1222,7 +1251,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     if (p < passes)
       rank_pass(p);
   if (!poisoned)
-    add_up_published<true, Units::kSets>(a, t, slice, tag, lane, wave_s, missing, block_sums);
+    add_up_published<true, Units::kSets>(a, t, slice, tag, lane, wave_s, missing, t.block_sums);
   LPLB_PLAN_STAMP(11);
   if (poisoned)
     missing[0] = 1;
@@ -1232,11 +1261,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   bool ok = missing[0] == 0;   // (the same in every thread)
   if (!ok && !poisoned && tid == 0)
     give_up(a, avail_state);
-  int32_t *my_bases = t.wave_total + wave_s * R;
+  int32_t *my_bases = t.wave_total + wave_s * (R + 1);
   if (ok) {
-    for (int q = tid; q < R; q += kPlanThreads)
+    for (int q = tid + 1; q <= R; q += kPlanThreads)
       set_total(t.reps[q], t.total[q]);
-    for (int q = lane; q < R; q += kWave)
+    for (int q = lane + 1; q <= R; q += kWave)
       my_bases[q] += t.before[q];
     if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word)
       say_that_all_arrived(a, tag, lane);
@@ -1252,7 +1281,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     }
     LPLB_PLAN_STAMP(3);
     LPLB_PLAN_STAMP(4);
-    collect_shares(a, t, slice, gen, avail_state, missing, tid);
+    collect_shares(a, t, slice, gen, avail_state, tid);
     __syncthreads();
     LPLB_PLAN_STAMP(5);
     ok = missing[1] == 0;
@@ -1268,12 +1297,12 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       const uint32_t e = token[p * K + c] & 0xffffu, k = token[p * K + c] >> 16;
-      const Route rt = t.route[e];
-      o[c] = rt.original;
+      const PlanRoute rt = t.route[e];
+      o[c] = rt.original();
       if (ok) {
-        const RepEntry x = t.reps[rt.rep];   // (without a replica: stays whatever the hash)
-        const int32_t h = ordinal_hash<true>(my_bases[min(rt.rep, R - 1)] + (int32_t)k, x.total, x.magic);
-        o[c] = h >= x.expected ? x.replica : rt.original;
+        const RepEntry x = t.reps[rt.set];   // (without a replica: stays whatever the hash)
+        const int32_t h = ordinal_hash<true>(my_bases[rt.set] + (int32_t)k, x.total, x.magic);
+        o[c] = h >= x.expected ? x.replica : rt.original();
       }
     }
     if ((p + 1) * K * kWave - 1 <= last) {
@@ -1320,6 +1349,7 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
+  fetch_arguments_now(a.idx, a.unit_blocks, a.sh.G, a.solve.workload, a.solve.n_group, a.solve.tagged_result, a.sync);
   // LDS: the LP waves' areas, the slice's tables
   constexpr size_t kLpArea = plan_lp_area_bytes<GM, DM>();
   const int n_lps = a.solve.n_units;
@@ -1327,28 +1357,28 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
   const int turn = (wave_s - n_lps) & (kPlanWaves - 1);   // this wave's place in the order of the indices
   auto records_of = [&](int place) { return t.records + (size_t)place * ((R + 1) * rank_record_bytes_single(K)); };
   unsigned char *my_records = records_of(turn);
-  const PlanTableLoads tl = issue_plan_table_loads(a, tid);
-  const int64_t w0 = (int64_t)turn * (K * kWave);
-  const bool has_tokens = w0 < a.n;
-  const int waves_with_tokens = (int)((a.n + K * kWave - 1) / (K * kWave));
+  const uint32_t n = (uint32_t)a.n, w0 = turn * (K * kWave);
+  const bool has_tokens = w0 < n;
+  const int waves_with_tokens = (int)((n + K * kWave - 1) / (K * kWave));
   int64_t raw[K];
-  load_chunks<K>(raw, a.idx, w0, a.n, lane);
+  load_chunks<K>(raw, a.idx, w0, n, lane);
+  const PlanTableLoads tl = issue_plan_table_loads(a, tid, wave_s, a.physical_counts);
   LPLB_PLAN_STAMP(0);
   uint32_t packed[(K + 1) / 2];
   // (called by the LP waves once their own table loads are on their way)
   auto count_the_tokens = [&]() -> bool {
-    clear_plan_tables<K>(a, t, tid);
+    clear_plan_tables<K>(t, tid);
     if (tid == 0)
       marked = 0;
     __syncthreads();
-    enter_plan_tables(a, t, tl, tid);
-    mask_chunks<K>(raw, w0, a.n, lane);
+    enter_plan_tables(a, t, tl, tid, wave_s);
+    mask_chunks<K>(raw, w0, n, lane);
     SliceTokens<K>::count(a, t, raw, packed);
     __syncthreads();
     if (has_tokens) {
       SliceTokens<K>::mark(a, t, my_records, packed, lane);
-      for (int q = lane; q < R; q += kWave) {   // (every wave enters the same values)
-        const SetOfPlan s = set_of_plan(a, R - 1 - q);
+      for (int q = lane + 1; q <= R; q += kWave) {   // (every wave enters the same values)
+        const SetOfPlan s = set_of_plan(a, q - 1);
         set_total(t.reps[q], t.hist[expert_of_set(a, t, q)]);
         t.reps[q].expected = s.ep_rank * a.sh.D + s.d;   // until the shares are there: where its share will be
       }
@@ -1381,9 +1411,9 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
     }
     const float wmax = wave_max_of_groups<true, true>((float)most);
     for (int e = tid - first; e < nl; e += kPlanThreads - first) {
-      const int32_t n = t.hist[e];
-      a.totals[e] = n;
-      a.solve.gw_out[e] = (float)n / wmax;
+      const int32_t count = t.hist[e];
+      a.totals[e] = count;
+      a.solve.gw_out[e] = (float)count / wmax;
     }
   }
   int32_t h[K];
@@ -1392,13 +1422,13 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
     SliceTokens<K>::starts_of_batch(a, my_records, lane, turn, records_of);
 #pragma unroll
     for (int c = 0; c < K; ++c)
-      h[c] = SliceTokens<K>::hash(t, my_records, nullptr, R, packed_expert(packed, c), c);
+      h[c] = SliceTokens<K>::hash(t, my_records, nullptr, packed_expert(packed, c), c);
   }
   if (wave_s < n_lps) {
     wait_for_waves(&marked, waves_with_tokens);   // (and its own shares have been stored)
     const int per_group = a.sh.G * a.sh.C * a.sh.D;
     for (int i = lane; i < per_group; i += kWave) {
-      RepEntry &x = t.reps[R - 1 - (wave_s * per_group + i)];
+      RepEntry &x = t.reps[wave_s * per_group + i + 1];
       x.expected = expected_on_original(share_of[x.expected], x.total);
     }
   }
@@ -1408,11 +1438,11 @@ __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArg
     int32_t o[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      const Route rt = t.route[packed_expert(packed, c)];
-      const RepEntry x = t.reps[rt.rep];
-      o[c] = h[c] >= x.expected ? x.replica : rt.original;
+      const PlanRoute rt = t.route[packed_expert(packed, c)];
+      const RepEntry x = t.reps[rt.set];
+      o[c] = h[c] >= x.expected ? x.replica : rt.original();
     }
-    store_chunks<K>(o, a.out, w0, a.n, lane);
+    store_chunks<K>(o, a.out, w0, n, lane);
   }
   if (a.physical_counts)
     plan_physical_counts(a, t, tl.physical_le0, true, tid);
