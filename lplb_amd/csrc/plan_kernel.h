@@ -965,9 +965,12 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
         agent_store(hist_rows + slice * a.hist_words + e2, tagged_word(tag, (uint32_t)both.x | (uint32_t)both.y << 16));
       }
     } else {
-      for (int q2 = tid - kHalf; q2 < set_lanes; q2 += kHalf) {
-        const int first = t.hist[2 * q2 < R ? expert_of_set(a, t, 2 * q2 + 1) : nl], second = t.hist[2 * q2 + 1 < R ? expert_of_set(a, t, 2 * q2 + 2) : nl];
-        agent_store(set_rows + slice * a.set_words + q2, tagged_word(tag, (uint32_t)first | (uint32_t)second << 16));
+      for (int i = tid - kHalf; i < 2 * set_lanes; i += kHalf) {   // lane = set, the word from the second of its two
+        const int e = t.set_expert[min(i, R - 1) + 1];
+        const int tokens = i < R && t.route[e].set == i + 1 ? t.hist[e] : 0;
+        const uint32_t both = (uint32_t)dpp_int<kQuadSwap1>(tokens) | (uint32_t)tokens << 16;
+        if (i & 1)
+          agent_store(set_rows + slice * a.set_words + i / 2, tagged_word(tag, both));
       }
     }
   } else if (slice == 0 && tid == 0) {
