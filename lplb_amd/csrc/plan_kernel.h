@@ -981,8 +981,13 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   // ---- what others have published, unit by unit: the batch's totals of this slice's share of the experts, if it is one of
   //      those that add them up and the LP waits for them; the tokens of each replicated set before this slice and in the whole batch.
   //      In between, while words are on their way, the tokens of each set in this slice's earlier chunks ----
-  if (!poisoned)
+  // (the waves that add up totals go first on their SIMDs meanwhile: run [32768 x 8] 10.0 -> 9.9 us, [100000 x 8] 11.8 -> 11.6)
+  if (!poisoned) {
+    if (slice < a.adders && wave_s >= kPlanWaves / 2)
+      __builtin_amdgcn_s_setprio(3);
     add_up_published<false, Units::kTotals>(a, t, slice, tag, lane, wave_s, missing, t.block_sums);
+    __builtin_amdgcn_s_setprio(2);
+  }
   SliceTokens<K>::mark(a, t, my_records, packed, lane);
   SliceTokens<K>::starts_in_wave(a, t, my_records, lane, wave_s);
   if (!poisoned)
@@ -1571,7 +1576,8 @@ template <int GM, int DM, bool EXACT> static int launch_plan_shape(PlanArgs &a, 
            : a.n <= 4 * per_chunk ? launch_plan_single<GM, DM, EXACT, 4>(a, s, done)
                                   : launch_plan_single<GM, DM, EXACT, 8>(a, s, done);
   }
-  return a.per <= 2 * kPlanThreads   ? launch_plan_slices<GM, DM, EXACT, 2>(a, s, done)
+  return a.per <= kPlanThreads       ? launch_plan_slices<GM, DM, EXACT, 1>(a, s, done)
+         : a.per <= 2 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 2>(a, s, done)
          : a.per <= 4 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 4>(a, s, done)
          : a.per <= 8 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 8>(a, s, done)
          : a.per <= kLongestSlice    ? launch_plan_slices<GM, DM, EXACT, 16>(a, s, done)
