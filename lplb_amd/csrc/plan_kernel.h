@@ -27,9 +27,10 @@
 // the counts do not wait for (ordinals inside a slice, the LP's topology) is done while they are on their way.
 // Per call, own histogram, before / after the counts went out ahead of the ordinals, units of 16-byte loads instead of sums by
 // the whole workgroup, and one batch of arguments: [8192 x 8] 10.9 -> 10.2 us, [262144 x 8] 19.3 -> 17.7, counts supplied
-// [8192 x 8] 8.1 -> 7.7.  What bounds it at [8192 x 8]: 2.7 us until the last slice's counts are out (0.9 of them until the last
-// workgroup has started), 2.0 until the LP has the totals, 4.1 of LP, 0.9 until its shares are seen, 0.6 until the last index
-// is stored.
+// [8192 x 8] 8.1 -> 7.7; ahead of everything that looks at the mapping as well (clear_plan_tables): 9.3, 15.2 and 6.8.  What bounds
+// it at [8192 x 8], from the first workgroup's start: 1.4 us until a slice's counts are out, 2.2 until the LP has the totals (0.4 the
+// adding wave's addresses, 0.5 its loads, 0.5 its sums and stores, 0.8 until the LP has seen them), 3.7 of LP, 0.3-0.5 until its
+// shares are seen, 0.5 until the last index is stored.
 // Words are written and read with agent-scope atomics (plan_sync.h).
 // The workgroups wait for each other, so the whole grid has to be resident: its size is bounded by what fits
 // the GPU, and the host admits a launch only while the plans still executing leave room for it.
