@@ -783,8 +783,10 @@ __device__ __forceinline__ void collect_shares(const PlanArgs &a, const SliceTab
     unsigned long long word = 0;
     int polls = 0;
     uint32_t got = 0;
-    while ((got = (uint32_t)((word = agent_load(word_at)) >> 32)) != tag_valid && got != tag_none && ++polls < a.max_polls)
-      __builtin_amdgcn_s_sleep(1);
+    // (no sleep between polls, each of which takes a trip to memory: a share is seen up to 64 clocks sooner, run [1024 x 8] 9.25 -> 9.1 us,
+    // [262144 x 8] 15.35 -> 15.25)
+    while ((got = (uint32_t)((word = agent_load(word_at)) >> 32)) != tag_valid && got != tag_none && ++polls < a.max_polls) {
+    }
     if (got == tag_valid) {
       t.reps[i + 1].expected = expected_on_original(__builtin_bit_cast(float, (uint32_t)word), t.total[i + 1]);
     } else {
