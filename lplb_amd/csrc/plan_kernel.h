@@ -48,7 +48,7 @@
 namespace lplb {
 
 constexpr int kPlanWaves = 8, kPlanThreads = kPlanWaves * kWave;
-constexpr int kPlanLdsLimit = 160 * 1024 - 8 * 1024;   // dynamic LDS; the kernels have static LDS besides
+constexpr int kPlanLdsLimit = 160 * 1024 - 7680;   // dynamic LDS; the kernels have up to 4.1 KiB of static LDS besides
 constexpr int kDefaultMaxPolls = 1 << 22;   // a few seconds of polling before a wait gives up
 // LPs per LP workgroup: waves 0..3 of a workgroup sit on the CU's four SIMDs, and an LP
 // wave is bound by instruction issue, so a fifth LP on the same CU would slow two of them
