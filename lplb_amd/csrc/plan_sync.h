@@ -47,9 +47,10 @@ __device__ inline void agent_store(int *p, int v) {
 __device__ inline void agent_store(unsigned long long *p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Two words, 16-byte aligned, past the caches with one store (each of the two lands in one piece).
+// Two words, 16-byte aligned, past the caches with one store (each of the two lands in one piece).  The data registers of a store of
+// more than 8 bytes may not be written by either of the next two instructions; the compiler sees to that behind its own stores only.
 __device__ inline void agent_store_pair(unsigned long long *p, u32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 __device__ inline int agent_add(int *p, int v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
