@@ -61,7 +61,7 @@ template <int GM, int DM> constexpr size_t plan_lp_area_bytes() {
   return lp_pivot_doubles<GM, DM>() * sizeof(double) + lp_tile_floats<GM, DM>() * sizeof(float);
 }
 
-// The counts an LP works on, in LDS, with the zeros behind them.
+// The counts an LP works on, in LDS, with the zeros behind them and at least one word more, the last.
 constexpr size_t counts_bytes(int n_logical) { return (size_t)(n_logical / 4 * 4 + 8) * sizeof(int32_t); }
 
 // One block of these per stream that plans (kSyncSlots of them per device), offsets in ints:
@@ -191,7 +191,7 @@ constexpr int kBlockSums = 17, kSliceFlags = 2 + kBlockSums;
 template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
   return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)kPlanWaves * (n_rep + 1) * slice_record_bytes(K) +
          (size_t)(n_logical + 2) * sizeof(PlanRoute) + (size_t)(n_logical + 16 + kSliceFlags) * sizeof(int32_t) +
-         (size_t)(3 + 2 * kPlanWaves) * (n_rep + 1) * sizeof(int32_t);
+         (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t);
 }
 // A long slice's records per (wave, replicated set): the bitmaps of a pass's chunks, and what a token's ordinal is made of (a
 // bitmap and the tokens before it), both padded for the LDS banks; sixteen sets are worked on at once.
@@ -199,7 +199,7 @@ constexpr int kLongBitsBytes = kLongChunks * 8 + 8, kLongRanksBytes = kLongChunk
 __host__ __device__ constexpr int long_slice_padded_sets(int n_rep) { return n_rep / 16 * 16 + 16; }   // at least one more: of tokens without a set
 __host__ __device__ constexpr size_t long_slice_records_at(int n_logical, int n_rep) {
   return ((size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)(n_logical + 2) * sizeof(PlanRoute) + (size_t)(n_logical + 16 + kSliceFlags) * sizeof(int32_t) +
-          (size_t)(3 + kPlanWaves) * (n_rep + 1) * sizeof(int32_t) + 15) / 16 * 16;
+          (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t) + 15) / 16 * 16;
 }
 inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
   return long_slice_records_at(n_logical, n_rep) +
@@ -213,10 +213,10 @@ struct SliceTables {
   int32_t *hist;            // [more than n_logical, a multiple of 16] the slice's histogram, then zeros; in the first slice at last the batch's
   int32_t *missing;         // [2] [0] some counts did not come, [1] some share will not come
   int32_t *block_sums;      // [kBlockSums] what the workgroup's units have added up of the totals, the last: how many of them have
-  int32_t *before, *total;  // [R + 1] tokens of the set before this slice, in the whole batch
-  int32_t *set_expert;      // [R + 1] the expert whose tokens the set has; n_logical (which has none): it has none
-  int32_t *wave_total;      // [waves][R + 1] ... in each wave
-  int32_t *base;            // [waves][R + 1] ... before each wave (not for long slices)
+  // By set, the first at [1]; [0], of no set, is an entry of what lies before:
+  int32_t *before, *total;  // tokens of the set before this slice, in the whole batch
+  int32_t *set_expert;      // the expert whose tokens the set has; n_logical (which has none): it has none
+  int32_t *of_wave;         // [waves][R] ... in each wave; later, with those before this slice, before each wave
 };
 template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, int nl, int R) {
   SliceTables t;
@@ -226,11 +226,10 @@ template <int K> __device__ inline SliceTables carve_tables(unsigned char *lds, 
   t.hist = reinterpret_cast<int32_t *>(t.records + (size_t)kPlanWaves * (R + 1) * slice_record_bytes(K));
   t.missing = t.hist + nl / 16 * 16 + 16;
   t.block_sums = t.missing + 2;
-  t.before = t.missing + kSliceFlags;
-  t.total = t.before + R + 1;
-  t.set_expert = t.total + R + 1;
-  t.wave_total = t.set_expert + R + 1;
-  t.base = t.wave_total + kPlanWaves * (R + 1);
+  t.before = t.missing + kSliceFlags - 1;
+  t.total = t.before + R;
+  t.set_expert = t.total + R;
+  t.of_wave = t.set_expert + R;
   if (K == 0)
     t.records = lds + long_slice_records_at(nl, R);
   return t;
@@ -298,7 +297,7 @@ template <int K> __device__ inline void clear_plan_tables(const SliceTables &t, 
     for (int i = tid; i < n16; i += kPlanThreads)
       reinterpret_cast<i32x4 *>(from)[i] = zero;
   };
-  clear(t.route, t.set_expert);   // (in a long slice the records, which lie elsewhere, are the waves' own)
+  clear(t.route, t.set_expert + 1);   // (in a long slice the records, which lie elsewhere, are the waves' own)
 }
 // Where an expert's tokens go when nothing is redirected and which replicated set (if any) it belongs to
 // (minilp.cu:466-496).  A workgroup barrier has to follow.
@@ -431,7 +430,7 @@ template <int K> struct SliceTokens {
     }
     own_slots_are_written();
   }
-  // The tokens of each set in the wave's earlier chunks into the slots, those in the whole wave into t.wave_total.  lane = set:
+  // The tokens of each set in the wave's earlier chunks into the slots, those in the whole wave into t.of_wave.  lane = set:
   // the chunks' pop-counts add up as they are read.  (lane = (set, chunk) with a scan over the lanes of a set takes as many instructions
   // at 16 sets and eight times as many at 128.  Counts supplied, [100000 x 8]: 64 sets 15.2 -> 12.8 us, 32 sets 12.1 -> 11.3; [16384 x 8]
   // with 128 sets 11.0 -> 10.2; [262144 x 8] with 16 sets 18.0 -> 17.9.)
@@ -448,20 +447,27 @@ template <int K> struct SliceTokens {
         slot(my_records, q, c)->start = before;
         before += __popcll(bits[c]);
       }
-      t.wave_total[wave_s * (R + 1) + q] = before;
+      t.of_wave[wave_s * R + q] = before;
     }
   }
-  // The tokens of each set before this wave's first into t.base.  The wave's own entries only: no barrier.
-  __device__ static void bases(const PlanArgs &a, const SliceTables &t, int lane, int wave_s) {
+  // What t.of_wave has becomes the tokens of each set before each wave's first, by the second half of the waves, a lane a set.  A
+  // workgroup barrier on either side.  (A table of its own for these takes 32 bytes a set: two slices of 16 chunks with 32 sets and 512
+  // experts did not fit a CU any more, and [262144 x 8] at 16 ranks ran as the chain.)
+  __device__ static void bases(const PlanArgs &a, const SliceTables &t, int tid) {
     const int R = a.n_rep;
-    for (int q = lane + 1; q <= R; q += kWave) {
-      int32_t base = t.before[q];
+    for (int q = tid - kPlanHalf + 1; q <= R; q += kPlanHalf) {
+      int32_t in_wave[kPlanWaves - 1];
 #pragma unroll
       for (int w = 0; w < kPlanWaves - 1; ++w)
-        base += w < wave_s ? t.wave_total[w * (R + 1) + q] : 0;
-      t.base[wave_s * (R + 1) + q] = base;
+        in_wave[w] = t.of_wave[w * R + q];
+      int32_t base = t.before[q];
+#pragma unroll
+      for (int w = 0; w < kPlanWaves; ++w) {
+        t.of_wave[w * R + q] = base;
+        if (w < kPlanWaves - 1)
+          base += in_wave[w];
+      }
     }
-    own_slots_are_written();
   }
   // The same where the workgroup holds the whole batch: from the bitmaps of the `turn` waves before this one, records_of(w)
   // their records.
@@ -823,8 +829,8 @@ __device__ inline void write_normalised_counts(const PlanArgs &a, const int32_t 
 // An LP workgroup of a plan: one wave per LP, the others help to collect the counts and write the normalised ones (by the LP waves
 // themselves, at their end, those took 0.8 us, and what is counted for the caller behind them came as much later).
 template <int GM, int DM, bool EXACT>
-__device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *smem_raw, int *rep_of_edge_all, int *missing,
-                                             unsigned long long gen_and_poison, int tid, int lane, int wave_s) {
+__device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *smem_raw, int *rep_of_edge_all, unsigned long long gen_and_poison,
+                                             int tid, int lane, int wave_s) {
   const int nl = a.sh.n_logical, pid = blockIdx.x;
   unsigned long long *shares = reinterpret_cast<unsigned long long *>(a.sync + kSharesAt);
   SolveArgs sa = a.solve;
@@ -838,6 +844,7 @@ __device__ __forceinline__ void lp_workgroup(const PlanArgs &a, unsigned char *s
   static_assert(kLpArea % 16 == 0, "the LP waves' areas keep 16-byte alignment");
   unsigned char *my_area = smem_raw + (size_t)min(wave_s, kLpsPerWorkgroup - 1) * kLpArea;
   float *staged = reinterpret_cast<float *>(smem_raw + kLpsPerWorkgroup * kLpArea);
+  int *const missing = reinterpret_cast<int *>(staged) + sa.staged_stride - 1;   // some counts did not come (own-histogram mode)
   sa.launch = (uint32_t)gen_and_poison;
   sa.gw_out = nullptr;   // (written by the waves without an LP)
   auto switched_off = [&]() { return (gen_and_poison >> 32) != 0; };
@@ -902,7 +909,6 @@ template <int GM, int DM, bool EXACT, int K>
 __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void plan_in_one_launch(PlanArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
-  __shared__ int lp_missing[1];   // LP workgroup: some counts did not come
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
@@ -917,7 +923,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 
   if (pid < a.n_lp_workgroups) {
     // ------------------------------------------------------------ the LPs
-    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, lp_missing, gen_and_poison, tid, lane, wave_s);
+    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, gen_and_poison, tid, lane, wave_s);
     LPLB_PLAN_STAMP(2);
     return;
   }
@@ -1009,9 +1015,11 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   __builtin_amdgcn_s_setprio(0);
   int32_t h[K];   // hashes of this thread's tokens: worked out while the LP is still running
   if (ok) {
-    for (int q = tid + 1; q <= R; q += kPlanThreads)
-      set_total(t.reps[q], t.total[q]);
-    SliceTokens<K>::bases(a, t, lane, wave_s);
+    if (wave_s < kPlanWaves / 2)
+      for (int q = tid + 1; q <= R; q += kPlanHalf)
+        set_total(t.reps[q], t.total[q]);
+    else
+      SliceTokens<K>::bases(a, t, tid);
     if (slice == 0 && wave_s == kPlanWaves - 1 && a.arrived_word)
       say_that_all_arrived(a, tag, lane);
     if (slice == 0 && !collect_totals(a, t.hist, tag, tid, wave_s)) {   // for the caller (and for the counts below)
@@ -1031,7 +1039,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
     // lanes on again: copied in no lane, lost in all.  97 registers this way at 8 ranks.  tests/test_host.py looks for such copies in the built library.
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      h[c] = SliceTokens<K>::hash(t, my_records, t.base + wave_s * (R + 1), packed_expert(packed, c), c);
+      h[c] = SliceTokens<K>::hash(t, my_records, t.of_wave + wave_s * R, packed_expert(packed, c), c);
       if (K > 8 && c % 8 == 7) {
 #pragma unroll
         for (int j = c - 7; j <= c; ++j)
@@ -1085,7 +1093,6 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   constexpr int K = kLongChunks;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __shared__ int rep_of_edge_all[kLpsPerWorkgroup * kWave];
-  __shared__ int lp_missing[1];
   const int nl = a.sh.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);   // wave-uniform
@@ -1093,7 +1100,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   fetch_arguments_now(a.idx, a.unit_blocks, a.sh.G, a.solve.workload, a.solve.n_group, a.solve.tagged_result, a.sync);
   unsigned long long gen_and_poison = agent_load(reinterpret_cast<const unsigned long long *>(a.sync));
   if (pid < a.n_lp_workgroups) {
-    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, lp_missing, gen_and_poison, tid, lane, wave_s);
+    lp_workgroup<GM, DM, EXACT>(a, smem_raw, rep_of_edge_all, gen_and_poison, tid, lane, wave_s);
     return;
   }
   const int slice = pid - a.n_lp_workgroups;
@@ -1189,7 +1196,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
         const int own = x < nl ? wave_hists[w * hist_len + x] : 0;
         const int before = group_exclusive_scan<kPlanWaves>(own, w);
         if (q < R)
-          t.wave_total[w * (R + 1) + q + 1] = before;   // (in a long slice: in the waves before)
+          t.of_wave[w * R + q + 1] = before;   // (in a long slice: in the waves before)
         const int first = row_shr<8>(before + own);
         if (i % 16 == 15)
           agent_store(set_rows + slice * a.set_words + i / 16, tagged_word(tag, (uint32_t)first | (uint32_t)(before + own) << 16));
@@ -1272,7 +1279,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   bool ok = missing[0] == 0;   // (the same in every thread)
   if (!ok && !poisoned && tid == 0)
     give_up(a, avail_state);
-  int32_t *my_bases = t.wave_total + wave_s * (R + 1);
+  int32_t *my_bases = t.of_wave + wave_s * R;
   if (ok) {
     for (int q = tid + 1; q <= R; q += kPlanThreads)
       set_total(t.reps[q], t.total[q]);
