@@ -11,8 +11,12 @@
 namespace lplb {
 
 static __device__ __attribute__((aligned(4096))) int g_plan_sync[kSyncInts];
-// Slices of the one-launch plan, in indices.
-constexpr int64_t kShortestSlice = 512;   // (the longest: kLongestSlice)
+// Slices of the one-launch plan, in indices (the longest: kLongestSlice).  While a wave adds up the counts of all slices (64) and the GPU
+// has no other plan, as short as 512 (run [2048 x 8] 9.2 -> 9.0 us, [4096 x 8] 9.3 -> 9.15, counts supplied [1024 x 8] 6.9 -> 6.75, at 32 ranks
+// [2048 x 8] 17.2 -> 16.75; [8192 x 8] in 128 slices 9.4 as in 64).  They take twice the workgroups, which a captured plan would keep for good
+// and other streams' plans would be refused for, ten times what is gained: of 16 ranks and [4096 x 8] six captured plans instead of eight
+// ran as one launch, of 32 ranks, where a CU holds one workgroup, three instead of six.
+constexpr int64_t kShortestSlice = 1024, kShortestSliceAlone = 512;
 static std::atomic<bool> g_cooperative{true};   // any thread may flip it while others plan
 static std::atomic<long long> g_one_launch_plans{0};
 // Test hook (lplb_plan_inject_fault): the next launch with a wait in it (one-launch plan, or scan and LP of a long
@@ -114,6 +118,8 @@ static int workgroups_per_cu(const void *kernel, KernelFootprint &known, int wav
   return min(by_registers, by_lds);
 }
 
+static bool cut_for_a_plan_alone(const PlanArgs &a) { return a.per <= kShortestSliceAlone && a.n > kShortestSliceAlone; }
+
 // Launches one variant, if the whole grid fits the GPU beside the plans that are still executing (a kernel whose
 // workgroups do not wait for others always does).  *done = false: it does not; nothing was enqueued.
 int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_others, PlanArgs &a, size_t lds, hipStream_t s,
@@ -146,7 +152,7 @@ int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_ot
       for (int i = 0; i < kSyncSlots; ++i)
         d->arrived[i] = 0;
     }
-    admitted = d->admission.admit(s, cost, capturing, d->arrived);
+    admitted = d->admission.admit(s, cost, capturing, d->arrived, cut_for_a_plan_alone(a));
     if (admitted.slot < 0)
       return LPLB_OK;
     a.sync = d->sync + (size_t)admitted.slot * kSlotInts;
@@ -178,6 +184,32 @@ int launch_plan(PlanKernel kernel, KernelFootprint &footprint, bool waits_for_ot
 
 // LP shapes that are built here: (8, 1) (8, 2) (8, 4) (16, 1) (16, 2) (32, 1) (32, 2) and what pads into them
 static bool lp_shape_is_built(int G, int D) { return G <= 8 ? D <= 4 : G <= 32 && D <= 2; }
+
+// The shortest of 1024, 2048, 4096, 8192 indices per slice (or of 512 and those) with which at most `most` slices, which is no more than
+// kMaxSlices, than the caller allows and than the GPU holds at once, cover the batch.  false: they cannot.
+static bool cut_into_slices(PlanArgs &a, int64_t shortest, int most) {
+  int64_t len = shortest;
+  while (len < kLongestSlice && (a.n + len - 1) / len > (len < kShortestSlice ? min(most, kUnitSlices) : most))
+    len *= 2;
+  a.per = slice_len(a.n, (int)min((a.n + len - 1) / len, (int64_t)most));
+  // Past that as many long slices as there may be, unless these are few: a caller that allows few workgroups keeps the chain.
+  // (So many may turn out not to be resident at once: up to 16 ranks `most` is for two per CU, and the tables of 32 sets and more
+  // leave room for one.  launch_plan refuses those.)
+  if (a.per > kLongestSlice && (a.per > kLongestOfLongSlices || most < kFewestLongSlices))
+    return false;
+  const int n = a.n_slices = (int)((a.n + a.per - 1) / a.per);   // (rounding the length up may have emptied the last ones)
+  a.adder_words = 8;
+  while (a.adder_words * n < a.hist_words)
+    a.adder_words *= 2;
+  a.adders = (a.hist_words + a.adder_words - 1) / a.adder_words;
+  a.n_share_copies = 1;
+  while (a.n_share_copies < kShareCopies && a.n_share_copies * 8 < n)
+    a.n_share_copies *= 2;
+  a.unit_lanes_log2 = n > 32 ? 2 : n > 16 ? 3 : n > 8 ? 4 : n > 4 ? 5 : 6;
+  a.unit_blocks = (n + kUnitSlices - 1) / kUnitSlices;
+  a.unit_block_bits = a.unit_blocks > 2 ? 2 : a.unit_blocks - 1;
+  return true;
+}
 
 // Tries the one-launch plan.  *done = false: shape or size outside what it covers, or no
 // room on the GPU right now; nothing was enqueued.
@@ -224,35 +256,18 @@ static int try_one_launch(const int64_t *idx, int64_t n_elements, const int32_t 
     if (rc != LPLB_OK || *done)
       return rc;
   }
-  // The shortest of 1024, 2048, 4096, 8192 indices per slice with which at most kMaxSlices slices, no more than
-  // the caller allows and no more than the GPU holds at once, cover the batch; 512 while a wave adds up the counts of all slices (run
-  // [2048 x 8] 9.2 -> 9.0 us, [4096 x 8] 9.3 -> 9.15, counts supplied [1024 x 8] 6.9 -> 6.75; [8192 x 8] in 128 slices 9.4 as in 64).
   a.n_lp_workgroups = (n_group + kLpsPerWorkgroup - 1) / kLpsPerWorkgroup;
   const int resident = (int)(kResidencyBudget * plan_workgroups_per_cu(G) * current_device_cu_count());
   const int most = min(min(n_blocks, kMaxSlices), resident - a.n_lp_workgroups);
   if (most < 1)
     return LPLB_OK;
-  int64_t len = kShortestSlice;
-  while (len < kLongestSlice && (n_elements + len - 1) / len > (len == kShortestSlice ? min(most, kUnitSlices) : most))
-    len *= 2;
-  a.per = slice_len(n_elements, (int)min((n_elements + len - 1) / len, (int64_t)most));
-  // Past that as many long slices as there may be, unless these are few: a caller that allows few workgroups keeps the chain.
-  // (So many may turn out not to be resident at once: up to 16 ranks `most` is for two per CU, and the tables of 32 sets and more
-  // leave room for one.  launch_plan refuses those.)
-  if (a.per > kLongestSlice && (a.per > kLongestOfLongSlices || most < kFewestLongSlices))
+  if (cut_into_slices(a, kShortestSliceAlone, most) && cut_for_a_plan_alone(a)) {
+    const int rc = launch_variant(a, s, done);
+    if (rc != LPLB_OK || *done)
+      return rc;
+  }
+  if (!cut_into_slices(a, kShortestSlice, most))
     return LPLB_OK;
-  a.n_slices = (int)((n_elements + a.per - 1) / a.per);   // (rounding the length up may have emptied the last ones)
-  a.adder_words = 8;
-  while (a.adder_words * a.n_slices < a.hist_words)
-    a.adder_words *= 2;
-  a.adders = (a.hist_words + a.adder_words - 1) / a.adder_words;
-  a.n_share_copies = 1;
-  while (a.n_share_copies < kShareCopies && a.n_share_copies * 8 < a.n_slices)
-    a.n_share_copies *= 2;
-  const int n = a.n_slices;
-  a.unit_lanes_log2 = n > 32 ? 2 : n > 16 ? 3 : n > 8 ? 4 : n > 4 ? 5 : 6;
-  a.unit_blocks = (n + kUnitSlices - 1) / kUnitSlices;
-  a.unit_block_bits = a.unit_blocks > 2 ? 2 : a.unit_blocks - 1;
   return launch_variant(a, s, done);
 }
 

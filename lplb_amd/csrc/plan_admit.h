@@ -25,7 +25,8 @@ public:
 
   // One launch that takes `cost` of the GPU's resident workgroups, on `stream`.  arrived[i]: number of the last launch of
   // slot i that has said that all of its workgroups have arrived (may be null until a launch outside a capture is admitted).
-  Admitted admit(const void *stream, float cost, bool capturing, const int *arrived) {
+  // if_alone: only while no other stream's plan may be executing, and if no graph keeps the share for good.
+  Admitted admit(const void *stream, float cost, bool capturing, const int *arrived, bool if_alone = false) {
     Admitted got;
     int slot = -1;
     for (int i = 0; i < SLOTS && slot < 0; ++i)
@@ -45,6 +46,8 @@ public:
     if (executing + cost > kResidencyBudget)
       return got;
     Slot &s = slots_[slot];
+    if (if_alone && (executing > 0.0f || capturing || s.captured))
+      return got;
     if (!s.used || s.stream != stream) {
       s.stream = stream;
       s.cost = 0.0f;

@@ -522,8 +522,8 @@ using A = lplb::PlanAdmission<8>;
 static A a;
 static A::Admitted last;
 extern "C" void reset() { a = A(); }
-extern "C" void admit(long stream, float cost, int capturing, const int *arrived, int *out) {
-  last = a.admit(reinterpret_cast<const void *>(stream), cost, capturing, arrived);
+extern "C" void admit(long stream, float cost, int capturing, const int *arrived, int if_alone, int *out) {
+  last = a.admit(reinterpret_cast<const void *>(stream), cost, capturing, arrived, if_alone);
   const int got[] = {last.slot, last.seq, last.wait_slices, last.wait_lps, last.wait_seq};
   for (int i = 0; i < 5; ++i) out[i] = got[i];
 }
@@ -541,9 +541,9 @@ extern "C" void idle() { a.device_is_idle(); }
             self.arrived = (ctypes.c_int * 8)()
             lib.reset()
 
-        def plan(self, stream, cost=0.1, capturing=False, slices=64, lps=1):
+        def plan(self, stream, cost=0.1, capturing=False, slices=64, lps=1, if_alone=False):
             out = (ctypes.c_int * 5)()
-            lib.admit(ctypes.c_long(stream), ctypes.c_float(cost), int(capturing), self.arrived, out)
+            lib.admit(ctypes.c_long(stream), ctypes.c_float(cost), int(capturing), self.arrived, int(if_alone), out)
             if out[0] >= 0:
                 lib.launched(int(capturing), slices, lps)
             return out[0], out[1], tuple(out[2:]) if out[2] else None
@@ -607,6 +607,24 @@ def test_forgetting_captured_plans_does_not_forget_a_plan_that_still_executes(ad
     adm.has_arrived(running)
     got = adm.plan(9, cost=0.4)
     assert got[0] == 0 and got[2] == (200, 3, running[1])
+
+
+def test_a_plan_takes_more_of_the_gpu_only_while_it_is_alone(admission):
+    """Short slices take twice the workgroups: only while no other stream's plan may be executing, and not where a captured graph
+    keeps the share, its own or that of one captured on the stream before."""
+    adm = admission()
+    other = adm.plan(1)
+    assert adm.plan(2, if_alone=True)[0] == -1 and adm.plan(2)[0] == 1
+    adm.idle()
+    assert adm.plan(3, if_alone=True)[0] == 2 and adm.plan(3, if_alone=True)[0] == 2   # (its own last one is ahead of it on the stream)
+    assert adm.plan(4, if_alone=True)[0] == -1
+    adm.idle()
+    assert adm.plan(3, if_alone=True, capturing=True)[0] == -1 and other[0] == 0
+    assert adm.plan(3, capturing=True)[0] == 2
+    assert adm.plan(3, if_alone=True)[0] == -1 and adm.plan(3)[0] == 2
+    adm.forget(3)
+    adm.idle()
+    assert adm.plan(3, if_alone=True)[0] == 2
 
 
 def test_as_many_streams_as_there_are_blocks_keep_one_each(admission):
