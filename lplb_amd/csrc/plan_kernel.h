@@ -1355,8 +1355,10 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 // Up to as many indices as leave the LP waves, which come last in the order of the indices, without any at eight chunks a wave.
 // One LP, in one workgroup / as slices: 3584 indices 7.6 / 8.9 us, 4096 9.7 / 8.9; two LPs, 3072 7.8 / 9.1, 3584 10.3 / 9.2; four, 2048
 // 8.4 / 9.25, 2560 11.0 / 9.25; (16, 2) 3584 10.9 / 12.1, 4096 13.9 / 12.1; (32, 2) 3584 18.3 / 19.4, 4096 22.7 / 19.4.  With eight LPs
-// every wave has one: 128 indices (two chunks in one wave) 8.5 / 9.2, 192 9.45 / 9.25.
+// every wave has one: 128 indices (two chunks in one wave) 8.5 / 9.2, 192 9.45 / 9.25.  Where the slices are refused, up to eight
+// chunks in every wave.
 constexpr int kSingleMaxLps = kPlanWaves;
+constexpr int64_t kSingleMaxIndices = 8 * kPlanThreads;
 constexpr int64_t single_max_indices(int n_lps) { return (n_lps < kPlanWaves ? 8 * (kPlanWaves - n_lps) : 2) * kWave; }
 template <int GM, int DM, bool EXACT, int K>
 __global__ __launch_bounds__(kPlanThreads, 2) void plan_in_one_workgroup(PlanArgs a) {
