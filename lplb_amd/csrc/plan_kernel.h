@@ -755,8 +755,7 @@ __device__ __forceinline__ void add_up_published(const PlanArgs &a, const SliceT
         }
         if (all_in && lane < unit_lanes && 2 * lane < my_words - at) {   // (words behind the last expert's have zeros and are not read)
           unsigned long long *to = totals + 2 * word0 + 4 * lane;
-          agent_store_pair(to, u32x4{sums[0], tag, sums[1], tag});
-          agent_store_pair(to + 2, u32x4{sums[2], tag, sums[3], tag});
+          agent_store_pairs(to, u32x4{sums[0], tag, sums[1], tag}, u32x4{sums[2], tag, sums[3], tag});
         }
       } else {
         missing[0] = 1;

@@ -321,7 +321,7 @@ def test_cross_workgroup_helpers_compile_to_the_forms_the_plan_relies_on(tmp_pat
 using namespace lplb;
 extern "C" __global__ void store_word(unsigned long long *word, unsigned tag, unsigned v) { agent_store(word + threadIdx.x, tagged_word(tag, v)); }
 extern "C" __global__ void load_word(const unsigned long long *word, unsigned long long *out) { out[threadIdx.x] = agent_load(word + threadIdx.x); }
-extern "C" __global__ void store_pair(unsigned long long *words, u32x4 v) { agent_store_pair(words + 2 * threadIdx.x, v); }
+extern "C" __global__ void store_pairs(unsigned long long *words, u32x4 v, u32x4 w) { agent_store_pairs(words + 4 * threadIdx.x, v, w); }
 extern "C" __global__ void store_int(int *p, int v) { agent_store(p + threadIdx.x, v); }
 extern "C" __global__ void load_int(const int *p, int *out) { out[threadIdx.x] = agent_load(p + threadIdx.x); }
 extern "C" __global__ void add_int(int *p) { agent_add(p + threadIdx.x, 3); }
@@ -339,14 +339,14 @@ extern "C" __global__ void collect(const unsigned long long *words, unsigned tag
                     f"-I{ROOT / 'lplb_amd' / 'csrc'}", str(probe), "-o", str(asm)], check=True, capture_output=True)
     text = asm.read_text()
     body = {name: text.split(f"\n{name}:")[1].split("s_endpgm")[0]
-            for name in ("store_word", "load_word", "store_pair", "store_int", "load_int", "add_int", "replace_int", "collect")}
+            for name in ("store_word", "load_word", "store_pairs", "store_int", "load_int", "add_int", "replace_int", "collect")}
     memory = {name: re.findall(r"(?:global|flat|buffer)_\w+ .*", code) for name, code in body.items()}
     for name, form in (("store_word", r"global_store_dwordx2 .* sc1$"), ("store_int", r"global_store_dword .* sc1$")):
         assert len(memory[name]) == 1 and re.match(form, memory[name][0]), (name, memory[name])      # one store, past the caches
-    # two words by one store; its data registers may not be written in the next two cycles, which the compiler does not see to
-    # for an instruction that it did not choose itself
-    pair_then_wait = r"global_store_dwordx4 .* sc1\n\ts_nop [1-9]"
-    assert len(memory["store_pair"]) == 1 and re.search(pair_then_wait, body["store_pair"]), body["store_pair"]
+    # two words by one store; its data registers may not be written by the next two instructions, which the compiler does not see
+    # to behind a store that it did not choose itself
+    pairs_then_wait = r"(\tglobal_store_dwordx4 .* sc1\n){2}\ts_nop [1-9]"
+    assert len(memory["store_pairs"]) == 2 and re.search(pairs_then_wait, body["store_pairs"]), body["store_pairs"]
     for name, form in (("load_word", r"global_load_dwordx2 .* sc1$"), ("load_int", r"global_load_dword .* sc1$")):
         assert re.match(form, memory[name][0]), (name, memory[name])
         assert sum("_load_" in m for m in memory[name]) == 1
@@ -364,9 +364,9 @@ extern "C" __global__ void collect(const unsigned long long *words, unsigned tag
             kernels += 1
             assert not any(op.startswith(("buffer_inv", "buffer_wbl2")) for _, op, _ in code), name
             for (_, op, _), (_, behind, _) in zip(code, code[1:]):
-                if re.match(r"global_store_dwordx4 .* sc1$", op):
+                if re.match(pair := r"global_store_dwordx4 .* sc1$", op):
                     pairs += 1
-                    assert re.match(r"s_nop [1-9]", behind), (name, op, behind)
+                    assert re.match(rf"s_nop [1-9]|{pair}", behind), (name, op, behind)
     assert kernels >= 14 * 6 + 14 + 1 and pairs >= 14 * 6 * 2, (kernels, pairs)
 
 
