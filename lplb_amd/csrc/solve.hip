@@ -45,7 +45,9 @@ static void launch_variant(SolveArgs a, hipStream_t s) {
   constexpr bool kKnown = takes_spread_form<GM, DM, ROWS, EPL>() || ROWS > 1;   // whether the kernel is built for either case
   if (a.staged_stride)
     launch(solve_groups<GM, DM, EXACT, ROWS, EPL, kKnown>, grid, block, lds, s, a);
-  else   // (more than 15 thousand experts, 3900 with four LPs per wave: one kernel, the padded one, serves every group that it holds)
+  else   // (more than 15 thousand experts, 3900 with four LPs per wave: one kernel, the padded one, serves every group that it holds; against one
+         // built for the group, us a batch: (8, 2) and 15872 experts 65.9 -> 64.4, (16, 2) and 17600 75.7 -> 74.9, (8, 1) and 16800 67.5 -> 68.4,
+         // (32, 2) and 16640 77.9 -> 79.6; four per wave, (16, 1), 1500 LPs, 3968 experts 128.9 -> 131.0)
     launch(solve_groups<GM, DM, EXACT && !kKnown, ROWS, EPL, false>, grid, block, 0, s, a);
 }
 
