@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
 static bool packing_pays(const SolveArgs &a) {
   const int n_cus = current_device_cu_count();
   const int n_simds = 4 * (n_cus > 0 ? n_cus : 256);
-  return packing_pays(a.G, a.D * a.C + a.n_fixed, a.n_experts, a.n_units / n_simds + (a.n_units % n_simds != 0), a.D);
+  return packing_pays(a.G, a.D, a.D * a.C + a.n_fixed, a.n_experts, a.n_units / n_simds + (a.n_units % n_simds != 0));
 }
 constexpr int kLdsLimit = 64 * 1024 - 2048;
 

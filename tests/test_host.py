@@ -409,7 +409,7 @@ def test_lps_are_packed_where_that_was_measured_to_pay(tmp_path):
     import subprocess
     (tmp_path / "pack.cpp").write_text('''
 #include "solve_pack.h"
-extern "C" int pays(int G, int per_rank, int n_experts, int per_simd) { return lplb::packing_pays(G, per_rank, n_experts, per_simd); }
+extern "C" int pays(int G, int D, int per_rank, int n_experts, int per_simd) { return lplb::packing_pays(G, D, per_rank, n_experts, per_simd); }
 ''')
     header = ROOT / "lplb_amd" / "csrc" / "solve_pack.h"
     subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{header.parent}",
@@ -417,23 +417,23 @@ extern "C" int pays(int G, int per_rank, int n_experts, int per_simd) { return l
     pays = ctypes.CDLL(str(tmp_path / "pack.so")).pays
     text = header.read_text()
     counts = [int(n) for n in re.search(r"of a rank, in all((?: +\d+)+) LPs", text).group(1).split()]
-    rows = re.findall(r"^//   \((\d+), \d+\) +(\d+) +(\d+) +((?:[\d.]+ / *[\d.]+ *)+)", text, flags=re.M)
-    assert len(rows) >= 10 and counts[0] == 2048
+    rows = re.findall(r"^//   \((\d+), (\d+)\) +(\d+) +(\d+) +((?:[\d.]+ / *[\d.]+ *)+)", text, flags=re.M)
+    assert len(rows) >= 17 and counts[0] == 2048 and {(G, D) for G, D, *_ in rows} >= {("8", "1"), ("8", "2"), ("16", "1")}
     chosen = set()
-    for G, per_rank, n_experts, times in rows:
+    for G, D, per_rank, n_experts, times in rows:
         both = [(float(lone), float(packed)) for lone, packed in re.findall(r"([\d.]+) / *([\d.]+)", times)]
         assert len(both) == len(counts)
         for n, (lone, packed) in zip(counts, both):
-            packs = pays(int(G), int(per_rank), int(n_experts), -(-n // 1024))
+            packs = pays(int(G), int(D), int(per_rank), int(n_experts), -(-n // 1024))
             chosen.add(packs)
             slower, faster = (packed, lone) if packs else (lone, packed)
-            assert slower <= 1.03 * faster, (G, per_rank, n_experts, n, lone, packed)
+            assert slower <= 1.03 * faster, (G, D, per_rank, n_experts, n, lone, packed)
     assert chosen == {0, 1}
-    assert not any(pays(G, per_rank, per_rank * G, 1) for G in range(1, 17) for per_rank in (1, 32, 1024))   # alone on its SIMD
+    assert not any(pays(G, D, per_rank, per_rank * G, 1) for G in range(1, 17) for D in (1, 2, 4) for per_rank in (1, 32, 1024))   # alone on its SIMD
     # the batches that the GPU's test takes for packed ones and for lone ones are
     for name, r2o, ep, n_logical, n_inst, packed in BATCHED_LPS:
         n_lps = n_inst * (ep // len(r2o))
-        assert pays(len(r2o), n_logical // ep, n_logical, -(-n_lps // 1024)) == packed, name
+        assert pays(len(r2o), np.asarray(r2o).shape[1], n_logical // ep, n_logical, -(-n_lps // 1024)) == packed, name
 
 
 def test_the_last_wave_to_add_up_totals_sees_what_the_others_have_added(tmp_path):
