@@ -936,10 +936,9 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   const uint32_t end = (uint32_t)min(a.n, a.per * (slice + 1)), w0 = (uint32_t)a.per * (uint32_t)slice + wave_s * (K * kWave);   // this wave's first index (uniform)
   LPLB_PLAN_STAMP(0);
   LPLB_SLICE_STAMP(0);
-  // Where a slice shares a CU with an LP workgroup (grids with more workgroups than CUs), its
-  // waves go first: the LP wave issues an instruction nearly every cycle it may, and a slice
-  // wave on the same SIMD would be starved for as long as the LP runs, with every other slice
-  // waiting for it.  The slices spend most of their time asleep, so the LP loses little.
+  // Where a slice shares a CU with an LP workgroup (grids with more workgroups than CUs), its waves go first until the counts are in:
+  // the LP wave issues an instruction nearly every cycle it may, also where counts are supplied and it has begun, and a slice wave on
+  // the same SIMD would be starved for as long as the LP runs, with every other slice waiting for it.
   __builtin_amdgcn_s_setprio(2);
 
   // ---- small table reads, the index loads right behind them, the tables while they are on their way ----
@@ -1122,7 +1121,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   const int passes = (wave_len + K * kWave - 1) / (K * kWave);
   LPLB_PLAN_STAMP(0);
   LPLB_SLICE_STAMP(0);
-  __builtin_amdgcn_s_setprio(2);
+  __builtin_amdgcn_s_setprio(2);   // (to the end: its ordinals take longer than the LP beside them; [1048576 x 8] 33.3 us with and without a step back)
 
   const PlanTableLoads tl = issue_plan_table_loads(a, tid, wave_s, slice == 0 && a.physical_counts);
   // (places past the last repeat it: without a branch the loads of the next pass stay on their way while one is counted)
