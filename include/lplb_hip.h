@@ -426,6 +426,12 @@ int lplb_place_experts_covers(int group_size, int dup_per_rank, int ep_size, int
 int lplb_place_experts(const void *history, int history_type, const int32_t *r2o, int group_size,
                        int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
                        int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream);
+/* The same with up to 384 experts to be packed at once. */
+int lplb_place_on_large_nodes_covers(int group_size, int dup_per_rank, int ep_size, int n_logical, int n_physical,
+                                     int n_nodes);
+int lplb_place_on_large_nodes(const void *history, int history_type, const int32_t *r2o, int group_size,
+                              int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
+                              int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream);
 
 /*
  * No counterpart in the reference.  enabled = 0 makes lplb_plan always run the

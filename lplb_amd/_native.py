@@ -68,6 +68,8 @@ _SIGNATURES = {
     "lplb_rebalance_experts": (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "lplb_build_mapping": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "lplb_place_experts_covers": (_i, [_i, _i, _i, _i, _i, _i]),
+    "lplb_place_on_large_nodes_covers": (_i, [_i, _i, _i, _i, _i, _i]),
+    "lplb_place_on_large_nodes": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "lplb_place_experts": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "lplb_plan_noalloc": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
 }
@@ -173,27 +175,33 @@ _HISTORY_TYPES = {torch.int32: 0, torch.int64: 1, torch.float32: 2, torch.float6
 
 
 @functools.lru_cache(maxsize=256)
-def placement_covers(group_size: int, dup_per_rank: int, ep_size: int, n_logical: int, n_physical: int, n_nodes: int) -> bool:
+def placement_covers(group_size: int, dup_per_rank: int, ep_size: int, n_logical: int, n_physical: int, n_nodes: int,
+                     large_nodes: bool = False) -> bool:
     """Whether place_experts has a kernel for this deployment.  (Kept: a call that is refused costs the host path as much as
     the question.)"""
-    return load().lplb_place_experts_covers(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes) != 0
+    lib = load()
+    covers = lib.lplb_place_on_large_nodes_covers if large_nodes else lib.lplb_place_experts_covers
+    return covers(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes) != 0
 
 
-def place_experts(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_physical: int, n_nodes: int) -> torch.Tensor | None:
+def place_experts(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_physical: int, n_nodes: int,
+                  large_nodes: bool = False) -> torch.Tensor | None:
     """build_redundancy_mapping for a history on the current device, by a kernel there: its three arrays as parts of
-    one int32 tensor [n_physical + 3 * n_logical] on that device, complete on return; None if the kernel does not cover it."""
+    one int32 tensor [n_physical + 3 * n_logical] on that device, complete on return; None if the kernel does not cover it.
+    large_nodes: also with more than 128 experts on a node."""
     kind = _HISTORY_TYPES.get(history.dtype)
     if kind is None or not history.is_contiguous() or _device_index(history) != torch.cuda.current_device():
         return None
     n_logical = history.numel()
     group_size, dup_per_rank = r2o.shape
-    if not placement_covers(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes):
+    if not placement_covers(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes, large_nodes):
         return None
     table = torch.empty(n_physical + 3 * n_logical, dtype=torch.int32, device=history.device)
     at = table.data_ptr()
-    _check(load().lplb_place_experts(history.data_ptr(), kind, r2o.data_ptr(), group_size, dup_per_rank, ep_size, n_logical,
-                                     n_physical, n_nodes, at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical),
-                                     _stream(history)))
+    lib = load()
+    place = lib.lplb_place_on_large_nodes if large_nodes else lib.lplb_place_experts
+    _check(place(history.data_ptr(), kind, r2o.data_ptr(), group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes,
+                 at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical), _stream(history)))
     return table
 
 

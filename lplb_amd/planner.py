@@ -136,7 +136,7 @@ class Planner:
                 or workload.numel() != self.n_logical_routed_experts or workload.device != self._r2o_placed.device
                 or torch.cuda.is_current_stream_capturing()):
             return None
-        return _native.place_experts(workload, self._r2o_placed, self.ep_size, self.n_routed_experts, n_nodes)
+        return _native.place_experts(workload, self._r2o_placed, self.ep_size, self.n_routed_experts, n_nodes, large_nodes=True)
 
     def count_workload(self, idx: torch.Tensor, n_sms: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Histogram of ``idx`` (values in [-1, n_logical), -1 ignored) over ``n_sms`` slices.

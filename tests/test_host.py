@@ -878,6 +878,17 @@ def test_a_deployment_that_the_gpu_does_not_place_allocates_nothing_there(monkey
     assert asked == [(8, 2, 8, 136, 152, 1)]
 
 
+def test_which_large_nodes_the_gpu_places():
+    """Up to 384 experts packed at once, and everything that the call for smaller nodes covers."""
+    covers = _native.load().lplb_place_on_large_nodes_covers
+    for name, (r2o, ep, n_logical, replicas, covered) in PLACEMENTS.items():
+        assert covers(*r2o.shape, ep, n_logical, n_logical + replicas * ep, ep // 8) == 1, name
+    for per_node, covered in ((136, 1), (256, 1), (384, 1), (392, 0)):
+        assert covers(8, 2, 8, per_node, per_node + 16, 1) == covered, per_node
+    assert covers(8, 2, 16, 512, 512 + 32, 2) == 1 and covers(8, 2, 16, 512, 512 + 32, 1) == 0   # a node each; both groups on one
+    assert covers(8, 2, 8, 129, 144, 1) == 0 and covers(0, 2, 8, 128, 144, 1) == 0               # no deployments
+
+
 def test_placement_reports_memory_that_runs_out():
     """No C++ exception leaves the library: a call whose working memory cannot be had fails like any other."""
     import subprocess
