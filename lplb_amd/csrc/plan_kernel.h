@@ -182,7 +182,7 @@ struct __attribute__((aligned(8))) PlanRoute {
 // One ranking slot per (wave, replicated set, chunk of 64 indices), K chunks per wave.
 constexpr int64_t kLongestSlice = 16 * kPlanThreads;   // 16 chunks per wave
 constexpr int kLongChunks = 8, kLongPasses = 8;        // of a long slice: chunks per wave and pass, passes
-constexpr int kFewestLongSlices = 64;
+constexpr int kFewestLongSlices = 64, kFewestSlicesInPasses = 32;   // past 8192 indices; up to them
 constexpr int64_t kLongestOfLongSlices = kLongPasses * kLongChunks * kPlanThreads;
 // (K = 0: a long slice, without its records, which lie behind the rest)
 constexpr int slice_record_bytes(int k) { return k > 0 ? rank_record_bytes_single(k) : 0; }
@@ -193,18 +193,24 @@ template <int K> static size_t plan_slice_lds_bytes(int n_logical, int n_rep) {
          (size_t)(n_logical + 2) * sizeof(PlanRoute) + (size_t)(n_logical + 16 + kSliceFlags) * sizeof(int32_t) +
          (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t);
 }
-// A long slice's records per (wave, replicated set): the bitmaps of a pass's chunks, and what a token's ordinal is made of (a
-// bitmap and the tokens before it), both padded for the LDS banks; sixteen sets are worked on at once.
-constexpr int kLongBitsBytes = kLongChunks * 8 + 8, kLongRanksBytes = kLongChunks * 16 + 16;
-__host__ __device__ constexpr int long_slice_padded_sets(int n_rep) { return n_rep / 16 * 16 + 16; }   // at least one more: of tokens without a set
+// A long slice's row per (wave, replicated set), and one for tokens without a set: the bitmaps of the chunks that are ranked at once
+// and the wave's tokens of the set so far (with 8 more bytes a row for the LDS banks).
+constexpr int kRankChunks = 4, kRankRowBytes = kRankChunks * 8 + 8;
+constexpr int kFewSets = 32;        // up to which slices of 16 chunks per wave that feed the LP have bitmaps of all chunks
+constexpr int kLongMaxSets = 255;   // sets of a long slice are bytes
 __host__ __device__ constexpr size_t long_slice_records_at(int n_logical, int n_rep) {
   return ((size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)(n_logical + 2) * sizeof(PlanRoute) + (size_t)(n_logical + 16 + kSliceFlags) * sizeof(int32_t) +
           (size_t)(3 + kPlanWaves) * n_rep * sizeof(int32_t) + 15) / 16 * 16;
 }
 inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
-  return long_slice_records_at(n_logical, n_rep) +
-         (size_t)kPlanWaves * (long_slice_padded_sets(n_rep) * (kLongBitsBytes + kLongRanksBytes + sizeof(int32_t)) + 2 * hist_words * sizeof(int32_t)) +
+  return long_slice_records_at(n_logical, n_rep) + (size_t)kPlanWaves * ((n_rep + 1) * kRankRowBytes + 2 * hist_words * sizeof(int32_t)) +
          (size_t)(n_logical + 16) / 16 * 16;
+}
+// Slices past kLongestSlice ask for more than that: 220 bytes a row, the sets padded to the next multiple of sixteen past their number.
+// It decides which batches are cut into those at all; tests/test_gpu_parity.py holds the chain to the rest.
+inline size_t longest_slices_lds_bytes(int n_logical, int n_rep, int hist_words) {
+  return long_slice_lds_bytes(n_logical, n_rep, hist_words) +
+         (size_t)kPlanWaves * ((n_rep / 16 * 16 + 16) * 220 - (n_rep + 1) * kRankRowBytes);
 }
 struct SliceTables {
   RepEntry *reps;           // [R + 1] by set; of set 0: a test that never sends a token away
@@ -1076,17 +1082,26 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   LPLB_SLICE_STAMP(3);
 }
 
-// Slices of more than kLongestSlice indices (batches of more than 256 x 8192 on 256 CUs): the same exchange, with the tokens of
-// a wave in passes of eight chunks.  The chain reads the indices twice and leaves the memory idle while its LP runs; here they
-// are read once and stay in registers (11 bits of expert, 12 of ordinal among the wave's tokens of the set), and the ordinals
-// are worked out while the LP is running.  At 8 ranks, as the chain and so: [1048576 x 8] 42 and 33.5-35.1 us; 2097153 indices in 256
-// slices 22.7 and 17.3, 4200000 30.5 and 23.3; 524289 in 64 slices 21.8 and 16.6, 1280000 27.9 and 22.4.  Read 9.3 and written 11.2 us
-// by kernels that do nothing else.  What bounds it: 10.5 us until the last index is
+// Slices of more than kLongestSlice indices (batches of more than 256 x 8192 on 256 CUs), and shorter ones with many replicated sets:
+// the same exchange, with the tokens of a wave in passes of eight chunks.  The chain reads the indices twice and leaves the memory
+// idle while its LP runs; here they are read once and stay in registers (11 bits of expert, 12 of ordinal among the wave's tokens of
+// the set), and the ordinals are worked out while the LP is running.  At 8 ranks, as the chain and so: [1048576 x 8] 42 and 33.5-35.1 us;
+// 2097153 indices in 256 slices 22.7 and 17.3, 4200000 30.5 and 23.3; 524289 in 64 slices 21.8 and 16.6, 1280000 27.9 and 22.4.
+// Read 9.3 and written 11.2 us by kernels that do nothing else.  What bounds it: 10.5 us until the last index is
 // counted, 4 until the LP has the totals, 5 until its shares are seen, then the choice and the stores (9) with the second half
 // of the ordinals between them: a pass of those is about 1 us a wave, waits for the LDS and instructions in
 // turn.  With every pass unrolled, for the registers' sake, the code is 58 KiB, nearly the instruction cache of two CUs.
 // The histogram is per wave: what is in the waves before then costs nothing more than the sums, and
 // a lookup of the set beside the histogram's update made the counting twice as long (the LDS serves them in turn).
+// Ordinals: a bitmap of a chunk says who is ahead of a token in the chunk, a running count per (wave, set) what is ahead of the chunk,
+// and a chunk's first token of a set adds to that.  The instructions do not go with the number of sets, and a row has 40 bytes where
+// bitmaps of 16 chunks with their starting ordinals have 272, of which 64 sets take a CU.
+// So, against the chain, 8 ranks in four and eight groups (64 and 128 sets): [131072 x 8] 18.2 -> 13.9 and 22.1 -> 15.9 us, [262144 x 8] 23.8 -> 16.5 and
+// 29.3 -> 18.5; 32 ranks (64 sets) [262144 x 8] 33.9 -> 27.1, counts supplied 34.8 -> 20.7.  16 sets at [1048576 x 8] 32.3 -> 32.1.
+// Against bitmaps of all 16 chunks (slices of 4097 to 8192): counts supplied, at 16, 32 and 64 sets [262144 x 8] 13.4 -> 12.7, 14.4 -> 13.7, 15.0 -> 15.0,
+// [196608 x 8] 12.9 -> 12.6, 14.1 -> 13.7, 16.0 -> 15.0; own counts, which leave later here (loads and table of sets ahead of them), 15.1 -> 15.2, 15.7 -> 15.5
+// and 14.35 -> 14.5, 14.7 -> 14.7, but 64 sets 16.0 -> 15.2.  Eight chunks (up to 4096) are the faster with bitmaps of all of them while
+// those fit: [131072 x 8] 11.9 and 12.7, counts supplied 9.9 and 10.1.
 template <int GM, int DM, bool EXACT>
 __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void plan_of_long_slices(PlanArgs a) {
   constexpr int K = kLongChunks;
@@ -1105,12 +1120,10 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   const int slice = pid - a.n_lp_workgroups;
   const SliceTables t = carve_tables<0>(smem_raw, nl, R);
   int *const missing = t.missing;
-  const int hist_len = 2 * a.hist_words, padded_sets = long_slice_padded_sets(R);
-  // [waves][padded_sets][kLongBitsBytes], [waves][padded_sets][kLongRanksBytes], [waves][padded_sets], [waves][hist_len], [n_logical + 1]
-  unsigned char *my_bits = t.records + wave_s * padded_sets * kLongBitsBytes;
-  unsigned char *my_ranks = t.records + kPlanWaves * padded_sets * kLongBitsBytes + wave_s * padded_sets * kLongRanksBytes;
-  int32_t *my_so_far = reinterpret_cast<int32_t *>(t.records + kPlanWaves * padded_sets * (kLongBitsBytes + kLongRanksBytes)) + wave_s * padded_sets;
-  int32_t *wave_hists = my_so_far + (kPlanWaves - wave_s) * padded_sets;
+  const int hist_len = 2 * a.hist_words, rows_bytes = (R + 1) * kRankRowBytes;
+  // [waves][R + 1][kRankRowBytes], [waves][hist_len], [n_logical + 1]
+  unsigned char *my_rows = t.records + wave_s * rows_bytes;
+  int32_t *wave_hists = reinterpret_cast<int32_t *>(t.records + kPlanWaves * rows_bytes);
   int32_t *my_hist = wave_hists + wave_s * hist_len;
   unsigned char *set_of_expert = reinterpret_cast<unsigned char *>(wave_hists + kPlanWaves * hist_len);   // four to a word: lanes rarely meet in a bank
   const int64_t begin = slice_begin(a.n, a.per, slice);
@@ -1133,12 +1146,10 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   };
   int64_t raw[2][K];
   load_pass(raw[0], 0);
-  for (int q = lane; q < padded_sets; q += kWave)
-    my_so_far[q] = 0;
   for (int e = lane; e < hist_len; e += kWave)
     my_hist[e] = 0;
-  for (int i = lane; i < padded_sets * kLongBitsBytes / 8; i += kWave)
-    reinterpret_cast<unsigned long long *>(my_bits)[i] = 0ull;
+  for (int i = lane; i < rows_bytes / 8; i += kWave)
+    reinterpret_cast<unsigned long long *>(my_rows)[i] = 0ull;
   clear_plan_tables<0>(t, tid);
   __syncthreads();
   enter_plan_tables(a, t, tl, tid, wave_s);
@@ -1211,57 +1222,51 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
   // ---- while the others' words are on their way: ordinals among the wave's tokens, pass by pass (the wave's own records: no barrier) ----
   __builtin_amdgcn_s_setprio(2);
   const uint32_t my_bit = 1u << lane % 32;
-  unsigned char *my_half_of_bits = my_bits + lane / 32 * 4;
-  const int c_of_lane = lane % K;
-  auto rank_pass = [&](int p) {
-    uint32_t set[K];
+  const int my_half = lane / 32 * 4;
+  auto rank_chunks = [&](uint32_t *mine) {
+    uint32_t set[kRankChunks];
+    unsigned char *row[kRankChunks];
+    bool in_set[kRankChunks];
     // (all reads ahead of the first update: the compiler keeps their order, and each would be waited for)
 #pragma unroll
-    for (int c = 0; c < K; ++c)
-      set[c] = set_of_expert[token[p * K + c]];
+    for (int c = 0; c < kRankChunks; ++c)
+      set[c] = set_of_expert[mine[c]];
 #pragma unroll
-    for (int c = 0; c < K; ++c) {
-      if (set[c] < (uint32_t)R)
-        atomicOr(reinterpret_cast<uint32_t *>(my_half_of_bits + __umul24(set[c], (uint32_t)kLongBitsBytes) + c * 8), my_bit);
+    for (int c = 0; c < kRankChunks; ++c) {
+      row[c] = my_rows + __umul24(set[c], (uint32_t)kRankRowBytes);
+      in_set[c] = set[c] < (uint32_t)R;
+      if (in_set[c])
+        atomicOr(reinterpret_cast<uint32_t *>(row[c] + c * 8 + my_half), my_bit);
     }
     SliceTokens<K>::own_slots_are_written();
-    // lane = (set, chunk), chunk fastest, two sets side by side; the bitmaps are empty again behind it
-    unsigned char *bits_at = my_bits + (lane / K) * kLongBitsBytes + c_of_lane * 8;
-    unsigned char *ranks_at = my_ranks + (lane / K) * kLongRanksBytes + c_of_lane * 16;
-    int32_t *so_far = my_so_far + lane / K;
-    constexpr int kSets = kWave / K;   // at once
-    for (int q0 = 0; q0 < R; q0 += 2 * kSets) {
-      unsigned long long bits[2];
-      int earlier[2], start[2], own[2];
+    uint2 bits[kRankChunks];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        bits[j] = *reinterpret_cast<const unsigned long long *>(bits_at + j * kSets * kLongBitsBytes);
-        earlier[j] = so_far[j * kSets];
-      }
+    for (int c = 0; c < kRankChunks; ++c)
+      bits[c] = *reinterpret_cast<const uint2 *>(row[c] + c * 8);
+    uint32_t before[kRankChunks], so_far[kRankChunks];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        own[j] = __popcll(bits[j]);
-        start[j] = earlier[j] + group_exclusive_scan<K>(own[j], c_of_lane);
-      }
+    for (int c = 0; c < kRankChunks; ++c)
+      before[c] = __builtin_amdgcn_mbcnt_hi(bits[c].y, __builtin_amdgcn_mbcnt_lo(bits[c].x, 0));
+    // The LDS serves a wave's instructions in the order they were issued: a chunk's tokens read what the chunks before it have added.
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        *reinterpret_cast<unsigned long long *>(bits_at + j * kSets * kLongBitsBytes) = 0ull;
-        *reinterpret_cast<i32x4 *>(ranks_at + j * kSets * kLongRanksBytes) = i32x4{(int)(uint32_t)bits[j], (int)(uint32_t)(bits[j] >> 32), start[j], 0};
-        if (c_of_lane == K - 1)
-          so_far[j * kSets] = start[j] + own[j];
+    for (int c = 0; c < kRankChunks; ++c) {
+      uint32_t *of_set = reinterpret_cast<uint32_t *>(row[c] + kRankChunks * 8);
+      so_far[c] = *of_set;
+      if (in_set[c] && before[c] == 0) {   // the chunk's first token of its set; its bitmap is empty again behind it
+        __hip_atomic_fetch_add(of_set, (uint32_t)(__popc(bits[c].x) + __popc(bits[c].y)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        *reinterpret_cast<uint2 *>(row[c] + c * 8) = uint2{0, 0};
       }
-      bits_at += 2 * kSets * kLongBitsBytes;
-      ranks_at += 2 * kSets * kLongRanksBytes;
-      so_far += 2 * kSets;
     }
-    SliceTokens<K>::own_slots_are_written();
 #pragma unroll
-    for (int c = 0; c < K; ++c) {
-      const i32x4 x = *reinterpret_cast<const i32x4 *>(my_ranks + __umul24(set[c], (uint32_t)kLongRanksBytes) + c * 16);
-      const uint32_t k = (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)x.y, __builtin_amdgcn_mbcnt_lo((uint32_t)x.x, (uint32_t)x.z));
-      token[p * K + c] |= k << 16;   // (without a set: whatever is there)
-      worked_out_here(token[p * K + c]);
+    for (int c = 0; c < kRankChunks; ++c) {
+      mine[c] |= (so_far[c] + before[c]) << 16;   // (without a set: whatever is there)
+      worked_out_here(mine[c]);
     }
+  };
+  auto rank_pass = [&](int p) {
+#pragma unroll
+    for (int c = 0; c < K; c += kRankChunks)
+      rank_chunks(token + p * K + c);
   };
 #pragma unroll
   for (int p = 0; p < kLongPasses / 2; ++p)
@@ -1557,14 +1562,15 @@ template <int GM, int DM> static int launch_scan_and_solve(const ScanSolveArgs &
 template <int GM, int DM, bool EXACT, int K>
 static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   const size_t lds_slice = K > 0 ? plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep)
-                                 : long_slice_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words);
+                           : a.per > kLongestSlice ? longest_slices_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words)
+                                                   : long_slice_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words);
   // LP workgroups: their waves' working areas, then the counts (one copy per LP, or one for all of the batch's own)
   const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
   const size_t one_copy = counts_bytes(a.sh.n_logical);
   const size_t all_copies = (size_t)min(a.solve.n_units, kLpsPerWorkgroup) * one_copy;
   const size_t lds = max(lds_slice, lp_areas + (a.local_counts ? one_copy : all_copies));
   a.solve.staged_stride = (int)(one_copy / sizeof(int32_t));
-  if (lds > (size_t)kPlanLdsLimit)
+  if (lds > (size_t)kPlanLdsLimit || (K == 0 && a.n_rep > kLongMaxSets))
     return LPLB_OK;
   static KernelFootprint footprint;
   if constexpr (K > 0)
@@ -1587,12 +1593,24 @@ template <int GM, int DM, bool EXACT> static int launch_plan_shape(PlanArgs &a, 
            : a.n <= 4 * per_chunk ? launch_plan_single<GM, DM, EXACT, 4>(a, s, done)
                                   : launch_plan_single<GM, DM, EXACT, 8>(a, s, done);
   }
-  return a.per <= kPlanThreads       ? launch_plan_slices<GM, DM, EXACT, 1>(a, s, done)
-         : a.per <= 2 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 2>(a, s, done)
-         : a.per <= 4 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 4>(a, s, done)
-         : a.per <= 8 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 8>(a, s, done)
-         : a.per <= kLongestSlice    ? launch_plan_slices<GM, DM, EXACT, 16>(a, s, done)
-                                     : launch_plan_slices<GM, DM, EXACT, 0>(a, s, done);
+  // Slices of up to 8192 indices in passes too, where there are many: whose tables fit no other way, or not twice on a CU; with 16
+  // chunks per wave also those that are the faster for it (plan_of_long_slices).
+  const bool many = a.n_slices >= kFewestSlicesInPasses;
+  const auto in_passes = [&]() { return launch_plan_slices<GM, DM, EXACT, 0>(a, s, done); };
+  if (a.per > kLongestSlice)
+    return in_passes();
+  int rc = LPLB_OK;
+  if (a.per > 8 * kPlanThreads && many && (!a.local_counts || a.n_rep > kFewSets)) {
+    rc = in_passes();
+    if (rc != LPLB_OK || *done)
+      return rc;
+  }
+  rc = a.per <= kPlanThreads       ? launch_plan_slices<GM, DM, EXACT, 1>(a, s, done)
+       : a.per <= 2 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 2>(a, s, done)
+       : a.per <= 4 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 4>(a, s, done)
+       : a.per <= 8 * kPlanThreads ? launch_plan_slices<GM, DM, EXACT, 8>(a, s, done)
+                                   : launch_plan_slices<GM, DM, EXACT, 16>(a, s, done);
+  return rc == LPLB_OK && !*done && many ? in_passes() : rc;
 }
 template <int GM, int DM> static int launch_plan_padded_or_not(PlanArgs &a, hipStream_t s, bool *done) {
   return a.sh.G == GM && a.sh.D == DM ? launch_plan_shape<GM, DM, true>(a, s, done) : launch_plan_shape<GM, DM, false>(a, s, done);
