@@ -55,17 +55,21 @@ template <typename Kernel> hipError_t allow_dynamic_lds(Kernel kernel, int bytes
 // Every kernel of the library is launched through here.  If the calling thread
 // armed a pair of events, the launch records the kernel's own begin and end
 // timestamps into them (not the time the launch was enqueued).
-template <typename Kernel, typename... Args>
-inline void launch_with_flags(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t stream,
+// (The launch syntax's own call pushes the configuration for a stub that takes it back: 2.42 us of the calling thread, 2.12 without.)
+template <typename... Params, typename... Args>
+inline void launch_with_flags(void (*kernel)(Params...), dim3 grid, dim3 block, size_t lds, hipStream_t stream,
                               unsigned flags, Args... args) {
   const LaunchEvents ev = take_launch_events();
-  if (ev.start || ev.stop || flags)
-    hipExtLaunchKernelGGL(kernel, grid, block, lds, stream, ev.start, ev.stop, flags, args...);
-  else
-    hipLaunchKernelGGL(kernel, grid, block, lds, stream, args...);
+  [&](Params... params) {
+    void *at[] = {const_cast<void *>(static_cast<const void *>(&params))...};
+    if (ev.start || ev.stop || flags)
+      (void)hipExtLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, at, lds, stream, ev.start, ev.stop, (int)flags);
+    else
+      (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, at, lds, stream);
+  }(args...);
 }
-template <typename Kernel, typename... Args>
-inline void launch(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t stream, Args... args) {
+template <typename... Params, typename... Args>
+inline void launch(void (*kernel)(Params...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, Args... args) {
   launch_with_flags(kernel, grid, block, lds, stream, 0u, args...);
 }
 
