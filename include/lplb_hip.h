@@ -490,6 +490,12 @@ int lplb_plan_one_launch_count(long long *count);
  */
 int lplb_plan_inject_fault(int extra_slices_expected, int max_polls);
 
+/*
+ * Test hook, no counterpart in the reference.  In the next lplb_count_idx that runs as one launch no slice waits for what the others
+ * publish: each counts the indices in front of it itself, as when a wait has run out.  The table is the same.
+ */
+int lplb_count_inject_fault(void);
+
 #ifdef __cplusplus
 }
 #endif

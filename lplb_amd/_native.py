@@ -62,6 +62,7 @@ _SIGNATURES = {
     "lplb_plan_poll_timeouts": (_i, [_vp, _vp]),
     "lplb_plan_one_launch_count": (_i, [_vp]),
     "lplb_plan_inject_fault": (_i, [_i, _i]),
+    "lplb_count_inject_fault": (_i, []),
     "lplb_plan": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
     "lplb_balanced_packing": (_i, [_vp, _i, _i, _i, _vp, _vp]),
     "lplb_replicate_experts": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp]),

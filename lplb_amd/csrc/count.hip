@@ -1,6 +1,7 @@
 // Per-expert token histogram with an inclusive prefix over slices.
 //
-// Two launches on the caller's stream:
+// Slices of up to 4096 indices, up to 256 of them: one launch on the caller's stream (count_and_scan, below).  Else, and in a
+// capture, two:
 //   1. slice_histogram: one workgroup per slice, LDS histogram (eight copies, chosen by lane)
 //      fed by coalesced 16-byte index loads, row p of the output = counts of slice p;
 //   2. prefix_over_slices: turns the rows into running sums down the slice axis,
@@ -20,6 +21,8 @@
 // the same both ways.
 // Callers that need only the totals of a short batch get them in one launch: slice_histogram with
 // TOTALS (slices add their counts to one vector) or expert_totals (every workgroup owns four experts).
+#include "map_kernel.h"
+#include "plan_sync.h"
 #include "scan.h"
 
 namespace lplb {
@@ -37,18 +40,12 @@ __host__ __device__ constexpr int histogram_stride(int n_experts, int copies) {
   return copies > 1 ? ((n_experts + 31) & ~31) + 4 : n_experts;
 }
 
-// TOTALS: instead of writing its row, a slice adds its counts to the one vector `counts` [n_experts]
-// (device-wide atomic adds, none for an expert the slice has no token of).  The launch sets the vector `clear` [n_experts]
-// (if given) to zero -- a caller that takes two vectors in turn never has to zero one --, or without TOTALS to kNoTotal,
-// for scan_and_solve.
-template <int COPIES, bool TOTALS>
-__global__ __launch_bounds__(1024) void slice_histogram(
-    const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per,
-    int32_t *__restrict__ counts, int32_t *__restrict__ clear) {
-  extern __shared__ int32_t hist[];
-  fetch_arguments_now(idx, n, n_experts, per, counts, clear);
+// The tokens of slice p into the histograms `hist` (LDS); ends with a workgroup barrier.  `meanwhile` is called while the first loads
+// are on their way.
+template <int COPIES, typename Meanwhile>
+__device__ __forceinline__ void count_slice(const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per, int p, int32_t *hist,
+                                            Meanwhile meanwhile) {
   const int tid = threadIdx.x, nt = blockDim.x;
-  const int p = blockIdx.x;
   const int stride = histogram_stride(n_experts, COPIES);
   int32_t *mine = hist + (tid % COPIES) * stride;
   auto count = [&](int64_t v) {
@@ -86,9 +83,7 @@ __global__ __launch_bounds__(1024) void slice_histogram(
   load_batch(even, 0);
   for (int e = tid; e < COPIES * stride; e += nt)
     hist[e] = 0;
-  if (clear)
-    for (int64_t e = (int64_t)p * nt + tid; e < n_experts; e += (int64_t)gridDim.x * nt)
-      clear[e] = TOTALS ? 0 : kNoTotal;
+  meanwhile();
   __syncthreads();
   for (int64_t i0 = 0; i0 < n_pairs; i0 += 2 * batch) {
     load_batch(odd, i0 + batch);
@@ -103,6 +98,26 @@ __global__ __launch_bounds__(1024) void slice_histogram(
   if (tid == 0 && ((end - begin - head) & 1))
     count(idx[end - 1]);
   __syncthreads();
+}
+
+// TOTALS: instead of writing its row, a slice adds its counts to the one vector `counts` [n_experts]
+// (device-wide atomic adds, none for an expert the slice has no token of).  The launch sets the vector `clear` [n_experts]
+// (if given) to zero -- a caller that takes two vectors in turn never has to zero one --, or without TOTALS to kNoTotal,
+// for scan_and_solve.
+template <int COPIES, bool TOTALS>
+__global__ __launch_bounds__(1024) void slice_histogram(
+    const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per,
+    int32_t *__restrict__ counts, int32_t *__restrict__ clear) {
+  extern __shared__ int32_t hist[];
+  fetch_arguments_now(idx, n, n_experts, per, counts, clear);
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int p = blockIdx.x;
+  const int stride = histogram_stride(n_experts, COPIES);
+  count_slice<COPIES>(idx, n, n_experts, per, p, hist, [&]() {
+    if (clear)
+      for (int64_t e = (int64_t)p * nt + tid; e < n_experts; e += (int64_t)gridDim.x * nt)
+        clear[e] = TOTALS ? 0 : kNoTotal;
+  });
   int32_t *row = TOTALS ? counts : counts + (int64_t)p * n_experts;
   if constexpr (!TOTALS) {
     for (int e = tid; e < n_experts; e += nt) {
@@ -162,6 +177,186 @@ __global__ __launch_bounds__(kScanThreads) void prefix_over_slices(int32_t *__re
   __shared__ ScanLds lds;
   fetch_arguments_now(counts, n_blocks, n_experts);
   scan_columns(counts, n_blocks, n_experts, blockIdx.x, lds, [](int, int32_t) {});
+}
+
+// ---- histogram and running sums in one launch ----
+// Up to kCountMaxSlices slices: a slice publishes its counts as soon as it has them, and the first of them turn a few columns of the
+// published rows into running sums each: a trip from CU to CU instead of a launch and a trip of the table through memory and back.
+// [32768 x 8] in 256 slices 6.2 -> 5.6 us as
+// kernels, of which 1.4 are the launch, 1.5 until the counts are out, 0.5 to 1 the trip, and one launch (2.1 us of the calling thread) less, which
+// is what the three calls waited for: 17.2 -> 14.9 us.
+// What crosses workgroups are words as in the one-launch plan (plan_sync.h): the launch's tag in the high half, two counts of 16
+// bits in the low half, so that nothing has to be cleared and words may arrive in any order.  The host gives every launch
+// of a device a number; it is the tag, and one of kCountRegions parts of the array in turn is the launch's.
+// Nothing has to be resident at once: only the workgroups with columns wait, a quarter of the grid at most, and should their
+// words not come within kCountPolls polls (a launch that is kept off the GPU for long, or that finds its region in use by one
+// kCountRegions launches later), they count those columns of all slices themselves.  So the rows are right in any case.
+constexpr int kCountMaxSlices = 256, kCountMaxExperts = 1024, kCountRegions = 8, kCountPolls = 1 << 14;
+// Up to 4096 indices a slice.  Longer ones keep the adding workgroups' loads waiting behind the indices', and the calling thread is not what
+// the three calls wait for any more: [131072 x 8] (4096) 18.1 -> 16.6 us, [262144 x 8] (8192) 19.6 in two launches, 20.1 in one, at 32 ranks
+// 32.1 and 32.7.
+constexpr int64_t kCountMaxSlice = 4096;
+static_assert(kCountMaxSlice < 65536, "two counts to a word");
+constexpr int kCountRegionWords = kCountMaxSlices * kCountMaxExperts / 2;
+static __device__ __attribute__((aligned(4096))) unsigned long long g_count_words[kCountRegions * kCountRegionWords];
+
+// A pair of words, 16-byte aligned, with one load past the caches (see agent_load_pairs), polled until both have the tag.  By whole
+// waves; false: they did not come, or a later launch has the region.
+__device__ inline bool poll_pair(u32x4 &v, const unsigned long long *p, uint32_t tag, int max_polls) {
+  bool in = false, later = false;
+  for (int polls = 0; polls < max_polls; ++polls) {
+    if (!in) {
+      asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
+      in = ((v.y ^ tag) | (v.w ^ tag)) == 0;
+      later = (int32_t)(v.y - tag) > 0 || (int32_t)(v.w - tag) > 0;
+    }
+    if (__all(in))
+      return true;
+    if (__any(later))
+      return false;
+    __builtin_amdgcn_s_sleep(2);
+  }
+  return false;
+}
+// Sum over the lanes up to this one.
+__device__ inline int32_t wave_inclusive_scan(int32_t v) {
+  v += row_shr<1>(v);
+  v += row_shr<2>(v);
+  v += row_shr<4>(v);
+  v += row_shr<8>(v);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142 /* row_bcast:15 */, 0xa, 0xf, false);
+  return v + __builtin_amdgcn_update_dpp(0, v, 0x143 /* row_bcast:31 */, 0xc, 0xf, false);
+}
+
+__host__ __device__ constexpr int padded_experts(int n) { return (n + 3) / 4 * 4; }
+// GROUPS of kCountMaxSlices threads; thread = (four columns, slice).
+template <int GROUPS>
+__global__ __launch_bounds__(GROUPS *kCountMaxSlices) void count_and_scan(const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per,
+                                                                          int n_slices, int32_t *__restrict__ counts, unsigned long long *rows,
+                                                                          uint32_t tag, int max_polls) {
+  constexpr int COPIES = kHistogramCopies, nt = GROUPS * kCountMaxSlices, kGroupWaves = kCountMaxSlices / kWave;
+  extern __shared__ int32_t hist[];
+  __shared__ int32_t of_wave[GROUPS][kGroupWaves][4];
+  __shared__ int missing;
+  fetch_arguments_now(idx, n, n_experts, per, n_slices, counts, rows, tag, max_polls);
+  const int tid = threadIdx.x, lane = tid % kWave, wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int p = blockIdx.x, group = wave_s / kGroupWaves, slice = tid % kCountMaxSlices;
+  const int words = padded_experts(n_experts) / 2, quads = words / 2, stride = histogram_stride(n_experts, COPIES);
+  count_slice<COPIES>(idx, n, n_experts, per, p, hist, [&]() {
+    if (tid == 0)
+      missing = 0;
+  });
+  auto counted = [&](int e) {
+    uint32_t sum = 0;
+    if (e < n_experts)
+#pragma unroll
+      for (int k = 0; k < COPIES; ++k)
+        sum += (uint32_t)hist[k * stride + e];
+    return sum;
+  };
+  for (int w = tid; w < words; w += nt)
+    agent_store(rows + p * words + w, (unsigned long long)tag << 32 | counted(2 * w) | counted(2 * w + 1) << 16);
+  for (int q0 = p * GROUPS; q0 < quads; q0 += n_slices * GROUPS) {
+    const int q = q0 + group;
+    int32_t c[4] = {};
+    if (q < quads) {
+      u32x4 v{};
+      if (!poll_pair(v, rows + min(slice, n_slices - 1) * words + 2 * q, tag, max_polls))
+        missing = 1;
+      if (slice < n_slices) {
+        c[0] = (int32_t)(v.x & 0xffffu), c[1] = (int32_t)(v.x >> 16);
+        c[2] = (int32_t)(v.z & 0xffffu), c[3] = (int32_t)(v.z >> 16);
+      }
+    }
+    __syncthreads();
+    if (missing) {   // words did not come: the columns are counted here, slice by slice
+      for (int i = tid; i < 4 * nt; i += nt)
+        hist[i] = 0;
+      __syncthreads();
+      for (int64_t i = tid; i < n; i += nt) {
+        const int64_t e = idx[i] - 4 * q0;
+        if ((uint64_t)e < 4 * GROUPS && e + 4 * q0 < n_experts)
+          atomicAdd(&hist[((int)e / 4 * kCountMaxSlices + (int)(i / per)) * 4 + (int)e % 4], 1);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        c[j] = hist[4 * tid + j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      c[j] = wave_inclusive_scan(c[j]);
+    if (lane == kWave - 1)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        of_wave[group][wave_s % kGroupWaves][j] = c[j];
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kGroupWaves - 1; ++w)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        c[j] += w < wave_s % kGroupWaves ? of_wave[group][w][j] : 0;
+    if (q < quads && slice < n_slices) {
+      int32_t *to = counts + (int64_t)slice * n_experts + 4 * q;
+      if (n_experts % 4 == 0 && (reinterpret_cast<uintptr_t>(counts) & 15) == 0) {
+        *reinterpret_cast<int4 *>(to) = int4{c[0], c[1], c[2], c[3]};
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (4 * q + j < n_experts)
+            to[j] = c[j];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Test hook (lplb_count_inject_fault): the next launch of count_and_scan waits for nothing, every slice counts for itself.
+static std::atomic<bool> g_count_fault{false};
+// *done = false: not a case for one launch; nothing was enqueued.  (A launch that is captured would carry its tag again when it is replayed.)
+static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int n_blocks, int32_t *counts, hipStream_t s, unsigned flags, bool *done) {
+  const int64_t per = slice_len(n, n_blocks);
+  if (n_blocks > kCountMaxSlices || n_experts > kCountMaxExperts || per > kCountMaxSlice)
+    return LPLB_OK;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
+    (void)hipGetLastError();   // (the launch behind this looks at it)
+    return LPLB_OK;
+  }
+  if (capture != hipStreamCaptureStatusNone)
+    return LPLB_OK;
+  static std::atomic<unsigned long long *> known[64];
+  static std::atomic<uint32_t> launches[64];
+  int dev = -1;
+  LPLB_HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64)
+    return LPLB_OK;
+  unsigned long long *words = known[dev].load(std::memory_order_acquire);
+  if (!words) {
+    LPLB_HIP_TRY(hipGetSymbolAddress(reinterpret_cast<void **>(&words), HIP_SYMBOL(g_count_words)));
+    known[dev].store(words, std::memory_order_release);
+  }
+  // (a word's tag is told from a later one's by its sign: after 2^31 launches the two-launch form takes over for good)
+  uint32_t number = launches[dev].load(std::memory_order_relaxed);
+  do {
+    if (number >= (uint32_t)INT32_MAX)
+      return LPLB_OK;
+  } while (!launches[dev].compare_exchange_weak(number, number + 1, std::memory_order_relaxed));
+  words += (size_t)(number % kCountRegions) * kCountRegionWords;
+  const int max_polls = g_count_fault.exchange(false) ? 0 : kCountPolls;
+  const int64_t batches = (per / 2 + kLoadsInFlight - 1) / kLoadsInFlight;   // (threads as for launch_slice_histogram)
+  const auto go = [&](auto kernel, int threads) {
+    const size_t ints = std::max(kHistogramCopies * histogram_stride(n_experts, kHistogramCopies), 4 * threads);
+    launch_with_flags(kernel, dim3(n_blocks), dim3(threads), ints * sizeof(int32_t), s, flags, idx, n, n_experts, per, n_blocks, counts, words,
+                      number + 1, max_polls);
+  };
+  if (batches <= 256)
+    go(count_and_scan<1>, 256);
+  else
+    go(count_and_scan<2>, 512);
+  LPLB_HIP_TRY(hipGetLastError());
+  *done = true;
+  return LPLB_OK;
 }
 
 // ---- totals only, for short batches: one launch, nothing shared between workgroups ----
@@ -247,7 +442,11 @@ int enqueue_histogram(const int64_t *idx, int64_t n_elements, int n_experts, int
 // that kernel waited for); the prefix launch is ordered after both.
 int enqueue_count(const int64_t *idx, int64_t n_elements, int n_experts, int n_blocks,
                   int32_t *counts_by_block, hipStream_t s, bool any_order) {
-  const int rc = launch_slice_histogram<false>(idx, n_elements, n_experts, n_blocks, counts_by_block, nullptr, s,
+  bool done = false;
+  int rc = try_count_and_scan(idx, n_elements, n_experts, n_blocks, counts_by_block, s, any_order ? hipExtAnyOrderLaunch : 0u, &done);
+  if (rc != LPLB_OK || done)
+    return rc;
+  rc = launch_slice_histogram<false>(idx, n_elements, n_experts, n_blocks, counts_by_block, nullptr, s,
                                                any_order ? hipExtAnyOrderLaunch : 0u);
   if (rc != LPLB_OK)
     return rc;
@@ -332,5 +531,10 @@ extern "C" int lplb_slice_histogram_series(const int64_t *const *idx, int64_t n_
       return rc;
     }
   }
+  return LPLB_OK;
+}
+
+extern "C" int lplb_count_inject_fault(void) {
+  lplb::g_count_fault = true;
   return LPLB_OK;
 }
