@@ -182,9 +182,10 @@ __global__ __launch_bounds__(kScanThreads) void prefix_over_slices(int32_t *__re
 // ---- histogram and running sums in one launch ----
 // Up to kCountMaxSlices slices: a slice publishes its counts as soon as it has them, and the first of them turn a few columns of the
 // published rows into running sums each: a trip from CU to CU instead of a launch and a trip of the table through memory and back.
-// [32768 x 8] in 256 slices 6.2 -> 5.6 us as
-// kernels, of which 1.4 are the launch, 1.5 until the counts are out, 0.5 to 1 the trip, and one launch (2.1 us of the calling thread) less, which
-// is what the three calls waited for: 17.2 -> 14.9 us.
+// [32768 x 8] in 256 slices 6.2 -> 4.8 us, and
+// one launch (2.1 us of the calling thread) less, which is what the three calls waited for.  What bounds it: the launch, the indices'
+// and the words' trip, instructions.  One copy of the histogram: a slice is 16 or 32 of a wave's instructions here, and eight copies
+// to clear and to add up cost more than lanes that wait for each other (eight 5.45 us, four 5.1, two 4.95, one 4.8).
 // What crosses workgroups are words as in the one-launch plan (plan_sync.h): the launch's tag in the high half, two counts of 16
 // bits in the low half, so that nothing has to be cleared and words may arrive in any order.  The host gives every launch
 // of a device a number; it is the tag, and one of kCountRegions parts of the array in turn is the launch's.
@@ -234,26 +235,19 @@ template <int GROUPS>
 __global__ __launch_bounds__(GROUPS *kCountMaxSlices) void count_and_scan(const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per,
                                                                           int n_slices, int32_t *__restrict__ counts, unsigned long long *rows,
                                                                           uint32_t tag, int max_polls) {
-  constexpr int COPIES = kHistogramCopies, nt = GROUPS * kCountMaxSlices, kGroupWaves = kCountMaxSlices / kWave;
+  constexpr int nt = GROUPS * kCountMaxSlices, kGroupWaves = kCountMaxSlices / kWave;
   extern __shared__ int32_t hist[];
   __shared__ int32_t of_wave[GROUPS][kGroupWaves][4];
   __shared__ int missing;
   fetch_arguments_now(idx, n, n_experts, per, n_slices, counts, rows, tag, max_polls);
   const int tid = threadIdx.x, lane = tid % kWave, wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int p = blockIdx.x, group = wave_s / kGroupWaves, slice = tid % kCountMaxSlices;
-  const int words = padded_experts(n_experts) / 2, quads = words / 2, stride = histogram_stride(n_experts, COPIES);
-  count_slice<COPIES>(idx, n, n_experts, per, p, hist, [&]() {
+  const int words = padded_experts(n_experts) / 2, quads = words / 2;
+  count_slice<1>(idx, n, n_experts, per, p, hist, [&]() {
     if (tid == 0)
       missing = 0;
   });
-  auto counted = [&](int e) {
-    uint32_t sum = 0;
-    if (e < n_experts)
-#pragma unroll
-      for (int k = 0; k < COPIES; ++k)
-        sum += (uint32_t)hist[k * stride + e];
-    return sum;
-  };
+  auto counted = [&](int e) { return e < n_experts ? (uint32_t)hist[e] : 0u; };
   for (int w = tid; w < words; w += nt)
     agent_store(rows + p * words + w, (unsigned long long)tag << 32 | counted(2 * w) | counted(2 * w + 1) << 16);
   for (int q0 = p * GROUPS; q0 < quads; q0 += n_slices * GROUPS) {
@@ -346,7 +340,7 @@ static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int 
   const int max_polls = g_count_fault.exchange(false) ? 0 : kCountPolls;
   const int64_t batches = (per / 2 + kLoadsInFlight - 1) / kLoadsInFlight;   // (threads as for launch_slice_histogram)
   const auto go = [&](auto kernel, int threads) {
-    const size_t ints = std::max(kHistogramCopies * histogram_stride(n_experts, kHistogramCopies), 4 * threads);
+    const size_t ints = std::max(n_experts, 4 * threads);
     launch_with_flags(kernel, dim3(n_blocks), dim3(threads), ints * sizeof(int32_t), s, flags, idx, n, n_experts, per, n_blocks, counts, words,
                       number + 1, max_polls);
   };
