@@ -5,7 +5,19 @@
 
 namespace lplb {
 
-// One wave per workgroup; ROWS LPs per wave.
+// The normalised counts of the experts from `first` on, `n` of them, each count over the largest of all: by a wave.
+__device__ inline void write_normalised_counts(const int32_t *__restrict__ counts, int n_experts, float *__restrict__ out, int first, int n, int lane) {
+  int32_t most = 0;
+#pragma unroll 4
+  for (int e = lane; e < n_experts; e += kWave)
+    most = max(most, counts[e]);
+  const float wmax = wave_max_of_groups<true, true>((float)most);
+#pragma unroll 4
+  for (int e = first + lane; e < first + n; e += kWave)
+    out[e] = (float)counts[e] / wmax;
+}
+
+// One wave solves; ROWS LPs per wave.
 //
 // Feasibility counter: updates of one address queue up behind each other in memory
 // (about 10 ns each: 2048 waves that each add their result take 20 us longer than
@@ -13,12 +25,25 @@ namespace lplb {
 // feasible with one add, and a wave takes back the LPs of its own that failed -- rare,
 // and the sum is the same.
 // STAGED: the counts fit in LDS.
-template <int GM, int DM, bool EXACT, int ROWS, int EPL, bool STAGED>
-__global__ __launch_bounds__(kWave) void solve_groups(SolveArgs a) {
+// HELPED: a second wave writes the group's normalised counts while the first solves.  By that one, at its end, one LP of 8 ranks takes
+// 5.25 us instead of 5.05, of 16 8.4 / 8.15, of 32 15.5 / 15.4; 1024 LPs of 8 ranks 6.3 / 6.0.  With more LPs than SIMDs the waves that solve
+// share those as it is (512 batches of four 7.15 / 7.25, 2048 LPs of 32 ranks 37 / 49).  A kernel of its own: as a condition at run time
+// it made LPs whose counts nobody wants 0.1 us slower.
+template <int GM, int DM, bool EXACT, int ROWS, int EPL, bool STAGED, bool HELPED = false>
+__global__ __launch_bounds__(HELPED ? 2 * kWave : kWave) void solve_groups(SolveArgs a) {
   extern __shared__ float staged_all[];   // a.staged_stride floats per LP of this wave
   __shared__ int rep_of_edge[EPL * kWave];
   __shared__ __attribute__((aligned(16))) double pivot_rows[lp_pivot_doubles<GM, DM, ROWS, EPL>()];
   __shared__ __attribute__((aligned(16))) float tile[lp_tile_floats<GM, DM, ROWS, EPL>()];
+  if constexpr (HELPED) {
+    if (threadIdx.x >= kWave) {
+      const int inst = blockIdx.x / a.n_group, per_group = a.n_experts / a.n_group;
+      write_normalised_counts(a.workload + (int64_t)inst * a.n_experts, a.n_experts, a.gw_out + (int64_t)inst * a.n_experts,
+                              (blockIdx.x - inst * a.n_group) * per_group, per_group, threadIdx.x - kWave);
+      return;
+    }
+    a.gw_out = nullptr;
+  }
   if (blockIdx.x == 0 && threadIdx.x == 0)
     atomicAdd(a.avail, a.n_units);
   const int first_unit = blockIdx.x * ROWS;
@@ -43,6 +68,11 @@ static void launch_variant(SolveArgs a, hipStream_t s) {
   a.staged_stride = lds <= kLdsLimit ? a.n_experts + 1 : 0;
   const dim3 grid((a.n_units + ROWS - 1) / ROWS), block(kWave);
   constexpr bool kKnown = takes_spread_form<GM, DM, ROWS, EPL>() || ROWS > 1;   // whether the kernel is built for either case
+  if constexpr (EXACT && ROWS == 1 && EPL == 1)   // (groups that fill no kernel are rare)
+    if (a.gw_out && a.staged_stride && a.n_units <= 4 * current_device_cu_count()) {
+      launch(solve_groups<GM, DM, EXACT, ROWS, EPL, kKnown, true>, grid, dim3(2 * kWave), lds, s, a);
+      return;
+    }
   if (a.staged_stride)
     launch(solve_groups<GM, DM, EXACT, ROWS, EPL, kKnown>, grid, block, lds, s, a);
   else   // (more than 15 thousand experts, 3900 with four LPs per wave: one kernel, the padded one, serves every group that it holds; against one
