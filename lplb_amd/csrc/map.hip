@@ -7,22 +7,27 @@
 // hashes k (minilp.cu:503-509).  The reference takes k from a shared-memory atomic
 // (minilp.cu:504), which fixes the set of ordinals per block but not which token
 // gets which.  Here k is canonical, and it is worked out only for the replicated
-// sets (a few per rank), which keeps the ranking state small: one 16-byte slot per
-// (wave, replicated set, chunk).
+// sets (a few per rank), which keeps the ranking state small: one row per (wave,
+// replicated set).
 //
 // A workgroup walks its slice in passes of n_waves * K consecutive 64-index chunks,
 // K per wave; the loads of two passes are in flight.  Per pass:
 //   A  every lane looks up its token's route; lanes with a replicated expert set
-//      their bit in the 64-bit bitmap of (wave, set, chunk);
+//      their bit in the 64-bit bitmap of (wave, set, chunk) and read it back: the lower
+//      lanes in it are ahead of the token in its chunk.  A running count per (wave, set),
+//      to which a chunk's first token of the set adds, is what is ahead in earlier chunks;
 //   -- workgroup barrier --
-//   B  lane (set, chunk) counts the bits of the same set and chunk in the waves
-//      before it (popcounts) and of the chunks before it in its own wave, which gives
-//      the ordinal of the chunk's first token of that set;
-//   C  a token's ordinal is that start plus the number of lower lanes in the bitmap
-//      (one 16-byte LDS read, two mbcnt); hash, compare, store.
-// Nothing in C depends on another chunk, so the K chunks of a wave overlap.
-// Bitmaps and running totals are double-buffered by pass parity, which leaves one
-// workgroup barrier per pass.  Nothing depends on execution order.
+//   B  what the waves before have counted, and the passes before, is what is ahead of a wave's
+//      first token: by every wave for itself, lane = set, up to 64 sets; by all waves together,
+//      thread = set, and another barrier, beyond;
+//   C  a token's ordinal is the sum of the three; hash, compare, store.
+// Counts are double-buffered by pass parity, which leaves one workgroup barrier per pass.
+// Neither the instructions of A and C nor, but for B, the LDS's go with the number of sets, and a row has 40 bytes for four chunks.
+// Histogram, LP and redirect of [1048576 x 8], with starting ordinals per (set, chunk) that every wave worked out from the
+// bitmaps of all waves before it (144 bytes a row, so that 64 sets left room for two chunks and 128 for one) -> so: in 256 slices 16 sets 41.9 -> 42.0 us,
+// 32 48.7 -> 42.7, 64 61.4 -> 44.2, 128 81.8 -> 51.5; in 64 slices 94 -> 88.5, 122 -> 92, 174 -> 100, 258 -> 121.  B by every wave for itself against by all together:
+// 64 sets 44.2 / 48.1, 128 51.6 / 51.5 and in 64 slices 135 / 121 (the bases of all waves take the room of eight chunks there).
+// Nothing depends on execution order.
 #include "map_kernel.h"
 
 namespace lplb {
@@ -177,7 +182,7 @@ __device__ inline void physical_counts_from_tables(const MapArgs &a, const Route
 
 // LDS bytes for n_logical experts, n_rep replicated sets, w waves and K chunks per wave and pass.
 static size_t map_lds_bytes(int n_logical, int n_rep, int w, int k) {
-  return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)w * (n_rep + 1) * rank_record_bytes(k) +
+  return (size_t)(n_rep + 1) * sizeof(RepEntry) + (size_t)w * (n_rep + 1) * (rank_row_bytes(k) + (n_rep <= kWave ? sizeof(int32_t) : 0)) +
          (size_t)(n_logical + 1) * sizeof(Route) + (size_t)2 * n_rep * sizeof(int32_t) +
          (size_t)2 * n_logical * sizeof(int32_t);
 }
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(kMaxWaves *kWave, SINGLE ? 8 : 4) void redirect_ind
   fetch_arguments_now(a.idx, a.o_weight, a.by_block, a.o2r, a.phy2log, a.n, a.per, a.n_logical, a.n_ranks, a.n_rep, a.G,
                       a.D, a.C, a.L, a.P, a.n_blocks, a.magic_L, a.magic_cd, a.magic_D, a.magic_G, a.out,
                       a.physical_counts);
-  constexpr int kRec = rank_record_bytes(K);
+  constexpr int kRow = rank_row_bytes(K);
   const int nl = a.n_logical, R = a.n_rep;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int lane = tid % kWave, n_waves = nt / kWave;
@@ -208,13 +213,16 @@ __global__ __launch_bounds__(kMaxWaves *kWave, SINGLE ? 8 : 4) void redirect_ind
     return;
 
   RepEntry *reps = reinterpret_cast<RepEntry *>(smem_raw);                          // [R + 1]
-  unsigned char *records = smem_raw + (size_t)(R + 1) * sizeof(RepEntry);          // [n_waves][R + 1][kRec]
-  const int wave_stride = (R + 1) * kRec;
-  Route *route = reinterpret_cast<Route *>(records + (size_t)n_waves * wave_stride);   // [nl + 1]
-  int32_t *carry = reinterpret_cast<int32_t *>(route + nl + 1);                     // [2][R]
+  unsigned char *rows = smem_raw + (size_t)(R + 1) * sizeof(RepEntry);             // [n_waves][R + 1][kRow]
+  const int wave_stride = (R + 1) * kRow;
+  Route *route = reinterpret_cast<Route *>(rows + (size_t)n_waves * wave_stride);   // [nl + 1]
+  int32_t *carry = reinterpret_cast<int32_t *>(route + nl + 1);                     // [2][R] tokens before this pass
   int32_t *staged = carry + 2 * R;   // [2][nl] tokens per expert: in the whole array, before this slice
-  unsigned char *my_records = records + (size_t)wave_s * wave_stride;
-  const unsigned long long my_bit = 1ull << lane;
+  const bool by_wave = R <= kWave;
+  int32_t *my_bases = staged + 2 * nl + wave_s * (R + 1);   // [n_waves][R + 1] tokens before this wave's first; only if by_wave
+  unsigned char *my_rows = rows + (size_t)wave_s * wave_stride;
+  const uint32_t my_bit = 1u << lane % 32;
+  const int my_half = lane / 32 * 4;
   const int32_t *last = a.by_block + (int64_t)(a.n_blocks - 1) * nl;
   const int32_t *prev = pid ? a.by_block + (int64_t)(pid - 1) * nl : nullptr;
   LPLB_MAP_STAMP(0);
@@ -246,10 +254,9 @@ __global__ __launch_bounds__(kMaxWaves *kWave, SINGLE ? 8 : 4) void redirect_ind
 
   // ---- tables ----
   {
-    const i32x4 zero{0, 0, 0, 0};
-    i32x4 *z = reinterpret_cast<i32x4 *>(records);
-    for (int i = tid; i < n_waves * wave_stride / 16; i += nt)
-      z[i] = zero;
+    uint2 *z = reinterpret_cast<uint2 *>(rows);
+    for (int i = tid; i < n_waves * wave_stride / 8; i += nt)
+      z[i] = uint2{0, 0};
   }
   tables_before_barrier(a, tl, route, reps, staged, last, prev, tid, nt);
   __syncthreads();
@@ -274,70 +281,100 @@ __global__ __launch_bounds__(kMaxWaves *kWave, SINGLE ? 8 : 4) void redirect_ind
     if constexpr (!SINGLE)
       if (pass + 2 * pass_len < end)
         issue_loads(raw, pass + 2 * pass_len);   // in flight during this pass and the next
-    // Phase A.
-    ChunkSlot *slot[K];
+    // Phase A.  (A wave's own rows: the LDS serves its instructions in the order they were issued.)
+    auto row = [&](int c) { return my_rows + __umul24((uint32_t)set[c], (uint32_t)kRow); };
+    auto of_set = [&](int c) { return reinterpret_cast<uint32_t *>(row(c) + 8 * K + 4 * PAR); };
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      if (set[c] < R)
+        atomicOr(reinterpret_cast<uint32_t *>(row(c) + c * 8 + my_half), my_bit);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    uint2 bits[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      bits[c] = *reinterpret_cast<const uint2 *>(row(c) + c * 8);
+    uint32_t ahead[K];
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      ahead[c] = __builtin_amdgcn_mbcnt_hi(bits[c].y, __builtin_amdgcn_mbcnt_lo(bits[c].x, 0));
+    uint32_t so_far[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      slot[c] = reinterpret_cast<ChunkSlot *>(my_records + __umul24((uint32_t)set[c], (uint32_t)kRec)) + (PAR * K + c);
-      if (set[c] < R)
-        atomicOr(reinterpret_cast<unsigned long long *>(slot[c]), my_bit);
+      so_far[c] = *of_set(c);
+      if (set[c] < R && ahead[c] == 0) {   // the chunk's first token of its set; its bitmap is empty again behind it
+        __hip_atomic_fetch_add(of_set(c), (uint32_t)(__popc(bits[c].x) + __popc(bits[c].y)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        *reinterpret_cast<uint2 *>(row(c) + c * 8) = uint2{0, 0};
+      }
     }
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      ahead[c] += so_far[c];
     LPLB_MAP_STAMP(2 + 4 * PAR);
     __syncthreads();
     LPLB_MAP_STAMP(3 + 4 * PAR);
-    // Phase B: lane = (set, chunk), chunk fastest.  The rows of the waves before this
-    // one are read four at a time (clamped addresses, masked values).
-    if (R > 0) {
-      const int c = lane % K;
-      for (int p0 = 0; p0 < R * K; p0 += kWave) {
-        const bool live = p0 + lane < R * K;
-        const int q = live ? (p0 + lane) / K : R;   // lanes past the end read the stand-in record (zeros)
-        unsigned char *first = records + __umul24((uint32_t)q, (uint32_t)kRec) + (PAR * K + c) * (int)sizeof(ChunkSlot);
-        const int32_t carried = carry[PAR * R + (live ? q : 0)];
-        const unsigned long long own_bits =
-            *reinterpret_cast<const unsigned long long *>(first + wave_s * wave_stride);
-        int earlier = 0;
+    // Phase B.  Four waves at a time (clamped addresses, masked values).
+    auto count_at = [&](int q) { return reinterpret_cast<int32_t *>(rows + __umul24((uint32_t)q, (uint32_t)kRow) + 8 * K + 4 * PAR); };
+    const int wave_ints = wave_stride / 4;
+    if (by_wave) {
+      for (int q0 = 0; q0 < R; q0 += kWave) {
+        const int q = min(q0 + lane, R - 1);
+        const int32_t *at = count_at(q);
+        int32_t base = carry[PAR * R + q];
         for (int w0 = 0; w0 < wave_s; w0 += 4) {
-          unsigned long long bits[4];
+          int32_t n[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u)
-            bits[u] = *reinterpret_cast<const unsigned long long *>(first + min(w0 + u, wave_s) * wave_stride);
+            n[u] = at[min(w0 + u, wave_s) * wave_ints];
 #pragma unroll
           for (int u = 0; u < 4; ++u)
-            earlier += w0 + u < wave_s ? __popcll(bits[u]) : 0;
+            base += w0 + u < wave_s ? n[u] : 0;
         }
-        const int own = __popcll(own_bits);
-        const int in_earlier_waves = group_sum<K>(earlier);
-        const int in_my_wave = group_sum<K>(own);
-        const int in_earlier_chunks = group_exclusive_scan<K>(own, c);
-        if (live) {
-          const int32_t base = carried + in_earlier_waves;
-          ChunkSlot *mine = reinterpret_cast<ChunkSlot *>(first + wave_s * wave_stride);
-          mine->start = base + in_earlier_chunks;
-          // the other parity's bitmap is free again: clear it for the pass after this one
-          *reinterpret_cast<unsigned long long *>(mine + (PAR ? -K : K)) = 0ull;
-          if (wave_s == n_waves - 1 && c == 0)
-            carry[(PAR ^ 1) * R + q] = base + in_my_wave;
-        }
+        my_bases[q] = base;
+        if (!SINGLE && wave_s == n_waves - 1)
+          carry[(PAR ^ 1) * R + q] = base + at[wave_s * wave_ints];
       }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+      for (int q = tid; q < R; q += nt) {
+        int32_t *at = count_at(q);
+        int32_t base = carry[PAR * R + q];
+        for (int w0 = 0; w0 < n_waves; w0 += 4) {
+          int32_t n[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            n[u] = at[min(w0 + u, n_waves - 1) * wave_ints];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (w0 + u < n_waves) {
+              at[(w0 + u) * wave_ints] = base;
+              base += n[u];
+            }
+        }
+        carry[(PAR ^ 1) * R + q] = base;
+      }
+      __syncthreads();
     }
-    __builtin_amdgcn_wave_barrier();
+    if constexpr (!SINGLE)   // the other parity's counts are free again: empty for the next pass
+      for (int q = lane; q < R; q += kWave)
+        *(count_at(q) + wave_s * wave_ints + (PAR ? -1 : 1)) = 0;
     LPLB_MAP_STAMP(4 + 4 * PAR);
     // Phase C: all LDS reads of the K chunks first, then the arithmetic, then the stores.
     const int64_t w0 = pass + wave_off;
     int64_t *dst = a.out + w0 + lane;
-    i32x4 s[K], x[K];
+    i32x4 x[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      s[c] = *reinterpret_cast<const i32x4 *>(slot[c]);         // bits_lo, bits_hi, start
+      so_far[c] = by_wave ? (uint32_t)my_bases[set[c]] : *of_set(c);   // (of no set: whatever is there)
       x[c] = *reinterpret_cast<const i32x4 *>(&reps[set[c]]);   // total, magic, expected, replica
     }
     int32_t o[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
-      const int32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)s[c].y,
-                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)s[c].x, (uint32_t)s[c].z));
-      const int32_t h = ordinal_hash<WRAP>(k, x[c].x, (uint32_t)x[c].y);
+      const int32_t h = ordinal_hash<WRAP>((int32_t)(ahead[c] + so_far[c]), x[c].x, (uint32_t)x[c].y);
       o[c] = h >= x[c].z ? x[c].w : original[c];
     }
     if (!TAIL || w0 + K * kWave <= end) {
@@ -762,9 +799,11 @@ static hipError_t launch_redirect(const MapArgs &a, dim3 grid, dim3 block, size_
   const int64_t pass_len = (int64_t)block.x * K;
   const bool whole = a.per % pass_len == 0 && a.n % pass_len == 0;
   const bool single = a.per <= pass_len;
-  if (single)
-    return whole ? launch_redirect_variant<K, WRAP, false, true>(a, grid, block, lds, s)
-                 : launch_redirect_variant<K, WRAP, true, true>(a, grid, block, lds, s);
+  if constexpr (K < 8) {   // (eight chunks per wave are for slices of two passes and more)
+    if (single)
+      return whole ? launch_redirect_variant<K, WRAP, false, true>(a, grid, block, lds, s)
+                   : launch_redirect_variant<K, WRAP, true, true>(a, grid, block, lds, s);
+  }
   return whole ? launch_redirect_variant<K, WRAP, false, false>(a, grid, block, lds, s)
                : launch_redirect_variant<K, WRAP, true, false>(a, grid, block, lds, s);
 }
@@ -882,7 +921,9 @@ static int map_checked(const int64_t *idx, const float *o_weight, const int32_t 
   // Waves per workgroup: one per 64-index chunk of the slice, at most 16 when there is
   // one workgroup per CU; with more workgroups than CUs smaller ones (8, then 4 waves)
   // share a CU.  A wave takes K chunks per pass; two passes are in flight, so that one
-  // pass's ranking and stores overlap the next one's loads.
+  // pass's ranking and stores overlap the next one's loads.  Four, unless half of the CUs have nothing
+  // to do: then the passes, not the memory, take the time, and eight are half as many (16 sets, histogram, LP and redirect of
+  // [1048576 x 8] in 64 slices 92.2 -> 88.5 us; in 256 slices 41.6 with four and 42.2 with eight).
   const int64_t chunks = (a.per + kWave - 1) / kWave;
   const int n_cus = current_device_cu_count();
   int max_waves = kMaxWaves;
@@ -890,7 +931,7 @@ static int map_checked(const int64_t *idx, const float *o_weight, const int32_t 
     max_waves >>= 1;
   int n_waves = chunks < max_waves ? (int)chunks : max_waves;
   const int64_t per_wave = (chunks + n_waves - 1) / n_waves;
-  int k = per_wave >= 8 ? 4 : per_wave >= 3 ? 2 : 1;
+  int k = per_wave >= 16 && 2 * n_blocks <= n_cus ? 8 : per_wave >= 8 ? 4 : per_wave >= 3 ? 2 : 1;
   while (k > 1 && map_lds_bytes(a.n_logical, a.n_rep, n_waves, k) > kLdsLimit)
     k >>= 1;
   while (n_waves > 1 && map_lds_bytes(a.n_logical, a.n_rep, n_waves, k) > kLdsLimit)
@@ -908,8 +949,10 @@ static int map_checked(const int64_t *idx, const float *o_weight, const int32_t 
     LPLB_MAP_CASE(1);
   } else if (k <= 2) {
     LPLB_MAP_CASE(2);
-  } else {
+  } else if (k <= 4) {
     LPLB_MAP_CASE(4);
+  } else {
+    LPLB_MAP_CASE(8);
   }
 #undef LPLB_MAP_CASE
   LPLB_HIP_TRY(err);

@@ -78,10 +78,9 @@ struct __attribute__((aligned(16))) ChunkSlot {
   int32_t unused;
 };
 
-// Bytes of the ranking record of one (wave, replicated set): K chunk slots for each of
-// the two pass parities, padded to an odd multiple of 16 bytes so that consecutive
-// sets start in different LDS banks.
-constexpr int rank_record_bytes(int k) { return 2 * k * (int)sizeof(ChunkSlot) + 16; }
+// Bytes of the row of one (wave, replicated set): the bitmaps of K chunks, then the wave's tokens of the set for each of the two
+// pass parities (which also lets consecutive rows start in different LDS banks).
+constexpr int rank_row_bytes(int k) { return k * 8 + 8; }
 
 // (499 k + 41) mod total with the sign rule of C (minilp.cu:505), k >= 0.
 // !WRAP: k < 2^24 and 499 k + 41 < 2^31 (the caller guarantees it).
