@@ -206,8 +206,9 @@ inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
   return long_slice_records_at(n_logical, n_rep) + (size_t)kPlanWaves * ((n_rep + 1) * kRankRowBytes + 2 * hist_words * sizeof(int32_t)) +
          (size_t)(n_logical + 16) / 16 * 16;
 }
-// Slices past kLongestSlice ask for more than that: 220 bytes a row, the sets padded to the next multiple of sixteen past their number.
-// It decides which batches are cut into those at all; tests/test_gpu_parity.py holds the chain to the rest.
+// Slices past kLongestSlice of more than 8 ranks, or with more than kFewSets sets, ask for more than that: 220 bytes a row, the sets padded to
+// the next multiple of sixteen past their number.  It decides which batches are cut into those at all; tests/test_gpu_parity.py holds the chain
+// to the rest.  (32 sets of 8 ranks, [1048576 x 8] as the chain and so: 44.6 and 32.8 us, [524288 x 8] 27.0 and 20.4.)
 inline size_t longest_slices_lds_bytes(int n_logical, int n_rep, int hist_words) {
   return long_slice_lds_bytes(n_logical, n_rep, hist_words) +
          (size_t)kPlanWaves * ((n_rep / 16 * 16 + 16) * 220 - (n_rep + 1) * kRankRowBytes);
@@ -1097,7 +1098,7 @@ __global__ __launch_bounds__(kPlanThreads, 2 * plan_workgroups_per_cu(GM)) void 
 // and a chunk's first token of a set adds to that.  The instructions do not go with the number of sets, and a row has 40 bytes where
 // bitmaps of 16 chunks with their starting ordinals have 272, of which 64 sets take a CU.
 // So, against the chain, 8 ranks in four and eight groups (64 and 128 sets): [131072 x 8] 18.2 -> 13.9 and 22.1 -> 15.9 us, [262144 x 8] 23.8 -> 16.5 and
-// 29.3 -> 18.5; 32 ranks (64 sets) [262144 x 8] 33.9 -> 27.1, counts supplied 34.8 -> 20.7.  16 sets at [1048576 x 8] 32.3 -> 32.1.
+// 29.3 -> 18.5, [196608 x 8] 15.8 -> 14.9 and 25.1 -> 17.9; 16 sets at [1048576 x 8] 32.3 -> 32.1.
 // Against bitmaps of all 16 chunks (slices of 4097 to 8192): counts supplied, at 16, 32 and 64 sets [262144 x 8] 13.4 -> 12.7, 14.4 -> 13.7, 15.0 -> 15.0,
 // [196608 x 8] 12.9 -> 12.6, 14.1 -> 13.7, 16.0 -> 15.0; own counts, which leave later here (loads and table of sets ahead of them), 15.1 -> 15.2, 15.7 -> 15.5
 // and 14.35 -> 14.5, 14.7 -> 14.7, but 64 sets 16.0 -> 15.2.  Eight chunks (up to 4096) are the faster with bitmaps of all of them while
@@ -1562,8 +1563,9 @@ template <int GM, int DM> static int launch_scan_and_solve(const ScanSolveArgs &
 template <int GM, int DM, bool EXACT, int K>
 static int launch_plan_slices(PlanArgs &a, hipStream_t s, bool *done) {
   const size_t lds_slice = K > 0 ? plan_slice_lds_bytes<K>(a.sh.n_logical, a.n_rep)
-                           : a.per > kLongestSlice ? longest_slices_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words)
-                                                   : long_slice_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words);
+                           : a.per <= kLongestSlice || (GM <= 8 && a.n_rep <= kFewSets)
+                               ? long_slice_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words)
+                               : longest_slices_lds_bytes(a.sh.n_logical, a.n_rep, a.hist_words);
   // LP workgroups: their waves' working areas, then the counts (one copy per LP, or one for all of the batch's own)
   const size_t lp_areas = kLpsPerWorkgroup * plan_lp_area_bytes<GM, DM>();
   const size_t one_copy = counts_bytes(a.sh.n_logical);
