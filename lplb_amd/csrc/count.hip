@@ -40,12 +40,12 @@ __host__ __device__ constexpr int histogram_stride(int n_experts, int copies) {
   return copies > 1 ? ((n_experts + 31) & ~31) + 4 : n_experts;
 }
 
-// The tokens of slice p into the histograms `hist` (LDS); ends with a workgroup barrier.  `meanwhile` is called while the first loads
+// The tokens of slice p into the histograms `hist` (LDS), by nt threads; ends with a workgroup barrier.  `meanwhile` is called while the first loads
 // are on their way.
 template <int COPIES, typename Meanwhile>
-__device__ __forceinline__ void count_slice(const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per, int p, int32_t *hist,
+__device__ __forceinline__ void count_slice(const int64_t *__restrict__ idx, int64_t n, int n_experts, int64_t per, int p, int nt, int32_t *hist,
                                             Meanwhile meanwhile) {
-  const int tid = threadIdx.x, nt = blockDim.x;
+  const int tid = threadIdx.x;
   const int stride = histogram_stride(n_experts, COPIES);
   int32_t *mine = hist + (tid % COPIES) * stride;
   auto count = [&](int64_t v) {
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(1024) void slice_histogram(
   const int tid = threadIdx.x, nt = blockDim.x;
   const int p = blockIdx.x;
   const int stride = histogram_stride(n_experts, COPIES);
-  count_slice<COPIES>(idx, n, n_experts, per, p, hist, [&]() {
+  count_slice<COPIES>(idx, n, n_experts, per, p, nt, hist, [&]() {
     if (clear)
       for (int64_t e = (int64_t)p * nt + tid; e < n_experts; e += (int64_t)gridDim.x * nt)
         clear[e] = TOTALS ? 0 : kNoTotal;
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(GROUPS *kCountMaxSlices) void count_and_scan(const 
   const int tid = threadIdx.x, lane = tid % kWave, wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int p = blockIdx.x, group = wave_s / kGroupWaves, slice = tid % kCountMaxSlices;
   const int words = padded_experts(n_experts) / 2, quads = words / 2;
-  count_slice<1>(idx, n, n_experts, per, p, hist, [&]() {
+  count_slice<1>(idx, n, n_experts, per, p, nt, hist, [&]() {
     if (tid == 0)
       missing = 0;
   });
