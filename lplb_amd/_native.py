@@ -285,10 +285,9 @@ class CompiledSolver:
 
     # -- csrc/plugin.cpp:491-578 -------------------------------------------------
     def solve(self, local_workload: torch.Tensor, r2o: torch.Tensor, phy2log: torch.Tensor,
-              avail_num: torch.Tensor, *, any_shape: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
-        """any_shape: local_workload is n_experts counts, not [n_group, group_size, L] (no counterpart in the reference)."""
+              avail_num: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         return _binding.solve(self.n_group, self.group_size, self.dup_per_rank, self.n_combined_experts,
-                              self.n_local_experts, self.step_rule, self.n_steps, local_workload, r2o, phy2log, avail_num, any_shape)
+                              self.n_local_experts, self.step_rule, self.n_steps, local_workload, r2o, phy2log, avail_num)
 
     def solve_batched(self, workloads: torch.Tensor, r2o: torch.Tensor, phy2log: torch.Tensor,
                       avail_num: torch.Tensor, want_global: bool = False):

@@ -194,21 +194,16 @@ PyObject *plan(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   });
 }
 
-// solve(shape..., local_workload, r2o, phy2log, avail_num, any_shape)
-// any_shape: the workload is n_experts counts of the solver's own groups, in whatever shape.
+// solve(shape..., local_workload, r2o, phy2log, avail_num)
 PyObject *solve(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
-  return guarded(n_args, 5, [&]() -> PyObject * {
+  return guarded(n_args, 4, [&]() -> PyObject * {
     const Shape s(args);
     args += kShapeArgs;
     const at::Tensor &workload = tensor(args[0], "local_workload"), &avail = tensor(args[3], "avail_num");
-    const bool any_shape = args[4] == Py_True;
     require(workload.is_cuda(), "local_workload on a GPU");
-    if (any_shape)
-      require(workload.numel() == s.n_experts && s.n_experts > 0, "local_workload.numel() == n_experts");
-    else
-      require(workload.dim() == 3, "local_workload.dim() == 3");
-    const int64_t n_group = any_shape ? s.n_group : workload.size(0), L = any_shape ? s.P - s.D * s.C : workload.size(2), n_pes = n_group * s.G;
-    require(any_shape || workload.size(1) == s.G, "group_size == local_workload.size(1)");
+    require(workload.dim() == 3, "local_workload.dim() == 3");
+    const int64_t n_group = workload.size(0), L = workload.size(2), n_pes = n_group * s.G;
+    require(workload.size(1) == s.G, "group_size == local_workload.size(1)");
     require(workload.scalar_type() == at::kInt, "local_workload.dtype == int32");
     require(workload.is_contiguous(), "local_workload.is_contiguous()");
     const at::Tensor &r2o = tensor(args[1], "r2o"), &phy2log = tensor(args[2], "phy2log");
@@ -222,7 +217,7 @@ PyObject *solve(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     require(avail.scalar_type() == at::kInt, "avail_num.dtype == int32");
     require(r2o.is_cuda() && phy2log.is_cuda() && avail.is_cuda(), "all tensors on the GPU");
     const at::Tensor r2o_c = r2o.contiguous(), phy2log_c = phy2log.contiguous();
-    const at::Tensor global = make({n_group, s.G, L}, at::kFloat, workload), result = make({n_group, s.G, s.D}, at::kFloat, workload);
+    const at::Tensor global = make(workload.sizes(), at::kFloat, workload), result = make({n_group, s.G, s.D}, at::kFloat, workload);
     const int64_t per_var = replicas / s.D;
     call_library([&] {
       return do_solve(ints(workload), floats(global), ints(r2o_c), ints(phy2log_c), (int)n_group, s.G, s.D, (int)per_var,

@@ -153,10 +153,11 @@ class Planner:
         :return: (share kept on the original rank, fp32 [n_group, group_size, num_redundants];
                   normalised global workload, fp32 [n_group, group_size, L]).
         """
+        workload = workload.view(self.n_group, self.group_size, self.n_local_logical_routed_experts)
         if self.ep_group is not None and not self.deep_ep_initialized:
-            workload = workload.view(self.n_group, self.group_size, self.n_local_logical_routed_experts).clone()
+            workload = workload.clone()
             torch.distributed.all_reduce(workload, group=self.ep_group)
-        return self.solver.solve(workload, self.r2o, self.phy2log, avail_counter, any_shape=True)
+        return self.solver.solve(workload, self.r2o, self.phy2log, avail_counter)
 
     def _prepared_mapping(self) -> torch.Tensor | None:
         """The redirect's mapping-only tables (which the reference rebuilds in every block of every launch,
