@@ -24,8 +24,8 @@
 // Counts are double-buffered by pass parity, which leaves one workgroup barrier per pass.
 // Neither the instructions of A and C nor, but for B, the LDS's go with the number of sets, and a row has 40 bytes for four chunks.
 // Histogram, LP and redirect of [1048576 x 8], with starting ordinals per (set, chunk) that every wave worked out from the
-// bitmaps of all waves before it (144 bytes a row, so that 64 sets left room for two chunks and 128 for one) -> so: in 256 slices 16 sets 41.9 -> 42.0 us,
-// 32 48.7 -> 42.7, 64 61.4 -> 44.2, 128 81.8 -> 51.5; in 64 slices 94 -> 88.5, 122 -> 92, 174 -> 100, 258 -> 121.  B by every wave for itself against by all together:
+// bitmaps of all waves before it (144 bytes a row, so that 64 sets left room for two chunks and 128 for one) -> so: in 256 slices 16 sets 41.9 -> 41.7 us,
+// 32 48.7 -> 42.5, 64 61.4 -> 44.2, 128 81.8 -> 51.4; in 64 slices 94 -> 86, 122 -> 90, 174 -> 98, 258 -> 120.  B by every wave for itself against by all together:
 // 64 sets 44.2 / 48.1, 128 51.6 / 51.5 and in 64 slices 135 / 121 (the bases of all waves take the room of eight chunks there).
 // Nothing depends on execution order.
 #include "map_kernel.h"
@@ -295,16 +295,18 @@ __global__ __launch_bounds__(kMaxWaves *kWave, SINGLE ? 8 : 4) void redirect_ind
 #pragma unroll
     for (int c = 0; c < K; ++c)
       bits[c] = *reinterpret_cast<const uint2 *>(row(c) + c * 8);
-    uint32_t ahead[K];
+    uint32_t ahead[K], in_chunk[K];
 #pragma unroll
-    for (int c = 0; c < K; ++c)
+    for (int c = 0; c < K; ++c) {
       ahead[c] = __builtin_amdgcn_mbcnt_hi(bits[c].y, __builtin_amdgcn_mbcnt_lo(bits[c].x, 0));
+      in_chunk[c] = (uint32_t)(__popc(bits[c].x) + __popc(bits[c].y));
+    }
     uint32_t so_far[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
       so_far[c] = *of_set(c);
       if (set[c] < R && ahead[c] == 0) {   // the chunk's first token of its set; its bitmap is empty again behind it
-        __hip_atomic_fetch_add(of_set(c), (uint32_t)(__popc(bits[c].x) + __popc(bits[c].y)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __hip_atomic_fetch_add(of_set(c), in_chunk[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
         *reinterpret_cast<uint2 *>(row(c) + c * 8) = uint2{0, 0};
       }
     }
@@ -362,20 +364,26 @@ __global__ __launch_bounds__(kMaxWaves *kWave, SINGLE ? 8 : 4) void redirect_ind
       for (int q = lane; q < R; q += kWave)
         *(count_at(q) + wave_s * wave_ints + (PAR ? -1 : 1)) = 0;
     LPLB_MAP_STAMP(4 + 4 * PAR);
-    // Phase C: all LDS reads of the K chunks first, then the arithmetic, then the stores.
+    // Phase C: all LDS reads of four chunks first (of eight they would not fit the registers), then the arithmetic; the stores.
     const int64_t w0 = pass + wave_off;
     int64_t *dst = a.out + w0 + lane;
-    i32x4 x[K];
-#pragma unroll
-    for (int c = 0; c < K; ++c) {
-      so_far[c] = by_wave ? (uint32_t)my_bases[set[c]] : *of_set(c);   // (of no set: whatever is there)
-      x[c] = *reinterpret_cast<const i32x4 *>(&reps[set[c]]);   // total, magic, expected, replica
-    }
+    constexpr int kAtOnce = K < 4 ? K : 4;
     int32_t o[K];
 #pragma unroll
-    for (int c = 0; c < K; ++c) {
-      const int32_t h = ordinal_hash<WRAP>((int32_t)(ahead[c] + so_far[c]), x[c].x, (uint32_t)x[c].y);
-      o[c] = h >= x[c].z ? x[c].w : original[c];
+    for (int c0 = 0; c0 < K; c0 += kAtOnce) {
+      i32x4 x[kAtOnce];
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        so_far[c0 + u] = by_wave ? (uint32_t)my_bases[set[c0 + u]] : *of_set(c0 + u);   // (of no set: whatever is there)
+        x[u] = *reinterpret_cast<const i32x4 *>(&reps[set[c0 + u]]);   // total, magic, expected, replica
+      }
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) {
+        const int32_t h = ordinal_hash<WRAP>((int32_t)(ahead[c0 + u] + so_far[c0 + u]), x[u].x, (uint32_t)x[u].y);
+        o[c0 + u] = h >= x[u].z ? x[u].w : original[c0 + u];
+      }
+      if (K > kAtOnce)
+        __builtin_amdgcn_sched_barrier(0);
     }
     if (!TAIL || w0 + K * kWave <= end) {
 #pragma unroll
