@@ -432,6 +432,11 @@ int lplb_place_on_large_nodes_covers(int group_size, int dup_per_rank, int ep_si
 int lplb_place_on_large_nodes(const void *history, int history_type, const int32_t *r2o, int group_size,
                               int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
                               int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream);
+/* ... in two parts, for a caller with something to do meanwhile: the first enqueues the kernel, the second returns when the tables are there. */
+int lplb_place_on_large_nodes_begin(const void *history, int history_type, const int32_t *r2o, int group_size,
+                                    int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
+                                    int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream);
+int lplb_place_wait(lplb_stream_t stream);
 
 /*
  * No counterpart in the reference.  enabled = 0 makes lplb_plan always run the

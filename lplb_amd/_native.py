@@ -71,6 +71,8 @@ _SIGNATURES = {
     "lplb_place_experts_covers": (_i, [_i, _i, _i, _i, _i, _i]),
     "lplb_place_on_large_nodes_covers": (_i, [_i, _i, _i, _i, _i, _i]),
     "lplb_place_on_large_nodes": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
+    "lplb_place_on_large_nodes_begin": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
+    "lplb_place_wait": (_i, [_vp]),
     "lplb_place_experts": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "lplb_plan_noalloc": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
 }
@@ -190,6 +192,16 @@ def place_experts(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_phys
     """build_redundancy_mapping for a history on the current device, by a kernel there: its three arrays as parts of
     one int32 tensor [n_physical + 3 * n_logical] on that device, complete on return; None if the kernel does not cover it.
     large_nodes: also with more than 128 experts on a node."""
+    begun = place_experts_begin(history, r2o, ep_size, n_physical, n_nodes, large_nodes)
+    if begun is None:
+        return None
+    place_wait(begun[1])
+    return begun[0]
+
+
+def place_experts_begin(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_physical: int, n_nodes: int,
+                        large_nodes: bool = True) -> tuple[torch.Tensor, int] | None:
+    """place_experts without the wait: the table and what to hand to place_wait before anything but this stream's work reads it."""
     kind = _HISTORY_TYPES.get(history.dtype)
     if kind is None or not history.is_contiguous() or _device_index(history) != torch.cuda.current_device():
         return None
@@ -198,12 +210,14 @@ def place_experts(history: torch.Tensor, r2o: torch.Tensor, ep_size: int, n_phys
     if not placement_covers(group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes, large_nodes):
         return None
     table = torch.empty(n_physical + 3 * n_logical, dtype=torch.int32, device=history.device)
-    at = table.data_ptr()
-    lib = load()
-    place = lib.lplb_place_on_large_nodes if large_nodes else lib.lplb_place_experts
-    _check(place(history.data_ptr(), kind, r2o.data_ptr(), group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes,
-                 at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical), _stream(history)))
-    return table
+    at, stream = table.data_ptr(), _stream(history)
+    _check(load().lplb_place_on_large_nodes_begin(history.data_ptr(), kind, r2o.data_ptr(), group_size, dup_per_rank, ep_size, n_logical,
+                                                  n_physical, n_nodes, at, at + 4 * n_physical, at + 4 * (n_physical + 2 * n_logical), stream))
+    return table, stream
+
+
+def place_wait(stream: int) -> None:
+    _check(load().lplb_place_wait(stream))
 
 
 class UnsupportedShape(RuntimeError):

@@ -6,7 +6,8 @@
 // On the host the arithmetic takes 11 us, but the history has to come over (a copy the host waits for) and the tables have to go
 // back (another).  Here nothing crosses: one launch, and the host waits once, because the tables are there for every stream
 // when the call returns.  update_redundancy_mapping of 256 experts on 32 ranks of 4 nodes, history on the GPU: 46.1 us by the host,
-// 24.2 here, of which the kernel is 5.3 (8.7, and 26.8 the call, with the lightest pack searched for in every step).  What bounds it is
+// 20.9 here, of which the kernel is 5.3 (8.7 with the lightest pack searched for in every step) and an empty kernel's launch and wait 11.1; 24.2
+// where the caller made the tables' views behind the wait instead of ahead of it.  What bounds it is
 // the packing, a serial chain of one step per expert of a node, 30 ns each (pack_node); the nodes are packed side by side, a wave
 // each.  With 256 experts on one node the kernel takes 13.2 us: 7.7 of packing, 2 of ranking every item by counting those ahead of it.
 #include "map_kernel.h"
@@ -16,7 +17,7 @@ namespace lplb {
 // lplb_place_experts has always refused more than this; lplb_place_on_large_nodes does not.
 constexpr int kPlaceMaxPerNode = 128;
 // The ranking's work is the square of a node's experts, and the host's arithmetic is a small part of a call there.  Per call, host /
-// here, into 8 packs: 256 experts of a node 45.5 / 32.4 us, 384 47.7 / 39.3, 512 49.7 / 47.3, 640 51.9 / 55.9; into 32 packs 256 46.6 / 35.3,
+// here (views behind the wait), into 8 packs: 256 experts of a node 45.5 / 32.4 us, 384 47.7 / 39.3, 512 49.7 / 47.3, 640 51.9 / 55.9; into 32 packs 256 46.6 / 35.3,
 // 512 50.5 / 52.7.  (What the caller waits for, one call and a synchronisation: 8 packs, 256 54.1 / 35.4, 512 58.4 / 50.0.)
 constexpr int kPlaceMaxPerLargeNode = 384;
 constexpr int kPlaceMaxExperts = 1024, kPlaceMaxPacks = 64, kPlaceMaxEdges = 2 * kWave;
@@ -260,6 +261,9 @@ static int place(const void *history, int history_type, const int32_t *r2o, int 
   default: return fail(LPLB_EINVAL, "place_experts: unknown history_type %d", history_type);
   }
   LPLB_HIP_TRY(hipGetLastError());
+  return LPLB_OK;
+}
+static int wait_for(hipStream_t s) {
   LPLB_HIP_TRY(hipStreamSynchronize(s));
   return LPLB_OK;
 }
@@ -278,12 +282,22 @@ extern "C" int lplb_place_on_large_nodes_covers(int group_size, int dup_per_rank
 extern "C" int lplb_place_experts(const void *history, int history_type, const int32_t *r2o, int group_size,
                                   int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
                                   int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream) {
-  return lplb::place(history, history_type, r2o, group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes, lplb::kPlaceMaxPerNode,
-                     phy2log, log2phy, logcnt, static_cast<hipStream_t>(stream));
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = lplb::place(history, history_type, r2o, group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes, lplb::kPlaceMaxPerNode,
+                             phy2log, log2phy, logcnt, s);
+  return rc == LPLB_OK ? lplb::wait_for(s) : rc;
 }
 extern "C" int lplb_place_on_large_nodes(const void *history, int history_type, const int32_t *r2o, int group_size,
                                          int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
                                          int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream) {
+  const int rc = lplb_place_on_large_nodes_begin(history, history_type, r2o, group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes,
+                                                 phy2log, log2phy, logcnt, stream);
+  return rc == LPLB_OK ? lplb_place_wait(stream) : rc;
+}
+extern "C" int lplb_place_on_large_nodes_begin(const void *history, int history_type, const int32_t *r2o, int group_size,
+                                               int dup_per_rank, int ep_size, int n_logical, int n_physical, int n_nodes,
+                                               int32_t *phy2log, int32_t *log2phy, int32_t *logcnt, lplb_stream_t stream) {
   return lplb::place(history, history_type, r2o, group_size, dup_per_rank, ep_size, n_logical, n_physical, n_nodes, lplb::kPlaceMaxPerLargeNode,
                      phy2log, log2phy, logcnt, static_cast<hipStream_t>(stream));
 }
+extern "C" int lplb_place_wait(lplb_stream_t stream) { return lplb::wait_for(static_cast<hipStream_t>(stream)); }

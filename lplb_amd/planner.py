@@ -119,24 +119,29 @@ class Planner:
         """
         # the three arrays are parts of one buffer
         n_phy, n_log, n_nodes = self.n_routed_experts, self.n_logical_routed_experts, max(1, self.ep_size // self.gpus_per_node)
-        table = self._mapping_where_the_history_is(workload, n_nodes)
-        if table is None:
+        begun = self._mapping_where_the_history_is(workload, n_nodes)
+        if begun is not None:
+            table, stream = begun
+        else:
             host = None if workload is None else workload.detach().cpu().numpy()
             staged = torch.empty(n_phy + 3 * n_log, dtype=torch.int32, pin_memory=self.device.type == "cuda")
             build_redundancy_mapping(self._r2o_host, self.ep_size, n_log, n_phy, host, n_nodes=n_nodes, out=staged.numpy())
             table = staged.to(self.device)
-        self.phy2log = table[:n_phy]
-        return self.phy2log, table[n_phy:n_phy + 2 * n_log].view(n_log, 2), table[n_phy + 2 * n_log:]
+        phy2log, log2phy, logcnt = table[:n_phy], table[n_phy:n_phy + 2 * n_log].view(n_log, 2), table[n_phy + 2 * n_log:]
+        if begun is not None:   # (the views were made while the GPU was at it)
+            _native.place_wait(stream)
+        self.phy2log = phy2log
+        return phy2log, log2phy, logcnt
 
-    def _mapping_where_the_history_is(self, workload: torch.Tensor | None, n_nodes: int) -> torch.Tensor | None:
-        """The mapping's tables made on the GPU, if the history is on the planner's and one kernel covers the deployment:
+    def _mapping_where_the_history_is(self, workload: torch.Tensor | None, n_nodes: int) -> tuple[torch.Tensor, int] | None:
+        """The mapping's tables under way on the GPU, if the history is on the planner's and one kernel covers the deployment:
         the history need not come to the host and the tables need not go back (the shape itself was checked when the planner
         was built).  Not inside a capture, where reading the history on the host is refused and this would wait."""
         if (workload is None or not workload.is_cuda or self.device.type != "cuda" or self._r2o_placed is None
                 or workload.numel() != self.n_logical_routed_experts or workload.device != self._r2o_placed.device
                 or torch.cuda.is_current_stream_capturing()):
             return None
-        return _native.place_experts(workload, self._r2o_placed, self.ep_size, self.n_routed_experts, n_nodes, large_nodes=True)
+        return _native.place_experts_begin(workload, self._r2o_placed, self.ep_size, self.n_routed_experts, n_nodes)
 
     def count_workload(self, idx: torch.Tensor, n_sms: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Histogram of ``idx`` (values in [-1, n_logical), -1 ignored) over ``n_sms`` slices.
