@@ -97,7 +97,7 @@ int lplb_copy_shape_series(const int64_t *const *src, int64_t *const *dst, int64
                            int streaming, void *const *start_events, void *const *stop_events,
                            lplb_stream_t stream);
 /*
- * Measurement aid, no counterpart in the reference: the first of lplb_count_idx's two kernels
+ * Measurement aid, no counterpart in the reference: the first kernel of lplb_count_idx's form with two
  * (the histogram per slice, rows not yet summed over the slices) alone, n_launches times as in
  * the series above.  A kernel that is followed at once by another one on the stream reads
  * 1.3-1.6 us longer by its own events than in a series of its own; this gives the latter.
