@@ -191,8 +191,9 @@ __global__ __launch_bounds__(kScanThreads) void prefix_over_slices(int32_t *__re
 // of a device a number; it is the tag, and one of kCountRegions parts of the array in turn is the launch's.
 // Nothing has to be resident at once: only the workgroups with columns wait, a quarter of the grid at most, and should their
 // words not come within kCountPolls polls (a launch that is kept off the GPU for long, or that finds its region in use by one
-// kCountRegions launches later), they count those columns of all slices themselves.  So the rows are right in any case.
-constexpr int kCountMaxSlices = 256, kCountMaxExperts = 1024, kCountRegions = 8, kCountPolls = 1 << 14;
+// kCountRegions launches later), they count those columns of all slices themselves.  So the rows are right in any case.  (1024 polls are
+// 0.5 ms and more, a few times what that counting takes.)
+constexpr int kCountMaxSlices = 256, kCountMaxExperts = 1024, kCountRegions = 8, kCountPolls = 1 << 10;
 // Up to 4096 indices a slice.  Longer ones keep the adding workgroups' loads waiting behind the indices', and the calling thread is not what
 // the three calls wait for any more: [131072 x 8] (4096) 18.1 -> 16.6 us, [262144 x 8] (8192) 19.6 in two launches, 20.1 in one, at 32 ranks
 // 32.1 and 32.7.
@@ -327,7 +328,10 @@ static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int 
     return LPLB_OK;
   unsigned long long *words = known[dev].load(std::memory_order_acquire);
   if (!words) {
-    LPLB_HIP_TRY(hipGetSymbolAddress(reinterpret_cast<void **>(&words), HIP_SYMBOL(g_count_words)));
+    if (hipGetSymbolAddress(reinterpret_cast<void **>(&words), HIP_SYMBOL(g_count_words)) != hipSuccess) {
+      (void)hipGetLastError();
+      return LPLB_OK;
+    }
     known[dev].store(words, std::memory_order_release);
   }
   // (a word's tag is told from a later one's by its sign: after 2^31 launches the two-launch form takes over for good)
