@@ -22,7 +22,9 @@
 // instructions.  With one lane per rank and edge (8, 2) took 1.15 us.
 // (A form in which rank i is lane i of every 16-lane row and holds its whole row, the elimination made of
 // fp64 multiply-adds with a row_newbcast operand, has pivots of 40 instead of 60 ns and no LDS in them; but
-// getting the rows into that shape costs 0.25 us a step more than it gains at 8 ranks.)
+// getting the rows into that shape costs 0.25 us a step more than it gains at 8 ranks.  At 16 and 32 ranks, where the
+// tile can be read in that shape for nothing, pivots in pairs, a lane with one or two rows and every fourth column: a step takes 0.13 and 0.42 us
+// longer, since a row's multiples are worked out by four lanes, not two, in the chain, and the next pair's columns take two stores.)
 #pragma once
 #include "solve_kernel.h"
 
