@@ -62,6 +62,13 @@ static bool packing_pays(const SolveArgs &a) {
 }
 constexpr int kLdsLimit = 64 * 1024 - 2048;
 
+// Whether the normalised counts go where counts are: one wave has read an only group's before it writes any, two would race.
+static bool normalised_in_place(const SolveArgs &a) {
+  const uintptr_t bytes = (uintptr_t)(a.n_units / a.n_group) * a.n_experts * sizeof(int32_t);
+  const uintptr_t from = reinterpret_cast<uintptr_t>(a.workload), to = reinterpret_cast<uintptr_t>(a.gw_out);
+  return from < to + bytes && to < from + bytes;
+}
+
 template <int GM, int DM, bool EXACT, int ROWS, int EPL = 1>
 static void launch_variant(SolveArgs a, hipStream_t s) {
   const size_t lds = (size_t)ROWS * (a.n_experts + 1) * sizeof(float);   // (one LP per wave has a zero behind its counts)
@@ -69,7 +76,7 @@ static void launch_variant(SolveArgs a, hipStream_t s) {
   const dim3 grid((a.n_units + ROWS - 1) / ROWS), block(kWave);
   constexpr bool kKnown = takes_spread_form<GM, DM, ROWS, EPL>() || ROWS > 1;   // whether the kernel is built for either case
   if constexpr (EXACT && ROWS == 1 && EPL == 1)   // (groups that fill no kernel are rare)
-    if (a.gw_out && a.staged_stride && a.n_units <= 4 * current_device_cu_count()) {
+    if (a.gw_out && a.staged_stride && a.n_units <= 4 * current_device_cu_count() && !normalised_in_place(a)) {
       launch(solve_groups<GM, DM, EXACT, ROWS, EPL, kKnown, true>, grid, dim3(2 * kWave), lds, s, a);
       return;
     }
