@@ -415,7 +415,8 @@ int lplb_build_mapping(const float *weight, const double *history, const int32_t
  * device pointers; returns when the tables are there.
  *
  *   history, history_type  [n_logical] of one of the types above
- *   r2o                    int32 [group_size, dup_per_rank], every column a permutation
+ *   r2o                    int32 [group_size, dup_per_rank], every column a permutation (nothing checks this: in a column that repeats a
+ *                          rank every slot has a copy, log2phy names one of several, and a rank left out has none)
  *
  * LPLB_EUNSUPPORTED (use lplb_build_mapping) beyond 1024 logical experts, 128 of them (unless a rank has one only) or 64
  * ranks to be packed at once, and where several groups share a node.  lplb_place_experts_covers says so beforehand: 1 if it

@@ -122,18 +122,23 @@ template <typename T> __global__ __launch_bounds__(kPlaceMaxExperts) void place_
   __shared__ __attribute__((aligned(16))) float node_weight[kPlaceMaxNodeWords];   // by node (padded), heaviest first
   __shared__ __attribute__((aligned(16))) int32_t node_places[kPlaceMaxNodeWords];
   __shared__ int32_t host_of[kPlaceMaxEdges];   // by rank and slot of a group: the rank that hosts the copy
-  __shared__ int not_simple, out_of_order;
+  __shared__ int not_simple, out_of_order, repeated;
   fetch_arguments_now(a.history, a.n_logical, a.magic_per_node);
   const int tid = threadIdx.x, nt = blockDim.x, lane = tid % kWave;
   const int wave_s = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int n = a.n_logical, per_node = a.per_node, padded = padded_to_four(per_node), room = a.L;
   if (tid == 0)
-    not_simple = out_of_order = 0;
+    not_simple = out_of_order = repeated = 0;
   __syncthreads();
-  for (int i = tid; i < a.G * a.D; i += nt) {
-    const int host = (int)fast_div((uint32_t)i, a.magic_D), from = a.r2o[i];
-    host_of[min(max(from < 0 ? from + a.G : from, 0), a.G - 1) * a.D + i - host * a.D] = host;   // (every column a permutation: checked on the host)
-  }
+  auto source_of = [&](int i) {   // by rank and slot of a group: the rank whose expert is copied there
+    const int from = a.r2o[i];
+    return min(max(from < 0 ? from + a.G : from, 0), a.G - 1);
+  };
+  static_assert(kPlaceMaxEdges <= kPlaceMaxExperts, "an edge per thread");
+  const int edge = nt - 1 - tid, my_host = (int)fast_div((uint32_t)edge, a.magic_D);   // (the last waves', which seldom have a node to pack)
+  const int my_edge = edge < a.G * a.D ? source_of(edge) * a.D + edge - my_host * a.D : -1;
+  if (my_edge >= 0)
+    host_of[my_edge] = my_host;
   for (int i = tid; i < n; i += nt) {
     const T v = static_cast<const T *>(a.history)[i];
     const float w = (float)v;
@@ -177,6 +182,9 @@ template <typename T> __global__ __launch_bounds__(kPlaceMaxExperts) void place_
     for (int i = tid; i < n; i += nt)
       packed[i] = i;
   }
+  // (where a column repeats a rank, that rank's entry has another host for all of its hosts but one; entries of ranks left out were never written)
+  if (my_edge >= 0 && host_of[my_edge] != my_host)
+    repeated = 1;
   __syncthreads();
   // ---- each rank's experts, heaviest first, equal ones in the order they were packed.  They were packed heaviest first: what is
   //      out of order is what only the packing, which rounds loads to 32 bits, took for equal ----
@@ -202,15 +210,25 @@ template <typename T> __global__ __launch_bounds__(kPlaceMaxExperts) void place_
       sorted = resorted;
     }
   }
-  // ---- physical experts: a rank's originals; of its first ones a copy on the rank that hosts the slot ----
+  // ---- physical experts: a rank's originals; of its first ones a copy on the rank that hosts the slot.  The values of r2o are the caller's:
+  //      with a rank repeated in a column its hosts are looked for one by one (none, or several, of which log2phy has the last), as host_of
+  //      says nothing about the ranks left out ----
   for (int i = tid; i < n; i += nt) {
     const int rank = (int)fast_div((uint32_t)i, a.magic_L), place = i - rank * a.L, e = sorted[i], phy = rank * a.P + place;
     int replica = -1;
     if (place < a.P - a.L) {
       const int d = place - (int)fast_div((uint32_t)place, a.magic_D) * a.D;
       const int group = (int)fast_div((uint32_t)rank, a.magic_G) * a.G;
-      replica = (group + host_of[(rank - group) * a.D + d]) * a.P + a.L + place;
-      a.phy2log[replica] = e;
+      if (!repeated) {
+        replica = (group + host_of[(rank - group) * a.D + d]) * a.P + a.L + place;
+        a.phy2log[replica] = e;
+      } else {
+        for (int host = 0; host < a.G; ++host)
+          if (source_of(host * a.D + d) == rank - group) {
+            replica = (group + host) * a.P + a.L + place;
+            a.phy2log[replica] = e;
+          }
+      }
     }
     a.phy2log[phy] = e;
     a.log2phy[2 * e] = phy;
