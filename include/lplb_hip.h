@@ -487,6 +487,8 @@ int lplb_plan_poll_timeouts(int32_t *dst, lplb_stream_t stream);
  * the chain of kernels).  For callers and tests that want to know which form they got.
  */
 int lplb_plan_one_launch_count(long long *count);
+/* The same of lplb_count_idx (the others, and all that are captured, are two launches). */
+int lplb_count_one_launch_count(long long *count);
 
 /*
  * Test hook, no counterpart in the reference.  The next plan with a wait in it (one

@@ -62,6 +62,7 @@ _SIGNATURES = {
     "lplb_plan_poll_timeouts": (_i, [_vp, _vp]),
     "lplb_plan_one_launch_count": (_i, [_vp]),
     "lplb_plan_inject_fault": (_i, [_i, _i]),
+    "lplb_count_one_launch_count": (_i, [_vp]),
     "lplb_count_inject_fault": (_i, []),
     "lplb_plan": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
     "lplb_balanced_packing": (_i, [_vp, _i, _i, _i, _vp, _vp]),
@@ -170,6 +171,13 @@ def plan_one_launch_count() -> int:
     """Plans of this process that ran as one kernel launch (the others ran the chain of kernels)."""
     count = ctypes.c_longlong(-1)
     _check(load().lplb_plan_one_launch_count(ctypes.byref(count)))
+    return count.value
+
+
+def count_one_launch_count() -> int:
+    """Histograms with running sums of this process that ran as one kernel launch (the others took two)."""
+    count = ctypes.c_longlong(-1)
+    _check(load().lplb_count_one_launch_count(ctypes.byref(count)))
     return count.value
 
 

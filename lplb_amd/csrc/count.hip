@@ -1,7 +1,7 @@
 // Per-expert token histogram with an inclusive prefix over slices.
 //
-// Slices of up to 4096 indices, up to 256 of them: one launch on the caller's stream (count_and_scan, below).  Else, and in a
-// capture, two:
+// Slices of up to 4096 indices, up to 256 of them and not too few for the experts: one launch on the caller's stream (count_and_scan,
+// below).  Else, and in a capture, two:
 //   1. slice_histogram: one workgroup per slice, LDS histogram (eight copies, chosen by lane)
 //      fed by coalesced 16-byte index loads, row p of the output = counts of slice p;
 //   2. prefix_over_slices: turns the rows into running sums down the slice axis,
@@ -199,6 +199,14 @@ constexpr int kCountMaxSlices = 256, kCountMaxExperts = 1024, kCountRegions = 8,
 // 32.1 and 32.7.
 constexpr int64_t kCountMaxSlice = 4096;
 static_assert(kCountMaxSlice < 65536, "two counts to a word");
+// The slices take the columns four at a time and in turn, by 256 or 512 threads one or two of those fours.  A round is a chain of a load past the
+// caches, sums over the wave and four barriers, 0.7 us with 256 threads and 0.9 with 512, where a second launch takes all columns at once: 256
+// experts in one slice are 64 rounds, 48 us instead of 6, 1024 experts 256 rounds and 188 us.  us a call in two launches / in one, call behind call:
+//   256 threads, slices of 2048:  two rounds, 256 experts in 32 slices 6.6 / 5.1, 1024 in 128 6.9 / 5.9; three, 256 in 22 6.6 / 5.9, 512 in 43 6.5 / 6.1,
+//     1024 in 86 6.8 / 6.4; four, 64 in 4 6.5 / 5.8, 256 in 16 6.6 / 6.8, 512 in 32 6.6 / 6.9, 1024 in 64 6.8 / 7.2
+//   512 threads, slices of 4096:  two rounds, 256 in 16 6.7 / 5.5, 1024 in 64 6.6 / 5.7; three, 256 in 11 6.6 / 6.4, 1024 in 43 6.6 / 6.6 (each waited
+//     for, 17.4 / 17.4 and 17.5 / 17.6); four, 256 in 8 6.6 / 7.3, 1024 in 32 6.6 / 7.5
+constexpr int most_count_rounds(int groups) { return groups == 1 ? 3 : 2; }
 constexpr int kCountRegionWords = kCountMaxSlices * kCountMaxExperts / 2;
 static __device__ __attribute__((aligned(4096))) unsigned long long g_count_words[kCountRegions * kCountRegionWords];
 
@@ -308,10 +316,15 @@ __global__ __launch_bounds__(GROUPS *kCountMaxSlices) void count_and_scan(const 
 
 // Test hook (lplb_count_inject_fault): the next launch of count_and_scan waits for nothing, every slice counts for itself.
 static std::atomic<bool> g_count_fault{false};
+static std::atomic<long long> g_one_launch_counts{0};
 // *done = false: not a case for one launch; nothing was enqueued.  (A launch that is captured would carry its tag again when it is replayed.)
 static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int n_blocks, int32_t *counts, hipStream_t s, unsigned flags, bool *done) {
   const int64_t per = slice_len(n, n_blocks);
   if (n_blocks > kCountMaxSlices || n_experts > kCountMaxExperts || per > kCountMaxSlice)
+    return LPLB_OK;
+  const int64_t batches = (per / 2 + kLoadsInFlight - 1) / kLoadsInFlight;   // (threads as for launch_slice_histogram)
+  const int groups = batches <= kCountMaxSlices ? 1 : 2, quads_of_a_round = n_blocks * groups;
+  if ((padded_experts(n_experts) / 4 + quads_of_a_round - 1) / quads_of_a_round > most_count_rounds(groups))
     return LPLB_OK;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
@@ -342,17 +355,18 @@ static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int 
   } while (!launches[dev].compare_exchange_weak(number, number + 1, std::memory_order_relaxed));
   words += (size_t)(number % kCountRegions) * kCountRegionWords;
   const int max_polls = g_count_fault.exchange(false) ? 0 : kCountPolls;
-  const int64_t batches = (per / 2 + kLoadsInFlight - 1) / kLoadsInFlight;   // (threads as for launch_slice_histogram)
-  const auto go = [&](auto kernel, int threads) {
+  const auto go = [&](auto kernel) {
+    const int threads = groups * kCountMaxSlices;
     const size_t ints = std::max(n_experts, 4 * threads);
     launch_with_flags(kernel, dim3(n_blocks), dim3(threads), ints * sizeof(int32_t), s, flags, idx, n, n_experts, per, n_blocks, counts, words,
                       number + 1, max_polls);
   };
-  if (batches <= 256)
-    go(count_and_scan<1>, 256);
+  if (groups == 1)
+    go(count_and_scan<1>);
   else
-    go(count_and_scan<2>, 512);
+    go(count_and_scan<2>);
   LPLB_HIP_TRY(hipGetLastError());
+  g_one_launch_counts.fetch_add(1, std::memory_order_relaxed);
   *done = true;
   return LPLB_OK;
 }
@@ -529,6 +543,12 @@ extern "C" int lplb_slice_histogram_series(const int64_t *const *idx, int64_t n_
       return rc;
     }
   }
+  return LPLB_OK;
+}
+
+extern "C" int lplb_count_one_launch_count(long long *count) {
+  LPLB_REQUIRE(count != nullptr, LPLB_EINVAL, "count_one_launch_count: null pointer");
+  *count = lplb::g_one_launch_counts.load(std::memory_order_relaxed);
   return LPLB_OK;
 }
 
