@@ -489,6 +489,11 @@ int lplb_plan_poll_timeouts(int32_t *dst, lplb_stream_t stream);
 int lplb_plan_one_launch_count(long long *count);
 /* The same of lplb_count_idx (the others, and all that are captured, are two launches). */
 int lplb_count_one_launch_count(long long *count);
+/*
+ * No counterpart in the reference.  *count receives how often slices of lplb_count_idx, as one launch on the current device, have counted for
+ * themselves because what they waited for did not come in time: a few when more than eight such launches overlap, else none.  Waits for the device.
+ */
+int lplb_count_recounts(int *count);
 
 /*
  * Test hook, no counterpart in the reference.  The next plan with a wait in it (one
@@ -499,8 +504,9 @@ int lplb_count_one_launch_count(long long *count);
 int lplb_plan_inject_fault(int extra_slices_expected, int max_polls);
 
 /*
- * Test hook, no counterpart in the reference.  In the next lplb_count_idx that runs as one launch no slice waits for what the others
- * publish: each counts the indices in front of it itself, as when a wait has run out.  The table is the same.
+ * Test hook, no counterpart in the reference.  If the next histogram with running sums (lplb_count_idx, or the chain of lplb_plan) is one launch,
+ * no slice of it waits for what the others publish: each counts all slices' indices for its columns itself, as when a wait has run out.  The
+ * table is the same.  One that is two launches uses the hook up without effect.
  */
 int lplb_count_inject_fault(void);
 

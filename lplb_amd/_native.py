@@ -63,6 +63,7 @@ _SIGNATURES = {
     "lplb_plan_one_launch_count": (_i, [_vp]),
     "lplb_plan_inject_fault": (_i, [_i, _i]),
     "lplb_count_one_launch_count": (_i, [_vp]),
+    "lplb_count_recounts": (_i, [_vp]),
     "lplb_count_inject_fault": (_i, []),
     "lplb_plan": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
     "lplb_balanced_packing": (_i, [_vp, _i, _i, _i, _vp, _vp]),
@@ -178,6 +179,13 @@ def count_one_launch_count() -> int:
     """Histograms with running sums of this process that ran as one kernel launch (the others took two)."""
     count = ctypes.c_longlong(-1)
     _check(load().lplb_count_one_launch_count(ctypes.byref(count)))
+    return count.value
+
+
+def count_recounts() -> int:
+    """How often slices of such a histogram have counted for themselves on the current device (waits for it)."""
+    count = ctypes.c_int(-1)
+    _check(load().lplb_count_recounts(ctypes.byref(count)))
     return count.value
 
 

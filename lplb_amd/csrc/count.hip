@@ -209,6 +209,7 @@ static_assert(kCountMaxSlice < 65536, "two counts to a word");
 constexpr int most_count_rounds(int groups) { return groups == 1 ? 3 : 2; }
 constexpr int kCountRegionWords = kCountMaxSlices * kCountMaxExperts / 2;
 static __device__ __attribute__((aligned(4096))) unsigned long long g_count_words[kCountRegions * kCountRegionWords];
+static __device__ int g_count_recounts;   // columns' turns that workgroups counted for themselves, since the library was loaded
 
 // A pair of words, 16-byte aligned, with one load past the caches (see agent_load_pairs), polled until both have the tag.  By whole
 // waves; false: they did not come, or a later launch has the region.
@@ -273,6 +274,8 @@ __global__ __launch_bounds__(GROUPS *kCountMaxSlices) void count_and_scan(const 
     }
     __syncthreads();
     if (missing) {   // words did not come: the columns are counted here, slice by slice
+      if (tid == 0)
+        atomicAdd(&g_count_recounts, 1);
       for (int i = tid; i < 4 * nt; i += nt)
         hist[i] = 0;
       __syncthreads();
@@ -314,11 +317,12 @@ __global__ __launch_bounds__(GROUPS *kCountMaxSlices) void count_and_scan(const 
   }
 }
 
-// Test hook (lplb_count_inject_fault): the next launch of count_and_scan waits for nothing, every slice counts for itself.
+// Test hook (lplb_count_inject_fault): if the next histogram with running sums is one launch, it waits for nothing, every slice counts for itself.
 static std::atomic<bool> g_count_fault{false};
 static std::atomic<long long> g_one_launch_counts{0};
 // *done = false: not a case for one launch; nothing was enqueued.  (A launch that is captured would carry its tag again when it is replayed.)
-static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int n_blocks, int32_t *counts, hipStream_t s, unsigned flags, bool *done) {
+static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int n_blocks, int32_t *counts, hipStream_t s, unsigned flags, int max_polls,
+                              bool *done) {
   const int64_t per = slice_len(n, n_blocks);
   if (n_blocks > kCountMaxSlices || n_experts > kCountMaxExperts || per > kCountMaxSlice)
     return LPLB_OK;
@@ -354,7 +358,6 @@ static int try_count_and_scan(const int64_t *idx, int64_t n, int n_experts, int 
       return LPLB_OK;
   } while (!launches[dev].compare_exchange_weak(number, number + 1, std::memory_order_relaxed));
   words += (size_t)(number % kCountRegions) * kCountRegionWords;
-  const int max_polls = g_count_fault.exchange(false) ? 0 : kCountPolls;
   const auto go = [&](auto kernel) {
     const int threads = groups * kCountMaxSlices;
     const size_t ints = std::max(n_experts, 4 * threads);
@@ -455,7 +458,8 @@ int enqueue_histogram(const int64_t *idx, int64_t n_elements, int n_experts, int
 int enqueue_count(const int64_t *idx, int64_t n_elements, int n_experts, int n_blocks,
                   int32_t *counts_by_block, hipStream_t s, bool any_order) {
   bool done = false;
-  int rc = try_count_and_scan(idx, n_elements, n_experts, n_blocks, counts_by_block, s, any_order ? hipExtAnyOrderLaunch : 0u, &done);
+  const int max_polls = g_count_fault.load(std::memory_order_relaxed) && g_count_fault.exchange(false) ? 0 : kCountPolls;
+  int rc = try_count_and_scan(idx, n_elements, n_experts, n_blocks, counts_by_block, s, any_order ? hipExtAnyOrderLaunch : 0u, max_polls, &done);
   if (rc != LPLB_OK || done)
     return rc;
   rc = launch_slice_histogram<false>(idx, n_elements, n_experts, n_blocks, counts_by_block, nullptr, s,
@@ -549,6 +553,15 @@ extern "C" int lplb_slice_histogram_series(const int64_t *const *idx, int64_t n_
 extern "C" int lplb_count_one_launch_count(long long *count) {
   LPLB_REQUIRE(count != nullptr, LPLB_EINVAL, "count_one_launch_count: null pointer");
   *count = lplb::g_one_launch_counts.load(std::memory_order_relaxed);
+  return LPLB_OK;
+}
+
+extern "C" int lplb_count_recounts(int *count) {
+  LPLB_REQUIRE(count != nullptr, LPLB_EINVAL, "count_recounts: null pointer");
+  void *at = nullptr;
+  LPLB_HIP_TRY(hipGetSymbolAddress(&at, HIP_SYMBOL(lplb::g_count_recounts)));
+  LPLB_HIP_TRY(hipDeviceSynchronize());
+  LPLB_HIP_TRY(hipMemcpy(count, at, sizeof(int), hipMemcpyDeviceToHost));
   return LPLB_OK;
 }
 
