@@ -29,6 +29,7 @@
 // 64 sets 44.2 / 48.1, 128 51.6 / 51.5 and in 64 slices 135 / 121 (the bases of all waves take the room of eight chunks there).
 // Nothing depends on execution order.
 #include "map_kernel.h"
+#include "redirect_chunks.h"
 
 namespace lplb {
 
@@ -928,10 +929,7 @@ static int map_checked(const int64_t *idx, const float *o_weight, const int32_t 
 
   // Waves per workgroup: one per 64-index chunk of the slice, at most 16 when there is
   // one workgroup per CU; with more workgroups than CUs smaller ones (8, then 4 waves)
-  // share a CU.  A wave takes K chunks per pass; two passes are in flight, so that one
-  // pass's ranking and stores overlap the next one's loads.  Four, unless half of the CUs have nothing
-  // to do: then the passes, not the memory, take the time, and eight are half as many (16 sets, histogram, LP and redirect of
-  // [1048576 x 8] in 64 slices 92.2 -> 88.5 us; in 256 slices 41.6 with four and 42.2 with eight).
+  // share a CU.  A wave takes K chunks per pass: redirect_chunks.h.
   const int64_t chunks = (a.per + kWave - 1) / kWave;
   const int n_cus = current_device_cu_count();
   int max_waves = kMaxWaves;
@@ -939,7 +937,7 @@ static int map_checked(const int64_t *idx, const float *o_weight, const int32_t 
     max_waves >>= 1;
   int n_waves = chunks < max_waves ? (int)chunks : max_waves;
   const int64_t per_wave = (chunks + n_waves - 1) / n_waves;
-  int k = per_wave >= 16 && 2 * n_blocks <= n_cus ? 8 : per_wave >= 8 ? 4 : per_wave >= 3 ? 2 : 1;
+  int k = redirect_chunks(per_wave, a.n_rep, n_blocks, n_cus);
   while (k > 1 && map_lds_bytes(a.n_logical, a.n_rep, n_waves, k) > kLdsLimit)
     k >>= 1;
   while (n_waves > 1 && map_lds_bytes(a.n_logical, a.n_rep, n_waves, k) > kLdsLimit)

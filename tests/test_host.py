@@ -436,6 +436,37 @@ extern "C" int pays(int G, int D, int per_rank, int n_experts, int per_simd) { r
         assert pays(len(r2o), np.asarray(r2o).shape[1], n_logical // ep, n_logical, -(-n_lps // 1024)) == packed, name
 
 
+def test_redirect_takes_as_many_chunks_per_pass_as_was_measured_to_pay(tmp_path):
+    """Four or eight chunks: the rule (lplb_amd/csrc/redirect_chunks.h) against the measurements that stand above it.  Nowhere may it choose
+    the form that was slower by more than 3 % (two runs of one form differ by up to that)."""
+    import subprocess
+    (tmp_path / "chunks.cpp").write_text('''
+#include "redirect_chunks.h"
+extern "C" int chunks(long long per_wave, int n_sets, int n_slices, int n_cus) { return lplb::redirect_chunks(per_wave, n_sets, n_slices, n_cus); }
+''')
+    header = ROOT / "lplb_amd" / "csrc" / "redirect_chunks.h"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{header.parent}",
+                    str(tmp_path / "chunks.cpp"), "-o", str(tmp_path / "chunks.so")], check=True, capture_output=True)
+    chunks = ctypes.CDLL(str(tmp_path / "chunks.so")).chunks
+    chunks.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    text = header.read_text()
+    per_wave = [int(n) for n in re.search(r"chunks of a wave in all: ([\d, ]+)", text).group(1).split(", ")]
+    rows = re.findall(r"^//  +(\d+) of +(\d+), +(\d+) +((?:[\d.]+ / *[\d.]+ *)+)", text, flags=re.M)
+    assert len(rows) == 15 and per_wave[0] == 16
+    chosen = set()
+    for sets, _experts, slices, times in rows:
+        both = [(float(four), float(eight)) for four, eight in re.findall(r"([\d.]+) / *([\d.]+)", times)]
+        assert len(both) == len(per_wave)
+        for n, (four, eight) in zip(per_wave, both):
+            k = chunks(n, int(sets), int(slices), 256)
+            chosen.add(k)
+            slower, faster = (eight, four) if k == 8 else (four, eight)
+            assert slower <= 1.03 * faster, (sets, slices, n, four, eight)
+    assert chosen == {4, 8}
+    assert [chunks(n, 16, 1, 256) for n in (1, 2, 3, 7, 8, 15)] == [1, 1, 2, 2, 4, 4]
+    assert not any(chunks(n, sets, 129, 256) == 8 or chunks(n, sets, 1, 0) == 8 for n in range(1, 600) for sets in (0, 16, 128))
+
+
 def test_the_last_wave_to_add_up_totals_sees_what_the_others_have_added(tmp_path):
     """With more than 64 slices several waves of a workgroup add to the same sums in LDS, count themselves, and the one that comes
     last reads the sums.  Nothing but fences keeps the compiler from moving the count ahead of a wave's own additions, or the
