@@ -182,17 +182,19 @@ __global__ __launch_bounds__(kScanThreads) void prefix_over_slices(int32_t *__re
 // ---- histogram and running sums in one launch ----
 // Up to kCountMaxSlices slices: a slice publishes its counts as soon as it has them, and the first of them turn a few columns of the
 // published rows into running sums each: a trip from CU to CU instead of a launch and a trip of the table through memory and back.
-// [32768 x 8] in 256 slices 6.2 -> 4.8 us, and
-// one launch (2.1 us of the calling thread) less, which is what the three calls waited for.  What bounds it: the launch, the indices'
+// [32768 x 8] in 256 slices 6.2 -> 4.8 us, and one launch (2.1 us of the calling thread) less, which is what the three calls waited for.
+// What bounds it: the launch, the indices'
 // and the words' trip, instructions.  One copy of the histogram: a slice is 16 or 32 of a wave's instructions here, and eight copies
 // to clear and to add up cost more than lanes that wait for each other (eight 5.45 us, four 5.1, two 4.95, one 4.8).
 // What crosses workgroups are words as in the one-launch plan (plan_sync.h): the launch's tag in the high half, two counts of 16
 // bits in the low half, so that nothing has to be cleared and words may arrive in any order.  The host gives every launch
 // of a device a number; it is the tag, and one of kCountRegions parts of the array in turn is the launch's.
-// Nothing has to be resident at once: only the workgroups with columns wait, a quarter of the grid at most, and should their
-// words not come within kCountPolls polls (a launch that is kept off the GPU for long, or that finds its region in use by one
-// kCountRegions launches later), they count those columns of all slices themselves.  So the rows are right in any case.  (1024 polls are
-// 0.5 ms and more, a few times what that counting takes.)
+// Nothing has to be resident at once: the workgroups with columns wait (the first of the grid, as many as there are fours of columns or,
+// with 512 threads, eights; with 1024 experts or few slices that is all of them), but not for long: should their words not come within
+// kCountPolls polls (a launch that is kept off the GPU for long, or that finds its region in use by one kCountRegions launches later), they
+// count those columns of all slices themselves, every waiting workgroup the whole batch once a round.  So every wait ends and the rows are
+// right in any case.  (1024 polls are 0.5 ms and more, a few times what that counting takes.)
+// A call that is captured takes two launches: a replay would carry the same tag.
 constexpr int kCountMaxSlices = 256, kCountMaxExperts = 1024, kCountRegions = 8, kCountPolls = 1 << 10;
 // Up to 4096 indices a slice.  Longer ones keep the adding workgroups' loads waiting behind the indices', and the calling thread is not what
 // the three calls wait for any more: [131072 x 8] (4096) 18.1 -> 16.6 us, [262144 x 8] (8192) 19.6 in two launches, 20.1 in one, at 32 ranks

@@ -4,7 +4,8 @@
 // It runs once per re-shuffle, on a few hundred numbers, between two batches: what it costs is the host time
 // of the call.  update_redundancy_mapping at 256 experts on 32 ranks, history on the GPU: 755 us as numpy loops
 // (one interpreted argmin per expert and pass) and three copies to the GPU, 42 us here, of which the arithmetic
-// is 12 and the two synchronising copies most of the rest (24 us with 64 experts per node and 35 with 256, which place.hip places on the GPU).  Behaviour follows the reference's embedded EPLB (lplb/eplb.py:6-190) and its
+// is 12 and the two synchronising copies most of the rest (20.9 us with 64 experts per node and 29
+// with 256, which place.hip places on the GPU).  Behaviour follows the reference's embedded EPLB (lplb/eplb.py:6-190) and its
 // use in the planner (lplb/planner.py:115-182); weights are 32-bit floats throughout, items of equal weight
 // are taken in index order and a tie between packs goes to the lowest (the reference sorts unstably).
 #include "error.h"

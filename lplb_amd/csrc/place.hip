@@ -18,7 +18,9 @@ namespace lplb {
 constexpr int kPlaceMaxPerNode = 128;
 // The ranking's work is the square of a node's experts, and the host's arithmetic is a small part of a call there.  Per call, host /
 // here (views behind the wait), into 8 packs: 256 experts of a node 45.5 / 32.4 us, 384 47.7 / 39.3, 512 49.7 / 47.3, 640 51.9 / 55.9; into 32 packs 256 46.6 / 35.3,
-// 512 50.5 / 52.7.  (What the caller waits for, one call and a synchronisation: 8 packs, 256 54.1 / 35.4, 512 58.4 / 50.0.)
+// 512 50.5 / 52.7.  (What the caller waits for, one call and a synchronisation: 8 packs, 256 54.1 / 35.4, 512 58.4 / 50.0.)  With weights that
+// are negative or not numbers, which loads are not, a step takes longer: 384 of a node, views ahead of the wait, 48.4 / 51.3, waited for 57.5 / 54.0;
+// without, 48.8 / 35.6 and 57.4 / 38.2.
 constexpr int kPlaceMaxPerLargeNode = 384;
 constexpr int kPlaceMaxExperts = 1024, kPlaceMaxPacks = 64, kPlaceMaxEdges = 2 * kWave;
 // Where a node's experts are laid side by side in fours (a node has two at least where there is something to pack), and four more.

@@ -182,7 +182,13 @@ struct __attribute__((aligned(8))) PlanRoute {
 // One ranking slot per (wave, replicated set, chunk of 64 indices), K chunks per wave.
 constexpr int64_t kLongestSlice = 16 * kPlanThreads;   // 16 chunks per wave
 constexpr int kLongChunks = 8, kLongPasses = 8;        // of a long slice: chunks per wave and pass, passes
-constexpr int kFewestLongSlices = 64, kFewestSlicesInPasses = 32;   // past 8192 indices; up to them
+constexpr int kFewestLongSlices = 64;   // past 8192 indices
+// Up to 8192 indices.  At 8 ranks, slices of 8192, us a plan in the other form / in passes, in 32, 64, 128 and 200 slices: counts supplied, 16 sets
+// 12.3 / 11.7, 12.3 / 11.7, 12.9 / 12.2, 13.6 / 12.9, 32 sets 12.5 / 11.9, 12.7 / 11.9, 13.3 / 12.6, 14.6 / 14.2, 64 sets 13.7 / 12.4, 14.0 / 12.5, 15.1 / 13.9, 16.3 / 15.5;
+// own counts, 64 sets 14.6 / 14.3, 14.9 / 14.5, 15.7 / 15.2, 16.5 / 15.6; 128 sets, as the chain in 31 slices and in passes in 32, 21.3 / 15.1.  Fewer slices
+// would gain as much, down to 8 (counts supplied, 16 sets 12.1 / 11.5; own counts, 128 sets 20.9 / 14.9), less or nothing with two (32 ranks on their
+// own counts 23.1 / 23.5); tests/test_gpu_parity.py names 31 slices with 80 sets as the chain's.
+constexpr int kFewestSlicesInPasses = 32;
 constexpr int64_t kLongestOfLongSlices = kLongPasses * kLongChunks * kPlanThreads;
 // (K = 0: a long slice, without its records, which lie behind the rest)
 constexpr int slice_record_bytes(int k) { return k > 0 ? rank_record_bytes_single(k) : 0; }
@@ -206,9 +212,13 @@ inline size_t long_slice_lds_bytes(int n_logical, int n_rep, int hist_words) {
   return long_slice_records_at(n_logical, n_rep) + (size_t)kPlanWaves * ((n_rep + 1) * kRankRowBytes + 2 * hist_words * sizeof(int32_t)) +
          (size_t)(n_logical + 16) / 16 * 16;
 }
-// Slices past kLongestSlice of more than 8 ranks, or with more than kFewSets sets, ask for more than that: 220 bytes a row, the sets padded to
-// the next multiple of sixteen past their number.  It decides which batches are cut into those at all; tests/test_gpu_parity.py holds the chain
-// to the rest.  (32 sets of 8 ranks, [1048576 x 8] as the chain and so: 44.6 and 32.8 us, [524288 x 8] 27.0 and 20.4.)
+// Slices past kLongestSlice of more than 8 ranks, or with more than kFewSets sets, ask for more than they use: 220 bytes a row, the sets padded to
+// the next multiple of sixteen past their number, which is what their tables once took.  It is a rule of dispatch in the guise of a size: by it such
+// batches are the chain where these would not fit a CU, or not on enough CUs at once, and those that are cut so hold that LDS for nothing.
+// tests/test_gpu_parity.py names as the chain's, of these, 16 ranks with 32 sets in 256 slices, 32 ranks with 64 sets and 256 experts, and 8 ranks with
+// 64 sets on their own counts (256 slices).  For 8 ranks with counts supplied or more than four groups no test does, and there the chain
+// is the slower: [1048576 x 8] in 256 slices, 64 sets 41.5 against 34.3 us, 128 sets 45.7 against 36.5.  (Up to kFewSets sets, 32 of 8 ranks,
+// [1048576 x 8] as the chain and so: 44.6 and 32.8 us, [524288 x 8] 27.0 and 20.4.)
 inline size_t longest_slices_lds_bytes(int n_logical, int n_rep, int hist_words) {
   return long_slice_lds_bytes(n_logical, n_rep, hist_words) +
          (size_t)kPlanWaves * ((n_rep / 16 * 16 + 16) * 220 - (n_rep + 1) * kRankRowBytes);
